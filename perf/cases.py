@@ -1,0 +1,624 @@
+"""The work that users of this framework have it do, as timed cases.
+
+Four kinds, each through the package's public entry points:
+
+  rollout  A scene held in a context.  One pass restores a snapshot's state
+           (x, v and, with the implicit viscosity, its warm-start direction),
+           advances `steps` steps and reads x and v back: a simulation loop
+           between two outputs.  One step a pass is the interactive loop, which
+           shows every step.
+  lanes    Requests served together: every scene of the mix is admitted to a
+           LanePool, advanced `steps` ticks, read (x, v) and retired.
+  mesh     Surface reconstruction of a particle set given by the host; the mesh
+           (vertices, triangles, normals or velocities as asked for) is read back
+           into the caller's arrays of fixed capacity, as SRTool's fields are.
+  lists    Neighbor lists of positions already in device memory, written to
+           device memory (the entry point that allocates nothing).
+
+Scene sizes follow nonnewton_amd.scenes and bench.py; lattice spacing 0.02,
+h 0.04, +-1% jitter.
+"""
+import ctypes
+import math
+
+import numpy as np
+import torch
+
+from nonnewton_amd import _lib as L
+from nonnewton_amd import scenes as S
+from nonnewton_amd.lanes import LanePool
+from nonnewton_amd.params import KIND_ELASTIC, KIND_FLUID, KIND_RIGID, KIND_STATIC, SceneParams
+from nonnewton_amd.surface import Surface
+
+SP = S.SPACING
+
+
+def _rollout(name, nx, ny, nz, steps, dt, **kw):
+    c = dict(kind="rollout", nx=nx, ny=ny, nz=nz, steps=steps, dt=dt, solver="explicit", model=-1, eta0=0.0, index=0.7,
+             elastic=0, rigid=0, plate=0, vy=0.0, radius=0.01, max_error=0.1, divergence=True, compensated=True,
+             warm=True)
+    c.update(kw)
+    if name:
+        c["name"] = name
+    return c
+
+
+def listed():
+    return [
+        # the interactive loop on a toy scene (216 fluid particles): one step,
+        # then the positions are shown.  Launches and latency decide.
+        _rollout("interactive_216", 6, 6, 6, 1, 1e-3),
+        # the plain dam break, 13,824 fluid particles, explicit viscosity
+        _rollout("dam_13824", 24, 24, 24, 10, 1e-3, max_error=0.05),
+        # a small served scene with an odd particle count: power law, implicit viscosity
+        _rollout("powerlaw_2717", 13, 19, 11, 10, 5e-4, solver="implicit", model=1, eta0=20.0, index=0.7),
+        # the large non-Newtonian dam break, 131,072 fluid particles, Cross model
+        _rollout("cross_131072", 64, 32, 64, 6, 5e-4, solver="implicit", model=2, eta0=50.0),
+        # an over-dense block thrown at the floor: the pressure solve iterates every step
+        _rollout("impact_9240", 22, 20, 21, 5, 1e-3, vy=-6.0, radius=0.011, max_error=0.02, divergence=False),
+        # the elastic block over its plate, 98,304 elastic particles, no fluid
+        _rollout("elastic_98304", 0, 0, 0, 10, 2e-4, elastic=98304, plate=200),
+        # two-way coupling: a pool and a rigid cube dropped into it
+        _rollout("rigid_7424", 24, 12, 24, 10, 5e-4, rigid=8),
+        # 64 mixed requests (2k-60k dynamic particles each) in three lanes, 50 steps each
+        dict(kind="lanes", name="serve_64", count=64, lo=2000, hi=60000, lanes=3, steps=50),
+        # the surface tool's example: a ring of a few thousand particles, with normals
+        dict(kind="mesh", name="mesh_ring_2000", shape="ring", n=2000, radius_ratio=6.0, anisotropic=True,
+             smooth=1, normals=True, velocity=False),
+        # a frame's fluid meshed: 128k particles, anisotropic, normals
+        dict(kind="mesh", name="mesh_block_128000", shape="block", n=128000, radius_ratio=6.0, anisotropic=True,
+             smooth=1, normals=True, velocity=False),
+        # the same tool with the velocity channels, an odd count, a smaller radius
+        dict(kind="mesh", name="mesh_velocity_30011", shape="block", n=30011, radius_ratio=4.0, anisotropic=True,
+             smooth=1, normals=False, velocity=True),
+        # neighbor lists for positions that live on the device
+        dict(kind="lists", name="lists_200000", n=200000),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choices(["rollout", "lanes", "mesh", "lists"], [6, 1, 2, 1])[0]
+    if kind == "lanes":
+        return dict(kind="lanes", count=rng.randint(3, 40), lo=1000, hi=_log_int(rng, 4000, 60000),
+                    lanes=rng.randint(1, 3), steps=rng.randint(20, 50))
+    if kind == "mesh":
+        vel = rng.random() < 0.3
+        return dict(kind="mesh", shape=rng.choice(["ring", "block"]), n=_log_int(rng, 500, 100000),
+                    radius_ratio=rng.choice([4.0, 5.0, 6.0]), anisotropic=vel or rng.random() < 0.8,
+                    smooth=rng.randint(0, 2), normals=rng.random() < 0.6, velocity=vel)
+    if kind == "lists":
+        return dict(kind="lists", n=_log_int(rng, 300, 200000))
+    sort = rng.choices(["explicit", "implicit", "elastic", "rigid", "impact"], [3, 5, 2, 1, 1])[0]
+    if sort == "elastic":
+        n = _log_int(rng, 500, 98304)
+        return _rollout(None, 0, 0, 0, rng.randint(1, 10), 2e-4, elastic=n, plate=int(math.sqrt(n)) // 2 + 40,
+                        compensated=rng.random() < 0.8)
+    if sort == "rigid":
+        a = rng.randint(10, 30)
+        return _rollout(None, a, rng.randint(4, 14), a + rng.randint(-2, 2), rng.randint(1, 10), 5e-4,
+                        rigid=rng.randint(3, 8))
+    if sort == "impact":
+        a = rng.randint(6, 22)
+        return _rollout(None, a, rng.randint(6, 20), a + rng.randint(0, 3), rng.randint(1, 5), 1e-3, vy=-6.0, radius=0.011,
+                        max_error=0.02, divergence=False)
+    n = _log_int(rng, 200, 131072)
+    a = max(4, int(round(n ** (1 / 3) * rng.uniform(0.8, 1.3))))
+    c = max(4, int(round(a * rng.uniform(0.7, 1.3))))
+    b = max(3, n // (a * c))
+    steps = rng.randint(1, 10) if n < 60000 else rng.randint(1, 5)
+    if sort == "explicit":
+        return _rollout(None, a, b, c, steps, rng.choice([5e-4, 1e-3]), compensated=rng.random() < 0.7,
+                        elastic=int(0.2 * n) if rng.random() < 0.25 else 0)
+    model = rng.choice([-1, 0, 1, 1, 2, 2, 3, 4, 5, 6])
+    return _rollout(None, a, b, c, steps, 5e-4, solver="implicit", model=model,
+                    eta0=math.exp(rng.uniform(math.log(0.1), math.log(100.0))), index=round(rng.uniform(0.5, 1.5), 3),
+                    warm=rng.random() < 0.8, elastic=int(0.2 * n) if rng.random() < 0.25 else 0)
+
+
+# ---------------------------------------------------------------------------
+# inputs
+# ---------------------------------------------------------------------------
+def _block_dims(n):
+    a = max(3, int(round(n ** (1 / 3))))
+    return a, -(-n // (a * a)), a
+
+
+def _scene(case, seed):
+    """Parameters, x, v, kind of a rollout's scene: a jittered fluid block on
+    the floor of a walled box with a swirl of about 0.3 m/s in it, an elastic
+    block beside it or a rigid cube above it; or an elastic block over a plate."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    kw = dict(dt=case["dt"], gravity=(0.0, -9.81, 0.0), particle_radius=case["radius"], max_error=case["max_error"],
+              enable_divergence_solver=case["divergence"], compensated=case["compensated"],
+              warm_start=int(case["warm"]), youngs_modulus=1e5, poisson_ratio=0.33)
+    if case["solver"] == "implicit":
+        kw.update(viscosity_method=1, weiler_tol=1e-4, weiler_max_iter=100)
+        if case["model"] >= 0:
+            e = case["eta0"]
+            kw.update(use_non_newtonian=True, non_newton_method=case["model"], viscosity0=e,
+                      viscosity_inf=e / 500.0, consistency_index=(e if case["model"] in (1, 6) else 1.0),
+                      power_index=case["index"], max_viscosity=1e4)
+        else:
+            kw.update(viscosity=max(case["eta0"], 0.01))
+    if not case["nx"]:  # the elastic block over a plate
+        p = case["plate"]
+        a, b, c = (48, 32, 64) if case["elastic"] == 98304 else _block_dims(case["elastic"])
+        cells = (p + 4, b + 28, p + 4)
+        plate = S.lattice((2 * SP, SP, 2 * SP), (p, 1, p))
+        o = (2 * SP + 0.5 * (p - a) * SP, SP + 0.05, 2 * SP + 0.5 * (p - c) * SP)
+        block = S.jitter(rng, S.lattice(o, (a, b, c))[: case["elastic"]])
+        sc = S.assemble("", SceneParams(domain_end=tuple(q * SP for q in cells), **kw), None, plate, block, 1)
+        sc.v[sc.kind == KIND_ELASTIC] = _swirl(rng, sc.x[sc.kind == KIND_ELASTIC])
+        return sc
+    nx, ny, nz = case["nx"], case["ny"], case["nz"]
+    ea = eb = ec = 0
+    if case["elastic"]:
+        ea, eb, ec = _block_dims(case["elastic"])
+    q = case["rigid"]
+    cells = (nx + 14 + (ea + 6 if ea else nx // 2), max(ny + 12 + q, eb + 8, ny * 3 // 2), max(nz, ec) + 8)
+    fluid = S.jitter(rng, S.lattice((3 * SP, 3 * SP, 3 * SP), (nx, ny, nz)))
+    el = None
+    if ea:
+        el = S.jitter(rng, S.lattice(((nx + 7) * SP, 3 * SP, 3 * SP), (ea, eb, ec))[: case["elastic"]])
+    body = []
+    if q:
+        body = [S.lattice((3 * SP + 0.5 * max(0, nx - q) * SP, (ny + 4) * SP, 3 * SP + 0.5 * max(0, nz - q) * SP), (q, q, q))]
+    sc = S.assemble("", SceneParams(domain_end=tuple(c * SP for c in cells), **kw), fluid, S.shell(cells), el, 1, rigid=body)
+    f = sc.kind == KIND_FLUID
+    sc.v[f] = _swirl(rng, sc.x[f])
+    sc.v[f, 1] += case["vy"]
+    sc.v[sc.kind >= KIND_RIGID, 1] = -0.5
+    return sc
+
+
+def _swirl(rng, x):
+    """A smooth velocity field of zero divergence, wavelength a fifth of a metre."""
+    k = 2 * np.pi / 0.2
+    a, b, c = rng.uniform(0, 2 * np.pi, 3)
+    return (0.3 * np.stack([np.sin(k * x[:, 1] + a), 0.3 * np.sin(k * x[:, 2] + b), np.sin(k * x[:, 0] + c)], 1)).astype(np.float32)
+
+
+def _points(case, seed):
+    """Particles to be meshed, spacing 0.02: a solid ring or a block, jittered."""
+    rng = np.random.Generator(np.random.PCG64(seed))
+    n = case["n"]
+    if case["shape"] == "ring":
+        r = (n * SP ** 3 / (2 * np.pi ** 2 * 3.0)) ** (1 / 3)  # tube radius; the ring's is 3 r
+        m = int(4 * r / SP) + 2
+        g = S.lattice((-m * SP, -(m // 2) * SP, -m * SP), (2 * m + 1, m + 1, 2 * m + 1))
+        t = (np.hypot(g[:, 0], g[:, 2]) - 3 * r) ** 2 + g[:, 1] ** 2
+        x = g[np.argsort(t, kind="stable")[:n]] + (m + 8) * SP
+    else:
+        a = max(3, int(round((n / 4) ** (1 / 3))))
+        x = S.lattice((0.2, 0.2, 0.2), (2 * a, -(-n // (4 * a * a)), 2 * a))[:n]
+    x = (x + rng.uniform(-0.15 * SP, 0.15 * SP, x.shape)).astype(np.float32)
+    return x, _swirl(rng, x)
+
+
+def prepare(case, seed):
+    if case["kind"] == "rollout":
+        sc = _scene(case, seed)
+        ctx = L.Context(sc.params, sc.n)
+        ctx.upload(sc.x, sc.kind, sc.v)
+        ctx.init()
+        return dict(case=case, ctx=ctx, x=sc.x, v=sc.v, zero=np.zeros_like(sc.v))
+    if case["kind"] == "lanes":
+        rng = np.random.Generator(np.random.PCG64(seed))
+        scs = S.mixed_batch(seed=3, count=case["count"], lo=case["lo"], hi=case["hi"])
+        for s in scs:
+            move = rng.uniform(-0.005 * SP, 0.005 * SP, s.x.shape).astype(np.float32)
+            s.x[s.kind != KIND_STATIC] += move[s.kind != KIND_STATIC]
+            s.v[s.kind == KIND_FLUID] = _swirl(rng, s.x[s.kind == KIND_FLUID])
+        order = sorted(range(len(scs)), key=lambda k: (-scs[k].n, k))
+        return dict(case=case, scenes=scs, order=order, pool=LanePool(64 << 30, lanes=case["lanes"]))
+    if case["kind"] == "mesh":
+        x, v = _points(case, seed)
+        surf = Surface(origin=(0.0, 0.0, 0.0), voxel_size=0.01, particle_radius=0.02,
+                       smooth_radius=0.01 * case["radius_ratio"], isolevel=0.0, anisotropic=case["anisotropic"],
+                       smooth_iterations=case["smooth"], normals=case["normals"], velocity=case["velocity"])
+        cap = max(8 * case["n"], 60000)
+        out = dict(vertices=np.zeros((cap, 3), np.float32), triangles=np.zeros((2 * cap, 3), np.int32),
+                   sizes=np.zeros(2, np.int32))
+        if case["normals"]:
+            out["normals"] = np.zeros((cap, 3), np.float32)
+        if case["velocity"]:
+            out["velocity"] = np.zeros((cap, 3), np.float32)
+        return dict(case=case, surf=surf, x=x, v=v if case["velocity"] else None, out=out)
+    n = case["n"]
+    rng = np.random.Generator(np.random.PCG64(seed))
+    a, b, c = _block_dims(n)
+    x = S.jitter(rng, S.lattice((3 * SP, 3 * SP, 3 * SP), (a, b, c))[:n], frac=0.2)
+    x = x[rng.permutation(n)] if n % 2 else x  # some callers number their particles in no spatial order
+    p = SceneParams(domain_end=tuple((m + 8) * SP for m in (a, b, c)))
+    dev = torch.device("cuda")
+    return dict(case=case, params=L.params_struct(p), x=torch.tensor(x, dtype=torch.float32, device=dev),
+                nbr=torch.empty((n, L.MAX_NEIGHBORS), dtype=torch.int32, device=dev),
+                cnt=torch.empty(n, dtype=torch.int32, device=dev), status=torch.zeros(1, dtype=torch.int32, device=dev))
+
+
+# ---------------------------------------------------------------------------
+# one pass
+# ---------------------------------------------------------------------------
+def run(state):
+    case = state["case"]
+    if case["kind"] == "rollout":
+        ctx = state["ctx"]
+        ctx.upload_field(L.FIELD_X, state["x"])
+        ctx.upload_field(L.FIELD_V, state["v"])
+        if case["solver"] == "implicit":
+            ctx.upload_field(L.FIELD_VISC_DIFF, state["zero"])
+        ctx.step(case["steps"])
+        return dict(x=ctx.download(L.FIELD_X), v=ctx.download(L.FIELD_V))
+    if case["kind"] == "lanes":
+        lp, scs = state["pool"], state["scenes"]
+        keys = {}
+        for k in state["order"]:
+            s = scs[k]
+            keys[k] = lp.admit(s.params, s.x, s.kind, s.v, n_elastic=s.n_elastic)
+        lp.run(case["steps"], [[] for _ in range(lp.lanes)])
+        x = [lp.read(keys[k], L.FIELD_X) for k in range(len(scs))]
+        v = [lp.read(keys[k], L.FIELD_V) for k in range(len(scs))]
+        for k in keys:
+            lp.retire(keys[k])
+        return dict(x=np.concatenate(x), v=np.concatenate(v))
+    if case["kind"] == "mesh":
+        surf, out = state["surf"], state["out"]
+        surf.run(state["x"], state["v"])
+        vert, tri, nrm = surf.mesh()
+        out["vertices"][: len(vert)] = vert
+        out["triangles"][: len(tri)] = tri
+        out["sizes"][:] = len(vert), len(tri)
+        if nrm is not None:
+            out["normals"][: len(vert)] = nrm
+        if case["velocity"]:
+            out["velocity"][: len(vert)] = surf.mesh_velocity()
+        return out
+    x, nbr, cnt, status = state["x"], state["nbr"], state["cnt"], state["status"]
+    L.check(L.load().nn_neighbors_noalloc(ctypes.byref(state["params"]), x.data_ptr(), case["n"], nbr.data_ptr(),
+                                          cnt.data_ptr(), L.MAX_NEIGHBORS, status.data_ptr(),
+                                          torch.cuda.current_stream().cuda_stream), "nn_neighbors_noalloc")
+    return dict(neighbors=nbr, counts=cnt, status=status)
+
+
+# ---------------------------------------------------------------------------
+# what a pass cannot do without
+# ---------------------------------------------------------------------------
+def _counts(case):
+    """fluid, elastic, rigid and all particles of a rollout's scene"""
+    nf = case["nx"] * case["ny"] * case["nz"]
+    if not nf:
+        return 0, case["elastic"], 0, case["elastic"] + case["plate"] ** 2
+    wall = 2 * (nf ** (2 / 3)) * 6
+    return nf, case["elastic"], case["rigid"] ** 3, int(nf + case["elastic"] + case["rigid"] ** 3 + wall)
+
+
+def _step_work(nf, ne, n, implicit, model):
+    """Bytes and operations of one step: positions and velocities read and
+    written once; per pair (30 of a fluid particle) the kernel and its gradient
+    once (25), density and factor (20), two divergence and two pressure sweeps
+    (10 each), surface tension and viscosity (20), the strain rate (30), and, in
+    the implicit solve, the pair scalar (20) and at least four products of 17;
+    per elastic pair (30) 27 + 36 + 70."""
+    per = 25 + 20 + 40 + 20 + (30 if model >= 0 else 0) + (20 + 4 * 17 if implicit else 0)
+    return dict(bytes=48.0 * (nf + ne) + 12.0 * (n - nf - ne), flops=30.0 * nf * per + 30.0 * ne * 133)
+
+
+def work(case):
+    if case["kind"] == "rollout":
+        nf, ne, nr, n = _counts(case)
+        w = _step_work(nf, ne + nr, n, case["solver"] == "implicit", case["model"])
+        return dict(bytes=48.0 * n + case["steps"] * w["bytes"], flops=case["steps"] * w["flops"])
+    if case["kind"] == "lanes":
+        mean = (case["hi"] - case["lo"]) / math.log(case["hi"] / case["lo"])
+        n = mean * case["count"]
+        w = _step_work(n, 0.05 * n, 1.75 * n, True, 1)
+        return dict(bytes=1.75 * n * 52 + case["steps"] * w["bytes"], flops=case["steps"] * w["flops"])
+    n = case["n"]
+    if case["kind"] == "mesh":
+        # positions in, a mesh of about one vertex and two triangles per surface
+        # voxel out; the field's value at every vertex within a particle's
+        # support: (4/3) pi ratio^3 vertices of 30 operations, twice that for a moment each
+        surface = 24.0 * n ** (2 / 3)
+        flops = n * 4.19 * case["radius_ratio"] ** 3 * 30
+        if case["anisotropic"]:
+            flops += n * 4.19 * (2 * case["radius_ratio"] / 2.0) ** 3 * 2 * 20
+        return dict(bytes=12.0 * n * (2 if case["velocity"] else 1) + surface * (36 + 12 * case["normals"] + 12 * case["velocity"]),
+                    flops=flops)
+    return dict(bytes=n * (12.0 + 240 + 4), flops=n * 27 * 8 * 8.0)
+
+
+# ---------------------------------------------------------------------------
+# the same steps in 64 bits, in plain numpy
+# ---------------------------------------------------------------------------
+def exact(case, seed):
+    """x and v of a rollout in 64 bits, by the same discretisation and stopping
+    rules.  None for the long ones and for the served mix (their steps would
+    take minutes), and for a mesh: a value near a threshold decides how many
+    vertices there are.  Neighbor lists are whole numbers."""
+    if case["kind"] != "rollout":
+        return None
+    nf, ne, nr, _ = _counts(case)
+    if case["steps"] * (nf * (4 if case["solver"] == "implicit" else 1) + 2 * ne) > 180000:
+        return None
+    x, v = _Rollout(_scene(case, seed)).advance(case["steps"])
+    return dict(x=x, v=v)
+
+
+class _Rollout:
+    def __init__(self, sc):
+        p = sc.params
+        self.p, self.kind = p, np.minimum(sc.kind, KIND_RIGID)
+        self.body = sc.kind - KIND_RIGID
+        self.x, self.v = sc.x.astype(np.float64), sc.v.astype(np.float64)
+        self.n = len(self.x)
+        self.h = 4.0 * p.particle_radius
+        self.fluid = self.kind == KIND_FLUID
+        self.dyn = (self.kind == KIND_ELASTIC) | (self.kind == KIND_RIGID)
+        d = 2.0 * p.particle_radius
+        self.vol0 = 0.8 * d ** 3
+        self.mass = self.vol0 * 1000.0
+        self.kw = 8.0 / math.pi / self.h ** 3
+        self.vdiff = np.zeros_like(self.x)
+        self.V = np.full(self.n, self.vol0)
+        self.search()
+        self.solid_volumes(self.kind == KIND_STATIC)
+        self.solid_volumes(self.dyn)
+        self.x0 = self.x.copy()
+        w = self.w(self.r)
+        self.V0 = self.mass / (self.mass * self.kw + self.sum(self.mass * w))
+        if (self.kind == KIND_ELASTIC).any():
+            el = self.kind == KIND_ELASTIC
+            need = el.copy()
+            need[self.j[el[self.i]]] = True
+            m = need[self.i]
+            self.rest = self.i[m], self.j[m]
+        self.bodies = [np.flatnonzero(self.body == b) for b in range(self.body.max() + 1)]
+
+    # pairs (i, j) with |x_i - x_j| < h, tested as 32-bit values, sorted by i
+    def search(self):
+        x, h = self.x, self.h
+        xf = x.astype(np.float32)
+        c = np.floor(x / h).astype(np.int64) + 1
+        g = c.max(0) + 2
+        key = (c[:, 0] * g[1] + c[:, 1]) * g[2] + c[:, 2]
+        order = np.argsort(key, kind="stable")
+        ks = key[order]
+        I, J = [], []
+        every = np.arange(self.n)
+        for dx in (-1, 0, 1):
+            for dy in (-1, 0, 1):
+                k0 = key + (dx * g[1] + dy) * g[2]
+                lo, hi = np.searchsorted(ks, k0 - 1, "left"), np.searchsorted(ks, k0 + 1, "right")
+                m = hi - lo
+                i = np.repeat(every, m)
+                at = np.arange(len(i)) - np.repeat(np.cumsum(m) - m, m) + np.repeat(lo, m)
+                j = order[at]
+                e = xf[i] - xf[j]
+                ss = e[:, 0] * e[:, 0] + e[:, 1] * e[:, 1] + e[:, 2] * e[:, 2]
+                ok = (np.sqrt(ss) < np.float32(h)) & (i != j)
+                I.append(i[ok])
+                J.append(j[ok])
+        i, j = np.concatenate(I), np.concatenate(J)
+        o = np.argsort(i, kind="stable")
+        self.i, self.j = i[o], j[o]
+        self.count = np.bincount(self.i, minlength=self.n)
+        self.d = x[self.i] - x[self.j]
+        self.r = np.sqrt((self.d ** 2).sum(1))
+        self.g = self.grad(self.d, self.r)
+
+    def w(self, r):
+        q = r / self.h
+        return np.where(q <= 0.5, self.kw * (6 * q ** 3 - 6 * q ** 2 + 1), np.where(q <= 1, 2 * self.kw * (1 - q) ** 3, 0.0))
+
+    def radial(self, r):
+        q = r / self.h
+        f = 6 * self.kw * np.where(q <= 0.5, q * (3 * q - 2), -((1 - q) ** 2))
+        return np.where((r > 1e-5) & (q <= 1), f / (np.maximum(r, 1e-5) * self.h), 0.0)
+
+    def grad(self, d, r):
+        return self.radial(r)[:, None] * d
+
+    def sum(self, a, i=None):
+        i = self.i if i is None else i
+        if a.ndim == 1:
+            return np.bincount(i, a, self.n)
+        return np.stack([np.bincount(i, a[:, k], self.n) for k in range(a.shape[1])], 1)
+
+    def solid_volumes(self, which):
+        if which.any():
+            solid = ~self.fluid[self.j]
+            vol = 3.0 / (self.kw + self.sum(np.where(solid, self.w(self.r), 0.0)))
+            self.V[which] = vol[which]
+
+    def divergence(self):
+        dv = self.v[self.i] - self.v[self.j]
+        return self.sum(self.V[self.j] * (dv * self.g).sum(1))
+
+    def push(self, k):
+        """v += dt sum_j V_j (k_i + k_j) grad W over fluid j, k_i alone over solid j"""
+        fj = self.fluid[self.j]
+        s = k[self.i] + np.where(fj, k[self.j], 0.0)
+        s = np.where(np.abs(s) > self.p.eps, s, 0.0) * self.V[self.j]
+        dv = self.p.dt * self.sum(s[:, None] * self.g)
+        self.v[self.fluid] += dv[self.fluid]
+
+    def step(self):
+        p, fl = self.p, self.fluid
+        self.search()
+        if self.dyn.any():
+            self.solid_volumes(self.dyn)
+        acc = np.where(self.dyn[:, None], np.array(p.gravity), 0.0)
+        if fl.any():
+            self.fluid_step(acc)
+        if (self.kind == KIND_ELASTIC).any():
+            acc += self.elastic()
+        for b in self.bodies:
+            for _ in range(max(0, p.coupling_interval)):
+                low = ~fl & (self.x[:, 1] < self.h)
+                self.x[low, 1] = self.h
+                q0 = self.x0[b] - self.x0[b].mean(0)
+                cm = self.x[b].mean(0)
+                self.x[b] = cm + q0 @ _polar(((self.x[b] - cm).T @ q0)[None])[0].T
+        self.v[self.dyn] += p.dt * acc[self.dyn]
+        self.advect()
+
+    def fluid_step(self, acc):
+        p, fl, dt, nf = self.p, self.fluid, self.p.dt, self.fluid.sum()
+        Vj, fj = self.V[self.j], fl[self.j]
+        fi = fl[self.i]
+        rho = np.where(fl, p.density0 * (self.V * self.kw + self.sum(Vj * self.w(self.r))), p.density0)
+        gp = -Vj[:, None] * self.g
+        sk = self.sum(np.where(fj, (gp ** 2).sum(1), 0.0)) + (self.sum(gp) ** 2).sum(1)
+        alpha = np.where(fl & (sk > 1e-6), -1.0 / np.maximum(sk, 1e-6), 0.0)
+
+        def rate():
+            return np.where(fl & (self.count >= 20), np.maximum(self.divergence(), 0.0), 0.0)
+
+        if p.enable_divergence_solver:
+            rd = rate()
+            for _ in range(max(1, p.max_iterations_v)):
+                self.push(rd * alpha / dt)
+                rd = rate()
+                if (p.density0 * rd).sum() / nf <= p.max_error_v * 0.01 * p.density0 / dt:
+                    break
+        implicit = p.viscosity_method == 1
+        eta = np.full(self.n, p.viscosity)
+        if p.use_non_newtonian:
+            vji = (self.v[self.j] - self.v[self.i])
+            t = vji[:, :, None] * self.g[:, None, :]
+            D = self.sum((self.mass * (t + t.transpose(0, 2, 1))).reshape(-1, 9)) * (0.5 / rho)[:, None]
+            eta = _viscosity(p, np.sqrt((D ** 2).sum(1)))
+        if implicit:
+            new = self.weiler(rho, eta * p.density0)
+        d2 = self.r ** 2
+        diam = 2.0 * p.particle_radius
+        a = np.tile(np.array(p.gravity), (self.n, 1))
+        tension = np.where(fj, np.where(d2 > np.float32(diam * diam), self.w(self.r), self.w(np.array([diam]))[0]), 0.0)
+        a -= p.surface_tension * self.sum(tension[:, None] * self.d)
+        if implicit:
+            a += (new - self.v) / dt
+            self.vdiff[fl] = (new - self.v)[fl]
+        else:
+            vx = ((self.v[self.i] - self.v[self.j]) * self.d).sum(1)
+            f = np.where(fj, 10 * p.viscosity * self.mass / rho[self.j] * vx / (d2 + 0.01 * self.h ** 2), 0.0)
+            a += self.sum(f[:, None] * self.g)
+        self.v[fl] += dt * a[fl]
+
+        def predicted():
+            return np.where(fl, np.maximum(rho / p.density0 + dt * self.divergence(), 1.0), 1.0)
+
+        da = predicted()
+        for _ in range(max(1, p.max_iterations)):
+            k = (da - 1.0) * alpha / dt ** 2
+            self.push(k)
+            if self.dyn.any():  # reactions on the dynamic solids
+                kf = np.where(fj & (np.abs(k[self.j]) > p.eps), k[self.j], 0.0)
+                acc += np.where(self.dyn[:, None], self.sum((self.V[self.i] * kf)[:, None] * self.g), 0.0)
+            da = predicted()
+            if (p.density0 * (da[fl] - 1.0)).sum() / nf <= p.max_error * 0.01 * p.density0:
+                break
+
+    def weiler(self, rho, mu):
+        p, fl, dt = self.p, self.fluid, self.p.dt
+        m = fl[self.i] & fl[self.j]
+        i, j, d, r = self.i[m], self.j[m], self.d[m], self.r[m]
+        s = 10 * 0.5 * (mu[i] + mu[j]) * self.mass / rho[j] / (r ** 2 + 0.01 * self.h ** 2) * self.radial(r)
+        f = (dt / rho)[:, None]
+
+        def A(u):
+            return u - f * self.sum((s * ((u[i] - u[j]) * d).sum(1))[:, None] * d, i)
+
+        blocks = np.eye(3) - f[:, :, None] * self.sum((s[:, None, None] * d[:, :, None] * d[:, None, :]).reshape(-1, 9), i).reshape(-1, 3, 3)
+        M = np.linalg.inv(blocks)
+        b = np.where(fl[:, None], self.v, 0.0)
+        x, res = b.copy(), b - A(b)
+        if p.warm_start & 1:
+            e = self.vdiff
+            z = A(e)
+            ez = (e * z).sum()
+            th = (e * res).sum() / ez if ez > 0 else 0.0
+            x, res = x + th * e, res - th * z
+        bb = (b * b).sum()
+        u = (M @ res[:, :, None])[:, :, 0]
+        pv, ga = u.copy(), (res * u).sum()
+        for _ in range(p.weiler_max_iter):
+            if (res * res).sum() <= p.weiler_tol ** 2 * bb:
+                break
+            w = A(pv)
+            al = ga / (pv * w).sum()
+            x, res = x + al * pv, res - al * w
+            u = (M @ res[:, :, None])[:, :, 0]
+            ga, old = (res * u).sum(), ga
+            pv = u + ga / old * pv
+        return x
+
+    def elastic(self):
+        p = self.p
+        i, j = self.rest
+        d, d0 = self.x[j] - self.x[i], self.x0[j] - self.x0[i]
+        r0 = np.sqrt((d0 ** 2).sum(1))
+        g = self.grad(d0, r0)
+        A = self.sum(((self.mass * self.w(r0))[:, None, None] * d[:, :, None] * d0[:, None, :]).reshape(-1, 9), i).reshape(-1, 3, 3)
+        R = _polar(A)
+        u = (R.transpose(0, 2, 1)[i] @ d[:, :, None])[:, :, 0] - d0
+        U = -self.sum((self.V0[j][:, None, None] * u[:, :, None] * g[:, None, :]).reshape(-1, 9), i).reshape(-1, 3, 3)
+        E = 0.5 * (U + U.transpose(0, 2, 1))
+        nu = p.poisson_ratio
+        k = p.youngs_modulus / ((1 + nu) * (1 - 2 * nu))
+        sig = k * 0.5 * (1 - 2 * nu) * E  # off the diagonal the shear modulus times the strain
+        tr = np.trace(E, axis1=1, axis2=2)
+        for a in range(3):
+            sig[:, a, a] = k * ((1 - 2 * nu) * E[:, a, a] + nu * tr)
+        gi = (self.V0[i] * self.V0[j])[:, None] * g
+        f = (R[j] @ -(sig[j] @ gi[:, :, None]) - R[i] @ (sig[i] @ gi[:, :, None]))[:, :, 0]
+        el = (self.kind == KIND_ELASTIC)[:, None]
+        return np.where(el, 0.5 * self.sum(f, i) / self.mass, 0.0)
+
+    def advect(self):
+        p, m = self.p, self.kind != KIND_STATIC
+        x = self.x[m] + p.dt * self.v[m]
+        v = self.v[m]
+        lo, hi = np.array(p.domain_start) + self.h, np.array(p.domain_end) - self.h
+        n = (x > hi).astype(float) - (x <= lo).astype(float)
+        x = np.where(x > hi, hi, np.where(x <= lo, lo, x))
+        ln = np.sqrt((n ** 2).sum(1))
+        hit = ln > 1e-6
+        n[hit] /= ln[hit][:, None]
+        v[hit] = (v - (1 + p.collision_coeff) * (v * n).sum(1)[:, None] * n)[hit] * p.sticky_coeff
+        self.x[m], self.v[m] = x, v
+
+    def advance(self, steps):
+        for _ in range(steps):
+            self.step()
+        return self.x, self.v
+
+
+def _polar(A):
+    U, s, Vt = np.linalg.svd(A)
+    U[:, :, 2] *= np.sign(np.linalg.det(U @ Vt))[:, None]
+    return U @ Vt
+
+
+def _viscosity(p, gam):
+    n, K, e0, ei, gc = p.power_index, p.consistency_index, p.viscosity0, p.viscosity_inf, p.critical_strain_rate
+    with np.errstate(divide="ignore", invalid="ignore"):
+        if p.non_newton_method == 1:
+            eta = K * gam ** (n - 1)
+        elif p.non_newton_method == 2:
+            eta = ei + (e0 - ei) / (1 + (K * gam) ** n)
+        elif p.non_newton_method == 3:
+            eta = (math.sqrt(p.mu_c) + np.sqrt(p.yield_stress / gam)) ** 2
+        elif p.non_newton_method == 4:
+            eta = ei + (e0 - ei) / (1 + (K * gam * gam) ** ((1 - n) / 2))
+        elif p.non_newton_method == 5:
+            eta = np.where(gam < gc, e0, gc * (e0 - ei) / gam + ei)
+        elif p.non_newton_method == 6:
+            eta = np.where(gam < gc, e0, (e0 * gc - K * gc ** n) / gam + K * gam ** (n - 1))
+        else:
+            eta = np.full_like(gam, e0)
+    eta = np.where(np.isnan(eta), p.max_viscosity, np.maximum(eta, 0.0))
+    return np.minimum(eta, p.max_viscosity)
