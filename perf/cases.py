@@ -87,9 +87,10 @@ def draw(rng):
                     lanes=rng.randint(1, 3), steps=rng.randint(20, 50))
     if kind == "mesh":
         vel = rng.random() < 0.3
+        aniso = vel or rng.random() < 0.8  # the isotropic field is contoured as it is (it has no negative values to smooth by)
         return dict(kind="mesh", shape=rng.choice(["ring", "block"]), n=_log_int(rng, 500, 100000),
-                    radius_ratio=rng.choice([4.0, 5.0, 6.0]), anisotropic=vel or rng.random() < 0.8,
-                    smooth=rng.randint(0, 2), normals=rng.random() < 0.6, velocity=vel)
+                    radius_ratio=rng.choice([4.0, 5.0, 6.0]), anisotropic=aniso,
+                    smooth=rng.randint(0, 2) if aniso else 0, normals=rng.random() < 0.6, velocity=vel)
     if kind == "lists":
         return dict(kind="lists", n=_log_int(rng, 300, 200000))
     sort = rng.choices(["explicit", "implicit", "elastic", "rigid", "impact"], [3, 5, 2, 1, 1])[0]
@@ -218,7 +219,8 @@ def prepare(case, seed):
     if case["kind"] == "mesh":
         x, v = _points(case, seed)
         surf = Surface(origin=(0.0, 0.0, 0.0), voxel_size=0.01, particle_radius=0.02,
-                       smooth_radius=0.01 * case["radius_ratio"], isolevel=0.0, anisotropic=case["anisotropic"],
+                       smooth_radius=0.01 * case["radius_ratio"], isolevel=0.0 if case["anisotropic"] else 0.2,
+                       anisotropic=case["anisotropic"],
                        smooth_iterations=case["smooth"], normals=case["normals"], velocity=case["velocity"])
         cap = max(8 * case["n"], 60000)
         out = dict(vertices=np.zeros((cap, 3), np.float32), triangles=np.zeros((2 * cap, 3), np.int32),
