@@ -125,6 +125,7 @@ class Batch {
   int kdepth[K_COUNT] = {};    // per-kernel gather depth (0 = the kernel's default), set by the autotuner
   int blk(int id) const { return kblock[id] ? kblock[id] : block; }
   int dep(int id) const { return kdepth[id]; }
+  int lanes(int id) const;  // lanes per particle of list sweep `id`
   hipStream_t stream;
   Dev d{};
   KernelTimer timer;

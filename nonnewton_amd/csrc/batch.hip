@@ -189,6 +189,7 @@ int derive_scene(SceneHost& s, std::string& err) {
   if (s.n_fluid > 0) f |= SF_HAS_FLUID;
   if (s.n_elastic > 0) f |= SF_HAS_ELASTIC;
   if (s.nbody > 0) f |= SF_HAS_RIGID;
+  if (c.h >= 0x1p-20f && c.h <= 0x1p20f) f |= SF_MIDRANGE;
   c.flags = f;
   c.n = s.n;
   c.n_fluid = s.n_fluid;
@@ -267,6 +268,26 @@ void Batch::release() {
 }
 
 DevRef Batch::dref() { return DevRef{d}; }
+
+// Lanes per particle of a list sweep, by the slots in use.  A sweep is bound by
+// its longest chain (a lane walking its list) until the device is full of
+// wavefronts, and by instructions after that, where every lane of a group
+// repeats the additions.  Microseconds a launch with 1 / 4 / 16 lanes, by
+// slots in use (one scene; the last column the 64-scene pool):
+//                  2,554          46,346         162,570        1,616,737
+//   build_lists    37 / 15 / 8    44 / 22 / 16   58 / 43 / 44   246 / 240 / 296
+//   density_alpha  13 / 9 / 7     15 / 12 / 17   22 / 25 / 51    96 / 129 / 385
+//   div_source     11 / 7 / 7     12 /  8 /  7   20 / 17 / 20    81 /  82 / 137
+//   nonpressure    24 / 11 / 8    28 / 16 / 15   46 / 34 / 39   156 / 176 / 258
+//   strain         13 / 9 / 6     16 / 12 / 15   27 / 24 / 39    97 / 118 / 231
+// (nonpressure of a scene with explicit viscosity.)  The search's limit is
+// higher: its lanes share candidates and repeat nothing.  One lane is left to
+// the three sweeps with the most sums, where four were slower.
+int Batch::lanes(int id) const {
+  if (d.Pn <= (id == K_BUILD_LISTS ? 131072 : 32768)) return 16;
+  const bool many_sums = id == K_DENSITY_ALPHA || id == K_NONPRESSURE || id == K_STRAIN;
+  return many_sums && d.Pn > 196608 ? 1 : 4;
+}
 
 void Batch::swap_sort_buffers() {
   std::swap(d.pos, d.pos_alt);
@@ -538,6 +559,10 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
     bytes_ = old_bytes;
     return rc;
   }
+  // the sort's keys and ranks are dead once the lists are being built: 16 W of
+  // the wavefronts' counts and densities fit in each (64 W words)
+  nd.wave_pairs = reinterpret_cast<int2*>(nd.rank);
+  nd.wave_rho = reinterpret_cast<float*>(nd.key);
   nd.scenes = scenes_dev;
   nd.wave_scene = ws;
   nd.s_wave_scene = sws;
@@ -802,7 +827,7 @@ int Batch::search_impl(int all) {
   TIMED(K_BUCKET, launch_bucket(dref(), blk(K_BUCKET), stream));
   TIMED(K_PLACE, launch_place(dref(), blk(K_PLACE), stream));
   swap_sort_buffers();
-  TIMED(K_BUILD_LISTS, launch_build_lists(dref(), blk(K_BUILD_LISTS), all, stream));
+  TIMED(K_BUILD_LISTS, launch_build_lists(dref(), blk(K_BUILD_LISTS), lanes(K_BUILD_LISTS), all, stream));
   lists_state_ = all ? 2 : 1;
   return NN_OK;
 }
@@ -923,8 +948,8 @@ int Batch::init_scenes(const std::vector<int>& which) {
   // the stress-set relayout does not carry neighbor lists (they hold absolute
   // slots); search again on the unchanged positions before the volume sweeps
   CHK(search_impl());
-  launch_bvol(dref(), block, 0, stream);
-  launch_bvol(dref(), block, 1, stream);
+  launch_bvol(dref(), block, lanes(K_BVOL), 0, stream);
+  launch_bvol(dref(), block, lanes(K_BVOL), 1, stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(stream));
   for (int k : which) scenes[k]->initialized = true;
@@ -959,13 +984,13 @@ int Batch::solver_loop(int which) {
   for (;;) {
     for (int c = 0; c < chunk; c++) {
       if (which == 0) {
-        TIMED(K_DIV_UPDATE, launch_div_update(dref(), blk(K_DIV_UPDATE), dep(K_DIV_UPDATE), stream));
-        TIMED(K_DIV_SOURCE, launch_div_source(dref(), blk(K_DIV_SOURCE), dep(K_DIV_SOURCE), stream));
-        launch_scene_finish(dref(), 0, stream);
+        TIMED(K_DIV_UPDATE, launch_div_update(dref(), blk(K_DIV_UPDATE), lanes(K_DIV_UPDATE), dep(K_DIV_UPDATE), stream));
+        TIMED(K_DIV_SOURCE, launch_div_source(dref(), blk(K_DIV_SOURCE), lanes(K_DIV_SOURCE), dep(K_DIV_SOURCE), stream));
+        launch_scene_finish(dref(), 0, lanes(K_DIV_SOURCE), stream);
       } else if (which == 1) {
-        TIMED(K_PRESS_UPDATE, launch_press_update(dref(), blk(K_PRESS_UPDATE), dep(K_PRESS_UPDATE), stream));
-        TIMED(K_PRESS_SOURCE, launch_press_source(dref(), blk(K_PRESS_SOURCE), dep(K_PRESS_SOURCE), 1, stream));
-        launch_scene_finish(dref(), 1, stream);
+        TIMED(K_PRESS_UPDATE, launch_press_update(dref(), blk(K_PRESS_UPDATE), lanes(K_PRESS_UPDATE), dep(K_PRESS_UPDATE), stream));
+        TIMED(K_PRESS_SOURCE, launch_press_source(dref(), blk(K_PRESS_SOURCE), lanes(K_PRESS_SOURCE), dep(K_PRESS_SOURCE), 1, stream));
+        launch_scene_finish(dref(), 1, lanes(K_PRESS_SOURCE), stream);
       }
     }
     done += chunk;
@@ -1041,28 +1066,28 @@ int Batch::step(std::vector<nn_step_stats>* stats) {
   // bodies: their ground collision moves positions after the search, so the
   // search positions would not survive to build those lists on demand
   CHK(search_impl(any_rigid_ ? 1 : 0));                                // :917
-  if (any_elastic_ || any_rigid_) TIMED(K_BVOL, launch_bvol(dref(), blk(K_BVOL), 1, stream));  // :918
+  if (any_elastic_ || any_rigid_) TIMED(K_BVOL, launch_bvol(dref(), blk(K_BVOL), lanes(K_BVOL), 1, stream));  // :918
   TIMED(K_CLEAR_ACC, launch_clear_acc(dref(), blk(K_CLEAR_ACC), stream));             // :920
   if (any_fluid_) {  // DFSPHSolver.substep, :1546-1555
-    TIMED(K_DENSITY_ALPHA, launch_density_alpha(dref(), blk(K_DENSITY_ALPHA), dep(K_DENSITY_ALPHA), stream));
+    TIMED(K_DENSITY_ALPHA, launch_density_alpha(dref(), blk(K_DENSITY_ALPHA), lanes(K_DENSITY_ALPHA), dep(K_DENSITY_ALPHA), stream));
     if (any_div_) {
       launch_solver_begin(dref(), 0, stream);
       CHK(solver_loop(0));
     }
-    if (any_strain_) TIMED(K_STRAIN, launch_strain(dref(), blk(K_STRAIN), dep(K_STRAIN), stream));
+    if (any_strain_) TIMED(K_STRAIN, launch_strain(dref(), blk(K_STRAIN), lanes(K_STRAIN), dep(K_STRAIN), stream));
     if (any_weiler_) {
       launch_solver_begin(dref(), 2, stream);
       TIMED(K_CG_INIT, launch_cg_init(dref(), blk(K_CG_INIT), stream));
-      if (any_warm_cg_) launch_scene_finish(dref(), 4, stream);
+      if (any_warm_cg_) launch_scene_finish(dref(), 4, 1, stream);
       TIMED(K_CG_GUESS, launch_cg_guess(dref(), blk(K_CG_GUESS), stream));
       TIMED(K_CG_MATVEC, launch_cg_matvec(dref(), blk(K_CG_MATVEC), dep(K_CG_MATVEC), 1, stream));
-      launch_scene_finish(dref(), 2, stream);
+      launch_scene_finish(dref(), 2, 1, stream);
       CHK(cg_loop());
     }
-    TIMED(K_NONPRESSURE, launch_nonpressure(dref(), blk(K_NONPRESSURE), dep(K_NONPRESSURE), stream));
+    TIMED(K_NONPRESSURE, launch_nonpressure(dref(), blk(K_NONPRESSURE), lanes(K_NONPRESSURE), dep(K_NONPRESSURE), stream));
     std::swap(d.vel, d.vel_alt);
     launch_solver_begin(dref(), 1, stream);
-    TIMED(K_PRESS_SOURCE, launch_press_source(dref(), blk(K_PRESS_SOURCE), dep(K_PRESS_SOURCE), 0, stream));
+    TIMED(K_PRESS_SOURCE, launch_press_source(dref(), blk(K_PRESS_SOURCE), lanes(K_PRESS_SOURCE), dep(K_PRESS_SOURCE), 0, stream));
     CHK(solver_loop(1));
   }
   if (any_elastic_) {  // Elasticity.substep, :1241-1244
@@ -1072,8 +1097,11 @@ int Batch::step(std::vector<nn_step_stats>* stats) {
   if (any_rigid_) CHK(rigid_step());  // :929-931
   TIMED(K_ADVECT, launch_advect(dref(), blk(K_ADVECT), stream));  // :933, :936-937
   std::swap(d.pos, d.pos_alt);  // pos_alt keeps the positions of this step's search
+  SceneState* pub = nullptr;
+  HIPCHK(hipHostGetDevicePointer((void**)&pub, h_state_, 0));
+  launch_publish(dref(), lanes(K_BUILD_LISTS), lanes(K_DENSITY_ALPHA), pub, stream);
   HIPCHK(hipGetLastError());
-  CHK(gather_state());
+  HIPCHK(hipStreamSynchronize(stream));
   CHK(timer.collect());
   int rc = NN_OK;
   if (stats) stats->resize(scenes.size());
@@ -1323,7 +1351,7 @@ int Batch::complete_lists() {
   if (lists_state_ == 0) return search_impl(1);  // laid out since: search the current positions
   Dev at_search = d;
   at_search.pos = d.pos_alt;
-  launch_build_lists(DevRef{at_search}, blk(K_BUILD_LISTS), 1, stream);
+  launch_build_lists(DevRef{at_search}, blk(K_BUILD_LISTS), lanes(K_BUILD_LISTS), 1, stream);
   HIPCHK(hipGetLastError());
   lists_state_ = 2;
   return NN_OK;

@@ -72,49 +72,219 @@ __device__ __forceinline__ float3 kern_grad(float h, float kG, float rx, float r
 // spair): groups of four positions, one int4 per particle and group.
 __device__ __forceinline__ long nb_word(long P, int i, int k) { return 4 * ((long)(k >> 2) * P + i) + (k & 3); }
 
-// Walk the neighbor list of particle i in list order, B entries at a time
-// (B a multiple of 4): the B list words are loaded together (B / 4 int4
-// groups), then the B neighbors' data (load(j)), and only then body(j, data)
-// runs for each in order.  The loads of a batch are independent, so a
-// wavefront has B gathers in flight instead of one; the order of the
-// per-neighbor terms (and so every sum) is unchanged.  Lanes past the end of
-// their list load their own particle's data and skip the body.
-template <int B, typename Load, typename Body>
-__device__ __forceinline__ void for_neighbors(const Dev& d, int i, int cnt, Load load, Body body) {
-  static_assert(B % 4 == 0, "whole groups of four list positions");
-  using T = decltype(load(0));
-  const long P = d.P;
-  const int4* groups = reinterpret_cast<const int4*>(d.nbr);
-  for (int k0 = 0; k0 < cnt; k0 += B) {
-    int j[B];
-    T v[B];
+// ---------------------------------------------------------------------------
+// The same roundings with fewer instructions.  hipcc's FP32 square root and
+// division are correctly rounded over the whole range; what they spend on
+// scaling (operands near overflow or underflow) a pair of particles never
+// needs.  Where a scene's h lies in [2^-20, 2^20] (SF_MIDRANGE) and a pair's
+// squared distance is above 1e-10 with no component in (0, 2^-100), the
+// sequences below give the same bits:
+//   sqrt_mid   v_sqrt_f32 (1 ulp), then the neighbor whose FMA residual shows
+//              it nearer
+//   recip_mid  v_rcp_f32 and one Newton step, shared by every quotient of one
+//              denominator
+//   div_mid    a y, then two residual corrections q + (a - b q) y (Markstein,
+//              IBM J. R&D 34, 1990); -0 / b comes out as +0, which only a sum
+//              that may itself be -0 can tell (pair_grad's SIGNED)
+// A gradient has one square root and four quotients of two denominators (h
+// and r h), about half of its instructions.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ float sqrt_mid(float x) {
+  const float s = __builtin_amdgcn_sqrtf(x);
+  const float dn = __int_as_float(__float_as_int(s) - 1), up = __int_as_float(__float_as_int(s) + 1);
+  const float rd = __builtin_fmaf(-dn, s, x), ru = __builtin_fmaf(-up, s, x);
+  float r = rd <= 0.0f ? dn : s;
+  r = ru > 0.0f ? up : r;
+  return r;
+}
+__device__ __forceinline__ float recip_mid(float b) {
+  const float y = __builtin_amdgcn_rcpf(b);
+  return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+__device__ __forceinline__ float div_mid(float a, float b, float y) {
+  float q = a * y;
+  q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+// some component nonzero and below 2^-100 in magnitude
+__device__ __forceinline__ bool any_tiny(float x, float y, float z) {
+  const unsigned tx = (__float_as_uint(x) << 1) - 1u, ty = (__float_as_uint(y) << 1) - 1u, tz = (__float_as_uint(z) << 1) - 1u;
+  return min(tx, min(ty, tz)) < (27u << 24) - 1u;  // 2^-100 has biased exponent 27
+}
+
+// The kernel's radius in the form the pairs use.
+struct KernH {
+  float h, yh;
+  bool mid;
+  __device__ __forceinline__ explicit KernH(const SceneDev& sc)
+      : h(sc.h), yh(recip_mid(sc.h)), mid((sc.flags & SF_MIDRANGE) != 0) {}
+};
+
+// kern_w and kern_grad's radial factor at q = |r| / h <= 1, both branches
+// formed and one selected
+__device__ __forceinline__ float w_of(float kW, float q) {
+  const float q2 = q * q, q3 = q2 * q, t = 1.0f - q;
+  const float in = kW * (6.0f * q3 - 6.0f * q2 + 1.0f), out = (kW * 2.0f) * (t * t * t);
+  const float w = q <= 0.5f ? in : out;
+  return q <= 1.0f ? w : 0.0f;
+}
+__device__ __forceinline__ float radial_of(float kG, float q) {
+  const float fa = 1.0f - q;
+  const float in = (kG * q) * (3.0f * q - 2.0f), out = kG * ((-fa) * fa);
+  const float f = q <= 0.5f ? in : out;
+  return q <= 1.0f ? f : 0.0f;
+}
+
+// One pair's |r| and gradient (kern_grad), and W (kern_w) where asked for;
+// `live` lanes get kern_grad's and kern_w's bits, others anything.  Without
+// SIGNED a zero component may have the other sign.
+template <bool WANT_W, bool SIGNED>
+__device__ __forceinline__ float3 pair_grad(const KernH& k, const SceneDev& sc, float rx, float ry, float rz, bool live,
+                                            float& rn, float& w) {
+  const float ss = rx * rx + ry * ry + rz * rz;
+  rn = sqrt_mid(ss);
+  const float q = div_mid(rn, k.h, k.yh);
+  const float den = rn * k.h;
+  const float y = recip_mid(den);
+  const float f = radial_of(sc.kG, q);
+  float ux = div_mid(rx, den, y), uy = div_mid(ry, den, y), uz = div_mid(rz, den, y);
+  if (SIGNED) {
+    ux = __builtin_copysignf(ux, rx);
+    uy = __builtin_copysignf(uy, ry);
+    uz = __builtin_copysignf(uz, rz);
+  }
+  float3 g = make_float3(f * ux, f * uy, f * uz);
+  if (WANT_W) w = w_of(sc.kW, q);
+  // 1e-10 < ss: |r| > 1e-5, so the gradient's own cut-off needs no test here;
+  // a pair past q = 1 (|r| rounds below h and |r| / h above 1) takes the plain form
+  if (__builtin_expect(live && (!k.mid || !(ss > 1.01e-10f) || !(q <= 1.0f) || any_tiny(rx, ry, rz)), 0)) {
+    rn = norm3(rx, ry, rz);
+    g = kern_grad(sc.h, sc.kG, rx, ry, rz, rn);
+    if (WANT_W) w = kern_w(sc.h, sc.kW, rn);
+  }
+  return g;
+}
+template <bool SIGNED = false>
+__device__ __forceinline__ float3 pair_grad(const KernH& k, const SceneDev& sc, float rx, float ry, float rz, bool live) {
+  float rn, w;
+  return pair_grad<false, SIGNED>(k, sc, rx, ry, rz, live, rn, w);
+}
+// W of one pair alone (kern_w of norm3)
+__device__ __forceinline__ float pair_w(const KernH& k, const SceneDev& sc, float rx, float ry, float rz, bool live) {
+  const float ss = rx * rx + ry * ry + rz * rz;
+  float w = w_of(sc.kW, div_mid(sqrt_mid(ss), k.h, k.yh));
+  if (__builtin_expect(live && (!k.mid || !(ss > 1.01e-10f)), 0)) w = kern_w(sc.h, sc.kW, norm3(rx, ry, rz));
+  return w;
+}
+
+// ---------------------------------------------------------------------------
+// Sweeps over a particle's list with G lanes per particle (1, 4 or 16, equal
+// to lane groups that DPP can broadcast in).  Lane q takes list positions q,
+// q + G, ...; each lane forms its own pair's terms and the group adds them in
+// list order, every lane reading the owning lane's term, so the sums are the
+// serial ones bit for bit whatever G is.
+// ---------------------------------------------------------------------------
+template <int G, int U>
+__device__ __forceinline__ float lane_bcast(float v) {
+  static_assert(G == 1 || G == 4 || G == 16, "lane groups");
+  if constexpr (G == 1) return v;
+  else if constexpr (G == 4)  // quad_perm [U, U, U, U]
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), U * 0x55, 0xf, 0xf, true));
+  else  // row_newbcast:U
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + U, 0xf, 0xf, true));
+}
+
+template <int G>
+__device__ __forceinline__ bool lane_slot_scene(const Dev& d, int& i, int& q, int& s) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  i = t / G;
+  q = t % G;
+  const int w = uniform(i >> 6);
+  if (w >= d.W) return false;
+  s = uniform(d.wave_scene[w]);
+  return s >= 0;
+}
+
+// x + NEUTRAL == x for every x, signed zeros included: what a lane without a
+// term contributes
+constexpr float NEUTRAL = -0.0f;
+
+template <int G, int N, int U, typename Add>
+__device__ __forceinline__ void add_in_order(const float (&t)[N], int left, Add& add) {
+  if constexpr (U < G) {
+    float b[N];
 #pragma unroll
-    for (int g = 0; g < B / 4; g++) {
-      const int k = k0 + 4 * g;
-      const int4 w = k < cnt ? groups[(long)(k >> 2) * P + i] : make_int4(i, i, i, i);
-      j[4 * g + 0] = w.x;
-      j[4 * g + 1] = k + 1 < cnt ? w.y : i;
-      j[4 * g + 2] = k + 2 < cnt ? w.z : i;
-      j[4 * g + 3] = k + 3 < cnt ? w.w : i;
-    }
-#pragma unroll
-    for (int u = 0; u < B; u++) v[u] = load(j[u]);
-#pragma unroll
-    for (int u = 0; u < B; u++)
-      if (k0 + u < cnt) body(j[u], v[u]);
+    for (int n = 0; n < N; n++) b[n] = lane_bcast<G, U>(t[n]);
+    add(b, U < left);
+    add_in_order<G, N, U + 1>(t, left, add);
   }
 }
 
-// Launch a sweep templated on its batch size B of for_neighbors (4, 8 or 16;
-// anything else is the default 8).  B changes how many gathers are in flight,
-// not the order of any sum.
-#define DEPTH_LAUNCH(kern, depth, grid, blk, st, ...)                          \
-  do {                                                                        \
-    switch (depth) {                                                          \
-      case 4: NN_LAUNCH(kern<4>, grid, blk, 0, st, __VA_ARGS__); break;        \
-      case 16: NN_LAUNCH(kern<16>, grid, blk, 0, st, __VA_ARGS__); break;      \
-      default: NN_LAUNCH(kern<8>, grid, blk, 0, st, __VA_ARGS__); break;       \
-    }                                                                         \
+// B positions per lane and batch: their list words are loaded together, then
+// the neighbors' data (load(j)), then term(j, data, live, t) forms the N terms
+// of each (a lane past the end of the list loads its own particle and is not
+// live) and add(t, ok) is called for every position in list order.
+template <int G, int B, int N, typename Load, typename Term, typename Add>
+__device__ __forceinline__ void for_pairs(const Dev& d, int i, int q, int cnt, Load load, Term term, Add add) {
+  using T = decltype(load(0));
+  const long P = d.P;
+  for (int k0 = 0; k0 < cnt; k0 += G * B) {
+    int j[B];
+    T v[B];
+    if constexpr (G == 1) {
+      static_assert(B % 4 == 0, "whole groups of four list positions");
+      const int4* groups = reinterpret_cast<const int4*>(d.nbr);
+#pragma unroll
+      for (int g = 0; g < B / 4; g++) {
+        const int k = k0 + 4 * g;
+        const int4 w = k < cnt ? groups[(long)(k >> 2) * P + i] : make_int4(i, i, i, i);
+        j[4 * g + 0] = w.x;
+        j[4 * g + 1] = k + 1 < cnt ? w.y : i;
+        j[4 * g + 2] = k + 2 < cnt ? w.z : i;
+        j[4 * g + 3] = k + 3 < cnt ? w.w : i;
+      }
+    } else {
+#pragma unroll
+      for (int b = 0; b < B; b++) {
+        const int k = k0 + b * G + q;
+        j[b] = k < cnt ? d.nbr[nb_word(P, i, k)] : i;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < B; b++) v[b] = load(j[b]);
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      const int left = cnt - (k0 + b * G);
+      if (left > 0) {
+        float t[N];
+        term(j[b], v[b], q < left, t);
+        add_in_order<G, N, 0>(t, left, add);
+      }
+    }
+  }
+}
+
+// Launch a sweep templated on its lanes per particle and positions per lane and
+// batch.  `depth` (4, 8 or 16; anything else is the default 8) is the list
+// positions a particle has in flight per batch, at least one per lane.  Neither
+// changes the order of a sum.
+#define SWEEP_LAUNCH_4(kern, lanes, depth, slots, block, st, ...)                                   \
+  do {                                                                                             \
+    const dim3 _g((unsigned)(((long)(slots) * (lanes) + (block) - 1) / (block))), _b(block);       \
+    switch ((lanes) * 100 + ((depth) == 4 || (depth) == 16 ? (depth) : 8)) {                       \
+      case 404: NN_LAUNCH((kern<4, 1>), _g, _b, 0, st, __VA_ARGS__); break;                        \
+      case 408: NN_LAUNCH((kern<4, 2>), _g, _b, 0, st, __VA_ARGS__); break;                        \
+      case 416: NN_LAUNCH((kern<4, 4>), _g, _b, 0, st, __VA_ARGS__); break;                        \
+      default: NN_LAUNCH((kern<16, 2>), _g, _b, 0, st, __VA_ARGS__); break;                        \
+    }                                                                                              \
+  } while (0)
+#define SWEEP_LAUNCH(kern, lanes, depth, slots, block, st, ...)                                     \
+  do {                                                                                             \
+    const dim3 _g1((unsigned)(((long)(slots) + (block) - 1) / (block))), _b1(block);               \
+    if ((lanes) != 1) SWEEP_LAUNCH_4(kern, lanes, depth, slots, block, st, __VA_ARGS__);           \
+    else if ((depth) == 4) NN_LAUNCH((kern<1, 4>), _g1, _b1, 0, st, __VA_ARGS__);                  \
+    else if ((depth) == 16) NN_LAUNCH((kern<1, 16>), _g1, _b1, 0, st, __VA_ARGS__);                \
+    else NN_LAUNCH((kern<1, 8>), _g1, _b1, 0, st, __VA_ARGS__);                                    \
   } while (0)
 
 struct PosVel {
@@ -143,6 +313,16 @@ struct KSum {
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// The same over values held once per G lanes, neighbors first: partials of
+// fewer particles (sweeps with several lanes per particle) combine further by
+// the same tree, so the sum over 64 particles has the same bits for every G.
+template <int G>
+__device__ __forceinline__ double tree_sum(double v) {
+#pragma unroll
+  for (int off = G; off <= 32; off <<= 1) v += __shfl_xor(v, off, 64);
   return v;
 }
 

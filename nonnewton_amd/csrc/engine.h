@@ -67,7 +67,8 @@ enum {
   SF_HAS_FLUID = 64,
   SF_HAS_ELASTIC = 128,
   SF_WARM_CG = 256,  // Weiler CG starts from v + (x - v) of the previous solve
-  SF_HAS_RIGID = 512
+  SF_HAS_RIGID = 512,
+  SF_MIDRANGE = 1024  // h within [2^-20, 2^20]: sqrt_mid and div_mid hold for its pairs
 };
 
 // Per-scene constants (device table).  Floats are the reference's FP32
@@ -111,7 +112,7 @@ struct SceneState {
   // the scene's first workgroup of that update
   int active_v, active_p, active_cg, cg_stop_at;
   int iter_v, iter_p, iter_cg, status;
-  unsigned counter, max_rho_bits;
+  unsigned max_rho_bits, pad_u;  // max_rho_bits, pairs and pairs_fluid: set by k_publish in the host copy
   unsigned long long pairs, pairs_fluid;
   double err_v, err_p;
   double cg_bb, cg_rr, cg_theta, pad_d;
@@ -167,6 +168,8 @@ struct Dev {
   int* cell_start;
   int* scan_tmp;
   double* partials;  // 8 arrays of 4W: wave partials (per 64 particles, or per 16 for four-lane sweeps)
+  int2* wave_pairs;  // list entries of a wavefront's particles: (of fluid and dynamic solids, of fluid)
+  float* wave_rho;   // largest density of a wavefront's particles; both one entry per lane of a particle and 64 slots
   const int2* cg_blocks;  // CG update workgroups: (scene, first wave), up to CG_UPD_WAVES waves of one scene each
   int* cg_list;           // 2 x W: waves of the scenes still iterating, by iteration parity
   int* cg_list_n;         // 2 counts
@@ -253,22 +256,22 @@ constexpr int SCAN_TILE_ITEMS = 2048;
 void launch_cell_count(const DevRef& d, int block, hipStream_t st);
 void launch_bucket(const DevRef& d, int block, hipStream_t st);
 void launch_place(const DevRef& d, int block, hipStream_t st);
-void launch_build_lists(const DevRef& d, int block, int all, hipStream_t st);  // all = 0: no static lists
-void launch_bvol(const DevRef& d, int block, int dynamic, hipStream_t st);
+void launch_build_lists(const DevRef& d, int block, int lanes, int all, hipStream_t st);  // all = 0: no static lists
+void launch_bvol(const DevRef& d, int block, int lanes, int dynamic, hipStream_t st);
 
-void launch_density_alpha(const DevRef& d, int block, int depth, hipStream_t st);
-void launch_div_update(const DevRef& d, int block, int depth, hipStream_t st);
-void launch_div_source(const DevRef& d, int block, int depth, hipStream_t st);
+void launch_density_alpha(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
+void launch_div_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
+void launch_div_source(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_solver_begin(const DevRef& d, int which, hipStream_t st);
-void launch_strain(const DevRef& d, int block, int depth, hipStream_t st);
+void launch_strain(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_cg_init(const DevRef& d, int block, hipStream_t st);
 void launch_cg_guess(const DevRef& d, int block, hipStream_t st);
 void launch_cg_matvec(const DevRef& d, int block, int depth, int start, hipStream_t st);  // depth 1, 2, 4, 8
 void launch_cg_matvec_list(const DevRef& d, int depth, int k, int grid, hipStream_t st);  // iteration k
 void launch_cg_update(const DevRef& d, int nblocks, int k, hipStream_t st);  // iteration k >= 1
-void launch_nonpressure(const DevRef& d, int block, int depth, hipStream_t st);
-void launch_press_source(const DevRef& d, int block, int depth, int reduce, hipStream_t st);
-void launch_press_update(const DevRef& d, int block, int depth, hipStream_t st);
+void launch_nonpressure(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
+void launch_press_source(const DevRef& d, int block, int lanes, int depth, int reduce, hipStream_t st);
+void launch_press_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_clear_acc(const DevRef& d, int block, hipStream_t st);
 void launch_elastic_init(const DevRef& d, int block, hipStream_t st);
 void launch_elastic_rot_stress(const DevRef& d, int block, hipStream_t st);
@@ -281,6 +284,7 @@ void launch_body_finish(const DevRef& d, int pass, int r, int c, hipStream_t st)
 void launch_rigid_place(const DevRef& d, int r, int c, hipStream_t st);
 void launch_advect(const DevRef& d, int block, hipStream_t st);
 void launch_step_begin(const DevRef& d, hipStream_t st);
-void launch_scene_finish(const DevRef& d, int which, hipStream_t st);  // 0 div, 1 press, 2 cg start, 3 cg iteration, 4 cg guess scale
+void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* host, hipStream_t st);
+void launch_scene_finish(const DevRef& d, int which, int lanes, hipStream_t st);  // 0 div, 1 press, 2 cg start, 3 cg iteration, 4 cg guess scale
 
 }  // namespace nn

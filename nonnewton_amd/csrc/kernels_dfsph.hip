@@ -1,12 +1,12 @@
 // kernels_dfsph.hip -- DFSPH sweeps over the cell-sorted particles
 // (DFSPHSolver, SPH/main.py:1519-1848; SPHBase, :908-1093).
 //
-// One lane per particle; each lane walks its neighbor list in list order, so
-// every per-particle sum is formed in the reference's serial order.  Solver
-// iterations never return to the host: the source sweeps reduce the average
-// density error per scene in FP64 (scene_reduce) and the last wavefront of a
-// scene decides termination, clearing the scene's active flag; later launches
-// of a finished scene return at once.
+// 1, 4 or 16 lanes per particle (Batch::lanes) share its neighbor list and add
+// their terms in list order (for_pairs), so every per-particle sum is formed in
+// the reference's serial order.  The source sweeps leave FP64 partials of the
+// average density error per scene; k_scene_finish adds them and decides
+// termination, clearing the scene's active flag; later launches of a finished
+// scene return at once.
 #include "device_common.h"
 
 namespace nn {
@@ -21,10 +21,6 @@ __device__ __forceinline__ float alpha_press(const SceneDev& sc, float a) {
 __global__ void k_step_begin(Dev d) {
   for (int s = threadIdx.x; s < d.nscenes; s += blockDim.x) {
     d.state[s].status = 0;
-    d.state[s].max_rho_bits = 0u;
-    d.state[s].counter = 0u;
-    d.state[s].pairs = 0ull;
-    d.state[s].pairs_fluid = 0ull;
   }
 }
 
@@ -41,53 +37,110 @@ __global__ void k_clear_acc(Dev d) {
 // compute_densities (:962-984), compute_DFSPH_factor (:1569-1608) and the first
 // compute_density_change of the divergence solve (:1610-1645), fused: all three
 // read the same neighbors and none reads what another writes.
-template <int B>
+template <int G, int B>
 __global__ void k_density_alpha(Dev d) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (!(sc.flags & SF_HAS_FLUID)) return;
   float rho_out = 0.0f;
   if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
+    const KernH kh(sc);
     const float4 xi = d.pos[i];
     const float4 vi = d.vel[i];
     const int cnt = d.nnbr[i];
     const bool comp = (sc.flags & SF_COMPENSATED) != 0;
     KSum den{0.0f, 0.0f};
-    float denp = 0.0f;
     float gix = 0.f, giy = 0.f, giz = 0.f, sk = 0.f, rd = 0.f;
-    for_neighbors<B>(
-        d, i, cnt, [&](int j) { return PosVel{d.pos[j], d.vel[j]}; },
-        [&](int, const PosVel& nj) {
+    for_pairs<G, B, 6>(
+        d, i, q, cnt, [&](int j) { return PosVel{d.pos[j], d.vel[j]}; },
+        [&](int, const PosVel& nj, bool live, float (&t)[6]) {
           const float4 xj = nj.x, vj = nj.v;
           const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-          const float rn = norm3(rx, ry, rz);
           const float Vj = fabsf(xj.w);
-          const float t = Vj * kern_w(sc.h, sc.kW, rn);
-          if (comp) den.add(t);
-          else denp += t;
-          const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, rn);
+          float rn, w;
+          const float3 g = pair_grad<true, false>(kh, sc, rx, ry, rz, live, rn, w);
           const float gpx = -Vj * g.x, gpy = -Vj * g.y, gpz = -Vj * g.z;
-          if (xj.w > 0.0f) sk += gpx * gpx + gpy * gpy + gpz * gpz;
-          gix -= gpx;
-          giy -= gpy;
-          giz -= gpz;
           const float dvx = vi.x - vj.x, dvy = vi.y - vj.y, dvz = vi.z - vj.z;
-          rd += Vj * (dvx * g.x + dvy * g.y + dvz * g.z);
+          t[0] = Vj * w;
+          t[1] = live && xj.w > 0.0f ? gpx * gpx + gpy * gpy + gpz * gpz : NEUTRAL;
+          t[2] = live ? -gpx : NEUTRAL;
+          t[3] = live ? -gpy : NEUTRAL;
+          t[4] = live ? -gpz : NEUTRAL;
+          t[5] = live ? Vj * (dvx * g.x + dvy * g.y + dvz * g.z) : NEUTRAL;
+        },
+        [&](const float (&t)[6], bool ok) {
+          KSum n = den;
+          if (comp) n.add(t[0]);
+          else n.s += t[0];
+          den.s = ok ? n.s : den.s;
+          den.c = ok ? n.c : den.c;
+          sk += t[1];
+          gix += t[2];
+          giy += t[3];
+          giz += t[4];
+          rd += t[5];
         });
     float rho = xi.w * sc.W0;
-    rho += comp ? den.s : denp;
+    rho += den.s;
     rho *= sc.rho0;
-    d.rho[i] = rho;
     rho_out = rho;
     sk += gix * gix + giy * giy + giz * giz;
     const float al = sk > 1e-6f ? -1.0f / sk : 0.0f;
     rd = rd > 0.0f ? rd : 0.0f;
     if (cnt < 20) rd = 0.0f;
-    d.sa[i] = make_float2(rd, al);
+    if (q == 0) {
+      d.rho[i] = rho;
+      d.sa[i] = make_float2(rd, al);
+    }
   }
   const float m = wave_max(rho_out);
-  if ((threadIdx.x & 63) == 0 && m > 0.0f) atomicMax(&d.state[s].max_rho_bits, __float_as_uint(m));
+  if ((threadIdx.x & 63) == 0) d.wave_rho[i / (64 / G)] = m;
+}
+
+// End of a step: per scene, the pair counts and the largest density of its
+// wavefronts (list_lanes and rho_lanes entries per 64 slots), then its state
+// into the host's pinned copy.  (With an atomic per wavefront on the scene's
+// words, the density sweep of 131,072 particles took 45 us instead of 22: each
+// atomic of one address costs about 13 ns.)
+constexpr int PUBLISH_THREADS = 256;
+__global__ __launch_bounds__(PUBLISH_THREADS) void k_publish(Dev d, int list_lanes, int rho_lanes, SceneState* host) {
+  __shared__ long long red[2][PUBLISH_THREADS / 64];
+  __shared__ float rmax[PUBLISH_THREADS / 64];
+  const int s = blockIdx.x, t = threadIdx.x;
+  const SceneDev& sc = d.scenes[s];
+  long long tot = 0, cf = 0;
+  float m = 0.0f;
+  for (int k = list_lanes * sc.wave_begin + t; k < list_lanes * sc.wave_end; k += PUBLISH_THREADS) {
+    const int2 c = d.wave_pairs[k];
+    tot += c.x;
+    cf += c.y;
+  }
+  if (sc.flags & SF_HAS_FLUID)
+    for (int k = rho_lanes * sc.wave_begin + t; k < rho_lanes * sc.wave_end; k += PUBLISH_THREADS) m = fmaxf(m, d.wave_rho[k]);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    tot += __shfl_xor(tot, off, 64);
+    cf += __shfl_xor(cf, off, 64);
+  }
+  m = wave_max(m);
+  if ((t & 63) == 0) {
+    red[0][t >> 6] = tot;
+    red[1][t >> 6] = cf;
+    rmax[t >> 6] = m;
+  }
+  __syncthreads();
+  if (t != 0) return;
+  SceneState st = d.state[s];
+  st.pairs = st.pairs_fluid = 0ull;
+  m = 0.0f;
+  for (int w = 0; w < PUBLISH_THREADS / 64; w++) {
+    st.pairs += (unsigned long long)red[0][w];
+    st.pairs_fluid += (unsigned long long)red[1][w];
+    m = fmaxf(m, rmax[w]);
+  }
+  st.max_rho_bits = __float_as_uint(m);
+  host[s] = st;
 }
 
 // which: 0 divergence, 1 pressure, 2 cg (cg_init activates scenes)
@@ -117,54 +170,72 @@ __global__ void k_solver_begin(Dev d, int which) {
       st.cg_bb = 0.0;
       if (s == 0) d.cg_list_n[0] = d.cg_list_n[1] = 0;
     }
-    st.counter = 0u;
     if (act) atomicAdd(&cnt, 1);
   }
   __syncthreads();
   if (threadIdx.x == 0) d.n_active[which] = cnt;
 }
 
+// sum_j of the velocity changes both solvers' updates make (:1721-1760,
+// :1799-1841): dt (k_i + k_j) V_j gradW_ij for a fluid neighbor, dt k_i V_j
+// gradW_ij for a solid one, each where the factor exceeds eps; kj(nj) is the
+// neighbor's factor.  SIGNED where the sums start at a velocity, which may be
+// -0, and not at +0.
+template <int G, int B, bool SIGNED, typename KJ>
+__device__ __forceinline__ void velocity_push(const Dev& d, const SceneDev& sc, const KernH& kh, int i, int q, int cnt,
+                                              float4 xi, float ki, KJ kj, float& ax, float& ay, float& az) {
+  const bool solid_on = fabsf(ki) > sc.eps;
+  for_pairs<G, B, 3>(
+      d, i, q, cnt, [&](int j) { const float2 t = d.sa[j]; return PosSrc{d.pos[j], t.x, t.y}; },
+      [&](int, const PosSrc& nj, bool live, float (&t)[3]) {
+        const float4 xj = nj.x;
+        const bool fluid = xj.w > 0.0f;
+        const float ksum = ki + kj(nj);
+        const bool on = live && (fluid ? fabsf(ksum) > sc.eps : solid_on);
+        t[0] = t[1] = t[2] = NEUTRAL;
+        if (on) {
+          const float3 g = pair_grad<SIGNED>(kh, sc, xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, true);
+          // v -= f (-V g) with f = dt ksum, v += f (-V g) with f = -dt ki
+          const float f = fluid ? -(sc.dt * ksum) : -sc.dt * ki;
+          const float Vj = fabsf(xj.w);
+          t[0] = f * (-Vj * g.x);
+          t[1] = f * (-Vj * g.y);
+          t[2] = f * (-Vj * g.z);
+        }
+      },
+      [&](const float (&t)[3], bool) {
+        ax += t[0];
+        ay += t[1];
+        az += t[2];
+      });
+}
+
+// One value per particle (held by its G lanes) summed over the particles of a
+// wavefront into partial array 0, entry G w + ... of 64-particle wave w.
+template <int G>
+__device__ __forceinline__ void lane_partial(const Dev& d, int i, double v) {
+  v = tree_sum<G>(v);
+  if ((threadIdx.x & 63) == 0) d.partials[i / (64 / G)] = v;
+}
+
 // divergence_solver_iteration_kernel, :1721-1760 (Jacobi: reads rho-dot and
 // alpha, writes v).  Reactions on dynamic solids are not formed: the second
 // clear_accelerations (:1552) erases them.
-template <int B>
+template <int G, int B>
 __global__ void k_div_update(Dev d) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (!d.state[s].active_v) return;
   if (i >= sc.p_begin + sc.n || kind_of(d.info[i]) != KIND_FLUID) return;
+  const KernH kh(sc);
   const float4 xi = d.pos[i];
   const float2 sai = d.sa[i];
   const float ki = sai.x * alpha_div(sc, sai.y);
-  const int cnt = d.nnbr[i];
   float dvx = 0.f, dvy = 0.f, dvz = 0.f;
-  for_neighbors<B>(
-      d, i, cnt, [&](int j) { const float2 t = d.sa[j]; return PosSrc{d.pos[j], t.x, t.y}; },
-      [&](int, const PosSrc& nj) {
-        const float4 xj = nj.x;
-        if (xj.w > 0.0f) {
-          const float kj = nj.src * alpha_div(sc, nj.alpha);
-          const float ksum = ki + kj;
-          if (fabsf(ksum) > sc.eps) {
-            const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-            const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, norm3(rx, ry, rz));
-            const float f = sc.dt * ksum;
-            const float Vj = xj.w;
-            dvx -= f * (-Vj * g.x);
-            dvy -= f * (-Vj * g.y);
-            dvz -= f * (-Vj * g.z);
-          }
-        } else if (fabsf(ki) > sc.eps) {
-          const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-          const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, norm3(rx, ry, rz));
-          const float f = -sc.dt * ki;
-          const float Vj = -xj.w;
-          dvx += f * (-Vj * g.x);
-          dvy += f * (-Vj * g.y);
-          dvz += f * (-Vj * g.z);
-        }
-      });
+  velocity_push<G, B, false>(d, sc, kh, i, q, d.nnbr[i], xi, ki, [&](const PosSrc& nj) { return nj.src * alpha_div(sc, nj.alpha); },
+                      dvx, dvy, dvz);
+  if (q != 0) return;
   float4 v = d.vel[i];
   v.x += dvx;
   v.y += dvy;
@@ -173,42 +244,43 @@ __global__ void k_div_update(Dev d) {
 }
 
 // sum_j V_j (v_i - v_j) . gradW_ij over all neighbors, and the count
-template <int B>
-__device__ __forceinline__ float velocity_divergence(const Dev& d, const SceneDev& sc, int i, float4 xi, int& cnt) {
+template <int G, int B>
+__device__ __forceinline__ float velocity_divergence(const Dev& d, const SceneDev& sc, int i, int q, float4 xi, int& cnt) {
+  const KernH kh(sc);
   const float4 vi = d.vel[i];
   cnt = d.nnbr[i];
   float acc = 0.f;
-  for_neighbors<B>(
-      d, i, cnt, [&](int j) { return PosVel{d.pos[j], d.vel[j]}; },
-      [&](int, const PosVel& nj) {
+  for_pairs<G, B, 1>(
+      d, i, q, cnt, [&](int j) { return PosVel{d.pos[j], d.vel[j]}; },
+      [&](int, const PosVel& nj, bool live, float (&t)[1]) {
         const float4 xj = nj.x, vj = nj.v;
-        const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-        const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, norm3(rx, ry, rz));
+        const float3 g = pair_grad(kh, sc, xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, live);
         const float dvx = vi.x - vj.x, dvy = vi.y - vj.y, dvz = vi.z - vj.z;
-        acc += fabsf(xj.w) * (dvx * g.x + dvy * g.y + dvz * g.z);
-      });
+        t[0] = live ? fabsf(xj.w) * (dvx * g.x + dvy * g.y + dvz * g.z) : NEUTRAL;
+      },
+      [&](const float (&t)[1], bool) { acc += t[0]; });
   return acc;
 }
 
 // compute_density_change (:1610-1645) + compute_density_error(0) (:1669-1675)
 // and the loop test of divergence_solve (:1695-1703)
-template <int B>
+template <int G, int B>
 __global__ void k_div_source(Dev d) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   SceneState* st = d.state + s;
   if (!st->active_v) return;
-  double v[1] = {0.0};
+  double v = 0.0;
   if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
     int cnt;
-    float rd = velocity_divergence<B>(d, sc, i, d.pos[i], cnt);
+    float rd = velocity_divergence<G, B>(d, sc, i, q, d.pos[i], cnt);
     rd = rd > 0.0f ? rd : 0.0f;
     if (cnt < 20) rd = 0.0f;
-    d.sa[i].x = rd;
-    v[0] = (double)sc.rho0 * (double)rd - 0.0;
+    if (q == 0) d.sa[i].x = rd;
+    v = (double)sc.rho0 * (double)rd - 0.0;
   }
-  wave_partials<1>(d, (int)(i >> 6), v);
+  lane_partial<G>(d, i, v);
 }
 
 // non-pressure forces (:1557-1567): surface tension (:1378-1414) and the
@@ -216,73 +288,92 @@ __global__ void k_div_source(Dev d) {
 // the implicit solver ran, then non_pressure_advect (:1843-1848).  The second
 // clear_accelerations (:1552) is folded in.  v is double-buffered: the sweep
 // reads vel and writes vel_alt.
-template <int B>
+template <int G, int B>
 __global__ void k_nonpressure(Dev d) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (i >= sc.p_begin + sc.n) return;
   const int kind = kind_of(d.info[i]);
   const float4 vi = d.vel[i];
   if (!(sc.flags & SF_HAS_FLUID)) {
-    d.vel_alt[i] = vi;
+    if (q == 0) d.vel_alt[i] = vi;
     return;
   }
-  const int P = d.P;
   const bool vis_on = (sc.flags & SF_VISCOSITY) != 0;
   const bool weiler = vis_on && (sc.flags & SF_WEILER);
   const bool expl = vis_on && !weiler;
   const bool bnu_on = vis_on && sc.bnu != 0.0f;
   if (kind == KIND_FLUID) {
+    const KernH kh(sc);
     const float4 xi = d.pos[i];
     const bool st_on = (sc.flags & SF_SURFACE_TENSION) != 0;
     const float rhoi = d.rho[i];
     float sx = 0.f, sy = 0.f, sz = 0.f, wvx = 0.f, wvy = 0.f, wvz = 0.f;
-    if (st_on || expl || bnu_on) {
-      const int cnt = d.nnbr[i];
+    // surface tension reads positions only: the velocities and densities are
+    // gathered only for a viscosity term formed here (two loops, so that the
+    // position-only one holds no velocity registers)
+    if (expl || bnu_on) {
       struct NJ {
         float4 x, v;
         float rho;
       };
-      // surface tension reads positions only: the velocities and densities
-      // are gathered only for a viscosity term formed here (two loops, so
-      // that the position-only one holds no velocity registers)
-      const bool need_v = expl || bnu_on;
-      auto body = [&](int, const NJ& nj) {
+      const int cnt = d.nnbr[i];
+      for_pairs<G, B, 6>(
+          d, i, q, cnt, [&](int j) { return NJ{d.pos[j], d.vel[j], d.rho[j]}; },
+          [&](int, const NJ& nj, bool live, float (&t)[6]) {
             const float4 xj = nj.x, vj = nj.v;
             const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-            if (xj.w > 0.0f) {
-              if (st_on) {
-                const float r2 = rx * rx + ry * ry + rz * rz;
-                const float w = r2 > sc.diam2 ? kern_w(sc.h, sc.kW, norm3(rx, ry, rz)) : sc.Wd;
-                sx -= sc.sig_m * rx * w;
-                sy -= sc.sig_m * ry * w;
-                sz -= sc.sig_m * rz * w;
-              }
-              if (expl) {
-                const float vxy = (vi.x - vj.x) * rx + (vi.y - vj.y) * ry + (vi.z - vj.z) * rz;
-                const float rn = norm3(rx, ry, rz);
-                const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, rn);
-                const float f = sc.ten_nu * (sc.mass / nj.rho) * vxy / (rn * rn + sc.visc_eps);
-                wvx += f * g.x;
-                wvy += f * g.y;
-                wvz += f * g.z;
-              }
-            } else if (bnu_on) {
-              const float vxy = (vi.x - vj.x) * rx + (vi.y - vj.y) * ry + (vi.z - vj.z) * rz;
-              const float rn = norm3(rx, ry, rz);
-              const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, rn);
-              const float f = sc.ten_bnu * (sc.rho0 * (-xj.w) / rhoi) * vxy / (rn * rn + sc.visc_eps);
-              wvx += f * g.x;
-              wvy += f * g.y;
-              wvz += f * g.z;
+            const bool fluid = xj.w > 0.0f;
+            float rn, w;
+            const float3 g = pair_grad<true, false>(kh, sc, rx, ry, rz, live, rn, w);
+#pragma unroll
+            for (int n = 0; n < 6; n++) t[n] = NEUTRAL;
+            if (live && fluid && st_on) {
+              const float r2 = rx * rx + ry * ry + rz * rz;
+              w = r2 > sc.diam2 ? w : sc.Wd;
+              t[0] = -(sc.sig_m * rx * w);
+              t[1] = -(sc.sig_m * ry * w);
+              t[2] = -(sc.sig_m * rz * w);
             }
-          };
-      if (need_v)
-        for_neighbors<B>(d, i, cnt, [&](int j) { return NJ{d.pos[j], d.vel[j], d.rho[j]}; }, body);
-      else
-        for_neighbors<B>(d, i, cnt, [&](int j) { return NJ{d.pos[j], make_float4(0.f, 0.f, 0.f, 0.f), 0.0f}; }, body);
+            if (live && (fluid ? expl : bnu_on)) {
+              const float vxy = (vi.x - vj.x) * rx + (vi.y - vj.y) * ry + (vi.z - vj.z) * rz;
+              const float num = fluid ? sc.mass : sc.rho0 * (-xj.w);
+              const float f = (fluid ? sc.ten_nu : sc.ten_bnu) * (num / (fluid ? nj.rho : rhoi)) * vxy / (rn * rn + sc.visc_eps);
+              t[3] = f * g.x;
+              t[4] = f * g.y;
+              t[5] = f * g.z;
+            }
+          },
+          [&](const float (&t)[6], bool) {
+            sx += t[0];
+            sy += t[1];
+            sz += t[2];
+            wvx += t[3];
+            wvy += t[4];
+            wvz += t[5];
+          });
+    } else if (st_on) {
+      const int cnt = d.nnbr[i];
+      for_pairs<G, B, 3>(
+          d, i, q, cnt, [&](int j) { return d.pos[j]; },
+          [&](int, const float4& xj, bool live, float (&t)[3]) {
+            const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
+            const float r2 = rx * rx + ry * ry + rz * rz;
+            const float far = pair_w(kh, sc, rx, ry, rz, live && r2 > sc.diam2);
+            const float w = r2 > sc.diam2 ? far : sc.Wd;
+            const bool on = live && xj.w > 0.0f;
+            t[0] = on ? -(sc.sig_m * rx * w) : NEUTRAL;
+            t[1] = on ? -(sc.sig_m * ry * w) : NEUTRAL;
+            t[2] = on ? -(sc.sig_m * rz * w) : NEUTRAL;
+          },
+          [&](const float (&t)[3], bool) {
+            sx += t[0];
+            sy += t[1];
+            sz += t[2];
+          });
     }
+    if (q != 0) return;
     float ax = sc.gx, ay = sc.gy, az = sc.gz;
     if (st_on) {
       ax += sx;
@@ -310,53 +401,65 @@ __global__ void k_nonpressure(Dev d) {
     d.vel_alt[i] = make_float4(vi.x + sc.dt * ax, vi.y + sc.dt * ay, vi.z + sc.dt * az, vi.w);
     return;
   }
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   if (dyn_solid(kind)) {
     float ax = sc.gx, ay = sc.gy, az = sc.gz;
     if (bnu_on) {  // reaction of the boundary viscosity (:1458-1460), gathered
+      struct NF {
+        float4 x, v;
+        float rho;
+      };
+      const KernH kh(sc);
       const float4 xi = d.pos[i];
       const float Vi = -xi.w;
-      const int cnt = d.nnbr[i];
-      for (int k = 0; k < cnt; k++) {
-        const int f = d.nbr[nb_word(P, i, k)];
-        const float4 xf = d.pos[f];
-        if (!(xf.w > 0.0f)) continue;
-        const float4 vf = d.vel[f];
-        const float rx = xf.x - xi.x, ry = xf.y - xi.y, rz = xf.z - xi.z;
-        const float vxy = (vf.x - vi.x) * rx + (vf.y - vi.y) * ry + (vf.z - vi.z) * rz;
-        const float rn = norm3(rx, ry, rz);
-        const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, rn);
-        const float ff = sc.ten_bnu * (sc.rho0 * Vi / d.rho[f]) * vxy / (rn * rn + sc.visc_eps);
-        ax += -(ff * g.x);
-        ay += -(ff * g.y);
-        az += -(ff * g.z);
-      }
+      for_pairs<G, B, 3>(
+          d, i, q, d.nnbr[i], [&](int j) { return NF{d.pos[j], d.vel[j], d.rho[j]}; },
+          [&](int, const NF& nf, bool live, float (&t)[3]) {
+            const float4 xf = nf.x, vf = nf.v;
+            t[0] = t[1] = t[2] = NEUTRAL;
+            if (live && xf.w > 0.0f) {
+              const float rx = xf.x - xi.x, ry = xf.y - xi.y, rz = xf.z - xi.z;
+              const float vxy = (vf.x - vi.x) * rx + (vf.y - vi.y) * ry + (vf.z - vi.z) * rz;
+              float rn, w;
+              const float3 g = pair_grad<false, true>(kh, sc, rx, ry, rz, true, rn, w);
+              const float ff = sc.ten_bnu * (sc.rho0 * Vi / nf.rho) * vxy / (rn * rn + sc.visc_eps);
+              t[0] = -(ff * g.x);
+              t[1] = -(ff * g.y);
+              t[2] = -(ff * g.z);
+            }
+          },
+          [&](const float (&t)[3], bool) {
+            ax += t[0];
+            ay += t[1];
+            az += t[2];
+          });
     }
-    d.acc[i] = make_float4(ax, ay, az, 0.f);
-  } else {
-    d.acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    acc = make_float4(ax, ay, az, 0.f);
   }
+  if (q != 0) return;
+  d.acc[i] = acc;
   d.vel_alt[i] = vi;
 }
 
 // compute_density_adv (:1647-1667) + compute_density_error(rho0) and the loop
 // test of pressure_solve (:1778-1784)
-template <int B>
+template <int G, int B>
 __global__ void k_press_source(Dev d, int reduce) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   SceneState* st = d.state + s;
   if (!st->active_p) return;
-  double v[1] = {0.0};
+  double v = 0.0;
   if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
     int cnt;
-    const float delta = velocity_divergence<B>(d, sc, i, d.pos[i], cnt);
+    const float delta = velocity_divergence<G, B>(d, sc, i, q, d.pos[i], cnt);
     float da = d.rho[i] / sc.rho0 + sc.dt * delta;
     da = da > 1.0f ? da : 1.0f;
-    d.sa[i].x = da;
-    v[0] = (double)sc.rho0 * (double)da - sc.rho0_d;
+    if (q == 0) d.sa[i].x = da;
+    v = (double)sc.rho0 * (double)da - sc.rho0_d;
   }
-  if (reduce) wave_partials<1>(d, (int)(i >> 6), v);
+  if (reduce) lane_partial<G>(d, i, v);
 }
 
 // Second stage of the per-scene reductions: one FINISH_THREADS-thread workgroup
@@ -368,11 +471,14 @@ __global__ void k_press_source(Dev d, int reduce) {
 // (The CG's per-iteration reduction is done inside k_cg_update.)
 // Thread t adds entries t, t + FINISH_THREADS, ... in order (two interleaved
 // chains); the wavefront sums are combined by a fixed pairwise tree: a fixed
-// order, the same bits every run.
+// order, the same bits every run.  The solvers' sweeps leave `lanes` partials
+// per 64 particles (lane_partial), which are first added by the tree the
+// sweep's wavefront would have continued, so an entry has the same bits for
+// every number of lanes.
 constexpr int FINISH_THREADS = NN_FINISH_THREADS;
 constexpr int FINISH_WAVES = FINISH_THREADS / 64;
 
-__global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int which) {
+__global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int which, int lanes) {
   __shared__ double red[4][FINISH_WAVES];
   const int s = blockIdx.x;
   const int t = threadIdx.x;
@@ -390,19 +496,32 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
   // partial arrays read and their granularity (4 = four-lane sweep, a
   // partial per 16 particles)
   const int nr = which == 2 ? 4 : (which == 4 ? 2 : 1);
+  const bool solver = which == 0 || which == 1;
   double tot[4] = {0.0, 0.0, 0.0, 0.0};
   for (int r = 0; r < nr; r++) {
     // the first matvec's partials (array 3) and cg_init's are per 16 particles
     const int g = which == 4 ? 4 : (which == 2 ? (r == 3 ? 4 : 1) : 1);
     const double* src = d.partials + (long)r * 4 * d.W;
     const int lo = g * sc.wave_begin, hi = g * sc.wave_end;
+    auto entry = [&](int k) {
+      if (!solver || lanes == 1) return src[k];
+      if (lanes == 4) return (src[4 * k] + src[4 * k + 1]) + (src[4 * k + 2] + src[4 * k + 3]);
+      double v[16];
+#pragma unroll
+      for (int e = 0; e < 16; e++) v[e] = src[16 * k + e];
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1)
+#pragma unroll
+        for (int e = 0; e < 16; e += 2 * off) v[e] += v[e + off];
+      return v[0];
+    };
     double a0 = 0.0, a1 = 0.0;
     int k = lo + t;
     for (; k + FINISH_THREADS < hi; k += 2 * FINISH_THREADS) {
-      a0 += src[k];
-      a1 += src[k + FINISH_THREADS];
+      a0 += entry(k);
+      a1 += entry(k + FINISH_THREADS);
     }
-    if (k < hi) a0 += src[k];
+    if (k < hi) a0 += entry(k);
     const double w = wave_sum(a0 + a1);
     if ((t & 63) == 0) red[r][t >> 6] = w;
   }
@@ -459,67 +578,47 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
 // pressure_solve_iteration_kernel, :1799-1841.  Fluid lanes update v in place
 // (nothing in the sweep reads v); dynamic-solid lanes gather the reaction
 // -vel_change/dt of every fluid neighbor (:1835-1841) into their acceleration.
-template <int B>
+template <int G, int B>
 __global__ void k_press_update(Dev d) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (!d.state[s].active_p) return;
   if (i >= sc.p_begin + sc.n) return;
   const int kind = kind_of(d.info[i]);
-  const int P = d.P;
-  const float4 xi = d.pos[i];
-  const int cnt = d.nnbr[i];
   if (kind == KIND_FLUID) {
+    const KernH kh(sc);
     const float2 sai = d.sa[i];
     const float ki = (sai.x - 1.0f) * alpha_press(sc, sai.y);
     float4 v = d.vel[i];
-    for_neighbors<B>(
-        d, i, cnt, [&](int j) { const float2 t = d.sa[j]; return PosSrc{d.pos[j], t.x, t.y}; },
-        [&](int, const PosSrc& nj) {
-          const float4 xj = nj.x;
-          if (xj.w > 0.0f) {
-            const float kj = (nj.src - 1.0f) * alpha_press(sc, nj.alpha);
-            const float ksum = ki + kj;
-            if (fabsf(ksum) > sc.eps) {
-              const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-              const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, norm3(rx, ry, rz));
-              const float f = sc.dt * ksum;
-              const float Vj = xj.w;
-              v.x -= f * (-Vj * g.x);
-              v.y -= f * (-Vj * g.y);
-              v.z -= f * (-Vj * g.z);
-            }
-          } else if (fabsf(ki) > sc.eps) {
-            const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-            const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, norm3(rx, ry, rz));
-            const float f = -sc.dt * ki;
-            const float Vj = -xj.w;
-            v.x += f * (-Vj * g.x);
-            v.y += f * (-Vj * g.y);
-            v.z += f * (-Vj * g.z);
-          }
-        });
-    d.vel[i] = v;
+    velocity_push<G, B, true>(d, sc, kh, i, q, d.nnbr[i], d.pos[i], ki,
+                              [&](const PosSrc& nj) { return (nj.src - 1.0f) * alpha_press(sc, nj.alpha); }, v.x, v.y, v.z);
+    if (q == 0) d.vel[i] = v;
   } else if (dyn_solid(kind)) {
+    const KernH kh(sc);
+    const float4 xi = d.pos[i];
     const float Vi = -xi.w;
     float4 a = d.acc[i];
-    for (int k = 0; k < cnt; k++) {
-      const int f = d.nbr[nb_word(P, i, k)];
-      const float4 xf = d.pos[f];
-      if (!(xf.w > 0.0f)) continue;
-      const float2 saf = d.sa[f];
-      const float kf = (saf.x - 1.0f) * alpha_press(sc, saf.y);
-      if (fabsf(kf) > sc.eps) {
-        const float rx = xf.x - xi.x, ry = xf.y - xi.y, rz = xf.z - xi.z;
-        const float3 g = kern_grad(sc.h, sc.kG, rx, ry, rz, norm3(rx, ry, rz));
-        const float fk = -sc.dt * kf;
-        a.x += -(fk * (-Vi * g.x)) * 1.0f / sc.dt;
-        a.y += -(fk * (-Vi * g.y)) * 1.0f / sc.dt;
-        a.z += -(fk * (-Vi * g.z)) * 1.0f / sc.dt;
-      }
-    }
-    d.acc[i] = a;
+    for_pairs<G, B, 3>(
+        d, i, q, d.nnbr[i], [&](int f) { const float2 t = d.sa[f]; return PosSrc{d.pos[f], t.x, t.y}; },
+        [&](int, const PosSrc& nf, bool live, float (&t)[3]) {
+          const float4 xf = nf.x;
+          const float kf = (nf.src - 1.0f) * alpha_press(sc, nf.alpha);
+          t[0] = t[1] = t[2] = NEUTRAL;
+          if (live && xf.w > 0.0f && fabsf(kf) > sc.eps) {
+            const float3 g = pair_grad<true>(kh, sc, xf.x - xi.x, xf.y - xi.y, xf.z - xi.z, true);
+            const float fk = -sc.dt * kf;
+            t[0] = -(fk * (-Vi * g.x)) * 1.0f / sc.dt;
+            t[1] = -(fk * (-Vi * g.y)) * 1.0f / sc.dt;
+            t[2] = -(fk * (-Vi * g.z)) * 1.0f / sc.dt;
+          }
+        },
+        [&](const float (&t)[3], bool) {
+          a.x += t[0];
+          a.y += t[1];
+          a.z += t[2];
+        });
+    if (q == 0) d.acc[i] = a;
   }
 }
 
@@ -578,35 +677,39 @@ static inline dim3 grid_of(const DevRef& d, int block) { return dim3((d.h.Pn + b
 void launch_step_begin(const DevRef& d, hipStream_t st) {
   NN_LAUNCH(k_step_begin, dim3(1), dim3(256), 0, st, d.h);
 }
+void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* host, hipStream_t st) {
+  if (d.h.nscenes > 0)
+    NN_LAUNCH(k_publish, dim3(d.h.nscenes), dim3(PUBLISH_THREADS), 0, st, d.h, list_lanes, rho_lanes, host);
+}
 void launch_clear_acc(const DevRef& d, int block, hipStream_t st) {
   NN_LAUNCH(k_clear_acc, grid_of(d, block), dim3(block), 0, st, d.h);
 }
-void launch_density_alpha(const DevRef& d, int block, int depth, hipStream_t st) {
-  DEPTH_LAUNCH(k_density_alpha, depth, grid_of(d, block), dim3(block), st, d.h);
+void launch_density_alpha(const DevRef& d, int block, int lanes, int depth, hipStream_t st) {
+  SWEEP_LAUNCH(k_density_alpha, lanes, depth, d.h.Pn, block, st, d.h);
 }
 void launch_solver_begin(const DevRef& d, int which, hipStream_t st) {
   NN_LAUNCH(k_solver_begin, dim3(1), dim3(256), 0, st, d.h, which);
 }
-void launch_div_update(const DevRef& d, int block, int depth, hipStream_t st) {
-  DEPTH_LAUNCH(k_div_update, depth, grid_of(d, block), dim3(block), st, d.h);
+void launch_div_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st) {
+  SWEEP_LAUNCH_4(k_div_update, lanes, depth, d.h.Pn, block, st, d.h);
 }
-void launch_div_source(const DevRef& d, int block, int depth, hipStream_t st) {
-  DEPTH_LAUNCH(k_div_source, depth, grid_of(d, block), dim3(block), st, d.h);
+void launch_div_source(const DevRef& d, int block, int lanes, int depth, hipStream_t st) {
+  SWEEP_LAUNCH_4(k_div_source, lanes, depth, d.h.Pn, block, st, d.h);
 }
-void launch_nonpressure(const DevRef& d, int block, int depth, hipStream_t st) {
-  DEPTH_LAUNCH(k_nonpressure, depth, grid_of(d, block), dim3(block), st, d.h);
+void launch_nonpressure(const DevRef& d, int block, int lanes, int depth, hipStream_t st) {
+  SWEEP_LAUNCH(k_nonpressure, lanes, depth, d.h.Pn, block, st, d.h);
 }
-void launch_press_source(const DevRef& d, int block, int depth, int reduce, hipStream_t st) {
-  DEPTH_LAUNCH(k_press_source, depth, grid_of(d, block), dim3(block), st, d.h, reduce);
+void launch_press_source(const DevRef& d, int block, int lanes, int depth, int reduce, hipStream_t st) {
+  SWEEP_LAUNCH_4(k_press_source, lanes, depth, d.h.Pn, block, st, d.h, reduce);
 }
-void launch_press_update(const DevRef& d, int block, int depth, hipStream_t st) {
-  DEPTH_LAUNCH(k_press_update, depth, grid_of(d, block), dim3(block), st, d.h);
+void launch_press_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st) {
+  SWEEP_LAUNCH_4(k_press_update, lanes, depth, d.h.Pn, block, st, d.h);
 }
 void launch_advect(const DevRef& d, int block, hipStream_t st) {
   NN_LAUNCH(k_advect, grid_of(d, block), dim3(block), 0, st, d.h);
 }
-void launch_scene_finish(const DevRef& d, int which, hipStream_t st) {
-  if (d.h.nscenes > 0) NN_LAUNCH(k_scene_finish, dim3(d.h.nscenes), dim3(FINISH_THREADS), 0, st, d.h, which);
+void launch_scene_finish(const DevRef& d, int which, int lanes, hipStream_t st) {
+  if (d.h.nscenes > 0) NN_LAUNCH(k_scene_finish, dim3(d.h.nscenes), dim3(FINISH_THREADS), 0, st, d.h, which, lanes);
 }
 
 }  // namespace nn

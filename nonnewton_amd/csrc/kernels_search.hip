@@ -206,114 +206,137 @@ __global__ void k_place(Dev d) {
   d.inv[sc.p_begin + my] = dest - sc.p_begin;
 }
 
+// The 9 runs' bounds from the lanes that loaded them, to every lane.
+template <int G, int R>
+__device__ __forceinline__ void run_table(const int* lo, const int* len, int base, int* first, int* shift, int& total) {
+  if constexpr (R < 9) {
+    const int b = __float_as_int(lane_bcast<G, R % G>(__int_as_float(lo[R / G])));
+    const int n = __float_as_int(lane_bcast<G, R % G>(__int_as_float(len[R / G])));
+    first[R] = total;
+    shift[R] = b + base - total;
+    total += n;
+    run_table<G, R + 1>(lo, len, base, first, shift, total);
+  }
+}
+
 // store_neighbors, SPH/main.py:836-847, over the sorted particles.  With
 // all == 0 (the search inside a step) static boundary particles get no list:
 // after the boundary volumes of the first search no sweep reads one.
+//
+// G lanes per particle.  The bounds of the 9 runs are loaded by the group at
+// once and the runs laid end to end: candidate c of the sequence is slot
+// c + shift[r] of the run r that holds it.  The lanes test candidates q, q + G,
+// ..., B rounds of loads in flight, and a hit's list position is the hits
+// before it: those of earlier rounds plus those of lower lanes (a ballot), so
+// the list keeps the reference's order.
+template <int G, int B>
 __global__ void k_build_lists(Dev d, int all) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
+  const bool mine = i < sc.p_begin + sc.n;
+  const int kind = mine ? kind_of(d.info[i]) : KIND_STATIC;
   int cnt = 0;
   int cx, cy, cz;
   const float4 xi = d.pos[i];
-  const bool want = i < sc.p_begin + sc.n && (all || kind_of(d.info[i]) != KIND_STATIC);
-  // list positions are collected in groups of four and each group is written
-  // as one int4 when complete (the last one possibly partial, its unused words
-  // never read)
-  int4 grp = make_int4(0, 0, 0, 0);
-  int4* groups = reinterpret_cast<int4*>(d.nbr);
-  if (want && cell_of(sc, xi, cx, cy, cz)) {
+  if (mine && (all || kind != KIND_STATIC) && cell_of(sc, xi, cx, cy, cz)) {
     const float thr2 = sc.thr2;
     const long P = d.P;
     const int z0 = cz > 0 ? cz - 1 : 0;
     const int z1 = cz + 1 < sc.gn2 ? cz + 1 : sc.gn2 - 1;
-    for (int dx = -1; dx <= 1; dx++) {
-      const int a = cx + dx;
-      if (a < 0 || a >= sc.gn0) continue;
-      for (int dy = -1; dy <= 1; dy++) {
-        const int b = cy + dy;
-        if (b < 0 || b >= sc.gn1) continue;
+    constexpr int RL = (9 + G - 1) / G;  // runs whose bounds a lane loads
+    int lo[RL], len[RL];
+#pragma unroll
+    for (int e = 0; e < RL; e++) {
+      const int r = q + e * G;
+      const int a = cx + r / 3 - 1, b = cy + r % 3 - 1;
+      lo[e] = len[e] = 0;
+      if (r < 9 && a >= 0 && a < sc.gn0 && b >= 0 && b < sc.gn1) {
         const int base = sc.cell_begin + (a * sc.gn1 + b) * sc.gn2;
-        const int j0 = d.cell_start[base + z0] + sc.shift;
-        const int j1 = d.cell_start[base + z1 + 1] + sc.shift;
-        // candidates in order, 8 positions loaded together
-        for (int jb = j0; jb < j1; jb += 8) {
-          float4 xj[8];
+        lo[e] = d.cell_start[base + z0];
+        len[e] = d.cell_start[base + z1 + 1] - lo[e];
+      }
+    }
+    int first[9], shift[9], total = 0;  // run r: candidates [first[r], first[r + 1])
+    run_table<G, 0>(lo, len, sc.shift, first, shift, total);
+    const int lane = threadIdx.x & 63;
+    const int below = (1 << q) - 1;
+    for (int c0 = 0; c0 < total; c0 += G * B) {
+      int j[B];
+      float4 xj[B];
 #pragma unroll
-          for (int u = 0; u < 8; u++) xj[u] = d.pos[jb + u < j1 ? jb + u : i];
+      for (int u = 0; u < B; u++) {
+        const int c = c0 + u * G + q;
+        int sh = shift[0];
 #pragma unroll
-          for (int u = 0; u < 8; u++) {
-            const int j = jb + u;
-            if (j >= j1 || j == i) continue;
-            const float ex = xi.x - xj[u].x, ey = xi.y - xj[u].y, ez = xi.z - xj[u].z;
-            const float ss = ex * ex + ey * ey + ez * ez;
-            // sqrt_rn(ss) < h  <=>  ss < thr2 (thr2: least float whose rounded sqrt >= h)
-            if (ss < thr2) {
-              if (cnt < MAX_NB) {
-                const int w = cnt & 3;
-                grp.x = w == 0 ? j : grp.x;
-                grp.y = w == 1 ? j : grp.y;
-                grp.z = w == 2 ? j : grp.z;
-                grp.w = w == 3 ? j : grp.w;
-                if (w == 3) groups[(long)(cnt >> 2) * P + i] = grp;
-              }
-              cnt++;
-            }
-          }
-        }
+        for (int r = 1; r < 9; r++) sh = c >= first[r] ? shift[r] : sh;
+        j[u] = c < total ? c + sh : i;
+      }
+#pragma unroll
+      for (int u = 0; u < B; u++) xj[u] = d.pos[j[u]];
+#pragma unroll
+      for (int u = 0; u < B; u++) {
+        const float ex = xi.x - xj[u].x, ey = xi.y - xj[u].y, ez = xi.z - xj[u].z;
+        const float ss = ex * ex + ey * ey + ez * ez;
+        // sqrt_rn(ss) < h  <=>  ss < thr2 (thr2: least float whose rounded sqrt >= h)
+        const bool hit = ss < thr2 && j[u] != i;
+        const int hits = (int)(__ballot(hit) >> (lane & ~(G - 1))) & ((1 << G) - 1);
+        const int at = cnt + __popc(hits & below);
+        cnt += __popc(hits);
+        if (hit && at < MAX_NB) d.nbr[nb_word(P, i, at)] = j[u];
       }
     }
     if (cnt > MAX_NB) {
-      atomicOr(&d.state[s].status, ST_NEIGHBOR_OVERFLOW);
+      if (q == 0) atomicOr(&d.state[s].status, ST_NEIGHBOR_OVERFLOW);
       cnt = MAX_NB;
     }
-    if (cnt & 3) groups[(long)(cnt >> 2) * P + i] = grp;
   }
+  if (mine && q == 0) d.nnbr[i] = cnt;
   // the step's pair counts cover the lists a step uses: fluid and dynamic
-  // solid particles (static boundary lists serve only the boundary volumes)
-  int cf = 0, tot = 0;
-  if (i < sc.p_begin + sc.n) {
-    d.nnbr[i] = cnt;
-    const int kind = kind_of(d.info[i]);
-    if (kind == KIND_FLUID) cf = cnt;
-    if (kind != KIND_STATIC) tot = cnt;
-  }
+  // solid particles (static boundary lists serve only the boundary volumes);
+  // a wavefront's counts go to its own entry (k_publish adds them: thousands of
+  // atomics on one word took longer than the search)
+  int tot = q == 0 && kind != KIND_STATIC ? cnt : 0, cf = q == 0 && kind == KIND_FLUID ? cnt : 0;
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
+  for (int off = 32; off >= G; off >>= 1) {
     tot += __shfl_xor(tot, off, 64);
     cf += __shfl_xor(cf, off, 64);
   }
-  if ((threadIdx.x & 63) == 0 && tot > 0) atomicAdd(&d.state[s].pairs, (unsigned long long)tot);
-  if ((threadIdx.x & 63) == 0 && cf > 0) atomicAdd(&d.state[s].pairs_fluid, (unsigned long long)cf);
+  if ((threadIdx.x & 63) == 0) d.wave_pairs[i / (64 / G)] = make_int2(tot, cf);
 }
 
 // compute_static/moving_boundary_volume, SPH/main.py:1010-1035:
 // V_b = 3 / (W0 + sum over solid neighbors of W); stored as -V (solid sign).
+template <int G, int B>
 __global__ void k_bvol(Dev d, int dynamic) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (i >= sc.p_begin + sc.n) return;
   const int kind = kind_of(d.info[i]);
   if (dynamic ? !dyn_solid(kind) : kind != KIND_STATIC) return;
+  const KernH kh(sc);
   const float4 xi = d.pos[i];
-  const int cnt = d.nnbr[i];
-  const int P = d.P;
   KSum ks{sc.W0, 0.0f};
-  float plain = sc.W0;
   const bool comp = (sc.flags & SF_COMPENSATED) != 0;
-  for (int k = 0; k < cnt; k++) {
-    const int j = d.nbr[nb_word(P, i, k)];
-    const float4 xj = d.pos[j];
-    if (xj.w < 0.0f) {
-      const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-      const float w = kern_w(sc.h, sc.kW, norm3(rx, ry, rz));
-      if (comp) ks.add(w);
-      else plain += w;
-    }
-  }
-  const float delta = comp ? ks.s : plain;
-  d.pos[i].w = -(1.0f / delta * 3.0f);
+  // (the volume of a neighbor may be rewritten meanwhile: only its sign, which
+  // stays, is read)
+  for_pairs<G, B, 2>(
+      d, i, q, d.nnbr[i], [&](int j) { return d.pos[j]; },
+      [&](int, const float4& xj, bool live, float (&t)[2]) {
+        const bool on = live && xj.w < 0.0f;
+        t[0] = pair_w(kh, sc, xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, on);
+        t[1] = on ? 1.0f : 0.0f;
+      },
+      [&](const float (&t)[2], bool) {
+        KSum n = ks;
+        if (comp) n.add(t[0]);
+        else n.s += t[0];
+        const bool on = t[1] != 0.0f;
+        ks.s = on ? n.s : ks.s;
+        ks.c = on ? n.c : ks.c;
+      });
+  if (q == 0) d.pos[i].w = -(1.0f / ks.s * 3.0f);
 }
 
 void launch_cell_count(const DevRef& d, int block, hipStream_t st) {
@@ -325,11 +348,13 @@ void launch_bucket(const DevRef& d, int block, hipStream_t st) {
 void launch_place(const DevRef& d, int block, hipStream_t st) {
   NN_LAUNCH(k_place, dim3((d.h.Pn + block - 1) / block), dim3(block), 0, st, d.h);
 }
-void launch_build_lists(const DevRef& d, int block, int all, hipStream_t st) {
-  NN_LAUNCH(k_build_lists, dim3((d.h.Pn + block - 1) / block), dim3(block), 0, st, d.h, all);
+void launch_build_lists(const DevRef& d, int block, int lanes, int all, hipStream_t st) {
+  const dim3 g((unsigned)(((long)d.h.Pn * lanes + block - 1) / block)), b(block);
+  if (lanes == 4) NN_LAUNCH((k_build_lists<4, 4>), g, b, 0, st, d.h, all);
+  else NN_LAUNCH((k_build_lists<16, 4>), g, b, 0, st, d.h, all);
 }
-void launch_bvol(const DevRef& d, int block, int dynamic, hipStream_t st) {
-  NN_LAUNCH(k_bvol, dim3((d.h.Pn + block - 1) / block), dim3(block), 0, st, d.h, dynamic);
+void launch_bvol(const DevRef& d, int block, int lanes, int dynamic, hipStream_t st) {
+  SWEEP_LAUNCH_4(k_bvol, lanes, 8, d.h.Pn, block, st, d.h, dynamic);
 }
 
 }  // namespace nn

@@ -38,10 +38,10 @@ __device__ __forceinline__ bool weiler_scene(const SceneDev& sc) {
 
 // NonNewton.calcStrainRate (:461-492, with the accumulation the reference
 // omits) + the viscosity model; mu for the implicit solver.
-template <int B>
+template <int G, int B>
 __global__ void k_strain(Dev d) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
+  int i, q, s;
+  if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (!(sc.flags & SF_HAS_FLUID)) return;
   const bool nn_on = (sc.flags & SF_NON_NEWTONIAN) != 0;
@@ -50,38 +50,48 @@ __global__ void k_strain(Dev d) {
   if (i >= sc.p_begin + sc.n || kind_of(d.info[i]) != KIND_FLUID) return;
   float eta = 0.0f;
   if (nn_on) {
+    const KernH kh(sc);
     const float4 xi = d.pos[i];
     const float4 vi = d.vel[i];
     const int cnt = d.nnbr[i];
-    float S[9];
+    // the tensor is symmetric, its two halves equal bit for bit (a sum of two
+    // products does not depend on their order): six sums
+    float S[6];
 #pragma unroll
-    for (int q = 0; q < 9; q++) S[q] = 0.0f;
-    for_neighbors<B>(
-        d, i, cnt, [&](int j) { return PosVel{d.pos[j], d.vel[j]}; },
-        [&](int, const PosVel& nj) {
+    for (int n = 0; n < 6; n++) S[n] = 0.0f;
+    for_pairs<G, B, 6>(
+        d, i, q, cnt, [&](int j) { return PosVel{d.pos[j], d.vel[j]}; },
+        [&](int, const PosVel& nj, bool live, float (&t)[6]) {
           const float4 xj = nj.x, vj = nj.v;
-          const float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
-          const float3 g3 = kern_grad(sc.h, sc.kG, rx, ry, rz, norm3(rx, ry, rz));
+          const float3 g3 = pair_grad(kh, sc, xi.x - xj.x, xi.y - xj.y, xi.z - xj.z, live);
           const float g[3] = {g3.x, g3.y, g3.z};
           const float vji[3] = {vj.x - vi.x, vj.y - vi.y, vj.z - vi.z};
+          int n = 0;
 #pragma unroll
           for (int a = 0; a < 3; a++)
 #pragma unroll
-            for (int b = 0; b < 3; b++) S[3 * a + b] += sc.mass * (vji[a] * g[b] + vji[b] * g[a]);
+            for (int b = a; b < 3; b++) t[n++] = live ? sc.mass * (vji[a] * g[b] + vji[b] * g[a]) : NEUTRAL;
+        },
+        [&](const float (&t)[6], bool) {
+#pragma unroll
+          for (int n = 0; n < 6; n++) S[n] += t[n];
         });
     const float f = 0.5f / d.rho[i];
+    const float M[9] = {S[0], S[1], S[2], S[1], S[3], S[4], S[2], S[4], S[5]};
     float n2 = 0.0f;
 #pragma unroll
-    for (int q = 0; q < 9; q++) {
-      const float t = f * S[q];
+    for (int e = 0; e < 9; e++) {
+      const float t = f * M[e];
       n2 += t * t;
     }
     const float gam = sqrtf(n2);
     eta = nn_model(sc, gam);
-    d.gam[i] = gam;
-    d.eta[i] = eta;
+    if (q == 0) {
+      d.gam[i] = gam;
+      d.eta[i] = eta;
+    }
   }
-  if (weiler) d.mu[i] = (nn_on ? eta : sc.nu) * sc.rho0;
+  if (weiler && q == 0) d.mu[i] = (nn_on ? eta : sc.nu) * sc.rho0;
 }
 
 // Start of a solve, b = v.  Pair scalars s_ij (stored), the inverse diagonal
@@ -554,8 +564,8 @@ static inline dim3 grid4_of(const DevRef& d, int block) {
   return dim3((4 * d.h.Pn + qb - 1) / qb);
 }
 
-void launch_strain(const DevRef& d, int block, int depth, hipStream_t st) {
-  DEPTH_LAUNCH(k_strain, depth, grid_of(d, block), dim3(block), st, d.h);
+void launch_strain(const DevRef& d, int block, int lanes, int depth, hipStream_t st) {
+  SWEEP_LAUNCH(k_strain, lanes, depth, d.h.Pn, block, st, d.h);
 }
 void launch_cg_init(const DevRef& d, int block, hipStream_t st) {
   NN_LAUNCH(k_cg_init, grid4_of(d, block), dim3(quad_block(block)), 0, st, d.h);
