@@ -79,8 +79,8 @@ __device__ __forceinline__ long nb_word(long P, int i, int k) { return 4 * ((lon
 // needs.  Where a scene's h lies in [2^-20, 2^20] (SF_MIDRANGE) and a pair's
 // squared distance is above 1e-10 with no component in (0, 2^-100), the
 // sequences below give the same bits:
-//   sqrt_mid   v_sqrt_f32 (1 ulp), then the neighbor whose FMA residual shows
-//              it nearer
+//   sqrt_mid   x rsq(x) and one residual correction (compared on this device
+//              with the correctly rounded root of every float in [2^-100, 2^100))
 //   recip_mid  v_rcp_f32 and one Newton step, shared by every quotient of one
 //              denominator
 //   div_mid    a y, then two residual corrections q + (a - b q) y (Markstein,
@@ -90,12 +90,9 @@ __device__ __forceinline__ long nb_word(long P, int i, int k) { return 4 * ((lon
 // and r h), about half of its instructions.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float sqrt_mid(float x) {
-  const float s = __builtin_amdgcn_sqrtf(x);
-  const float dn = __int_as_float(__float_as_int(s) - 1), up = __int_as_float(__float_as_int(s) + 1);
-  const float rd = __builtin_fmaf(-dn, s, x), ru = __builtin_fmaf(-up, s, x);
-  float r = rd <= 0.0f ? dn : s;
-  r = ru > 0.0f ? up : r;
-  return r;
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float g = x * y;
+  return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
 }
 __device__ __forceinline__ float recip_mid(float b) {
   const float y = __builtin_amdgcn_rcpf(b);

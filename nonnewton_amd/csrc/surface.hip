@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "batch.h"
+#include "device_common.h"
 
 namespace nn {
 namespace sr {
@@ -57,14 +58,14 @@ struct K {
   long nvox, nvert, nblock;
   const float* pos;  // 3 per particle, caller order
   const float* vel;  // 3 per particle when the velocity channels are on, else null
-  unsigned long long* vacc;  // 3 per vertex (velocity channels)
-  float *vfield, *mvel;      // 3 per vertex, 3 per mesh vertex
+  float *vfield, *mvel;  // 3 per vertex, 3 per mesh vertex
+  int mid;                   // the smooth radius lies where sqrt_mid and div_mid hold
   float cvs3;                // voxel_size^3 (contribution_coeff, :1165)
   int* pvox;         // 3 per particle: its voxel
   int *vcount, *vstart, *vslot, *vlist;
-  float *G, *xbar, *detG;
+  float *G, *xbar;
   unsigned char* active;
-  unsigned long long* acc;
+  float4* rec;  // REC_QUADS per entry of vlist
   float *field0, *field, *tmp;
   int *flag, *cube_id, *tcount, *tstart;
   float *verts, *normals;
@@ -77,9 +78,6 @@ struct K {
 // ------------------------------------------------------------------ helpers
 
 __device__ __forceinline__ float norm3f(float x, float y, float z) { return sqrtf(x * x + y * y + z * z); }
-// a value every lane of the wavefront holds (lets the compiler use scalar loads)
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
 // exp for the bilateral weights (x <= 0 there).  Cody-Waite reduction
 // x = k ln2 + r with ln2 split into a 16-bit high part (k ln2_hi exact) and a
 // low part, the degree-7 Taylor polynomial of e^r in Horner form, exact
@@ -181,19 +179,6 @@ __device__ __forceinline__ float poly6(const K& k, float rx, float ry, float rz,
     tmp = tmp * tmp * tmp * tmp * h;
     res = k.acoef * res / tmp;
   }
-  return res;
-}
-// cubic_spline_kernel (:1115-1124), "+ 1" where the reference puts it
-__device__ __forceinline__ float aniso_w(const K& k, const float* G, float det, float dx, float dy, float dz) {
-  const float a = G[0] * dx + G[1] * dy + G[2] * dz;
-  const float b = G[3] * dx + G[4] * dy + G[5] * dz;
-  const float c = G[6] * dx + G[7] * dy + G[8] * dz;
-  const float q = norm3f(a, b, c);
-  float res = 0.0f;
-  if (0.0f < q && q <= 0.5f)
-    res = k.c48 * det * (q * q * q - q * q) + 1.0f;
-  else if (0.5f < q && q <= 1.0f)
-    res = k.c16 * det * (1.0f - q) * (1.0f - q) * (1.0f - q);
   return res;
 }
 __device__ __forceinline__ unsigned long long fix_of(float v) {
@@ -338,6 +323,20 @@ __device__ __forceinline__ void vrange(const K& k, int x, int y, int z, int& b, 
   e = k.vstart[q + 1];
 }
 
+template <int G, int U>
+__device__ __forceinline__ int lane_bcast_i(int v) {
+  return __float_as_int(lane_bcast<G, U>(__int_as_float(v)));
+}
+// lane r's (first, shift) of G runs laid end to end: the shift of the run that holds candidate c
+template <int G, int U>
+__device__ __forceinline__ int shift_at(int c, int first, int shift, int sh) {
+  if constexpr (U < G) {
+    const int f = lane_bcast_i<G, U>(first), s = lane_bcast_i<G, U>(shift);
+    return shift_at<G, U + 1>(c, first, shift, c >= f ? s : sh);
+  }
+  return sh;
+}
+
 // The particles a sweep of pre_process_data visits, in its order (voxel dx,
 // dy, dz nested, z fastest, then the voxel's list), restricted to the voxels
 // that can hold a particle closer than r2: a voxel's particles are contiguous
@@ -345,98 +344,153 @@ __device__ __forceinline__ void vrange(const K& k, int x, int y, int z, int& b, 
 // column is one range.  A skipped particle has w = 0 and adds +0 to every sum
 // (rows and column ends are trimmed with a margin of 1e-3 voxel around each
 // voxel and 1e-4 of r2), so the sums are those of the full loop bit for bit.
-template <typename F>
-__device__ __forceinline__ void for_reach(const K& k, const int* v, float x0, float x1, float x2, float r2, F f) {
+//
+// G lanes per particle (4 or 16): they find the ranges of G columns at a time,
+// lay them end to end, and take candidates q, q + G, ...; term(entry of vlist
+// or -1, t) forms a candidate's N terms and the group adds them in order.
+template <int G, int N, typename Term>
+__device__ __forceinline__ void for_reach(const K& k, int q, const int* v, float x0, float x1, float x2, float r2,
+                                          float (&acc)[N], Term term) {
   const int R = k.R, off = k.off;
   const float reach = r2 * 1.0001f;
   const float reach2 = reach * reach;
   const float m = 1e-3f * k.vs;
-  for (int dx = 0; dx < R; dx++) {
-    const int x = v[0] + dx - off;
-    if (x < 0 || x < k.vlo[0] || x >= k.vlo[0] + k.vdim[0]) continue;
-    const float lx = (float)x * k.vs + k.o[0] - m, hx = lx + k.vs + 2.0f * m;
-    const float gx = fmaxf(0.0f, fmaxf(lx - x0, x0 - hx));
-    for (int dy = 0; dy < R; dy++) {
-      const int y = v[1] + dy - off;
-      if (y < 0 || y < k.vlo[1] || y >= k.vlo[1] + k.vdim[1]) continue;
+  for (int col0 = 0; col0 < R * R; col0 += G) {
+    const int col = col0 + q;
+    int b = 0, len = 0;
+    const int x = v[0] + col / R - off, y = v[1] + col % R - off;
+    if (col < R * R && x >= 0 && x >= k.vlo[0] && x < k.vlo[0] + k.vdim[0] && y >= 0 && y >= k.vlo[1] && y < k.vlo[1] + k.vdim[1]) {
+      const float lx = (float)x * k.vs + k.o[0] - m, hx = lx + k.vs + 2.0f * m;
+      const float gx = fmaxf(0.0f, fmaxf(lx - x0, x0 - hx));
       const float ly = (float)y * k.vs + k.o[1] - m, hy = ly + k.vs + 2.0f * m;
       const float gy = fmaxf(0.0f, fmaxf(ly - x1, x1 - hy));
       const float rest = reach2 - (gx * gx + gy * gy);
-      if (!(rest > 0.0f)) continue;
-      const float zr = sqrtf(rest);
-      int z0 = (int)floorf((x2 - zr - k.o[2]) / k.vs) - 1;
-      int z1 = (int)floorf((x2 + zr - k.o[2]) / k.vs) + 1;
-      z0 = max(max(z0, v[2] - off), max(0, k.vlo[2]));
-      z1 = min(min(z1, v[2] - off + R - 1), k.vlo[2] + k.vdim[2] - 1);
-      if (z0 > z1) continue;
-      const long base = ((long)(x - k.vlo[0]) * k.vdim[1] + (y - k.vlo[1])) * k.vdim[2] - k.vlo[2];
-      const int b = k.vstart[base + z0], e = k.vstart[base + z1 + 1];
-      for (int mm = b; mm < e; mm++) f(k.vlist[mm]);
+      if (rest > 0.0f) {
+        const float zr = sqrtf(rest);
+        int z0 = (int)floorf((x2 - zr - k.o[2]) / k.vs) - 1;
+        int z1 = (int)floorf((x2 + zr - k.o[2]) / k.vs) + 1;
+        z0 = max(max(z0, v[2] - off), max(0, k.vlo[2]));
+        z1 = min(min(z1, v[2] - off + R - 1), k.vlo[2] + k.vdim[2] - 1);
+        if (z0 <= z1) {
+          const long base = ((long)(x - k.vlo[0]) * k.vdim[1] + (y - k.vlo[1])) * k.vdim[2] - k.vlo[2];
+          b = k.vstart[base + z0];
+          len = k.vstart[base + z1 + 1] - b;
+        }
+      }
+    }
+    // inclusive scan of the lengths over the group
+    int incl = len;
+#pragma unroll
+    for (int d = 1; d < G; d <<= 1) {
+      const int u = __shfl_up(incl, d, G);
+      if (q >= d) incl += u;
+    }
+    const int first = incl - len, shift = b - first;
+    const int total = lane_bcast_i<G, G - 1>(incl);
+    for (int c0 = 0; c0 < total; c0 += G) {
+      const int c = c0 + q;
+      const int e = c + shift_at<G, 0>(c, first, shift, 0);
+      float t[N];
+      term(c < total ? e : -1, t);
+      auto add = [&](const float (&b)[N], bool) {
+#pragma unroll
+        for (int n = 0; n < N; n++) acc[n] += b[n];
+      };
+      add_in_order<G, N, 0>(t, G, add);
     }
   }
 }
 
+// Record of list entry m (particle j = vlist[m]), for the field's tiles:
+//   (x_bar, det G), (G row 0, support radius), (G row 1, voxel x), (G row 2,
+//   voxel y), (voxel z, position)
+// Beyond the support radius the anisotropic value is exactly 0: there
+// |G d| > 1.  G = V diag(1 / (h s)) V^T with V orthonormal to FP32 rounding,
+// so |G d| >= |d| / (h max |s|) less a few ulp; 1% covers them.
+constexpr int REC_QUADS = 5;
+constexpr int ANISO_THREADS = 64;
+constexpr long ANISO_WIDE = 32768;  // 16 lanes and 4 take the same time at 32,000 particles
+
 // pre_process_data (:1007-1112) for particle i >= 1 (particle 0 keeps G = 0,
-// x_bar = 0: the reference's loop starts at 1 and reset() zeroes both)
+// x_bar = 0: the reference's loop starts at 1 and reset() zeroes both), in
+// the order of the voxel lists.  16 lanes per particle while they are few, 4
+// once the device is full (a lane repeats its group's additions and searches
+// its group's columns): 2,000 particles take 0.14 ms against 2.0 with one lane
+// each walking about 900 neighbors twice, 128,000 take 1.78 with 4 lanes, 2.60
+// with 16 and 3.05 with one.
+template <int L>
 __global__ void k_aniso(K k) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= k.n) return;
+  const int m = (blockIdx.x * blockDim.x + threadIdx.x) / L, q = threadIdx.x & (L - 1);
+  if (m >= k.n) return;  // whole groups leave together
+  const int i = k.vlist[m];
   float* G = k.G + 9 * (long)i;
   float* xb = k.xbar + 3 * (long)i;
-  if (i == 0) {
-    for (int a = 0; a < 9; a++) G[a] = 0.0f;
-    for (int a = 0; a < 3; a++) xb[a] = 0.0f;
-    k.detG[0] = 0.0f;
-    return;
-  }
+  float4* rec = k.rec + (long)REC_QUADS * m;
   const float* xi = k.pos + 3 * (long)i;
   const float x0 = xi[0], x1 = xi[1], x2 = xi[2];
   int v[3];
   voxel_of(k, xi, v);
-  const float r2 = 2.0f * k.sr;
-  float tw = 0.0f, w0 = 0.0f, w1 = 0.0f, w2 = 0.0f;
-  for_reach(k, v, x0, x1, x2, r2, [&](int j) {
-    const float* xj = k.pos + 3 * (long)j;
-    const float y0 = xj[0], y1 = xj[1], y2 = xj[2];
-    const float nr = norm3f(x0 - y0, x1 - y1, x2 - y2);
-    float w = 0.0f;
-    if (nr < r2) {
-      const float t = nr / r2;
-      w = 1.0f - t * t * t;
+  if (i == 0) {
+    if (q == 0) {
+      for (int a = 0; a < 9; a++) G[a] = 0.0f;
+      for (int a = 0; a < 3; a++) xb[a] = 0.0f;
+      rec[0] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      rec[1] = make_float4(0.0f, 0.0f, 0.0f, -1.0f);  // q = 0 everywhere: no value anywhere
+      rec[2] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(v[0]));
+      rec[3] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(v[1]));
+      rec[4] = make_float4(__int_as_float(v[2]), x0, x1, x2);
     }
-    tw += w;
-    w0 += w * y0;
-    w1 += w * y1;
-    w2 += w * y2;
+    return;
+  }
+  const float r2 = 2.0f * k.sr;
+  const float r2y = recip_mid(r2);
+  auto weight = [&](float y0, float y1, float y2) {
+    const float dx = x0 - y0, dy = x1 - y1, dz = x2 - y2;
+    const float ss = dx * dx + dy * dy + dz * dz;
+    float nr = sqrt_mid(ss);
+    float t = div_mid(nr, r2, r2y);
+    if (__builtin_expect(!(ss > 1e-30f) || !k.mid, 0)) {
+      nr = sqrtf(ss);
+      t = nr / r2;
+    }
+    return nr < r2 ? 1.0f - t * t * t : 0.0f;
+  };
+  float sw[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for_reach<L, 4>(k, q, v, x0, x1, x2, r2, sw, [&](int e, float (&t)[4]) {
+    const float* xj = k.pos + 3 * (long)(e >= 0 ? k.vlist[e] : i);
+    const float y0 = xj[0], y1 = xj[1], y2 = xj[2];
+    const float w = weight(y0, y1, y2);
+    t[0] = e >= 0 ? w : NEUTRAL;
+    t[1] = e >= 0 ? w * y0 : NEUTRAL;
+    t[2] = e >= 0 ? w * y1 : NEUTRAL;
+    t[3] = e >= 0 ? w * y2 : NEUTRAL;
   });
+  const float tw = sw[0];
+  float w0 = sw[1], w1 = sw[2], w2 = sw[3];
   if (tw != 0.0f) {
     w0 /= tw;
     w1 /= tw;
     w2 /= tw;
   }
-  xb[0] = k.lam1 * x0 + k.lam * w0;
-  xb[1] = k.lam1 * x1 + k.lam * w1;
-  xb[2] = k.lam1 * x2 + k.lam * w2;
+  const float b0 = k.lam1 * x0 + k.lam * w0, b1 = k.lam1 * x1 + k.lam * w1, b2 = k.lam1 * x2 + k.lam * w2;
+  // C is symmetric bit for bit (w (a b) and w (b a)): six sums, and the
+  // neighbors (w > 0) counted beside them
   int nn = 0;
-  float C[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  for_reach(k, v, x0, x1, x2, r2, [&](int j) {
-    const float* xj = k.pos + 3 * (long)j;
+  float cs[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  for_reach<L, 6>(k, q, v, x0, x1, x2, r2, cs, [&](int e, float (&t)[6]) {
+    const float* xj = k.pos + 3 * (long)(e >= 0 ? k.vlist[e] : i);
     const float y0 = xj[0], y1 = xj[1], y2 = xj[2];
-    const float nr = norm3f(x0 - y0, x1 - y1, x2 - y2);
-    float w = 0.0f;
-    if (nr < r2) {
-      const float t = nr / r2;
-      w = 1.0f - t * t * t;
-    }
-    if (w > 0.0f) {
-      nn++;
-      const float dp[3] = {y0 - w0, y1 - w1, y2 - w2};
+    const float w = weight(y0, y1, y2);
+    const bool on = e >= 0 && w > 0.0f;
+    nn += __popc((unsigned)(__ballot(on) >> (threadIdx.x & 63 & ~(L - 1))) & ((1u << L) - 1u));
+    const float dp[3] = {y0 - w0, y1 - w1, y2 - w2};
+    int n = 0;
 #pragma unroll
-      for (int a = 0; a < 3; a++)
+    for (int a = 0; a < 3; a++)
 #pragma unroll
-        for (int c = 0; c < 3; c++) C[3 * a + c] += w * (dp[a] * dp[c]);
-    }
+      for (int c = a; c < 3; c++) t[n++] = on ? w * (dp[a] * dp[c]) : NEUTRAL;
   });
+  float C[9] = {cs[0], cs[1], cs[2], cs[1], cs[3], cs[4], cs[2], cs[4], cs[5]};
   if (tw != 0.0f)
 #pragma unroll
     for (int a = 0; a < 9; a++) C[a] /= tw;
@@ -458,6 +512,7 @@ __global__ void k_aniso(K k) {
         }
       }
   float g[9];
+  float radius = 1.01f;
   if (tw == 0.0f) {
 #pragma unroll
     for (int a = 0; a < 9; a++) g[a] = (a % 4) == 0 ? 1.0f : 0.0f;
@@ -472,6 +527,7 @@ __global__ void k_aniso(K k) {
     } else {
       sg[0] = sg[1] = sg[2] = k.kn;
     }
+    radius = 1.01f * k.sr * fmaxf(fabsf(sg[0]), fmaxf(fabsf(sg[1]), fabsf(sg[2])));
     const float ih = 1.0f / k.sr;
     float P[9];
 #pragma unroll
@@ -482,10 +538,27 @@ __global__ void k_aniso(K k) {
     for (int a = 0; a < 3; a++)
 #pragma unroll
       for (int b = 0; b < 3; b++) g[3 * a + b] = P[3 * a] * V[3 * b] + P[3 * a + 1] * V[3 * b + 1] + P[3 * a + 2] * V[3 * b + 2];
+    // a support radius is only trusted where V came out orthonormal
+    float e = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int b = 0; b < 3; b++)
+        e = fmaxf(e, fabsf(V[a] * V[b] + V[3 + a] * V[3 + b] + V[6 + a] * V[6 + b] - (a == b ? 1.0f : 0.0f)));
+    if (!(e < 1e-3f)) radius = INFINITY;
   }
+  if (q != 0) return;
 #pragma unroll
   for (int a = 0; a < 9; a++) G[a] = g[a];
-  k.detG[i] = g[0] * (g[4] * g[8] - g[7] * g[5]) - g[3] * (g[1] * g[8] - g[7] * g[2]) + g[6] * (g[1] * g[5] - g[4] * g[2]);
+  xb[0] = b0;
+  xb[1] = b1;
+  xb[2] = b2;
+  const float det = g[0] * (g[4] * g[8] - g[7] * g[5]) - g[3] * (g[1] * g[8] - g[7] * g[2]) + g[6] * (g[1] * g[5] - g[4] * g[2]);
+  rec[0] = make_float4(b0, b1, b2, det);
+  rec[1] = make_float4(g[0], g[1], g[2], radius);
+  rec[2] = make_float4(g[3], g[4], g[5], __int_as_float(v[0]));
+  rec[3] = make_float4(g[6], g[7], g[8], __int_as_float(v[1]));
+  rec[4] = make_float4(__int_as_float(v[2]), x0, x1, x2);
 }
 
 // The blocks the two field passes write: every vertex >= 0 of the particle's
@@ -513,159 +586,299 @@ __global__ void k_mark(K k) {
   }
 }
 
-// The field at the vertices of one 8^3 tile, one thread per vertex, summed
-// over every particle whose boxes can reach the tile: the particles of voxels
-// c in [T - R + off, T + 7 + off] per axis (T = the tile's first vertex).  The
-// workgroup lists the candidate voxel columns and their particle counts (a
-// scan in LDS), then stages the candidates' data in LDS 512 at a time (each
-// thread finds its candidate's column by bisection), and every thread adds
-// what each staged particle gives its vertex: the poly6 value when
-// |v - c_j| <= 1 per axis, the anisotropic value times the multiplicity of the
-// reference's voxel-corner loop when v is in j's box.  The contributions are
-// 2^-32 fixed-point integers, so the sum is the one any order of the
-// reference's atomics would give exactly.  Tiles of unwritten blocks store 0.
+// The field at the vertices of one 8^3 tile, one workgroup of 8 wavefronts per
+// tile.  All contributions are 2^-32 fixed-point integers, so their sum is the
+// one any order of the reference's atomics would give exactly.
+//
+// FIELD_ANISO: the anisotropic values of the particles whose boxes reach the
+// tile (voxels c in [T - R + off, T + 7 + off] per axis, T the tile's first
+// vertex).  The workgroup lists the candidate voxel columns and their particle
+// counts, stages the candidates' records in LDS 512 at a time, dropping those
+// whose support radius ends before the tile, and each wavefront takes every
+// eighth of them: a lane holds the 8 vertices of one (x, y) column, so the
+// x and y parts of G d are formed once for 8 values, a vertex plane outside
+// the particle's box is skipped by the whole wavefront, and the multiplicity
+// of the reference's voxel-corner loop is a shift (1, 2, 4 or 8).  The
+// wavefronts' sums meet in LDS.  What bounds it is VALU issue: about 45
+// instructions a value, in 26 of every 33 planes and 26^2 of every 33^2
+// columns; 128,000 particles take 4.3 ms against 10.7 with one vertex per
+// lane and every candidate evaluated at all 512.
+// The fixed-point form of v: the double v + 1.5 2^20 has an ulp of 2^-32, so
+// its bits less those of 1.5 2^20 are rint(v 2^32), for |v| < 2^19.  Each lane
+// adds up |v|; only if some total reaches 2^19 or is not a number is the tile
+// summed again in the general form (fix_of, with its error flag).
+//
+// FIELD_VELOCITY: the poly6-weighted velocity of the particles within h
+// (generate_smooth_fluid_field_with_velocity_impl, :1160-1190), same layout.
+//
+// Every tile then has the isotropic poly6 values added (in FIELD_ANISO or, for
+// the isotropic field, FIELD_ISO), one thread per vertex over the 27 voxels
+// around it.  Tiles of unwritten blocks store 0.
+enum { FIELD_ISO = 0, FIELD_ANISO = 1, FIELD_VELOCITY = 2 };
 constexpr int TILE = 8;
-constexpr int GATHER_THREADS = TILE * TILE * TILE;
+constexpr int FIELD_THREADS = TILE * TILE * TILE;
+constexpr int FIELD_WAVES = FIELD_THREADS / 64;
 constexpr int MAX_COLS = 1536;  // (TILE + R)^2 columns, R + 1 <= 32
-__global__ __launch_bounds__(GATHER_THREADS) void k_field(K k) {
-  __shared__ int col_off[MAX_COLS + 1];
-  __shared__ int col_begin[MAX_COLS];
-  __shared__ float s_pos[3][GATHER_THREADS], s_xb[3][GATHER_THREADS], s_g[9][GATHER_THREADS], s_det[GATHER_THREADS];
-  __shared__ int s_c[3][GATHER_THREADS];
-  __shared__ float s_vel[3][GATHER_THREADS];
+constexpr float FIX_ROOM = 524288.0f;  // 2^19
+
+__device__ __forceinline__ unsigned long long fix_fast(float v) {
+  const double t = (double)v + 1572864.0;  // 1.5 2^20
+  return (unsigned long long)__double_as_longlong(t) - 0x4138000000000000ull;
+}
+
+// multiplicity of axis position v for a particle of voxel c, as a shift: 0, 1, or -1 for none
+__device__ __forceinline__ int mult_shift(int v, int c, int off, int R) { return mult_axis(v, c, off, R) - 1; }
+
+// cubic_spline_kernel (:1115-1124) at q = |G d|, "+ 1" where the reference puts it
+__device__ __forceinline__ float aniso_of(float c48d, float c16d, float q) {
+  const float in = c48d * (q * q * q - q * q) + 1.0f;
+  const float out = c16d * (1.0f - q) * (1.0f - q) * (1.0f - q);
+  const float r = q <= 0.5f ? in : out;
+  return 0.0f < q && q <= 1.0f ? r : 0.0f;
+}
+
+// one staged particle's values at the 8 vertices of each lane's column
+template <bool GENERAL>
+__device__ __forceinline__ void aniso_column(const K& k, const float4 (&r)[REC_QUADS], const int* T, int vx, int vy, float px,
+                                             float py, unsigned long long (&acc)[TILE], float& total, bool& bad) {
+  const int c0 = uniform(__float_as_int(r[2].w)), c1 = uniform(__float_as_int(r[3].w)), c2 = uniform(__float_as_int(r[4].x));
+  const int sx = mult_shift(vx, c0, k.off, k.R), sy = mult_shift(vy, c1, k.off, k.R);
+  if (sx < 0 || sy < 0) return;
+  const int sxy = sx + sy;
+  const float dx = r[0].x - px, dy = r[0].y - py;
+  const float ta = r[1].x * dx + r[1].y * dy, tb = r[2].x * dx + r[2].y * dy, tc = r[3].x * dx + r[3].y * dy;
+  const float c48d = k.c48 * r[0].w, c16d = k.c16 * r[0].w;
+#pragma unroll
+  for (int z = 0; z < TILE; z++) {
+    const int sz = mult_shift(T[2] + z, c2, k.off, k.R);
+    if (sz < 0) continue;  // uniform
+    const float dz = r[0].z - ((float)(T[2] + z) * k.vs + k.o[2]);
+    const float a = ta + r[1].z * dz, b = tb + r[2].z * dz, c = tc + r[3].z * dz;
+    const float ss = a * a + b * b + c * c;
+    if (!GENERAL && __all(ss > 1.0f)) continue;  // q = 1 gives 0 too
+    float q = GENERAL ? sqrtf(ss) : sqrt_mid(ss);
+    if (!GENERAL && __builtin_expect(ss < 1e-30f, 0)) q = sqrtf(ss);
+    const float w = k.vol * aniso_of(c48d, c16d, q);
+    if (GENERAL) {
+      if (!(fabsf(w) <= MAX_CONTRIB)) bad = true;
+      else acc[z] += fix_of(w) << (sxy + sz);
+    } else {
+      total += fabsf(w);
+      acc[z] += fix_fast(w) << (sxy + sz);
+    }
+  }
+}
+
+// one staged particle's poly6-weighted velocity at the 8 vertices of each lane's column
+__device__ __forceinline__ void velocity_column(const K& k, const float4& p4, const float4& v4, int c0, int c1, const int* T,
+                                                int vx, int vy, float px, float py, unsigned long long (&acc)[3][TILE],
+                                                bool& bad) {
+  const int sx = mult_shift(vx, c0, k.off, k.R), sy = mult_shift(vy, c1, k.off, k.R);
+  if (sx < 0 || sy < 0) return;
+  const int c2 = uniform(__float_as_int(p4.x));
+  const float rx = p4.y - px, ry = p4.z - py;
+  if (__all(rx * rx + ry * ry > 1.0001f * k.sr * k.sr)) return;
+#pragma unroll
+  for (int z = 0; z < TILE; z++) {
+    const int sz = mult_shift(T[2] + z, c2, k.off, k.R);
+    if (sz < 0) continue;
+    const float rz = p4.w - ((float)(T[2] + z) * k.vs + k.o[2]);
+    if (fabsf(rz) > 1.0001f * k.sr) continue;  // uniform; poly6 is 0 there
+    const float f = poly6(k, rx, ry, rz, k.sr) * k.cvs3;
+    const float u[3] = {v4.x * f, v4.y * f, v4.z * f};
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      if (!(fabsf(u[c]) <= MAX_CONTRIB)) bad = true;
+      else acc[c][z] += fix_of(u[c]) << (sx + sy + sz);
+    }
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(FIELD_THREADS) void k_field(K k) {
+  constexpr int QUADS = MODE == FIELD_VELOCITY ? 3 : REC_QUADS;
+  __shared__ int col_off[MODE == FIELD_ISO ? 1 : MAX_COLS + 1];
+  __shared__ int col_begin[MODE == FIELD_ISO ? 1 : MAX_COLS];
+  __shared__ float4 stage[MODE == FIELD_ISO ? 1 : QUADS * FIELD_THREADS];
+  __shared__ unsigned long long sum[MODE == FIELD_VELOCITY ? 3 : 1][FIELD_THREADS];
+  __shared__ int wave_tot[FIELD_WAVES];
+  __shared__ int kept;
   const int tb = blockIdx.x;
   const int tdy = k.gdim[1] / TILE, tdz = k.gdim[2] / TILE;
   const int tx = tb / (tdy * tdz), ty = (tb / tdz) % tdy, tz = tb % tdz;
   const int t = threadIdx.x;
-  const int gx = tx * TILE + (t >> 6), gy = ty * TILE + ((t >> 3) & 7), gz = tz * TILE + (t & 7);
-  const long q = gidx(k, gx, gy, gz);
+  const long q = gidx(k, tx * TILE + (t >> 6), ty * TILE + ((t >> 3) & 7), tz * TILE + (t & 7));
   if (!k.active[bidx(k, tx * TILE, ty * TILE, tz * TILE)]) {  // a tile lies in one block
-    k.acc[q] = 0ull;
-    if (k.vel)
-      for (int c = 0; c < 3; c++) k.vacc[3 * q + c] = 0ull;
+    if (MODE == FIELD_VELOCITY) {
+      for (int c = 0; c < 3; c++) k.vfield[3 * q + c] = 0.0f;
+    } else {
+      k.field0[q] = 0.0f;
+      k.field[q] = 0.0f;
+    }
     return;
   }
-  const int vx = gx + k.glo[0], vy = gy + k.glo[1], vz = gz + k.glo[2];
-  float p[3];
-  vpos(k, vx, vy, vz, p);
-  const int R = k.R, off = k.off;
   const int T[3] = {tx * TILE + k.glo[0], ty * TILE + k.glo[1], tz * TILE + k.glo[2]};
-  unsigned long long va[3] = {0ull, 0ull, 0ull};
-  int clo[3], chi[3];
-  for (int a = 0; a < 3; a++) {
-    clo[a] = k.aniso ? T[a] - R + off : T[a] - 1;
-    chi[a] = k.aniso ? T[a] + TILE - 1 + off : T[a] + TILE;
-    clo[a] = max(clo[a], k.vlo[a]);
-    chi[a] = min(chi[a], k.vlo[a] + k.vdim[a] - 1);
-  }
-  const int ncx = max(0, chi[0] - clo[0] + 1), ncy = max(0, chi[1] - clo[1] + 1);
-  const int ncol = clo[2] <= chi[2] ? ncx * ncy : 0;  // <= MAX_COLS (checked on the host)
-  // columns: particle counts, then an inclusive scan (Hillis-Steele over
-  // GATHER_THREADS-wide rounds with a carry)
-  int carry = 0;
-  for (int c0 = 0; c0 < ncol; c0 += GATHER_THREADS) {
-    const int c = c0 + t;
-    int cnt = 0;
-    if (c < ncol) {
-      const int cx = clo[0] + c / ncy, cy = clo[1] + c % ncy;
-      const long base = ((long)(cx - k.vlo[0]) * k.vdim[1] + (cy - k.vlo[1])) * k.vdim[2] - k.vlo[2];
-      const int b = k.vstart[base + clo[2]], e = k.vstart[base + chi[2] + 1];
-      col_begin[c] = b;
-      cnt = e - b;
-    }
-    __shared__ int scan[GATHER_THREADS];
-    scan[t] = cnt;
-    __syncthreads();
-    for (int d = 1; d < GATHER_THREADS; d <<= 1) {
-      const int u = t >= d ? scan[t - d] : 0;
-      __syncthreads();
-      scan[t] += u;
-      __syncthreads();
-    }
-    if (c < ncol) col_off[c + 1] = carry + scan[t];
-    if (c0 == 0 && t == 0) col_off[0] = 0;
-    carry += scan[GATHER_THREADS - 1];
-    __syncthreads();
-  }
-  const int total = ncol > 0 ? carry : 0;
-  unsigned long long acc = 0ull;
+  const int R = k.R, off = k.off;
   bool bad = false;
-  for (int s0 = 0; s0 < total; s0 += GATHER_THREADS) {
-    const int idx = s0 + t;
-    if (idx < total) {
-      int lo = 0, hi = ncol - 1;  // the column c with col_off[c] <= idx < col_off[c + 1]
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (col_off[mid] <= idx) lo = mid;
-        else hi = mid - 1;
+  if (MODE == FIELD_VELOCITY)
+    for (int c = 0; c < 3; c++) sum[c][t] = 0ull;
+  if (MODE != FIELD_VELOCITY) {  // the isotropic part, one vertex per thread
+    const int vx = T[0] + (t >> 6), vy = T[1] + ((t >> 3) & 7), vz = T[2] + (t & 7);
+    float p[3];
+    vpos(k, vx, vy, vz, p);
+    const int z0 = max(vz - 1, k.vlo[2]), z1 = min(vz + 1, k.vlo[2] + k.vdim[2] - 1);
+    unsigned long long acc = 0ull;
+    if (z0 <= z1)
+      for (int x = max(vx - 1, k.vlo[0]); x <= min(vx + 1, k.vlo[0] + k.vdim[0] - 1); x++)
+        for (int y = max(vy - 1, k.vlo[1]); y <= min(vy + 1, k.vlo[1] + k.vdim[1] - 1); y++) {
+          const long base = ((long)(x - k.vlo[0]) * k.vdim[1] + (y - k.vlo[1])) * k.vdim[2] - k.vlo[2];
+          for (int m = k.vstart[base + z0]; m < k.vstart[base + z1 + 1]; m++) {
+            const float* xj = k.pos + 3 * (long)k.vlist[m];
+            const float w = k.vol * poly6(k, xj[0] - p[0], xj[1] - p[1], xj[2] - p[2], k.sr);
+            if (!(fabsf(w) <= MAX_CONTRIB)) bad = true;
+            else acc += fix_of(w);
+          }
+        }
+    sum[0][t] = acc;
+  }
+  if constexpr (MODE != FIELD_ISO) {
+    // candidate columns: the voxels whose boxes (or, for the velocities, whose
+    // spheres of h) can reach the tile
+    const int near = (int)(k.sr / k.vs) + 2;
+    int clo[3], chi[3];
+    for (int a = 0; a < 3; a++) {
+      clo[a] = T[a] - R + off;
+      chi[a] = T[a] + TILE - 1 + off;
+      if (MODE == FIELD_VELOCITY) {
+        clo[a] = max(clo[a], T[a] - near);
+        chi[a] = min(chi[a], T[a] + TILE - 1 + near);
       }
-      const int j = k.vlist[col_begin[lo] + (idx - col_off[lo])];
-      s_pos[0][t] = k.pos[3 * (long)j];
-      s_pos[1][t] = k.pos[3 * (long)j + 1];
-      s_pos[2][t] = k.pos[3 * (long)j + 2];
-      s_c[0][t] = k.pvox[3 * (long)j];
-      s_c[1][t] = k.pvox[3 * (long)j + 1];
-      s_c[2][t] = k.pvox[3 * (long)j + 2];
-      if (k.aniso) {
-        s_xb[0][t] = k.xbar[3 * (long)j];
-        s_xb[1][t] = k.xbar[3 * (long)j + 1];
-        s_xb[2][t] = k.xbar[3 * (long)j + 2];
+      clo[a] = max(clo[a], k.vlo[a]);
+      chi[a] = min(chi[a], k.vlo[a] + k.vdim[a] - 1);
+    }
+    const int ncx = max(0, chi[0] - clo[0] + 1), ncy = max(0, chi[1] - clo[1] + 1);
+    const int ncol = clo[2] <= chi[2] ? ncx * ncy : 0;  // <= MAX_COLS (checked on the host)
+    // their particle counts, scanned: wavefront scans, then the wavefronts' totals
+    int carry = 0;
+    if (t == 0) col_off[0] = 0;
+    for (int c0 = 0; c0 < ncol; c0 += FIELD_THREADS) {
+      const int c = c0 + t;
+      int cnt = 0;
+      if (c < ncol) {
+        const int cx = clo[0] + c / ncy, cy = clo[1] + c % ncy;
+        const long base = ((long)(cx - k.vlo[0]) * k.vdim[1] + (cy - k.vlo[1])) * k.vdim[2] - k.vlo[2];
+        const int b = k.vstart[base + clo[2]];
+        col_begin[c] = b;
+        cnt = k.vstart[base + chi[2] + 1] - b;
+      }
+      int incl = cnt;
 #pragma unroll
-        for (int a = 0; a < 9; a++) s_g[a][t] = k.G[9 * (long)j + a];
-        s_det[t] = k.detG[j];
-        if (k.vel)
-          for (int a = 0; a < 3; a++) s_vel[a][t] = k.vel[3 * (long)j + a];
+      for (int d = 1; d < 64; d <<= 1) {
+        const int u = __shfl_up(incl, d, 64);
+        if ((t & 63) >= d) incl += u;
       }
+      __syncthreads();  // the previous round's totals are read
+      if ((t & 63) == 63) wave_tot[t >> 6] = incl;
+      __syncthreads();
+      int before = carry, all = 0;
+      for (int w = 0; w < FIELD_WAVES; w++) {
+        if (w < (t >> 6)) before += wave_tot[w];
+        all += wave_tot[w];
+      }
+      if (c < ncol) col_off[c + 1] = before + incl;
+      carry += all;
     }
     __syncthreads();
-    const int nst = min(GATHER_THREADS, total - s0);
-#pragma unroll 4
-    for (int r = 0; r < nst; r++) {
-      const int c0 = s_c[0][r], c1 = s_c[1][r], c2 = s_c[2][r];
-      if (abs(vx - c0) <= 1 && abs(vy - c1) <= 1 && abs(vz - c2) <= 1) {
-        const float w = k.vol * poly6(k, s_pos[0][r] - p[0], s_pos[1][r] - p[1], s_pos[2][r] - p[2], k.sr);
-        if (!(fabsf(w) <= MAX_CONTRIB)) bad = true;
-        else acc += fix_of(w);
-      }
-      if (!k.aniso) continue;
-      const int mm = mult_axis(vx, c0, off, R) * mult_axis(vy, c1, off, R) * mult_axis(vz, c2, off, R);
-      if (mm == 0) continue;
-      float g[9];
-#pragma unroll
-      for (int a = 0; a < 9; a++) g[a] = s_g[a][r];
-      const float w = k.vol * aniso_w(k, g, s_det[r], s_xb[0][r] - p[0], s_xb[1][r] - p[1], s_xb[2][r] - p[2]);
-      if (!(fabsf(w) <= MAX_CONTRIB)) bad = true;
-      else acc += (unsigned long long)mm * fix_of(w);
-      if (k.vel) {  // generate_smooth_fluid_field_with_velocity_impl (:1160-1190)
-        const float f = poly6(k, s_pos[0][r] - p[0], s_pos[1][r] - p[1], s_pos[2][r] - p[2], k.sr) * k.cvs3;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          const float u = s_vel[c][r] * f;
-          if (!(fabsf(u) <= MAX_CONTRIB)) bad = true;
-          else va[c] += (unsigned long long)mm * fix_of(u);
-        }
-      }
+    const int total = carry;
+    const int lane = t & 63, wave = uniform(t >> 6);
+    const int vx = T[0] + (lane >> 3), vy = T[1] + (lane & 7);
+    const float px = (float)vx * k.vs + k.o[0], py = (float)vy * k.vs + k.o[1];
+    // the tile's box of vertices
+    float tlo[3], thi[3];
+    for (int a = 0; a < 3; a++) {
+      tlo[a] = (float)T[a] * k.vs + k.o[a];
+      thi[a] = (float)(T[a] + TILE - 1) * k.vs + k.o[a];
     }
+    unsigned long long acc[MODE == FIELD_VELOCITY ? 3 : 1][TILE];
+    // a second round, in the general form, only where the first was out of range
+    for (int round = 0; round < 2; round++) {
+      for (int c = 0; c < (MODE == FIELD_VELOCITY ? 3 : 1); c++)
+#pragma unroll
+        for (int z = 0; z < TILE; z++) acc[c][z] = 0ull;
+      float abs_total = 0.0f;
+      for (int s0 = 0; s0 < total; s0 += FIELD_THREADS) {
+        if (t == 0) kept = 0;
+        __syncthreads();
+        const int idx = s0 + t;
+        if (idx < total) {
+          int lo = 0, hi = ncol - 1;  // the column c with col_off[c] <= idx < col_off[c + 1]
+          while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (col_off[mid] <= idx) lo = mid;
+            else hi = mid - 1;
+          }
+          const int m = col_begin[lo] + (idx - col_off[lo]);
+          const float4* rec = k.rec + (long)REC_QUADS * m;
+          if (MODE == FIELD_ANISO) {
+            const float4 r0 = rec[0], r1 = rec[1];
+            const float gx = fmaxf(0.0f, fmaxf(tlo[0] - r0.x, r0.x - thi[0]));
+            const float gy = fmaxf(0.0f, fmaxf(tlo[1] - r0.y, r0.y - thi[1]));
+            const float gz = fmaxf(0.0f, fmaxf(tlo[2] - r0.z, r0.z - thi[2]));
+            const bool out = r1.w < 0.0f || gx * gx + gy * gy + gz * gz > 1.001f * r1.w * r1.w;
+            if (!out) {
+              const int at = atomicAdd(&kept, 1);
+              stage[at] = r0;
+              stage[FIELD_THREADS + at] = r1;
+              stage[2 * FIELD_THREADS + at] = rec[2];
+              stage[3 * FIELD_THREADS + at] = rec[3];
+              stage[4 * FIELD_THREADS + at] = rec[4];
+            }
+          } else {
+            const int at = atomicAdd(&kept, 1);
+            const float* u = k.vel + 3 * (long)k.vlist[m];
+            stage[at] = rec[4];
+            stage[FIELD_THREADS + at] = make_float4(u[0], u[1], u[2], 0.0f);
+            stage[2 * FIELD_THREADS + at] = make_float4(rec[2].w, rec[3].w, 0.0f, 0.0f);
+          }
+        }
+        __syncthreads();
+        const int nst = kept;
+        for (int r = wave; r < nst; r += FIELD_WAVES) {
+          if constexpr (MODE == FIELD_ANISO) {
+            float4 rr[REC_QUADS];
+#pragma unroll
+            for (int e = 0; e < REC_QUADS; e++) rr[e] = stage[e * FIELD_THREADS + r];
+            if (round == 0) aniso_column<false>(k, rr, T, vx, vy, px, py, acc[0], abs_total, bad);
+            else aniso_column<true>(k, rr, T, vx, vy, px, py, acc[0], abs_total, bad);
+          } else {
+            const float4 c4 = stage[2 * FIELD_THREADS + r];
+            velocity_column(k, stage[r], stage[FIELD_THREADS + r], uniform(__float_as_int(c4.x)), uniform(__float_as_int(c4.y)),
+                            T, vx, vy, px, py, acc, bad);
+          }
+        }
+        __syncthreads();
+      }
+      if (MODE != FIELD_ANISO || !__syncthreads_or(!(abs_total < FIX_ROOM))) break;
+    }
+    for (int c = 0; c < (MODE == FIELD_VELOCITY ? 3 : 1); c++)
+#pragma unroll
+      for (int z = 0; z < TILE; z++) atomicAdd(&sum[c][(lane << 3) + z], acc[c][z]);
     __syncthreads();
   }
-  k.acc[q] = acc;
-  if (k.vel)
-    for (int c = 0; c < 3; c++) k.vacc[3 * q + c] = va[c];
+  if (MODE == FIELD_VELOCITY) {
+    for (int c = 0; c < 3; c++) k.vfield[3 * q + c] = (float)((double)(long long)sum[c][t] * FIX_INV);
+  } else {
+    const float v = (float)((double)(long long)sum[0][t] * FIX_INV);
+    k.field0[q] = v;
+    k.field[q] = v;
+  }
   if (bad) atomicOr(k.err, ERR_RANGE);
 }
 
-__global__ void k_convert(K k) {
-  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= k.nvert) return;
-  const int gz = (int)(q % k.gdim[2]), gy = (int)((q / k.gdim[2]) % k.gdim[1]), gx = (int)(q / ((long)k.gdim[1] * k.gdim[2]));
-  float v = 0.0f;
-  if (k.active[bidx(k, gx, gy, gz)]) v = (float)((double)(long long)k.acc[q] * FIX_INV);
-  k.field0[q] = v;
-  k.field[q] = v;
-  if (k.vel) {
-    const bool act = k.active[bidx(k, gx, gy, gz)];
-    for (int c = 0; c < 3; c++) k.vfield[3 * q + c] = act ? (float)((double)(long long)k.vacc[3 * q + c] * FIX_INV) : 0.0f;
-  }
+// a velocity that is not finite gives no finite contribution anywhere in its particle's box
+__global__ void k_check_velocities(K k) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 3L * k.n && !isfinite(k.vel[i])) atomicOr(k.err, ERR_RANGE);
 }
 
 // Blocked FP64 statistic of the negative values, one workgroup per block in
@@ -1144,10 +1357,10 @@ struct Surface {
   nn_surface_params prm{};
   K k{};
   hipStream_t st = nullptr;
-  DBuf<float> pos, vel, G, xbar, detG, field0, field, tmp, verts, normals, vfield, mvel;
+  DBuf<float> pos, vel, G, xbar, field0, field, tmp, verts, normals, vfield, mvel;
   DBuf<int> vcount, vstart, vslot, vlist, pvox, flag, cube_id, tcount, tstart, faces, err, bounds, scratch;
   DBuf<unsigned char> active;
-  DBuf<unsigned long long> acc, vacc;
+  DBuf<float4> rec;
   DBuf<double> stats, part;
   DBuf<long long> pcount;
   long nverts = 0, ntris = 0, nactive = 0;
@@ -1156,12 +1369,11 @@ struct Surface {
   int64_t budget = 0;  // device bytes a run may use (0 = no limit)
 
   ~Surface() {
-    for (auto* b : {&pos, &vel, &G, &xbar, &detG, &field0, &field, &tmp, &verts, &normals, &vfield, &mvel}) b->release();
+    for (auto* b : {&pos, &vel, &G, &xbar, &field0, &field, &tmp, &verts, &normals, &vfield, &mvel}) b->release();
     for (auto* b : {&vcount, &vstart, &vslot, &vlist, &pvox, &flag, &cube_id, &tcount, &tstart, &faces, &err, &bounds, &scratch})
       b->release();
     active.release();
-    acc.release();
-    vacc.release();
+    rec.release();
     stats.release();
     part.release();
     pcount.release();
@@ -1303,9 +1515,8 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   SR_HIP(S.pvox.ensure(3 * n), "nn_surface_run: alloc");
   SR_HIP(S.G.ensure(9 * n), "nn_surface_run: alloc");
   SR_HIP(S.xbar.ensure(3 * n), "nn_surface_run: alloc");
-  SR_HIP(S.detG.ensure(n), "nn_surface_run: alloc");
+  if (k.aniso) SR_HIP(S.rec.ensure(REC_QUADS * (size_t)n), "nn_surface_run: alloc");
   SR_HIP(S.active.ensure(nblock), "nn_surface_run: alloc");
-  SR_HIP(S.acc.ensure(nvert), "nn_surface_run: alloc");
   SR_HIP(S.field0.ensure(nvert), "nn_surface_run: alloc");
   SR_HIP(S.field.ensure(nvert), "nn_surface_run: alloc");
   SR_HIP(S.tmp.ensure(nvert), "nn_surface_run: alloc");
@@ -1316,9 +1527,7 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   SR_HIP(S.part.ensure(nblock), "nn_surface_run: alloc");
   SR_HIP(S.pcount.ensure(nblock), "nn_surface_run: alloc");
   if (k.vel) {
-    SR_HIP(S.vacc.ensure(3 * nvert), "nn_surface_run: alloc");
     SR_HIP(S.vfield.ensure(3 * nvert), "nn_surface_run: alloc");
-    k.vacc = S.vacc.p;
     k.vfield = S.vfield.p;
   }
   k.vcount = S.vcount.p;
@@ -1328,9 +1537,8 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   k.pvox = S.pvox.p;
   k.G = S.G.p;
   k.xbar = S.xbar.p;
-  k.detG = S.detG.p;
+  k.rec = S.rec.p;
   k.active = S.active.p;
-  k.acc = S.acc.p;
   k.field0 = S.field0.p;
   k.field = S.field.p;
   k.tmp = S.tmp.p;
@@ -1346,11 +1554,19 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   hipLaunchKernelGGL(k_vsort, dim3(grid1(nvox, 256)), dim3(256), 0, S.st, k);
   if ((rc = device_error(S))) return rc;
   // anisotropic kernel and field
-  if (k.aniso) hipLaunchKernelGGL(k_aniso, dim3(grid1(n, 64)), dim3(64), 0, S.st, k);
+  if (k.aniso) {
+    if (n <= ANISO_WIDE) hipLaunchKernelGGL(k_aniso<16>, dim3(grid1(16 * n, ANISO_THREADS)), dim3(ANISO_THREADS), 0, S.st, k);
+    else hipLaunchKernelGGL(k_aniso<4>, dim3(grid1(4 * n, ANISO_THREADS)), dim3(ANISO_THREADS), 0, S.st, k);
+  }
   hipLaunchKernelGGL(k_fill_u8, dim3(grid1(nblock, 256)), dim3(256), 0, S.st, k.active, nblock);
   hipLaunchKernelGGL(k_mark, dim3(grid1(n, 256)), dim3(256), 0, S.st, k);
-  hipLaunchKernelGGL(k_field, dim3((unsigned)(nvert / GATHER_THREADS)), dim3(GATHER_THREADS), 0, S.st, k);
-  hipLaunchKernelGGL(k_convert, dim3(grid1(nvert, 256)), dim3(256), 0, S.st, k);
+  const dim3 tiles((unsigned)(nvert / FIELD_THREADS)), ft(FIELD_THREADS);
+  if (k.aniso) hipLaunchKernelGGL(k_field<FIELD_ANISO>, tiles, ft, 0, S.st, k);
+  else hipLaunchKernelGGL(k_field<FIELD_ISO>, tiles, ft, 0, S.st, k);
+  if (k.vel) {
+    hipLaunchKernelGGL(k_check_velocities, dim3(grid1(3 * n, 256)), dim3(256), 0, S.st, k);
+    hipLaunchKernelGGL(k_field<FIELD_VELOCITY>, tiles, ft, 0, S.st, k);
+  }
   if ((rc = device_error(S))) return rc;
   // smoothing
   hipLaunchKernelGGL(k_stats, dim3((unsigned)nblock), dim3(ST_THREADS), 0, S.st, k, 0, S.part.p, S.pcount.p);
@@ -1504,6 +1720,7 @@ int32_t nn_surface_create(const nn_surface_params* p, nn_surface** out) {
   k.c2pi = (float)(2 * M_PI);
   k.cvs3 = (float)(p->voxel_size * p->voxel_size * p->voxel_size);
   k.aniso = p->anisotropic ? 1 : 0;
+  k.mid = k.sr >= 0x1p-20f && k.sr <= 0x1p20f ? 1 : 0;
   k.R = (int)ceilf(4.0f * k.sr / k.vs) + 1;  // smooth_range, :1137
   k.off = k.R / 2;
   if (k.aniso && (k.R < 1 || k.R + 1 > nn::sr::BLOCK)) {

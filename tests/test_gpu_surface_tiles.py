@@ -1,0 +1,98 @@
+"""The field's tiles and the grouped anisotropy against the oracle bit for bit
+where they branch: one and two particles, particle counts on both sides of the
+lanes' limit, particles exactly on grid vertices, a cluster whose
+contributions are too large for the tiles' short fixed-point form (and one
+beyond the range that is an error), a smooth radius outside the range of the
+short square roots, and a velocity that is not finite."""
+import numpy as np
+import pytest
+
+from nonnewton_amd import _lib as L
+from nonnewton_amd.surface import Surface
+from oracle import surface as O
+
+pytestmark = pytest.mark.gpu
+
+
+def check(x, vel=None, **kw):
+    s = Surface(velocity=vel is not None, **kw)
+    info = s.run(x, vel)
+    o = O.reconstruct(x, velocity=vel, **kw) if vel is not None else O.reconstruct(x, **kw)
+    if kw.get("anisotropic", True):
+        G, xb = s.aniso()
+        assert np.array_equal(G, o["G"], equal_nan=True) and np.array_equal(xb, o["xbar"])
+    assert np.array_equal(s.field(0), o["field0"])
+    assert np.array_equal(s.field(1), o["field"], equal_nan=True)
+    v, f, _ = s.mesh()
+    assert np.array_equal(v, o["vertices"]) and np.array_equal(f, o["faces"])
+    s.close()
+    return info, o
+
+
+def block(n, seed, sp=0.02, frac=0.15):
+    a = max(1, int(round(n ** (1 / 3))))
+    k = np.arange(n)
+    x = np.stack([k // (a * a), k // a % a, k % a], 1) * sp + 0.21
+    return (x + np.random.Generator(np.random.PCG64(seed)).uniform(-frac * sp, frac * sp, x.shape)).astype(np.float32)
+
+
+@pytest.mark.parametrize("n", [1, 2, 17, 1000, 32768, 32769])
+def test_counts(n):
+    check(block(n, n), voxel_size=0.02, particle_radius=0.02, smooth_radius=0.04, normals=True)
+
+
+@pytest.mark.parametrize("aniso", [True, False])
+def test_particles_on_vertices(aniso):
+    """An exact lattice whose points are vertices: zero offsets from them."""
+    g = np.arange(9) * np.float32(0.03125) + np.float32(0.25)
+    x = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3).astype(np.float32)
+    check(x, voxel_size=0.015625, particle_radius=0.03, smooth_radius=0.0625, anisotropic=aniso,
+          isolevel=0.0 if aniso else 0.2, smooth_iterations=1 if aniso else 0)
+
+
+def cluster(std):
+    rng = np.random.Generator(np.random.PCG64(11))
+    x = np.array([0.4, 0.4, 0.4]) + rng.normal(0, std, (400, 3))
+    return np.concatenate([0.9 + rng.uniform(0, 0.3, (20, 3)), x]).astype(np.float32)
+
+
+def test_large_contributions():
+    """About 4e5 a value and 6e7 a vertex: the tile is summed in the general form."""
+    _, o = check(cluster(0.0025), voxel_size=0.01, particle_radius=0.02, smooth_radius=0.06)
+    assert np.abs(o["field0"]).max() > 2.0 ** 25
+
+
+def test_contributions_out_of_range():
+    with pytest.raises(L.NNError) as e:
+        s = Surface(voxel_size=0.01, particle_radius=0.02, smooth_radius=0.06)
+        s.run(cluster(0.002))
+    assert e.value.code == L.NN_E_NAN
+
+
+@pytest.mark.parametrize("n", [20, 300])
+@pytest.mark.parametrize("scale", [2.0 ** -17, 2.0 ** 26])
+def test_smooth_radius_outside_the_midrange(scale, n):
+    """20 particles have too few neighbors for an anisotropic kernel; those of
+    300 are far out of range at these scales, which the oracle refuses too."""
+    x = (block(n, 5) * np.float32(scale)).astype(np.float32)
+    kw = dict(voxel_size=0.015625 * scale, particle_radius=0.02 * scale, smooth_radius=0.0625 * scale)
+    if n == 20:
+        check(x, **kw)
+        return
+    with pytest.raises(O.SurfaceError):
+        O.reconstruct(x, **kw)
+    with pytest.raises(L.NNError) as e:
+        Surface(**kw).run(x)
+    assert e.value.code == L.NN_E_NAN
+
+
+def test_velocity_not_finite():
+    x = block(200, 6)
+    v = np.zeros_like(x)
+    s = Surface(voxel_size=0.02, particle_radius=0.02, smooth_radius=0.05, velocity=True)
+    s.run(x, v)
+    v[77, 1] = np.inf
+    with pytest.raises(L.NNError) as e:
+        s.run(x, v)
+    assert e.value.code == L.NN_E_NAN
+    s.close()
