@@ -71,19 +71,23 @@ def test_contributions_out_of_range():
 
 @pytest.mark.parametrize("n", [20, 300])
 @pytest.mark.parametrize("scale", [2.0 ** -17, 2.0 ** 26])
-def test_smooth_radius_outside_the_midrange(scale, n):
-    """20 particles have too few neighbors for an anisotropic kernel; those of
-    300 are far out of range at these scales, which the oracle refuses too."""
+def test_scales_whose_kernels_overflow_are_refused(scale, n):
+    """h^9 leaves FP32: the oracle refuses these, and so does the device."""
     x = (block(n, 5) * np.float32(scale)).astype(np.float32)
     kw = dict(voxel_size=0.015625 * scale, particle_radius=0.02 * scale, smooth_radius=0.0625 * scale)
-    if n == 20:
-        check(x, **kw)
-        return
     with pytest.raises(O.SurfaceError):
         O.reconstruct(x, **kw)
     with pytest.raises(L.NNError) as e:
         Surface(**kw).run(x)
     assert e.value.code == L.NN_E_NAN
+
+
+def test_smooth_radius_below_the_midrange():
+    """h = 2^-22 in a coarse grid: no vertex lies within h of a particle, but
+    the particles, some 1e-7 apart, are each other's neighbors."""
+    rng = np.random.Generator(np.random.PCG64(8))
+    x = (0.01 + rng.uniform(-2e-7, 2e-7, (30, 3))).astype(np.float32)
+    check(x, voxel_size=0.5, particle_radius=0.02, smooth_radius=2.0 ** -22)
 
 
 def test_velocity_not_finite():
