@@ -141,6 +141,7 @@ class Batch {
   int C_cap_ = 0;    // cells allocated
   int scene_cap_ = 0;
   int n_cg_blocks_ = 0;  // entries of d.cg_blocks
+  int solve_waves_ = -1;  // waves k_cg_solve may have (-1: not looked up yet)
   std::vector<void*> deferred_;
   int scan_blocks_ = 0;
   SceneState* h_state_ = nullptr;  // pinned, h_state_cap_ entries
@@ -162,6 +163,8 @@ class Batch {
   // 2 complete
   int lists_state_ = 0;
   int solver_loop(int which);
+  int cg_start();
+  int cg_solve(bool& done);
   int cg_loop();
   int build_stress_set(const std::vector<int>& which);
   int gather_state();

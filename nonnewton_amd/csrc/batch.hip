@@ -523,8 +523,8 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   A(nd.partials, 32 * (size_t)nd.W);
   int2* cgb = nullptr;
   A(cgb, (size_t)nd.W / CG_UPD_WAVES + Sc + 1);
-  A(nd.cg_list, 2 * (size_t)nd.W);
-  A(nd.cg_list_n, 2);
+  A(nd.cg_list, 3 * (size_t)nd.W);
+  A(nd.cg_list_n, 3);
   A(nd.n_active, 4);
   A(nd.wx, Pc);
   A(nd.wr, Pc);
@@ -1003,24 +1003,60 @@ int Batch::solver_loop(int which) {
   return NN_OK;
 }
 
-// The Weiler CG iterations: update k (which first forms the scene sums of
-// iteration k - 1 and stops converged scenes) and matvec k, for k = 1 ..
-// limit, then update limit + 1, which only tests the last residual.  Enqueued
-// in chunks -- first the previous step's iteration count plus two, then four
-// -- with one 4-byte read of the active-scene counter per chunk; iterations
-// past convergence are near-empty launches.
+// The Weiler CG.  A batch of one scene of few waves (with a workgroup for each
+// and no more than the compute units): one launch, k_cg_solve, which may give
+// up waiting.  An iteration then takes 6.3 us at 27 waves, 7.0 at 102 and 8.0
+// at 222, against 13 to 15 as two launches.  Otherwise update k (which first forms
+// the scene sums of iteration k - 1 and stops converged scenes) and matvec k,
+// for k = 1 .. limit, then update limit + 1, which only tests the last
+// residual.  Enqueued in chunks -- first the previous step's iteration count
+// plus two, then four -- with one 4-byte read of the active-scene counter per
+// chunk; iterations past convergence are near-empty launches.
+int Batch::cg_start() {
+  h_active_[3] = 0;
+  launch_solver_begin(dref(), 2, stream);
+  TIMED(K_CG_INIT, launch_cg_init(dref(), blk(K_CG_INIT), stream));
+  if (any_warm_cg_) launch_scene_finish(dref(), 4, 1, stream);
+  TIMED(K_CG_GUESS, launch_cg_guess(dref(), blk(K_CG_GUESS), stream));
+  TIMED(K_CG_MATVEC, launch_cg_matvec_start(dref(), blk(K_CG_MATVEC), dep(K_CG_MATVEC), stream));
+  launch_scene_finish(dref(), 2, 1, stream);
+  return NN_OK;
+}
+
+int Batch::cg_solve(bool& done) {
+  done = false;
+  if (solve_waves_ < 0) {  // its workgroups wait for one another: no more than compute units
+    int dev = 0, cus = 0;
+    HIPCHK(hipGetDevice(&dev));
+    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    solve_waves_ = std::min(cus, CG_SOLVE_WAVES);
+  }
+  if (dep(K_CG_MATVEC) != 0) return NN_OK;  // a gather depth was asked for: it is k_cg_matvec's
+  if (scenes.size() != 1 || scenes[0]->dev.wave_begin != 0 || scenes[0]->dev.wave_end > solve_waves_) return NN_OK;
+  if (timer.on) timer.seen[K_CG_UPDATE]++;  // one launch does the work of both
+  TIMED(K_CG_MATVEC, launch_cg_solve(dref(), scenes[0]->dev.wave_end, stream));
+  HIPCHK(hipMemcpyAsync(h_active_, d.n_active, 4 * sizeof(int), hipMemcpyDeviceToHost, stream));
+  HIPCHK(hipStreamSynchronize(stream));
+  done = h_active_[3] == 0;
+  if (!done) solve_waves_ = 0;  // the device is shared: this batch does not try again
+  return NN_OK;
+}
+
 int Batch::cg_loop() {
   int pred = 1;
-  long total_waves = 0;
+  long last_waves = 0;
   for (auto& sp : scenes) {
-    pred = std::max(pred, sp->last_iter[2]);
     const int f = sp->dev.flags;
-    if ((f & SF_HAS_FLUID) && (f & SF_VISCOSITY) && (f & SF_WEILER)) total_waves += sp->dev.wave_end - sp->dev.wave_begin;
+    if (!((f & SF_HAS_FLUID) && (f & SF_VISCOSITY) && (f & SF_WEILER))) continue;
+    if (sp->last_iter[2] > pred) last_waves = 0;
+    pred = std::max(pred, sp->last_iter[2]);
+    if (sp->last_iter[2] == pred) last_waves += sp->dev.wave_end - sp->dev.wave_begin;
   }
   // waves expected to still iterate at iteration k, from each scene's count
-  // in the previous step (plus a margin): while they are many the matvec runs
-  // on the full grid, once they are few on a grid sized to them (the list of
-  // waves the update writes holds the exact set either way)
+  // in the previous step (plus a margin; past every count, the scenes that had
+  // the most): the matvec's grid (its list of waves holds the exact set either
+  // way; a grid of 64 workgroups for a scene of 131,072 particles that iterated
+  // longer than it had before took 141 us a product instead of 16)
   auto expected_waves = [&](int k) {
     long w = 0;
     for (auto& sp : scenes) {
@@ -1028,7 +1064,7 @@ int Batch::cg_loop() {
       if ((f & SF_HAS_FLUID) && (f & SF_VISCOSITY) && (f & SF_WEILER) && sp->last_iter[2] + 2 >= k)
         w += sp->dev.wave_end - sp->dev.wave_begin;
     }
-    return w;
+    return std::max(w, last_waves);
   };
   const int maxit = std::max(1, max_iter_[2]);
   const int last = maxit + 1;
@@ -1037,13 +1073,7 @@ int Batch::cg_loop() {
     for (int c = 0; c < chunk && k <= last; c++, k++) {
       TIMED(K_CG_UPDATE, launch_cg_update(dref(), n_cg_blocks_, k, stream));
       if (k > maxit) continue;
-      const long ew = expected_waves(k);
-      if (4 * ew >= total_waves) {
-        TIMED(K_CG_MATVEC, launch_cg_matvec(dref(), blk(K_CG_MATVEC), dep(K_CG_MATVEC), 0, stream));
-      } else {
-        const int grid = (int)std::min<long>(std::max<long>(ew, 64), 2048);
-        TIMED(K_CG_MATVEC, launch_cg_matvec_list(dref(), dep(K_CG_MATVEC), k, grid, stream));
-      }
+      TIMED(K_CG_MATVEC, launch_cg_matvec(dref(), dep(K_CG_MATVEC), k, (int)expected_waves(k), stream));
     }
     if (k > last) break;
     HIPCHK(hipMemcpyAsync(h_active_, d.n_active + 2, sizeof(int), hipMemcpyDeviceToHost, stream));
@@ -1076,13 +1106,13 @@ int Batch::step(std::vector<nn_step_stats>* stats) {
     }
     if (any_strain_) TIMED(K_STRAIN, launch_strain(dref(), blk(K_STRAIN), lanes(K_STRAIN), dep(K_STRAIN), stream));
     if (any_weiler_) {
-      launch_solver_begin(dref(), 2, stream);
-      TIMED(K_CG_INIT, launch_cg_init(dref(), blk(K_CG_INIT), stream));
-      if (any_warm_cg_) launch_scene_finish(dref(), 4, 1, stream);
-      TIMED(K_CG_GUESS, launch_cg_guess(dref(), blk(K_CG_GUESS), stream));
-      TIMED(K_CG_MATVEC, launch_cg_matvec(dref(), blk(K_CG_MATVEC), dep(K_CG_MATVEC), 1, stream));
-      launch_scene_finish(dref(), 2, 1, stream);
-      CHK(cg_loop());
+      CHK(cg_start());
+      bool done = false;
+      CHK(cg_solve(done));
+      if (!done) {
+        if (h_active_[3]) CHK(cg_start());  // given up by k_cg_solve: from the start again
+        CHK(cg_loop());
+      }
     }
     TIMED(K_NONPRESSURE, launch_nonpressure(dref(), blk(K_NONPRESSURE), lanes(K_NONPRESSURE), dep(K_NONPRESSURE), stream));
     std::swap(d.vel, d.vel_alt);

@@ -330,18 +330,18 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 
 // Per-scene FP64 reductions, first stage: every wavefront of a participating
-// scene stores its NR partial sums into partial arrays base..base+NR-1 (plain
-// stores, no fences).  The second stage is k_scene_finish, one workgroup per
-// scene in the next launch, which adds the partials in a fixed order: the
-// totals are the same on every run and do not depend on the order in which
-// wavefronts ran.
-template <int NR>
-__device__ __forceinline__ void wave_partials(const Dev& d, int wave, double (&v)[NR], int base = 0) {
+// scene stores the sums of its particles' NR values (each held by the lane 0,
+// or by all, of a particle's G lanes) in partial arrays base..base+NR-1, G
+// entries per 64 particles (plain stores, no fences).  A later launch adds
+// them in a fixed order: the totals are the same on every run and do not
+// depend on the order in which wavefronts ran.
+template <int G, int NR>
+__device__ __forceinline__ void lane_partials(const Dev& d, int i, double (&v)[NR], int base) {
 #pragma unroll
-  for (int r = 0; r < NR; r++) v[r] = wave_sum(v[r]);
+  for (int r = 0; r < NR; r++) v[r] = tree_sum<G>(v[r]);
   if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-    for (int r = 0; r < NR; r++) d.partials[(long)(base + r) * 4 * d.W + wave] = v[r];
+    for (int r = 0; r < NR; r++) d.partials[(long)(base + r) * 4 * d.W + i / (64 / G)] = v[r];
   }
 }
 

@@ -167,13 +167,13 @@ struct Dev {
   int* cell_count;
   int* cell_start;
   int* scan_tmp;
-  double* partials;  // 8 arrays of 4W: wave partials (per 64 particles, or per 16 for four-lane sweeps)
+  double* partials;  // 8 arrays of 4W: wave partials (per 64 particles, or per 16 for four-lane sweeps; the solvers' 16-lane sweeps fill 16W)
   int2* wave_pairs;  // list entries of a wavefront's particles: (of fluid and dynamic solids, of fluid)
   float* wave_rho;   // largest density of a wavefront's particles; both one entry per lane of a particle and 64 slots
   const int2* cg_blocks;  // CG update workgroups: (scene, first wave), up to CG_UPD_WAVES waves of one scene each
-  int* cg_list;           // 2 x W: waves of the scenes still iterating, by iteration parity
-  int* cg_list_n;         // 2 counts
-  int* n_active;     // [0] divergence, [1] pressure, [2] cg
+  int* cg_list;           // 3 x W: waves of the scenes that iteration k leaves iterating, at k % 3
+  int* cg_list_n;         // 3 counts
+  int* n_active;     // [0] divergence, [1] pressure, [2] cg, [3] k_cg_solve gave up waiting
   // Weiler CG: 3-vectors packed at 12 bytes (the sweeps stream them and the
   // matvec gathers u and the position of every neighbor)
   float3* wx;  // iterate x
@@ -266,9 +266,11 @@ void launch_solver_begin(const DevRef& d, int which, hipStream_t st);
 void launch_strain(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_cg_init(const DevRef& d, int block, hipStream_t st);
 void launch_cg_guess(const DevRef& d, int block, hipStream_t st);
-void launch_cg_matvec(const DevRef& d, int block, int depth, int start, hipStream_t st);  // depth 1, 2, 4, 8
-void launch_cg_matvec_list(const DevRef& d, int depth, int k, int grid, hipStream_t st);  // iteration k
+void launch_cg_matvec_start(const DevRef& d, int block, int depth, hipStream_t st);  // depth 1, 2, 4, 8
 void launch_cg_update(const DevRef& d, int nblocks, int k, hipStream_t st);  // iteration k >= 1
+void launch_cg_matvec(const DevRef& d, int depth, int k, int grid, hipStream_t st);
+constexpr int CG_SOLVE_WAVES = 256;  // one workgroup per compute unit of the device
+void launch_cg_solve(const DevRef& d, int waves, hipStream_t st);  // the whole solve of a batch of one scene
 void launch_nonpressure(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_press_source(const DevRef& d, int block, int lanes, int depth, int reduce, hipStream_t st);
 void launch_press_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st);

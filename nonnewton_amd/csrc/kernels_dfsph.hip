@@ -168,12 +168,15 @@ __global__ void k_solver_begin(Dev d, int which) {
       st.iter_cg = 0;
       st.cg_rr = 0.0;
       st.cg_bb = 0.0;
-      if (s == 0) d.cg_list_n[0] = d.cg_list_n[1] = 0;
+      if (s == 0) d.cg_list_n[0] = d.cg_list_n[1] = d.cg_list_n[2] = 0;
     }
     if (act) atomicAdd(&cnt, 1);
   }
   __syncthreads();
-  if (threadIdx.x == 0) d.n_active[which] = cnt;
+  if (threadIdx.x == 0) {
+    d.n_active[which] = cnt;
+    if (which == 2) d.n_active[3] = 0;
+  }
 }
 
 // sum_j of the velocity changes both solvers' updates make (:1721-1760,
@@ -208,14 +211,6 @@ __device__ __forceinline__ void velocity_push(const Dev& d, const SceneDev& sc, 
         ay += t[1];
         az += t[2];
       });
-}
-
-// One value per particle (held by its G lanes) summed over the particles of a
-// wavefront into partial array 0, entry G w + ... of 64-particle wave w.
-template <int G>
-__device__ __forceinline__ void lane_partial(const Dev& d, int i, double v) {
-  v = tree_sum<G>(v);
-  if ((threadIdx.x & 63) == 0) d.partials[i / (64 / G)] = v;
 }
 
 // divergence_solver_iteration_kernel, :1721-1760 (Jacobi: reads rho-dot and
@@ -271,16 +266,16 @@ __global__ void k_div_source(Dev d) {
   const SceneDev& sc = d.scenes[s];
   SceneState* st = d.state + s;
   if (!st->active_v) return;
-  double v = 0.0;
+  double v[1] = {0.0};
   if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
     int cnt;
     float rd = velocity_divergence<G, B>(d, sc, i, q, d.pos[i], cnt);
     rd = rd > 0.0f ? rd : 0.0f;
     if (cnt < 20) rd = 0.0f;
     if (q == 0) d.sa[i].x = rd;
-    v = (double)sc.rho0 * (double)rd - 0.0;
+    v[0] = (double)sc.rho0 * (double)rd - 0.0;
   }
-  lane_partial<G>(d, i, v);
+  lane_partials<G, 1>(d, i, v, 0);
 }
 
 // non-pressure forces (:1557-1567): surface tension (:1378-1414) and the
@@ -450,16 +445,16 @@ __global__ void k_press_source(Dev d, int reduce) {
   const SceneDev& sc = d.scenes[s];
   SceneState* st = d.state + s;
   if (!st->active_p) return;
-  double v = 0.0;
+  double v[1] = {0.0};
   if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
     int cnt;
     const float delta = velocity_divergence<G, B>(d, sc, i, q, d.pos[i], cnt);
     float da = d.rho[i] / sc.rho0 + sc.dt * delta;
     da = da > 1.0f ? da : 1.0f;
     if (q == 0) d.sa[i].x = da;
-    v = (double)sc.rho0 * (double)da - sc.rho0_d;
+    v[0] = (double)sc.rho0 * (double)da - sc.rho0_d;
   }
-  if (reduce) lane_partial<G>(d, i, v);
+  if (reduce) lane_partials<G, 1>(d, i, v, 0);
 }
 
 // Second stage of the per-scene reductions: one FINISH_THREADS-thread workgroup
@@ -471,10 +466,10 @@ __global__ void k_press_source(Dev d, int reduce) {
 // (The CG's per-iteration reduction is done inside k_cg_update.)
 // Thread t adds entries t, t + FINISH_THREADS, ... in order (two interleaved
 // chains); the wavefront sums are combined by a fixed pairwise tree: a fixed
-// order, the same bits every run.  The solvers' sweeps leave `lanes` partials
-// per 64 particles (lane_partial), which are first added by the tree the
-// sweep's wavefront would have continued, so an entry has the same bits for
-// every number of lanes.
+// order, the same bits every run.  A sweep with several lanes per particle
+// leaves that many partials per 64 particles (`lanes` of the solvers' sweeps),
+// which are first added by the tree that sweep's wavefront would have
+// continued, so an entry has the same bits for every number of lanes.
 constexpr int FINISH_THREADS = NN_FINISH_THREADS;
 constexpr int FINISH_WAVES = FINISH_THREADS / 64;
 
@@ -493,19 +488,17 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
     default: part = weiler && (sc.flags & SF_WARM_CG); break;  // 4
   }
   if (!part) return;  // uniform over the workgroup
-  // partial arrays read and their granularity (4 = four-lane sweep, a
-  // partial per 16 particles)
+  // partial arrays read, and the entries each has per 64 particles (cg_init
+  // and the first matvec, array 3, run four lanes per particle)
   const int nr = which == 2 ? 4 : (which == 4 ? 2 : 1);
-  const bool solver = which == 0 || which == 1;
   double tot[4] = {0.0, 0.0, 0.0, 0.0};
   for (int r = 0; r < nr; r++) {
-    // the first matvec's partials (array 3) and cg_init's are per 16 particles
-    const int g = which == 4 ? 4 : (which == 2 ? (r == 3 ? 4 : 1) : 1);
+    const int per = which < 2 ? lanes : (which == 4 || r == 3 ? 4 : 1);
     const double* src = d.partials + (long)r * 4 * d.W;
-    const int lo = g * sc.wave_begin, hi = g * sc.wave_end;
+    const int lo = sc.wave_begin, hi = sc.wave_end;
     auto entry = [&](int k) {
-      if (!solver || lanes == 1) return src[k];
-      if (lanes == 4) return (src[4 * k] + src[4 * k + 1]) + (src[4 * k + 2] + src[4 * k + 3]);
+      if (per == 1) return src[k];
+      if (per == 4) return (src[4 * k] + src[4 * k + 1]) + (src[4 * k + 2] + src[4 * k + 3]);
       double v[16];
 #pragma unroll
       for (int e = 0; e < 16; e++) v[e] = src[16 * k + e];
@@ -526,7 +519,6 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
     if ((t & 63) == 0) red[r][t >> 6] = w;
   }
   __syncthreads();
-  if (t != 0) return;
   for (int r = 0; r < nr; r++) {  // fixed pairwise tree over the wave sums
     double w[FINISH_WAVES];
 #pragma unroll
@@ -537,6 +529,7 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
       for (int q = 0; q + span < FINISH_WAVES; q += 2 * span) w[q] += w[q + span];
     tot[r] = w[0];
   }
+  if (t != 0) return;
   if (which == 0) {
     const double err = tot[0] / sc.nf_d;
     const int ran = st->iter_v + 1;
