@@ -1218,6 +1218,17 @@ int Batch::download(int k, int field, void* host, size_t bytes) {
     return NN_E_ARG;
   }
   if (field == NN_FIELD_NUM_NEIGHBORS) CHK(complete_lists());
+  // three-component fields: into original order on the device (vel_alt is free
+  // between steps), then one copy
+  if (field == NN_FIELD_X || field == NN_FIELD_V || field == NN_FIELD_ACCELERATION || field == NN_FIELD_VISC_DIFF) {
+    const float4* p = field == NN_FIELD_V ? d.vel : field == NN_FIELD_ACCELERATION ? d.acc : field == NN_FIELD_VISC_DIFF ? d.vdiff : d.pos;
+    float* ordered = reinterpret_cast<float*>(d.vel_alt + pb);
+    launch_gather3(p + pb, d.inv + pb, n, ordered, stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(host, ordered, bytes, hipMemcpyDeviceToHost, stream));
+    HIPCHK(hipStreamSynchronize(stream));
+    return NN_OK;
+  }
   std::vector<int> info(n);
   HIPCHK(hipMemcpyAsync(info.data(), d.info + pb, sizeof(int) * n, hipMemcpyDeviceToHost, stream));
   float* out = (float*)host;
@@ -1243,26 +1254,11 @@ int Batch::download(int k, int field, void* host, size_t bytes) {
   std::vector<float> f1;
   std::vector<int> i1;
   switch (field) {
-    case NN_FIELD_X:
-    case NN_FIELD_V:
-    case NN_FIELD_ACCELERATION:
-    case NN_FIELD_VISC_DIFF:
-    case NN_FIELD_VOLUME: {
-      const float4* p = field == NN_FIELD_V ? d.vel : field == NN_FIELD_ACCELERATION ? d.acc
-                        : field == NN_FIELD_VISC_DIFF ? d.vdiff : d.pos;
-      HIPCHK(slot_f4(p, f4));
+    case NN_FIELD_VOLUME:
+      HIPCHK(slot_f4(d.pos, f4));
       HIPCHK(hipStreamSynchronize(stream));
-      for (int t = 0; t < n; t++) {
-        const int id = info[t] & 0x0FFFFFFF;
-        if (field == NN_FIELD_VOLUME) out[id] = std::fabs(f4[t].w);
-        else {
-          out[3 * id] = f4[t].x;
-          out[3 * id + 1] = f4[t].y;
-          out[3 * id + 2] = f4[t].z;
-        }
-      }
+      for (int t = 0; t < n; t++) out[info[t] & 0x0FFFFFFF] = std::fabs(f4[t].w);
       return NN_OK;
-    }
     case NN_FIELD_X0:
     case NN_FIELD_REST_VOLUME: {
       f4.resize(n);
@@ -1354,20 +1350,11 @@ int Batch::upload_field(int k, int field, const void* host, size_t bytes) {
     set_error("only x, v and the Weiler warm-start direction (float[n][3]) can be uploaded");
     return NN_E_ARG;
   }
-  std::vector<int> info(n);
-  std::vector<float4> f4(n);
   float4* p = field == NN_FIELD_X ? d.pos : field == NN_FIELD_V ? d.vel : d.vdiff;
-  HIPCHK(hipMemcpyAsync(info.data(), d.info + pb, sizeof(int) * n, hipMemcpyDeviceToHost, stream));
-  HIPCHK(hipMemcpyAsync(f4.data(), p + pb, sizeof(float4) * n, hipMemcpyDeviceToHost, stream));
-  HIPCHK(hipStreamSynchronize(stream));
-  const float* in = (const float*)host;
-  for (int t = 0; t < n; t++) {
-    const int id = info[t] & 0x0FFFFFFF;
-    f4[t].x = in[3 * id];
-    f4[t].y = in[3 * id + 1];
-    f4[t].z = in[3 * id + 2];
-  }
-  HIPCHK(hipMemcpyAsync(p + pb, f4.data(), sizeof(float4) * n, hipMemcpyHostToDevice, stream));
+  float* ordered = reinterpret_cast<float*>(d.vel_alt + pb);  // free between steps
+  HIPCHK(hipMemcpyAsync(ordered, host, bytes, hipMemcpyHostToDevice, stream));
+  launch_scatter3(ordered, d.inv + pb, n, p + pb, stream);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(stream));
   return NN_OK;
 }
