@@ -526,4 +526,17 @@ __device__ __forceinline__ float nn_model(const SceneDev& c, float gam) {
   return eta;
 }
 
+// The 9 runs' bounds from the lanes that loaded them, to every lane.
+template <int G, int R>
+__device__ __forceinline__ void run_table(const int* lo, const int* len, int base, int* first, int* shift, int& total) {
+  if constexpr (R < 9) {
+    const int b = __float_as_int(lane_bcast<G, R % G>(__int_as_float(lo[R / G])));
+    const int n = __float_as_int(lane_bcast<G, R % G>(__int_as_float(len[R / G])));
+    first[R] = total;
+    shift[R] = b + base - total;
+    total += n;
+    run_table<G, R + 1>(lo, len, base, first, shift, total);
+  }
+}
+
 }  // namespace nn

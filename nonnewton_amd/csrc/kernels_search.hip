@@ -40,8 +40,8 @@ void launch_fill_f4(float4* p, long n, float4 v, hipStream_t st) {
 
 // Fields of float[n][3] in original order (inv: slot of an id).  Reordered by
 // the host, particle by particle over two arrays copied each way, an upload of
-// 138,304 particles took 0.4 ms and a download 0.25 ms; the kernels take 3 to
-// 5 us and the copies what the link needs for 12 bytes a particle.
+// 168,218 particles took 402 us and a download 360 us; through these kernels
+// (3 to 5 us) and one copy of 12 bytes a particle, 86 and 152 us.
 __global__ void k_gather3(const float4* slots, const int* inv, int n, float* ordered) {
   const int id = blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= n) return;
@@ -231,19 +231,6 @@ __global__ void k_place(Dev d) {
   d.info_alt[dest] = inf;
   if (sc.flags & SF_WARM_CG) d.vdiff_alt[dest] = d.vdiff[i];
   d.inv[sc.p_begin + my] = dest - sc.p_begin;
-}
-
-// The 9 runs' bounds from the lanes that loaded them, to every lane.
-template <int G, int R>
-__device__ __forceinline__ void run_table(const int* lo, const int* len, int base, int* first, int* shift, int& total) {
-  if constexpr (R < 9) {
-    const int b = __float_as_int(lane_bcast<G, R % G>(__int_as_float(lo[R / G])));
-    const int n = __float_as_int(lane_bcast<G, R % G>(__int_as_float(len[R / G])));
-    first[R] = total;
-    shift[R] = b + base - total;
-    total += n;
-    run_table<G, R + 1>(lo, len, base, first, shift, total);
-  }
 }
 
 // store_neighbors, SPH/main.py:836-847, over the sorted particles.  With

@@ -2,8 +2,8 @@
 // (meta.ns.run_search() + meta.ns.neighbors, SPH/main.py:815-847) for
 // positions already in device memory, written to device memory, with no
 // device allocation: the search's scratch (cell counts, cell starts, scan
-// partials, cell keys, the particles in cell order) lives in one file-scope
-// __device__ array per device, at a fixed maximum size.
+// partials, cell keys, the particles by cell and in cell order) lives in one
+// file-scope __device__ array per device, at a fixed maximum size.
 //
 // Order and test are those of the context's search: cell = truncation of x / h
 // (pos_to_index, :805-807), the 27 cells visited dx slowest and dz fastest,
@@ -14,18 +14,21 @@
 #include <mutex>
 
 #include "batch.h"
+#include "device_common.h"
 
 namespace nn {
 
 constexpr long NA_MAX_PARTICLES = 1L << 20;
 constexpr long NA_MAX_CELLS = 1L << 22;
+constexpr int NA_WIDE = 131072;  // up to here 16 lanes per particle (Batch::lanes of the search)
 constexpr long na_round(long w) { return (w + 63) / 64 * 64; }  // 256-byte sections
 constexpr long NA_COUNTS = 0;                                                  // NA_MAX_CELLS + 1 ints
 constexpr long NA_STARTS = NA_COUNTS + na_round(NA_MAX_CELLS + 1);             // NA_MAX_CELLS + 1 ints
 constexpr long NA_SUMS = NA_STARTS + na_round(NA_MAX_CELLS + 1);               // scan partials
 constexpr long NA_KEY = NA_SUMS + na_round((NA_MAX_CELLS + 1 + SCAN_TILE_ITEMS - 1) / SCAN_TILE_ITEMS);
-constexpr long NA_SORTED = NA_KEY + na_round(NA_MAX_PARTICLES);                // particles in cell order
-constexpr long NA_WORDS = NA_SORTED + na_round(NA_MAX_PARTICLES);              // 10.5M ints = 42 MB
+constexpr long NA_BUCKET = NA_KEY + na_round(NA_MAX_PARTICLES);                // particles by cell, in arrival order
+constexpr long NA_SORTED = NA_BUCKET + na_round(NA_MAX_PARTICLES);             // float4 (x, index) in cell order
+constexpr long NA_WORDS = NA_SORTED + 4 * na_round(NA_MAX_PARTICLES);          // 14.7M ints = 59 MB
 
 // The scratch of nn_neighbors_noalloc.  Host code never names it directly:
 // scratch_base() returns the device's address from hipGetSymbolAddress.
@@ -46,86 +49,122 @@ __device__ __forceinline__ int na_key(const float* x, int i, float h, int g0, in
   return (cx * g1 + cy) * g2 + cz;
 }
 
-__global__ void k_na_count(const float* x, int n, float h, int g0, int g1, int g2, int* key, int* counts,
-                           int* status) {
+// Cell key and arrival rank in the cell (kept in the sorted section, which is
+// written only after the ranks were read).  A particle outside the grid is in
+// no cell: its list is empty.
+__global__ void k_na_count(const float* x, int n, float h, int g0, int g1, int g2, int* key, int* counts, int* arrival,
+                           int* nbr, int* count, int cap, int* status) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int k = na_key(x, i, h, g0, g1, g2);
   key[i] = k;
-  if (k < 0) atomicOr(status, ST_OUT_OF_GRID);
-  else atomicAdd(&counts[k], 1);
-}
-
-// every particle into its cell's range (in arrival order; k_na_order sorts)
-__global__ void k_na_bucket(const int* key, int n, const int* starts, int* cursor, int* sorted) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int k = key[i];
-  if (k >= 0) sorted[starts[k] + atomicAdd(&cursor[k], 1)] = i;
-}
-
-// one thread per cell: its particles in increasing index (insertion sort of
-// at most MAX_PIC entries; a fuller cell is reported and left unsorted)
-__global__ void k_na_order(const int* starts, int ncells, int* sorted, int* status) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncells) return;
-  const int b = starts[c], e = starts[c + 1];
-  if (e - b > MAX_PIC) {
-    atomicOr(status, ST_CELL_OVERFLOW);
+  if (k >= 0) {
+    arrival[i] = atomicAdd(&counts[k], 1);
     return;
   }
-  for (int a = b + 1; a < e; a++) {
-    const int v = sorted[a];
-    int q = a - 1;
-    while (q >= b && sorted[q] > v) {
-      sorted[q + 1] = sorted[q];
-      q--;
-    }
-    sorted[q + 1] = v;
-  }
+  atomicOr(status, ST_OUT_OF_GRID);
+  for (int m = 0; m < cap; m++) nbr[(long)i * cap + m] = -1;
+  count[i] = 0;
 }
 
-// store_neighbors (:836-847) for particle i in caller order: the 9 runs of
-// (cx+dx, cy+dy, cz-1..cz+1) cells in cell order, -1 padding up to cap
-__global__ void k_na_lists(const float* x, int n, float h, float thr2, int g0, int g1, int g2, const int* key,
-                           const int* starts, const int* sorted, int* nbr, int* count, int cap, int* status) {
+// every particle into its cell's range, in arrival order
+__global__ void k_na_bucket(const int* key, int n, const int* starts, const int* arrival, int* bucket) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  int* row = nbr + (long)i * cap;
-  int cnt = 0;
   const int k = key[i];
-  if (k >= 0) {
-    const int cz = k % g2, cy = (k / g2) % g1, cx = k / (g1 * g2);
-    const float xi = x[3 * (long)i], yi = x[3 * (long)i + 1], zi = x[3 * (long)i + 2];
-    const int z0 = cz > 0 ? cz - 1 : 0;
-    const int z1 = cz + 1 < g2 ? cz + 1 : g2 - 1;
-    for (int dx = -1; dx <= 1; dx++) {
-      const int a = cx + dx;
-      if (a < 0 || a >= g0) continue;
-      for (int dy = -1; dy <= 1; dy++) {
-        const int bb = cy + dy;
-        if (bb < 0 || bb >= g1) continue;
-        const int base = (a * g1 + bb) * g2;
-        const int j0 = starts[base + z0], j1 = starts[base + z1 + 1];
-        for (int t = j0; t < j1; t++) {
-          const int j = sorted[t];
-          if (j == i) continue;
-          const float ex = xi - x[3 * (long)j], ey = yi - x[3 * (long)j + 1], ez = zi - x[3 * (long)j + 2];
-          const float ss = ex * ex + ey * ey + ez * ez;
-          if (ss < thr2) {
-            if (cnt < MAX_NB) row[cnt] = j;
-            cnt++;
-          }
-        }
-      }
+  if (k >= 0) bucket[starts[k] + arrival[i]] = i;
+}
+
+// Position and index into cell order: a particle's place in its cell is the
+// number of lower indices there (a cell with more than MAX_PIC particles is
+// reported and left in arrival order).  One thread per cell sorting its range
+// by insertion took 27 us for 200,000 particles, a serial chain through memory
+// per cell, and left the lists to gather each position through its index; this
+// and the arrival order take 7.5 + 3.7 us.
+__global__ void k_na_place(const float* x, const int* starts, int ncells, const int* key, const int* bucket,
+                           float4* sorted, int* status) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= starts[ncells]) return;
+  const int i = bucket[t];
+  const int k = key[i];
+  const int b = starts[k], e = starts[k + 1];
+  int dest = t;
+  if (e - b > MAX_PIC) {
+    atomicOr(status, ST_CELL_OVERFLOW);
+  } else {
+    dest = b;
+    for (int a = b; a < e; a++) dest += bucket[a] < i;
+  }
+  sorted[dest] = make_float4(x[3 * (long)i], x[3 * (long)i + 1], x[3 * (long)i + 2], __int_as_float(i));
+}
+
+// store_neighbors (:836-847) for the particle in place t of the cell order: the
+// 9 runs of (cx+dx, cy+dy, cz-1..cz+1) cells, -1 padding up to cap.  G lanes
+// per particle share the runs as in the context's search (k_build_lists).  With
+// one thread per particle in caller order each candidate was a dependent index
+// load and a gather of 3 floats: 198 us for 200,000 particles, now 59, of
+// which writing the 48 MB of rows is 11.
+template <int G, int B>
+__global__ void k_na_lists(float thr2, int g0, int g1, int g2, const int* key, const int* starts,
+                           const float4* sorted, int* nbr, int* count, int cap, int* status) {
+  const long tid = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = (int)(tid / G), q = (int)(tid % G);
+  if (t >= starts[g0 * g1 * g2]) return;
+  const float4 xi = sorted[t];
+  const int i = __float_as_int(xi.w);
+  int* row = nbr + (long)i * cap;
+  const int k = key[i];
+  const int cz = k % g2, cy = (k / g2) % g1, cx = k / (g1 * g2);
+  const int z0 = cz > 0 ? cz - 1 : 0;
+  const int z1 = cz + 1 < g2 ? cz + 1 : g2 - 1;
+  constexpr int RL = (9 + G - 1) / G;  // runs whose bounds a lane loads
+  int lo[RL], len[RL];
+#pragma unroll
+  for (int e = 0; e < RL; e++) {
+    const int r = q + e * G;
+    const int a = cx + r / 3 - 1, b = cy + r % 3 - 1;
+    lo[e] = len[e] = 0;
+    if (r < 9 && a >= 0 && a < g0 && b >= 0 && b < g1) {
+      const int base = (a * g1 + b) * g2;
+      lo[e] = starts[base + z0];
+      len[e] = starts[base + z1 + 1] - lo[e];
+    }
+  }
+  int first[9], shift[9], total = 0;
+  run_table<G, 0>(lo, len, 0, first, shift, total);
+  const int lane = threadIdx.x & 63;
+  const int below = (1 << q) - 1;
+  int cnt = 0;
+  for (int c0 = 0; c0 < total; c0 += G * B) {
+    int p[B];
+    float4 xj[B];
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      const int c = c0 + u * G + q;
+      int sh = shift[0];
+#pragma unroll
+      for (int r = 1; r < 9; r++) sh = c >= first[r] ? shift[r] : sh;
+      p[u] = c < total ? c + sh : t;
+    }
+#pragma unroll
+    for (int u = 0; u < B; u++) xj[u] = sorted[p[u]];
+#pragma unroll
+    for (int u = 0; u < B; u++) {
+      const float ex = xi.x - xj[u].x, ey = xi.y - xj[u].y, ez = xi.z - xj[u].z;
+      const float ss = ex * ex + ey * ey + ez * ez;
+      const bool hit = ss < thr2 && p[u] != t;
+      const int hits = (int)(__ballot(hit) >> (lane & ~(G - 1))) & ((1 << G) - 1);
+      const int at = cnt + __popc(hits & below);
+      cnt += __popc(hits);
+      if (hit && at < MAX_NB) row[at] = __float_as_int(xj[u].w);
     }
   }
   if (cnt > MAX_NB) {
-    atomicOr(status, ST_NEIGHBOR_OVERFLOW);
+    if (q == 0) atomicOr(status, ST_NEIGHBOR_OVERFLOW);
     cnt = MAX_NB;
   }
-  for (int m = cnt; m < cap; m++) row[m] = -1;
-  count[i] = cnt;
+  for (int m = cnt + q; m < cap; m += G) row[m] = -1;
+  if (q == 0) count[i] = cnt;
 }
 
 // Address of this device's scratch, looked up once per device with the device
@@ -200,7 +239,9 @@ extern "C" int32_t nn_neighbors_noalloc(const nn_params* params, const float* x,
   int* starts = base + NA_STARTS;
   int* sums = base + NA_SUMS;
   int* key = base + NA_KEY;
-  int* sorted = base + NA_SORTED;
+  int* bucket = base + NA_BUCKET;
+  float4* sorted = reinterpret_cast<float4*>(base + NA_SORTED);
+  int* arrival = base + NA_SORTED;
   const int nc = (int)cells;
   const int ni = (int)n;
   const int T = 256;
@@ -208,15 +249,19 @@ extern "C" int32_t nn_neighbors_noalloc(const nn_params* params, const float* x,
   hipLaunchKernelGGL(k_na_zero, dim3((unsigned)((nc + 1 + T - 1) / T)), dim3(T), 0, st, counts, (long)nc + 1, status);
   if (ni > 0) {
     hipLaunchKernelGGL(k_na_count, dim3((ni + T - 1) / T), dim3(T), 0, st, x, ni, hf, (int)g[0], (int)g[1], (int)g[2],
-                       key, counts, status);
+                       key, counts, arrival, nbr, count, cap, status);
   }
   launch_scan_i32(counts, nc + 1, sums, starts, st);
   if (ni > 0) {
-    hipLaunchKernelGGL(k_na_zero, dim3((unsigned)((nc + T - 1) / T)), dim3(T), 0, st, counts, (long)nc, nullptr);
-    hipLaunchKernelGGL(k_na_bucket, dim3((ni + T - 1) / T), dim3(T), 0, st, key, ni, starts, counts, sorted);
-    hipLaunchKernelGGL(k_na_order, dim3((nc + T - 1) / T), dim3(T), 0, st, starts, nc, sorted, status);
-    hipLaunchKernelGGL(k_na_lists, dim3((ni + T - 1) / T), dim3(T), 0, st, x, ni, hf, thr2, (int)g[0], (int)g[1],
-                       (int)g[2], key, starts, sorted, nbr, count, cap, status);
+    const dim3 per_particle((ni + T - 1) / T);
+    hipLaunchKernelGGL(k_na_bucket, per_particle, dim3(T), 0, st, key, ni, starts, arrival, bucket);
+    hipLaunchKernelGGL(k_na_place, per_particle, dim3(T), 0, st, x, starts, nc, key, bucket, sorted, status);
+    const auto lists = [&](auto kern, int lanes) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)(((long)ni * lanes + T - 1) / T)), dim3(T), 0, st, thr2, (int)g[0],
+                         (int)g[1], (int)g[2], key, starts, sorted, nbr, count, cap, status);
+    };
+    if (ni <= NA_WIDE) lists(k_na_lists<16, 4>, 16);
+    else lists(k_na_lists<4, 4>, 4);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "nn_neighbors_noalloc launch");
