@@ -284,7 +284,8 @@ DevRef Batch::dref() { return DevRef{d}; }
 // higher: its lanes share candidates and repeat nothing.  One lane is left to
 // the three sweeps with the most sums, where four were slower.
 int Batch::lanes(int id) const {
-  if (d.Pn <= (id == K_BUILD_LISTS ? 131072 : 32768)) return 16;
+  const int slots = id == K_ELASTIC_ROT_STRESS || id == K_ELASTIC_FORCE ? d.NSn : d.Pn;
+  if (slots <= (id == K_BUILD_LISTS ? 131072 : 32768)) return 16;
   const bool many_sums = id == K_DENSITY_ALPHA || id == K_NONPRESSURE || id == K_STRAIN;
   return many_sums && d.Pn > 196608 ? 1 : 4;
 }
@@ -1121,8 +1122,8 @@ int Batch::step(std::vector<nn_step_stats>* stats) {
     CHK(solver_loop(1));
   }
   if (any_elastic_) {  // Elasticity.substep, :1241-1244
-    TIMED(K_ELASTIC_ROT_STRESS, launch_elastic_rot_stress(dref(), blk(K_ELASTIC_ROT_STRESS), stream));
-    TIMED(K_ELASTIC_FORCE, launch_elastic_force(dref(), blk(K_ELASTIC_FORCE), stream));
+    TIMED(K_ELASTIC_ROT_STRESS, launch_elastic_rot_stress(dref(), lanes(K_ELASTIC_ROT_STRESS), stream));
+    TIMED(K_ELASTIC_FORCE, launch_elastic_force(dref(), lanes(K_ELASTIC_FORCE), stream));
   }
   if (any_rigid_) CHK(rigid_step());  // :929-931
   TIMED(K_ADVECT, launch_advect(dref(), blk(K_ADVECT), stream));  // :933, :936-937

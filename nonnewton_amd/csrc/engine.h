@@ -279,8 +279,8 @@ void launch_press_source(const DevRef& d, int block, int lanes, int depth, int r
 void launch_press_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_clear_acc(const DevRef& d, int block, hipStream_t st);
 void launch_elastic_init(const DevRef& d, int block, hipStream_t st);
-void launch_elastic_rot_stress(const DevRef& d, int block, hipStream_t st);
-void launch_elastic_force(const DevRef& d, int block, hipStream_t st);
+void launch_elastic_rot_stress(const DevRef& d, int lanes, hipStream_t st);
+void launch_elastic_force(const DevRef& d, int lanes, hipStream_t st);
 // rigid body r of every scene, substep c (RigidBodySolver.substep, :1112-1115):
 // ground collision, centre of mass, A and its rotation, projection
 void launch_rigid_ground(const DevRef& d, int r, int c, hipStream_t st);

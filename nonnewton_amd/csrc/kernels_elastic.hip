@@ -31,65 +31,132 @@ __global__ void k_elastic_init(Dev d) {
   d.x0[sc.p_begin + id_of(d.info[i])] = make_float4(xi.x, xi.y, xi.z, sc.mass / den);
 }
 
-__device__ __forceinline__ bool member(const Dev& d, int& q, int& s) {
-  q = blockIdx.x * blockDim.x + threadIdx.x;
-  const int w = uniform(q >> 6);
-  if (w >= d.SW) return false;
-  s = uniform(d.s_wave_scene[w]);
-  if (s < 0) return false;
-  return d.s_pid[q] >= 0;
+// The stress set's sweeps: 64 members per workgroup, G lanes per member (4 or
+// 16, as the list sweeps), so that every wavefront of a workgroup belongs to one
+// scene.
+template <int G>
+__device__ __forceinline__ bool member(const Dev& d, int& m, int& q, int& lane, int& s) {
+  m = threadIdx.x / G;
+  lane = threadIdx.x % G;
+  q = blockIdx.x * 64 + m;
+  s = uniform(d.s_wave_scene[blockIdx.x]);
+  return s >= 0;  // the same for the whole workgroup
 }
+
+// B positions per lane and batch over the rest list of member q: load(id),
+// term(data, live, t), add(t), as for_pairs
+template <int G, int B, int N, typename Load, typename Term, typename Add>
+__device__ __forceinline__ void for_rest(const Dev& d, int q, int lane, int cnt, int own, Load load, Term term, Add add) {
+  using T = decltype(load(0));
+  const long NS = d.NS;
+  for (int k0 = 0; k0 < cnt; k0 += G * B) {
+    int id[B];
+    T v[B];
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      const int k = k0 + b * G + lane;
+      id[b] = k < cnt ? d.rest[k * NS + q] : own;
+    }
+#pragma unroll
+    for (int b = 0; b < B; b++) v[b] = load(id[b]);
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      const int left = cnt - (k0 + b * G);
+      if (left > 0) {
+        float t[N];
+        term(v[b], lane < left, t);
+        add_in_order<G, N, 0>(t, left, add);
+      }
+    }
+  }
+}
+
+struct RestPair {
+  float4 x, x0;
+};
 
 // computeRotations_kernel (:1249-1274) and computeStress_kernel (:1285-1323),
 // fused: the stress of particle i uses only its own rotation.
-__global__ void k_elastic_rot_stress(Dev d) {
-  int q, s;
-  if (!member(d, q, s)) return;
+//
+// With one lane per member this was bound by latency: three dependent gathers
+// per rest neighbor, a serial chain of 18 Jacobi rotations, and 1.5 wavefronts
+// a SIMD to hide them (98,304 members).  The lanes share the gathers of both
+// passes; the rotations are formed once per member, by the workgroup's first
+// wavefront (64 members, all lanes busy), through LDS.  36.4 -> 30.0 us, now
+// bound by its instructions (about 2,400 a wavefront, six wavefronts a SIMD: 23
+// us); workgroups placed so that each XCD has one part of the set took 33.0.
+template <int G>
+__global__ __launch_bounds__(64 * G) void k_elastic_rot_stress(Dev d) {
+  __shared__ float M[9][64];
+  int m, q, lane, s;
+  if (!member<G>(d, m, q, lane, s)) return;
   const SceneDev& sc = d.scenes[s];
+  const KernH kh(sc);
   const int pb = sc.p_begin;
   const int pid = d.s_pid[q];
-  const int i = pb + d.inv[pb + pid];
-  const float4 xi = d.pos[i];
-  const float4 xi0 = d.x0[pb + pid];
-  const int cnt = d.rest_cnt[q];
-  const int NS = d.NS;
+  const int own = pid < 0 ? 0 : pid;
+  const int cnt = pid < 0 ? 0 : d.rest_cnt[q];
+  const float4 xi = d.pos[pb + d.inv[pb + own]];
+  const float4 xi0 = d.x0[pb + own];
+  const auto load = [&](int id) { return RestPair{d.pos[pb + d.inv[pb + id]], d.x0[pb + id]}; };
   float A[9];
 #pragma unroll
   for (int k = 0; k < 9; k++) A[k] = 0.0f;
-  for (int k = 0; k < cnt; k++) {
-    const int jid = d.rest[(long)k * NS + q];
-    const float4 xj = d.pos[pb + d.inv[pb + jid]];
-    const float4 xj0 = d.x0[pb + jid];
-    const float dd[3] = {xj.x - xi.x, xj.y - xi.y, xj.z - xi.z};
-    const float d0[3] = {xj0.x - xi0.x, xj0.y - xi0.y, xj0.z - xi0.z};
-    const float w = sc.mass * kern_w(sc.h, sc.kW, norm3(d0[0], d0[1], d0[2]));
+  for_rest<G, 2, 9>(
+      d, q, lane, cnt, own, load,
+      [&](const RestPair& p, bool live, float* t) {
+        const float dd[3] = {p.x.x - xi.x, p.x.y - xi.y, p.x.z - xi.z};
+        const float d0[3] = {p.x0.x - xi0.x, p.x0.y - xi0.y, p.x0.z - xi0.z};
+        const float w = sc.mass * pair_w(kh, sc, d0[0], d0[1], d0[2], live);
 #pragma unroll
-    for (int a = 0; a < 3; a++)
+        for (int a = 0; a < 3; a++)
 #pragma unroll
-      for (int b = 0; b < 3; b++) A[3 * a + b] += w * (dd[a] * d0[b]);
+          for (int b = 0; b < 3; b++) t[3 * a + b] = live ? w * (dd[a] * d0[b]) : NEUTRAL;
+      },
+      [&](const float* t, bool) {
+#pragma unroll
+        for (int k = 0; k < 9; k++) A[k] += t[k];
+      });
+  if (lane == 0) {
+#pragma unroll
+    for (int k = 0; k < 9; k++) M[k][m] = A[k];
   }
+  __syncthreads();
   float R[9];
-  polar3(A, R);
+  if (threadIdx.x < 64) {
+#pragma unroll
+    for (int k = 0; k < 9; k++) A[k] = M[k][threadIdx.x];
+    polar3(A, R);
+#pragma unroll
+    for (int k = 0; k < 9; k++) M[k][threadIdx.x] = R[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 9; k++) R[k] = M[k][m];
   float U[9];
 #pragma unroll
   for (int k = 0; k < 9; k++) U[k] = 0.0f;
-  for (int k = 0; k < cnt; k++) {
-    const int jid = d.rest[(long)k * NS + q];
-    const float4 xj = d.pos[pb + d.inv[pb + jid]];
-    const float4 xj0 = d.x0[pb + jid];
-    const float dd[3] = {xj.x - xi.x, xj.y - xi.y, xj.z - xi.z};
-    const float d0[3] = {xj0.x - xi0.x, xj0.y - xi0.y, xj0.z - xi0.z};
-    float u[3];
+  for_rest<G, 2, 9>(
+      d, q, lane, cnt, own, load,
+      [&](const RestPair& p, bool live, float* t) {
+        const float dd[3] = {p.x.x - xi.x, p.x.y - xi.y, p.x.z - xi.z};
+        const float d0[3] = {p.x0.x - xi0.x, p.x0.y - xi0.y, p.x0.z - xi0.z};
+        float u[3];
 #pragma unroll
-    for (int a = 0; a < 3; a++) u[a] = R[a] * dd[0] + R[3 + a] * dd[1] + R[6 + a] * dd[2] - d0[a];
-    const float3 g3 = kern_grad(sc.h, sc.kG, d0[0], d0[1], d0[2], norm3(d0[0], d0[1], d0[2]));
-    const float g[3] = {g3.x, g3.y, g3.z};
-    const float vj0 = xj0.w;
+        for (int a = 0; a < 3; a++) u[a] = R[a] * dd[0] + R[3 + a] * dd[1] + R[6 + a] * dd[2] - d0[a];
+        const float3 g3 = pair_grad(kh, sc, d0[0], d0[1], d0[2], live);
+        const float g[3] = {g3.x, g3.y, g3.z};
+        const float vj0 = p.x0.w;
 #pragma unroll
-    for (int a = 0; a < 3; a++)
+        for (int a = 0; a < 3; a++)
 #pragma unroll
-      for (int b = 0; b < 3; b++) U[3 * a + b] -= (vj0 * u[a]) * g[b];
-  }
+          for (int b = 0; b < 3; b++) t[3 * a + b] = live ? -((vj0 * u[a]) * g[b]) : NEUTRAL;
+      },
+      [&](const float* t, bool) {
+#pragma unroll
+        for (int k = 0; k < 9; k++) U[k] += t[k];
+      });
+  if (lane != 0 || pid < 0) return;
   const float e[6] = {U[0], U[4], U[8], 0.5f * (U[1] + U[3]), 0.5f * (U[2] + U[6]), 0.5f * (U[5] + U[7])};
   const float Cd = sc.C_diag, Co = sc.C_off, Cs = sc.C_shear;
   const float C[6][6] = {{Cd, Co, Co, 0.f, 0.f, 0.f}, {Co, Cd, Co, 0.f, 0.f, 0.f}, {Co, Co, Cd, 0.f, 0.f, 0.f},
@@ -115,13 +182,22 @@ __device__ __forceinline__ void sym_mat_vec(const float* M, const float* v, floa
   out[2] = M[4] * v[0] + M[5] * v[1] + M[2] * v[2];
 }
 
+struct RestStress {
+  float4 x0, b0, b1, b2, b3;
+};
+
 // computeForces_kernel, :1334-1375, for elastic particles: a += f / m.
-__global__ void k_elastic_force(Dev d) {
-  int q, s;
-  if (!member(d, q, s)) return;
+// Bound by the gather of 80 bytes per rest neighbor (98,304 members: 0.26 GB in
+// 21.4 us; with one lane per member 23.3).
+template <int G>
+__global__ __launch_bounds__(64 * G) void k_elastic_force(Dev d) {
+  int m, q, lane, s;
+  if (!member<G>(d, m, q, lane, s)) return;
   const SceneDev& sc = d.scenes[s];
+  const KernH kh(sc);
   const int pb = sc.p_begin;
   const int pid = d.s_pid[q];
+  if (pid < 0) return;
   const int i = pb + d.inv[pb + pid];
   if (kind_of(d.info[i]) != KIND_ELASTIC) return;
   const float4 xi0 = d.x0[pb + pid];
@@ -130,41 +206,45 @@ __global__ void k_elastic_force(Dev d) {
   const float4 a0 = ri[0], a1 = ri[1], a2 = ri[2], a3 = ri[3];
   const float Ri[9] = {a0.x, a0.y, a0.z, a1.x, a1.y, a1.z, a2.x, a2.y, a2.z};
   const float si[6] = {a0.w, a1.w, a2.w, a3.x, a3.y, a3.z};
-  const int cnt = d.rest_cnt[q];
-  const int NS = d.NS;
   float fi[3] = {0.f, 0.f, 0.f};
-  for (int k = 0; k < cnt; k++) {
-    const int jid = d.rest[(long)k * NS + q];
-    const int qj = sc.s_begin + d.s_of[pb + jid];
-    const float4 xj0 = d.x0[pb + jid];
-    const float4* rj = d.rs + 4L * qj;
-    const float4 b0 = rj[0], b1 = rj[1], b2 = rj[2], b3 = rj[3];
-    const float Rj[9] = {b0.x, b0.y, b0.z, b1.x, b1.y, b1.z, b2.x, b2.y, b2.z};
-    const float sj[6] = {b0.w, b1.w, b2.w, b3.x, b3.y, b3.z};
-    const float d0[3] = {xj0.x - xi0.x, xj0.y - xi0.y, xj0.z - xi0.z};
-    const float3 g3 = kern_grad(sc.h, sc.kG, d0[0], d0[1], d0[2], norm3(d0[0], d0[1], d0[2]));
-    const float g[3] = {g3.x, g3.y, g3.z};
-    const float vj0 = xj0.w;
-    float dji[3], dij[3], sdji[3], sdij[3], fij[3], fji[3];
+  for_rest<G, 1, 3>(
+      d, q, lane, d.rest_cnt[q], pid,
+      [&](int id) {
+        const float4* rj = d.rs + 4L * (sc.s_begin + d.s_of[pb + id]);
+        return RestStress{d.x0[pb + id], rj[0], rj[1], rj[2], rj[3]};
+      },
+      [&](const RestStress& p, bool live, float* t) {
+        const float Rj[9] = {p.b0.x, p.b0.y, p.b0.z, p.b1.x, p.b1.y, p.b1.z, p.b2.x, p.b2.y, p.b2.z};
+        const float sj[6] = {p.b0.w, p.b1.w, p.b2.w, p.b3.x, p.b3.y, p.b3.z};
+        const float d0[3] = {p.x0.x - xi0.x, p.x0.y - xi0.y, p.x0.z - xi0.z};
+        const float3 g3 = pair_grad(kh, sc, d0[0], d0[1], d0[2], live);
+        const float g[3] = {g3.x, g3.y, g3.z};
+        const float vj0 = p.x0.w;
+        float dji[3], dij[3], sdji[3], sdij[3], fij[3], fji[3];
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      dji[c] = vi0 * g[c];
-      dij[c] = -vj0 * g[c];
-    }
-    sym_mat_vec(sj, dji, sdji);
-    sym_mat_vec(si, dij, sdij);
+        for (int c = 0; c < 3; c++) {
+          dji[c] = vi0 * g[c];
+          dij[c] = -vj0 * g[c];
+        }
+        sym_mat_vec(sj, dji, sdji);
+        sym_mat_vec(si, dij, sdij);
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      fij[c] = -vj0 * sdji[c];
-      fji[c] = -vi0 * sdij[c];
-    }
+        for (int c = 0; c < 3; c++) {
+          fij[c] = -vj0 * sdji[c];
+          fji[c] = -vi0 * sdij[c];
+        }
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-      const float t1 = Rj[3 * a] * fij[0] + Rj[3 * a + 1] * fij[1] + Rj[3 * a + 2] * fij[2];
-      const float t2 = Ri[3 * a] * fji[0] + Ri[3 * a + 1] * fji[1] + Ri[3 * a + 2] * fji[2];
-      fi[a] += t1 - t2;
-    }
-  }
+        for (int a = 0; a < 3; a++) {
+          const float t1 = Rj[3 * a] * fij[0] + Rj[3 * a + 1] * fij[1] + Rj[3 * a + 2] * fij[2];
+          const float t2 = Ri[3 * a] * fji[0] + Ri[3 * a + 1] * fji[1] + Ri[3 * a + 2] * fji[2];
+          t[a] = live ? t1 - t2 : NEUTRAL;
+        }
+      },
+      [&](const float* t, bool) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) fi[a] += t[a];
+      });
+  if (lane != 0) return;
   float4 acc = d.acc[i];
   fi[0] = 0.5f * fi[0];
   fi[1] = 0.5f * fi[1];
@@ -178,13 +258,17 @@ __global__ void k_elastic_force(Dev d) {
 void launch_elastic_init(const DevRef& d, int block, hipStream_t st) {
   NN_LAUNCH(k_elastic_init, dim3((d.h.Pn + block - 1) / block), dim3(block), 0, st, d.h);
 }
-void launch_elastic_rot_stress(const DevRef& d, int block, hipStream_t st) {
+void launch_elastic_rot_stress(const DevRef& d, int lanes, hipStream_t st) {
   if (d.h.NSn <= 0) return;
-  NN_LAUNCH(k_elastic_rot_stress, dim3((d.h.NSn + block - 1) / block), dim3(block), 0, st, d.h);
+  const dim3 g((d.h.NSn + 63) / 64);
+  if (lanes == 16) NN_LAUNCH(k_elastic_rot_stress<16>, g, dim3(1024), 0, st, d.h);
+  else NN_LAUNCH(k_elastic_rot_stress<4>, g, dim3(256), 0, st, d.h);
 }
-void launch_elastic_force(const DevRef& d, int block, hipStream_t st) {
+void launch_elastic_force(const DevRef& d, int lanes, hipStream_t st) {
   if (d.h.NSn <= 0) return;
-  NN_LAUNCH(k_elastic_force, dim3((d.h.NSn + block - 1) / block), dim3(block), 0, st, d.h);
+  const dim3 g((d.h.NSn + 63) / 64);
+  if (lanes == 16) NN_LAUNCH(k_elastic_force<16>, g, dim3(1024), 0, st, d.h);
+  else NN_LAUNCH(k_elastic_force<4>, g, dim3(256), 0, st, d.h);
 }
 
 }  // namespace nn
