@@ -564,6 +564,7 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   // the wavefronts' counts and densities fit in each (64 W words)
   nd.wave_pairs = reinterpret_cast<int2*>(nd.rank);
   nd.wave_rho = reinterpret_cast<float*>(nd.key);
+  nd.cg_waves = nd.bucket;  // the search's, dead after it
   nd.scenes = scenes_dev;
   nd.wave_scene = ws;
   nd.s_wave_scene = sws;

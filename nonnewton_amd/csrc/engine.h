@@ -112,7 +112,8 @@ struct SceneState {
   // the scene's first workgroup of that update
   int active_v, active_p, active_cg, cg_stop_at;
   int iter_v, iter_p, iter_cg, status;
-  unsigned max_rho_bits, pad_u;  // max_rho_bits, pairs and pairs_fluid: set by k_publish in the host copy
+  unsigned max_rho_bits;  // this, pairs and pairs_fluid: set by k_publish in the host copy
+  int cg_nw;              // waves with fluid particles, listed in cg_waves
   unsigned long long pairs, pairs_fluid;
   double err_v, err_p;
   double cg_bb, cg_rr, cg_theta, pad_d;
@@ -170,6 +171,7 @@ struct Dev {
   double* partials;  // 8 arrays of 4W: wave partials (per 64 particles, or per 16 for four-lane sweeps; the solvers' 16-lane sweeps fill 16W)
   int2* wave_pairs;  // list entries of a wavefront's particles: (of fluid and dynamic solids, of fluid)
   float* wave_rho;   // largest density of a wavefront's particles; both one entry per lane of a particle and 64 slots
+  int* cg_waves;     // per Weiler scene, from its wave_begin: its waves with fluid particles
   const int2* cg_blocks;  // CG update workgroups: (scene, first wave), up to CG_UPD_WAVES waves of one scene each
   int* cg_list;           // 3 x W: waves of the scenes that iteration k leaves iterating, at k % 3
   int* cg_list_n;         // 3 counts

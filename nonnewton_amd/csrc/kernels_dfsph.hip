@@ -529,6 +529,24 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
       for (int q = 0; q + span < FINISH_WAVES; q += 2 * span) w[q] += w[q + span];
     tot[r] = w[0];
   }
+  if (which == 2) {  // the waves that the CG's iterations go over
+    __shared__ int fluid[FINISH_WAVES];
+    int n = 0;
+    for (int j0 = sc.wave_begin; j0 < sc.wave_end; j0 += FINISH_THREADS) {
+      const bool f = j0 + t < sc.wave_end && d.cg_list[j0 + t];
+      const unsigned long long m = __ballot(f);
+      if ((t & 63) == 0) fluid[t >> 6] = __popcll(m);
+      __syncthreads();
+      int at = n + __popcll(m & ((1ull << (t & 63)) - 1ull));
+      for (int q = 0; q < FINISH_WAVES; q++) {
+        if (q < t >> 6) at += fluid[q];
+        n += fluid[q];
+      }
+      if (f) d.cg_waves[sc.wave_begin + at] = j0 + t;
+      __syncthreads();
+    }
+    if (t == 0) st->cg_nw = n;
+  }
   if (t != 0) return;
   if (which == 0) {
     const double err = tot[0] / sc.nf_d;

@@ -105,10 +105,11 @@ __device__ __forceinline__ float3 precondition(float4 w0, float2 w1, float3 r) {
                      w0.z * r.x + w1.x * r.y + w1.y * r.z);
 }
 
-// Partial arrays of iteration k: (r.r, r.u), by parity, since update k + 1
-// reads them while writing its own, and u.w.
+// Partial arrays of iteration k, one entry per 64 slots: (r.r, r.u), by parity,
+// since update k + 1 reads them while writing its own, and u.w (in words that
+// neither those arrays nor k_cg_solve's use).
 __device__ __forceinline__ int cg_rr(int k) { return 4 + 2 * (k & 1); }
-constexpr int CG_UW = 3;
+constexpr long CG_UW = 31;  // times d.W
 
 // x0 = b + theta e, r = r0 - theta A e.
 __global__ void k_cg_init(Dev d) {
@@ -250,8 +251,12 @@ __global__ void k_cg_guess(Dev d) {
     v[2] = (double)r.x * (double)u.x + (double)r.y * (double)u.y + (double)r.z * (double)u.z;
   }
   lane_partials<1, 3>(d, i, v, 0);
-  if ((threadIdx.x & 63) < 12)  // k_cg_solve's words, of no iteration yet
+  // the partials of the iterations, of k_cg_solve's words or of waves that
+  // k_cg_update and k_cg_matvec pass by; the waves that they go over
+  const bool fluid = __any(kind_of(d.info[i]) == KIND_FLUID && i < sc.p_begin + sc.n);
+  if ((threadIdx.x & 63) < 16)
     reinterpret_cast<unsigned long long*>(d.partials)[(16L + (threadIdx.x & 63)) * d.W + (i >> 6)] = 0ull;
+  if ((threadIdx.x & 63) == 0) d.cg_list[i >> 6] = fluid;
 }
 
 // w = A u of particle i by its four lanes (u gathered from the neighbors, in
@@ -265,22 +270,29 @@ __global__ void k_cg_guess(Dev d) {
 // u is never read there.  Returns u.w of the particle (lane 0; else 0).
 template <int D>
 __device__ __forceinline__ double matvec_row(const Dev& d, const SceneDev& sc, int i, int q) {
+  const long P = d.P;
+  // one round of loads: the particle's own data and its lanes' first positions
+  // (every slot has room for MAX_NB; those past the list's end are replaced)
+  static_assert(4 * D <= MAX_NB, "list positions of the first batch");
+  int jn[D];
+  float sn[D];
+#pragma unroll
+  for (int e = 0; e < D; e++) {
+    jn[e] = d.nbr[nb_word(P, i, q + 4 * e)];
+    sn[e] = d.spair[nb_word(P, i, q + 4 * e)];
+  }
+  const XU own = d.xu[i];
+  const int cnt = d.nnbr[i];
+  const float rho = d.rho[i];
   const bool valid = i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID;
   float ax = 0.f, ay = 0.f, az = 0.f;
-  float3 ui = make_float3(0.f, 0.f, 0.f);
+  const float3 xi = own.p, ui = own.u;
   if (valid) {
-    const XU own = d.xu[i];
-    const float3 xi = own.p;
-    ui = own.u;
-    const int cnt = d.nnbr[i];
-    const long P = d.P;
-    int jn[D];
-    float sn[D];
 #pragma unroll
     for (int e = 0; e < D; e++) {
       const bool in = q + 4 * e < cnt;
-      jn[e] = in ? d.nbr[nb_word(P, i, q + 4 * e)] : i;
-      sn[e] = in ? d.spair[nb_word(P, i, q + 4 * e)] : 0.0f;
+      jn[e] = in ? jn[e] : i;
+      sn[e] = in ? sn[e] : 0.0f;
     }
     for (int k = q; k < cnt; k += 4 * D) {
       int j[D];
@@ -322,7 +334,7 @@ __device__ __forceinline__ double matvec_row(const Dev& d, const SceneDev& sc, i
   ay = quad_sum(ay);
   az = quad_sum(az);
   if (!valid || q != 0) return 0.0;
-  const float f = sc.dt / d.rho[i];
+  const float f = sc.dt / rho;
   const float wx = ui.x - f * ax, wy = ui.y - f * ay, wz = ui.z - f * az;
   d.ww[i] = make_float3(wx, wy, wz);
   return (double)ui.x * (double)wx + (double)ui.y * (double)wy + (double)ui.z * (double)wz;
@@ -359,7 +371,7 @@ __global__ __launch_bounds__(MVL_THREADS) void k_cg_matvec(Dev d, int k) {
     if ((threadIdx.x & 63) == 0) red[flip][threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0)
-      d.partials[(long)CG_UW * 4 * d.W + w] = (red[flip][0] + red[flip][1]) + (red[flip][2] + red[flip][3]);
+      d.partials[CG_UW * d.W + w] = (red[flip][0] + red[flip][1]) + (red[flip][2] + red[flip][3]);
   }
 }
 
@@ -373,18 +385,23 @@ __device__ __forceinline__ void scene_sums(const Dev& d, const SceneDev& sc, int
                                            double (&tot)[3]) {
   const int t = threadIdx.x;
   const double* src[3] = {d.partials + (long)cg_rr(k - 1) * 4 * d.W, d.partials + (long)(cg_rr(k - 1) + 1) * 4 * d.W,
-                          d.partials + (long)CG_UW * 4 * d.W};
+                          d.partials + CG_UW * d.W};
   const int lo = sc.wave_begin, hi = sc.wave_end;
+  double a[3][2] = {};
+  for (int j = lo + t; j < hi; j += 2 * SUM_THREADS) {  // six loads in flight
+    double e[3][2];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+      for (int r = 0; r < 3; r++) e[r][c] = j + c * SUM_THREADS < hi ? src[r][j + c * SUM_THREADS] : 0.0;
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+      for (int r = 0; r < 3; r++) a[r][c] += e[r][c];
+  }
 #pragma unroll
   for (int r = 0; r < 3; r++) {
-    double a0 = 0.0, a1 = 0.0;
-    int j = lo + t;
-    for (; j + SUM_THREADS < hi; j += 2 * SUM_THREADS) {
-      a0 += src[r][j];
-      a1 += src[r][j + SUM_THREADS];
-    }
-    if (j < hi) a0 += src[r][j];
-    const double w = wave_sum(a0 + a1);
+    const double w = wave_sum(a[r][0] + a[r][1]);
     if ((t & 63) == 0) red[r][t >> 6] = w;
   }
   __syncthreads();
@@ -413,12 +430,13 @@ __device__ __forceinline__ bool cg_decide(const Dev& d, const SceneDev& sc, Scen
     be = 0.0;
     return true;
   }
+  const int q = (k - 1) & 1;
+  const double bb = st->cg_bb, ga_old = st->cg_gamma2[q], al_old = st->cg_alpha2[q];
   double tot[3];
   scene_sums(d, sc, k, red, tot);
-  const int q = (k - 1) & 1;
   const double rr = tot[0], ga = tot[1], de = tot[2];
   const int it = k - 1;
-  const bool conv = rr <= sc.cg_tol2 * st->cg_bb;
+  const bool conv = rr <= sc.cg_tol2 * bb;
   if (conv || it >= sc.max_iter_cg) {
     if (lead) {
       st->iter_cg = it;
@@ -429,8 +447,8 @@ __device__ __forceinline__ bool cg_decide(const Dev& d, const SceneDev& sc, Scen
     }
     return false;
   }
-  be = ga / st->cg_gamma2[q];
-  al = ga / (de - be * ga / st->cg_alpha2[q]);
+  be = ga / ga_old;
+  al = ga / (de - be * ga / al_old);
   if (lead) {
     st->iter_cg = it;
     st->cg_rr = rr;
@@ -443,19 +461,27 @@ __device__ __forceinline__ bool cg_decide(const Dev& d, const SceneDev& sc, Scen
 // a scene that iterates on lists its waves for what follows in iteration k
 __device__ __forceinline__ void cg_list_scene(const Dev& d, const SceneDev& sc, int k) {
   __shared__ int base;
-  const int nw = sc.wave_end - sc.wave_begin;
+  const int nw = d.state[&sc - d.scenes].cg_nw;
   if (threadIdx.x == 0) base = atomicAdd(&d.cg_list_n[k % 3], nw);
   __syncthreads();
   int* out = d.cg_list + (long)(k % 3) * d.W + base;
-  for (int m = threadIdx.x; m < nw; m += SUM_THREADS) out[m] = sc.wave_begin + m;
+  for (int m = threadIdx.x; m < nw; m += SUM_THREADS) out[m] = d.cg_waves[sc.wave_begin + m];
 }
 
 // Iteration k of the CG with the scene's reduction of iteration k - 1 done in
 // the same launch (no separate reduction kernel per iteration).  Workgroup =
-// up to CG_UPD_WAVES waves of one scene (d.cg_blocks).  Every workgroup takes
-// the scene's decision (cg_decide) and then p = u + beta p, s = w + beta s,
-// x += alpha p, r -= alpha s, u = M r, with partials (r.r, r.u) into arrays
-// cg_rr(k) and the next.
+// up to CG_UPD_WAVES of the scene's waves with fluid (cg_waves; d.cg_blocks has
+// room for all its waves).  Every workgroup takes the scene's decision
+// (cg_decide) and then p = u + beta p, s = w + beta s, x += alpha p,
+// r -= alpha s, u = M r, with partials (r.r, r.u) into arrays cg_rr(k) and the
+// next.
+//
+// 20 MB in and out at 131,072 particles: 4.3 us at the rate of a large copy,
+// and a chain of loads through the tables and the sums before it.  Requested
+// after the decision, with the sums' loads four at a time, the vectors made the
+// update take 11.8 us; requested before it, with the sums' loads together, 10.6
+// (workgroups of 4 or 16 waves: 10.9, 10.1).  Waves without fluid, a fifth
+// there and half of a small scene's, made up a tenth of a 64-scene pool's tick.
 constexpr int UPD_THREADS = 64 * CG_UPD_WAVES;
 static_assert(UPD_THREADS == SUM_THREADS, "scene_sums runs in k_cg_update's workgroups");
 
@@ -478,37 +504,40 @@ __global__ __launch_bounds__(UPD_THREADS) void k_cg_update(Dev d, int k) {
   if (blockIdx.x == 0 && t == 0) d.cg_list_n[(k + 1) % 3] = 0;  // for iteration k + 1
   const int stop = st->cg_stop_at;
   if (!st->active_cg || (stop != 0 && stop < k)) return;  // uniform over the workgroup
+  // waves [m0, m0 + CG_UPD_WAVES) of the scene's waves with fluid
+  const int m0 = e.y - sc.wave_begin, m = m0 + (t >> 6), nw = st->cg_nw;
+  if (m0 != 0 && m0 >= nw) return;
+  // the particle's vectors are requested before the decision that scales them
+  const int w = d.cg_waves[sc.wave_begin + min(m, nw - 1)];
+  const int i = w * 64 + (t & 63);
+  const int inf = d.info[i];
+  const float3 ww = d.ww[i], po = d.wp[i], so = d.ws[i];
+  float3 x = d.wx[i], r = d.wr[i];
+  const float4 w0 = d.wd0[i];
+  const float2 w1 = d.wd1[i];
   double al, be;
   if (!cg_decide(d, sc, st, k, e.y == sc.wave_begin && t == 0, red, al, be)) return;
   if (e.y == sc.wave_begin) cg_list_scene(d, sc, k);
-  const bool first = k == 1;
   const float alf = (float)al, bef = (float)be;
-  const int w = e.y + (t >> 6);
-  if (w >= sc.wave_end) return;  // whole waves past the scene
-  const int i = w * 64 + (t & 63);
+  if (m >= nw) return;  // whole waves past the list
   double v[2] = {0.0, 0.0};
-  if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
-    const float3 u = d.xu[i].u;
-    const float3 ww = d.ww[i];
+  if (i < sc.p_begin + sc.n && kind_of(inf) == KIND_FLUID) {
+    const float3 u = precondition(w0, w1, r);  // as the last update stored it for the matvec
     float3 p, sv;
-    if (first) {
+    if (k == 1) {
       p = u;
       sv = ww;
     } else {
-      const float3 po = d.wp[i];
-      const float3 so = d.ws[i];
       p = make_float3(u.x + bef * po.x, u.y + bef * po.y, u.z + bef * po.z);
       sv = make_float3(ww.x + bef * so.x, ww.y + bef * so.y, ww.z + bef * so.z);
     }
-    float3 x = d.wx[i];
-    float3 r = d.wr[i];
     x.x += alf * p.x;
     x.y += alf * p.y;
     x.z += alf * p.z;
     r.x -= alf * sv.x;
     r.y -= alf * sv.y;
     r.z -= alf * sv.z;
-    const float3 z = precondition(d.wd0[i], d.wd1[i], r);
+    const float3 z = precondition(w0, w1, r);
     d.wp[i] = p;
     d.ws[i] = sv;
     d.wx[i] = x;
