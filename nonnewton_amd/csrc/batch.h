@@ -144,9 +144,15 @@ class Batch {
   int solve_waves_ = -1;  // waves k_cg_solve may have (-1: not looked up yet)
   std::vector<void*> deferred_;
   int scan_blocks_ = 0;
-  SceneState* h_state_ = nullptr;  // pinned, h_state_cap_ entries
+  // pinned, h_state_cap_ entries each, with their device addresses: scene states
+  // and report words (ticket in the high half), and the fields' staging memory
+  SceneState *h_state_ = nullptr, *state_dev_ = nullptr;
+  unsigned long long *h_report_ = nullptr, *report_dev_ = nullptr;
   int h_state_cap_ = 0;
-  int* h_active_ = nullptr;        // pinned
+  unsigned ticket_ = 0;
+  float *h_stage_ = nullptr, *stage_dev_ = nullptr;
+  int stage();
+  int await(int n, unsigned& bits);
   bool any_fluid_ = false, any_elastic_ = false, any_weiler_ = false, any_strain_ = false, any_div_ = false;
   bool any_warm_cg_ = false, any_rigid_ = false;
   int max_body_ = 0, max_coupling_ = 0;  // over the scenes with rigid bodies
@@ -164,7 +170,7 @@ class Batch {
   int lists_state_ = 0;
   int solver_loop(int which);
   int cg_start();
-  int cg_solve(bool& done);
+  int cg_solve(bool& done, bool& gave_up);
   int cg_loop();
   int build_stress_set(const std::vector<int>& which);
   int gather_state();

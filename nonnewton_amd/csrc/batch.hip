@@ -4,6 +4,7 @@
 #include "batch.h"
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 
@@ -233,7 +234,7 @@ Batch::Batch(hipStream_t st) : stream(st) {}
 Batch::~Batch() {
   release();
   if (h_state_) (void)hipHostFree(h_state_);
-  if (h_active_) (void)hipHostFree(h_active_);
+  if (h_stage_) (void)hipHostFree(h_stage_);
 }
 
 // The arrays of a layout are carved from one device allocation (256-byte
@@ -584,15 +585,20 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   NB_cap_ = NBc;
   scene_cap_ = Sc;
   scan_blocks_ = nscan;
-  // pinned host copies of the scene states, for as many scenes as the layout
-  // holds (a staging batch holds one; hipHostFree synchronizes the device)
+  // pinned host copies of the scene states and their report words, for as many
+  // scenes as the layout holds (a staging batch holds one; hipHostFree
+  // synchronizes the device)
   if (!h_state_ || h_state_cap_ < Sc) {
     if (h_state_) HIPCHK(hipHostFree(h_state_));
     h_state_ = nullptr;
-    HIPCHK(hipHostMalloc((void**)&h_state_, sizeof(SceneState) * (size_t)std::max(Sc, 1), hipHostMallocDefault));
-    h_state_cap_ = std::max(Sc, 1);
+    const size_t cap = (size_t)std::max(Sc, 1);
+    HIPCHK(hipHostMalloc((void**)&h_state_, (sizeof(SceneState) + sizeof(*h_report_)) * cap, hipHostMallocDefault));
+    h_report_ = reinterpret_cast<unsigned long long*>(h_state_ + cap);
+    std::fill(h_report_, h_report_ + cap, 0ull);
+    h_state_cap_ = (int)cap;
+    HIPCHK(hipHostGetDevicePointer((void**)&state_dev_, h_state_, 0));
+    report_dev_ = reinterpret_cast<unsigned long long*>(state_dev_ + cap);
   }
-  if (!h_active_) HIPCHK(hipHostMalloc((void**)&h_active_, sizeof(int) * 4, hipHostMallocDefault));
   CHK(upload_tables(nd));
   HIPCHK(hipMemsetAsync(nd.state, 0, sizeof(SceneState) * std::max<size_t>(Sc, 1), stream));
   launch_fill_i32(nd.info, Pc, -1, stream);
@@ -849,6 +855,34 @@ int Batch::search() {
   return NN_OK;
 }
 
+// Waits until each of the first n report words carries the last ticket; bits:
+// the or of what they report.  Polling them costs 6 us less than a copy of the
+// counter and a wait for the stream (six small launches and the wait: 19.5 us
+// against 26); a wait that lasts is left to the stream's, which also returns
+// the errors of launches that cannot report.
+int Batch::await(int n, unsigned& bits) {
+  HIPCHK(hipGetLastError());
+  bits = 0;
+  bool synced = false;
+  const auto start = std::chrono::steady_clock::now();
+  for (int k = 0, polls = 0; k < n;) {
+    const unsigned long long v = __atomic_load_n(h_report_ + k, __ATOMIC_ACQUIRE);
+    if ((unsigned)(v >> 32) == ticket_) {
+      bits |= (unsigned)v;
+      k++;
+    } else if (synced) {
+      set_error("a launch did not report its end");
+      return NN_E_HIP;
+    } else if (++polls % 64 == 0 && std::chrono::steady_clock::now() - start > std::chrono::microseconds(300)) {
+      HIPCHK(hipStreamSynchronize(stream));
+      synced = true;
+    } else {
+      __builtin_ia32_pause();
+    }
+  }
+  return NN_OK;
+}
+
 int Batch::gather_state() {
   const size_t ns = scenes.size();
   if (ns > 4096) {
@@ -976,30 +1010,33 @@ int Batch::rigid_step() {
 }
 
 // Runs solver iterations until no scene is active: the first chunk is the
-// previous step's count, later chunks two at a time; each chunk ends with one
-// 4-byte read of the active-scene counter.
+// previous step's count, later chunks four at a time; the last scene finish of a
+// chunk reports each scene's active flag to the host.
 int Batch::solver_loop(int which) {
   int pred = 1;
   for (auto& sp : scenes) pred = std::max(pred, sp->last_iter[which]);
   const int maxit = std::max(1, max_iter_[which]);
   int done = 0, chunk = std::min(pred, maxit);
   for (;;) {
+    ticket_++;
+    const int reporting = done + chunk < maxit ? chunk - 1 : -1;  // its scene finish reports
     for (int c = 0; c < chunk; c++) {
+      unsigned long long* report = c == reporting ? report_dev_ : nullptr;
       if (which == 0) {
         TIMED(K_DIV_UPDATE, launch_div_update(dref(), blk(K_DIV_UPDATE), lanes(K_DIV_UPDATE), dep(K_DIV_UPDATE), stream));
         TIMED(K_DIV_SOURCE, launch_div_source(dref(), blk(K_DIV_SOURCE), lanes(K_DIV_SOURCE), dep(K_DIV_SOURCE), stream));
-        launch_scene_finish(dref(), 0, lanes(K_DIV_SOURCE), stream);
+        launch_scene_finish(dref(), 0, lanes(K_DIV_SOURCE), report, ticket_, stream);
       } else if (which == 1) {
         TIMED(K_PRESS_UPDATE, launch_press_update(dref(), blk(K_PRESS_UPDATE), lanes(K_PRESS_UPDATE), dep(K_PRESS_UPDATE), stream));
         TIMED(K_PRESS_SOURCE, launch_press_source(dref(), blk(K_PRESS_SOURCE), lanes(K_PRESS_SOURCE), dep(K_PRESS_SOURCE), 1, stream));
-        launch_scene_finish(dref(), 1, lanes(K_PRESS_SOURCE), stream);
+        launch_scene_finish(dref(), 1, lanes(K_PRESS_SOURCE), report, ticket_, stream);
       }
     }
     done += chunk;
     if (done >= maxit) break;
-    HIPCHK(hipMemcpyAsync(h_active_, d.n_active + which, sizeof(int), hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    if (*h_active_ <= 0) break;
+    unsigned active = 0;
+    CHK(await((int)scenes.size(), active));
+    if (!active) break;
     chunk = std::min(4, maxit - done);
   }
   return NN_OK;
@@ -1012,21 +1049,20 @@ int Batch::solver_loop(int which) {
 // the scene sums of iteration k - 1 and stops converged scenes) and matvec k,
 // for k = 1 .. limit, then update limit + 1, which only tests the last
 // residual.  Enqueued in chunks -- first the previous step's iteration count
-// plus two, then four -- with one 4-byte read of the active-scene counter per
-// chunk; iterations past convergence are near-empty launches.
+// plus two, then four -- with one report of the active-scene counter per chunk;
+// iterations past convergence are near-empty launches.
 int Batch::cg_start() {
-  h_active_[3] = 0;
   launch_solver_begin(dref(), 2, stream);
   TIMED(K_CG_INIT, launch_cg_init(dref(), blk(K_CG_INIT), stream));
-  if (any_warm_cg_) launch_scene_finish(dref(), 4, 1, stream);
+  if (any_warm_cg_) launch_scene_finish(dref(), 4, 1, nullptr, 0, stream);
   TIMED(K_CG_GUESS, launch_cg_guess(dref(), blk(K_CG_GUESS), stream));
   TIMED(K_CG_MATVEC, launch_cg_matvec_start(dref(), blk(K_CG_MATVEC), dep(K_CG_MATVEC), stream));
-  launch_scene_finish(dref(), 2, 1, stream);
+  launch_scene_finish(dref(), 2, 1, nullptr, 0, stream);
   return NN_OK;
 }
 
-int Batch::cg_solve(bool& done) {
-  done = false;
+int Batch::cg_solve(bool& done, bool& gave_up) {
+  done = gave_up = false;
   if (solve_waves_ < 0) {  // its workgroups wait for one another: no more than compute units
     int dev = 0, cus = 0;
     HIPCHK(hipGetDevice(&dev));
@@ -1037,9 +1073,11 @@ int Batch::cg_solve(bool& done) {
   if (scenes.size() != 1 || scenes[0]->dev.wave_begin != 0 || scenes[0]->dev.wave_end > solve_waves_) return NN_OK;
   if (timer.on) timer.seen[K_CG_UPDATE]++;  // one launch does the work of both
   TIMED(K_CG_MATVEC, launch_cg_solve(dref(), scenes[0]->dev.wave_end, stream));
-  HIPCHK(hipMemcpyAsync(h_active_, d.n_active, 4 * sizeof(int), hipMemcpyDeviceToHost, stream));
-  HIPCHK(hipStreamSynchronize(stream));
-  done = h_active_[3] == 0;
+  unsigned bits = 0;
+  launch_report_active(dref(), 3, report_dev_, ++ticket_, stream);
+  CHK(await(1, bits));
+  gave_up = bits != 0;
+  done = !gave_up;
   if (!done) solve_waves_ = 0;  // the device is shared: this batch does not try again
   return NN_OK;
 }
@@ -1078,9 +1116,10 @@ int Batch::cg_loop() {
       TIMED(K_CG_MATVEC, launch_cg_matvec(dref(), dep(K_CG_MATVEC), k, (int)expected_waves(k), stream));
     }
     if (k > last) break;
-    HIPCHK(hipMemcpyAsync(h_active_, d.n_active + 2, sizeof(int), hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    if (*h_active_ <= 0) break;
+    unsigned active = 0;
+    launch_report_active(dref(), 2, report_dev_, ++ticket_, stream);
+    CHK(await(1, active));
+    if (!active) break;
     chunk = 4;
   }
   return NN_OK;
@@ -1109,10 +1148,10 @@ int Batch::step(std::vector<nn_step_stats>* stats) {
     if (any_strain_) TIMED(K_STRAIN, launch_strain(dref(), blk(K_STRAIN), lanes(K_STRAIN), dep(K_STRAIN), stream));
     if (any_weiler_) {
       CHK(cg_start());
-      bool done = false;
-      CHK(cg_solve(done));
+      bool done = false, gave_up = false;
+      CHK(cg_solve(done, gave_up));
       if (!done) {
-        if (h_active_[3]) CHK(cg_start());  // given up by k_cg_solve: from the start again
+        if (gave_up) CHK(cg_start());  // given up by k_cg_solve: from the start again
         CHK(cg_loop());
       }
     }
@@ -1129,11 +1168,10 @@ int Batch::step(std::vector<nn_step_stats>* stats) {
   if (any_rigid_) CHK(rigid_step());  // :929-931
   TIMED(K_ADVECT, launch_advect(dref(), blk(K_ADVECT), stream));  // :933, :936-937
   std::swap(d.pos, d.pos_alt);  // pos_alt keeps the positions of this step's search
-  SceneState* pub = nullptr;
-  HIPCHK(hipHostGetDevicePointer((void**)&pub, h_state_, 0));
-  launch_publish(dref(), lanes(K_BUILD_LISTS), lanes(K_DENSITY_ALPHA), pub, stream);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(stream));
+  launch_publish(dref(), lanes(K_BUILD_LISTS), lanes(K_DENSITY_ALPHA), state_dev_, report_dev_, ++ticket_, stream);
+  unsigned none = 0;
+  CHK(await((int)scenes.size(), none));
+  if (timer.on) HIPCHK(hipStreamSynchronize(stream));
   CHK(timer.collect());
   int rc = NN_OK;
   if (stats) stats->resize(scenes.size());
@@ -1207,6 +1245,20 @@ static int field_width(int field) {
   }
 }
 
+// Pinned memory through which the kernels read and write the fields of small
+// scenes themselves.  Microseconds of an upload / a download by field size,
+// this way and with a copy to or from device memory:
+//             5 KB      134 KB    329 KB    886 KB    1.9 MB     3.4 MB
+//   kernels   11 / 11   15 / 17   21 / 27   41 / 51   93 / 139   142 / 238
+//   copies    20 / 27   74 / 82   36 / 40   60 / 68   91 / 145   141 / 274
+constexpr size_t STAGE_BYTES = 1 << 20;
+int Batch::stage() {
+  if (h_stage_) return NN_OK;
+  HIPCHK(hipHostMalloc((void**)&h_stage_, STAGE_BYTES, hipHostMallocDefault));
+  HIPCHK(hipHostGetDevicePointer((void**)&stage_dev_, h_stage_, 0));
+  return NN_OK;
+}
+
 int Batch::download(int k, int field, void* host, size_t bytes) {
   SceneHost& s = *scenes[k];
   const int w = field_width(field);
@@ -1224,6 +1276,15 @@ int Batch::download(int k, int field, void* host, size_t bytes) {
   // between steps), then one copy
   if (field == NN_FIELD_X || field == NN_FIELD_V || field == NN_FIELD_ACCELERATION || field == NN_FIELD_VISC_DIFF) {
     const float4* p = field == NN_FIELD_V ? d.vel : field == NN_FIELD_ACCELERATION ? d.acc : field == NN_FIELD_VISC_DIFF ? d.vdiff : d.pos;
+    if (bytes <= STAGE_BYTES) {
+      CHK(stage());
+      launch_gather3(p + pb, d.inv + pb, n, stage_dev_, stream);
+      launch_report_active(dref(), -1, report_dev_, ++ticket_, stream);
+      unsigned none = 0;
+      CHK(await(1, none));
+      std::memcpy(host, h_stage_, bytes);
+      return NN_OK;
+    }
     float* ordered = reinterpret_cast<float*>(d.vel_alt + pb);
     launch_gather3(p + pb, d.inv + pb, n, ordered, stream);
     HIPCHK(hipGetLastError());
@@ -1353,6 +1414,14 @@ int Batch::upload_field(int k, int field, const void* host, size_t bytes) {
     return NN_E_ARG;
   }
   float4* p = field == NN_FIELD_X ? d.pos : field == NN_FIELD_V ? d.vel : d.vdiff;
+  if (bytes <= STAGE_BYTES) {
+    CHK(stage());
+    std::memcpy(h_stage_, host, bytes);
+    launch_scatter3(stage_dev_, d.inv + pb, n, p + pb, stream);
+    launch_report_active(dref(), -1, report_dev_, ++ticket_, stream);
+    unsigned none = 0;
+    return await(1, none);
+  }
   float* ordered = reinterpret_cast<float*>(d.vel_alt + pb);  // free between steps
   HIPCHK(hipMemcpyAsync(ordered, host, bytes, hipMemcpyHostToDevice, stream));
   launch_scatter3(ordered, d.inv + pb, n, p + pb, stream);

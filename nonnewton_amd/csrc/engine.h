@@ -291,7 +291,11 @@ void launch_body_finish(const DevRef& d, int pass, int r, int c, hipStream_t st)
 void launch_rigid_place(const DevRef& d, int r, int c, hipStream_t st);
 void launch_advect(const DevRef& d, int block, hipStream_t st);
 void launch_step_begin(const DevRef& d, hipStream_t st);
-void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* host, hipStream_t st);
-void launch_scene_finish(const DevRef& d, int which, int lanes, hipStream_t st);  // 0 div, 1 press, 2 cg start, 3 cg iteration, 4 cg guess scale
+void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* host, unsigned long long* report,
+                    unsigned ticket, hipStream_t st);
+// reports whether n_active[which] is not zero (which < 0: only the ticket)
+void launch_report_active(const DevRef& d, int which, unsigned long long* report, unsigned ticket, hipStream_t st);
+// 0 div, 1 press, 2 cg start, 4 cg guess scale; 0 and 1 report each scene's active flag if `report` is given
+void launch_scene_finish(const DevRef& d, int which, int lanes, unsigned long long* report, unsigned ticket, hipStream_t st);
 
 }  // namespace nn

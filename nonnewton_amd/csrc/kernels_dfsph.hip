@@ -98,13 +98,25 @@ __global__ void k_density_alpha(Dev d) {
   if ((threadIdx.x & 63) == 0) d.wave_rho[i / (64 / G)] = m;
 }
 
+// A report to the host: one word of its pinned memory, which it polls, with the
+// ticket it waits for in the high half.
+__device__ __forceinline__ void report_word(unsigned long long* word, unsigned ticket, unsigned bits) {
+  __hip_atomic_store(word, ((unsigned long long)ticket << 32) | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// (a launch of its own: the end of the launches before it is what it reports)
+__global__ void k_report_active(Dev d, int which, unsigned long long* report, unsigned ticket) {
+  if (threadIdx.x == 0) report_word(report, ticket, which >= 0 && d.n_active[which] > 0);
+}
+
 // End of a step: per scene, the pair counts and the largest density of its
 // wavefronts (list_lanes and rho_lanes entries per 64 slots), then its state
 // into the host's pinned copy.  (With an atomic per wavefront on the scene's
 // words, the density sweep of 131,072 particles took 45 us instead of 22: each
-// atomic of one address costs about 13 ns.)
-constexpr int PUBLISH_THREADS = 256;
-__global__ __launch_bounds__(PUBLISH_THREADS) void k_publish(Dev d, int list_lanes, int rho_lanes, SceneState* host) {
+// atomic of one address costs about 13 ns.)  1,024 threads: 4.7 us at 138,304
+// particles, 10.0 with 256.
+constexpr int PUBLISH_THREADS = 1024;
+__global__ __launch_bounds__(PUBLISH_THREADS) void k_publish(Dev d, int list_lanes, int rho_lanes, SceneState* host,
+                                                             unsigned long long* report, unsigned ticket) {
   __shared__ long long red[2][PUBLISH_THREADS / 64];
   __shared__ float rmax[PUBLISH_THREADS / 64];
   const int s = blockIdx.x, t = threadIdx.x;
@@ -141,6 +153,8 @@ __global__ __launch_bounds__(PUBLISH_THREADS) void k_publish(Dev d, int list_lan
   }
   st.max_rho_bits = __float_as_uint(m);
   host[s] = st;
+  // after the state: released to the host
+  __hip_atomic_store(report + s, (unsigned long long)ticket << 32, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // which: 0 divergence, 1 pressure, 2 cg (cg_init activates scenes)
@@ -473,7 +487,8 @@ __global__ void k_press_source(Dev d, int reduce) {
 constexpr int FINISH_THREADS = NN_FINISH_THREADS;
 constexpr int FINISH_WAVES = FINISH_THREADS / 64;
 
-__global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int which, int lanes) {
+__global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int which, int lanes, unsigned long long* report,
+                                                                unsigned ticket) {
   __shared__ double red[4][FINISH_WAVES];
   const int s = blockIdx.x;
   const int t = threadIdx.x;
@@ -487,7 +502,10 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
     case 2: part = weiler; break;
     default: part = weiler && (sc.flags & SF_WARM_CG); break;  // 4
   }
-  if (!part) return;  // uniform over the workgroup
+  if (!part) {  // uniform over the workgroup
+    if (report && t == 0) report_word(report + s, ticket, 0);
+    return;
+  }
   // partial arrays read, and the entries each has per 64 particles (cg_init
   // and the first matvec, array 3, run four lanes per particle)
   const int nr = which == 2 ? 4 : (which == 4 ? 2 : 1);
@@ -558,6 +576,7 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
       if (!(err <= sc.eta_v)) st->status |= ST_NOCONV;
       atomicSub(&d.n_active[0], 1);
     }
+    if (report) report_word(report + s, ticket, !(err <= sc.eta_v || ran >= sc.max_iter_v));
   } else if (which == 1) {
     const double err = tot[0] / sc.nf_d;
     const int ran = st->iter_p + 1;
@@ -568,6 +587,7 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
       if (!(err <= sc.eta_p)) st->status |= ST_NOCONV;
       atomicSub(&d.n_active[1], 1);
     }
+    if (report) report_word(report + s, ticket, !(err <= sc.eta_p || ran >= sc.max_iter_p));
   } else if (which == 4) {
     // tot: e.r0, e.Ae
     st->cg_theta = tot[1] > 0.0 ? tot[0] / tot[1] : 0.0;
@@ -688,9 +708,13 @@ static inline dim3 grid_of(const DevRef& d, int block) { return dim3((d.h.Pn + b
 void launch_step_begin(const DevRef& d, hipStream_t st) {
   NN_LAUNCH(k_step_begin, dim3(1), dim3(256), 0, st, d.h);
 }
-void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* host, hipStream_t st) {
+void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* host, unsigned long long* report,
+                    unsigned ticket, hipStream_t st) {
   if (d.h.nscenes > 0)
-    NN_LAUNCH(k_publish, dim3(d.h.nscenes), dim3(PUBLISH_THREADS), 0, st, d.h, list_lanes, rho_lanes, host);
+    NN_LAUNCH(k_publish, dim3(d.h.nscenes), dim3(PUBLISH_THREADS), 0, st, d.h, list_lanes, rho_lanes, host, report, ticket);
+}
+void launch_report_active(const DevRef& d, int which, unsigned long long* report, unsigned ticket, hipStream_t st) {
+  NN_LAUNCH(k_report_active, dim3(1), dim3(64), 0, st, d.h, which, report, ticket);
 }
 void launch_clear_acc(const DevRef& d, int block, hipStream_t st) {
   NN_LAUNCH(k_clear_acc, grid_of(d, block), dim3(block), 0, st, d.h);
@@ -719,8 +743,9 @@ void launch_press_update(const DevRef& d, int block, int lanes, int depth, hipSt
 void launch_advect(const DevRef& d, int block, hipStream_t st) {
   NN_LAUNCH(k_advect, grid_of(d, block), dim3(block), 0, st, d.h);
 }
-void launch_scene_finish(const DevRef& d, int which, int lanes, hipStream_t st) {
-  if (d.h.nscenes > 0) NN_LAUNCH(k_scene_finish, dim3(d.h.nscenes), dim3(FINISH_THREADS), 0, st, d.h, which, lanes);
+void launch_scene_finish(const DevRef& d, int which, int lanes, unsigned long long* report, unsigned ticket, hipStream_t st) {
+  if (d.h.nscenes > 0)
+    NN_LAUNCH(k_scene_finish, dim3(d.h.nscenes), dim3(FINISH_THREADS), 0, st, d.h, which, lanes, report, ticket);
 }
 
 }  // namespace nn

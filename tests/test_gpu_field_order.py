@@ -47,3 +47,22 @@ def test_fields_keep_their_order(counts, n):
     assert np.array_equal(ctx.download(L.FIELD_X).reshape(-1, 3).view(np.uint32), marks)
     assert np.array_equal(ctx.download(L.FIELD_VOLUME), volume)
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [87380, 87381, 87382])
+def test_fields_on_either_side_of_the_staging_size(n):
+    """1 MiB of a field is 87,381 particles."""
+    sc = scenes.tiny_box(seed=2, fluid_counts=(3, 3, 3), cells=(100, 100, 100))
+    rng = np.random.Generator(np.random.PCG64(n))
+    x = scenes.lattice((0.1, 0.1, 0.1), (45, 45, 45)).astype(np.float32)
+    sc.x = np.ascontiguousarray(x[rng.permutation(len(x))[:n]])
+    sc.kind, sc.v = np.zeros(n, np.int32), np.zeros((n, 3), np.float32)
+    ctx = L.Context(sc.params, sc.n)
+    ctx.upload(sc.x, sc.kind, sc.v)
+    ctx.init()  # the slots are in cell order now
+    assert np.array_equal(ctx.download(L.FIELD_X).reshape(-1, 3), sc.x)
+    marks = (np.arange(3 * n, dtype=np.uint32) * 2654435761 & 0x7FFFFFFF).reshape(-1, 3)
+    ctx.upload_field(L.FIELD_V, marks.view(np.float32))
+    assert np.array_equal(ctx.download(L.FIELD_V).reshape(-1, 3).view(np.uint32), marks)
+    assert np.array_equal(ctx.download(L.FIELD_X).reshape(-1, 3), sc.x)
+    ctx.close()
