@@ -155,7 +155,7 @@ class Batch {
   int await(int n, unsigned& bits);
   bool any_fluid_ = false, any_elastic_ = false, any_weiler_ = false, any_strain_ = false, any_div_ = false;
   bool any_warm_cg_ = false, any_rigid_ = false;
-  int max_body_ = 0, max_coupling_ = 0;  // over the scenes with rigid bodies
+  int max_body_ = 0, max_coupling_ = 0, max_body_waves_ = 0;  // over the scenes with rigid bodies
   int NB_cap_ = 0;                       // body-table entries allocated
   int rigid_step();
   int max_iter_[3] = {1, 1, 1};

@@ -304,7 +304,7 @@ void Batch::swap_sort_buffers() {
 void Batch::derive_members() {
   long base = 0;
   any_fluid_ = any_elastic_ = any_weiler_ = any_strain_ = any_div_ = any_warm_cg_ = any_rigid_ = false;
-  max_body_ = max_coupling_ = 0;
+  max_body_ = max_coupling_ = max_body_waves_ = 0;
   max_iter_[0] = max_iter_[1] = max_iter_[2] = 1;
   for (auto& sp : scenes) {
     SceneHost& s = *sp;
@@ -330,6 +330,8 @@ void Batch::derive_members() {
       any_rigid_ = true;
       max_body_ = std::max(max_body_, s.dev.nbody);
       max_coupling_ = std::max(max_coupling_, s.dev.coupling);
+      for (size_t b = 0; b + 1 < s.body_off.size(); b++)
+        max_body_waves_ = std::max(max_body_waves_, round_up64(s.body_off[b + 1] - s.body_off[b]) / 64);
     }
     max_iter_[0] = std::max(max_iter_[0], s.dev.max_iter_v);
     max_iter_[1] = std::max(max_iter_[1], s.dev.max_iter_p);
@@ -994,8 +996,14 @@ int Batch::init_scenes(const std::vector<int>& which) {
 
 // RigidBodySolver.substep for every scene's bodies (:929-931): body rank r
 // of all scenes together, coupling_interval substeps each (a scene with fewer
-// bodies or substeps sits the extra launches out).
+// bodies or substeps sits the extra launches out); small bodies in one launch.
 int Batch::rigid_step() {
+  if (max_body_waves_ <= RB_WHOLE) {
+    if (max_coupling_ > 0) launch_rigid_ground(dref(), 0, 0, stream);
+    launch_rigid_bodies(dref(), stream);
+    HIPCHK(hipGetLastError());
+    return NN_OK;
+  }
   for (int r = 0; r < max_body_; r++)
     for (int c = 0; c < max_coupling_; c++) {
       launch_rigid_ground(dref(), r, c, stream);

@@ -398,8 +398,16 @@ __device__ __forceinline__ void jacobi_rot(float* S, float* V, int p, int q) {
   float apq = S[3 * p + q];
   if (apq == 0.0f) return;
   float theta = (S[3 * q + q] - S[3 * p + p]) / (2.0f * apq);
-  float tt = (theta >= 0.0f ? 1.0f : -1.0f) / (fabsf(theta) + sqrtf(theta * theta + 1.0f));
-  float c = 1.0f / sqrtf(tt * tt + 1.0f);
+  const float sg = theta >= 0.0f ? 1.0f : -1.0f;
+  float tt;
+  if (fabsf(theta) < 0x1p49f) {  // operands within the shorter forms' range
+    const float den = fabsf(theta) + sqrt_mid(theta * theta + 1.0f);
+    tt = div_mid(sg, den, recip_mid(den));
+  } else {
+    tt = sg / (fabsf(theta) + sqrtf(theta * theta + 1.0f));
+  }
+  const float den = sqrt_mid(tt * tt + 1.0f);  // |tt| <= 1
+  float c = div_mid(1.0f, den, recip_mid(den));
   float sn = tt * c;
 #pragma unroll
   for (int k = 0; k < 3; k++) {

@@ -49,6 +49,7 @@ constexpr int CG_UPD_WAVES = NN_UPD_WAVES;
 
 enum { KIND_FLUID = 0, KIND_STATIC = 1, KIND_ELASTIC = 2, KIND_RIGID = 3 };
 constexpr int MAX_BODIES = 4096;  // rigid bodies per scene
+constexpr int RB_WHOLE = 64;      // waves of a body that one workgroup projects by itself
 enum {
   ST_NEIGHBOR_OVERFLOW = 1,
   ST_CELL_OVERFLOW = 2,
@@ -285,6 +286,7 @@ void launch_elastic_rot_stress(const DevRef& d, int lanes, hipStream_t st);
 void launch_elastic_force(const DevRef& d, int lanes, hipStream_t st);
 // rigid body r of every scene, substep c (RigidBodySolver.substep, :1112-1115):
 // ground collision, centre of mass, A and its rotation, projection
+void launch_rigid_bodies(const DevRef& d, hipStream_t st);
 void launch_rigid_ground(const DevRef& d, int r, int c, hipStream_t st);
 void launch_rigid_sum(const DevRef& d, int pass, int r, int c, hipStream_t st);
 void launch_body_finish(const DevRef& d, int pass, int r, int c, hipStream_t st);
