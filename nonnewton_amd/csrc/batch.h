@@ -162,7 +162,7 @@ class Batch {
 
   int alloc_arena(std::vector<std::pair<void**, size_t>>& req);
   void release();
-  int search_impl(int all = 1);
+  int search_impl(int all, int begin);
   int complete_lists();
   // neighbor lists: 0 none valid (new layout), 1 built by a step's search
   // (static particles without lists; that search's positions in pos_alt),

@@ -830,12 +830,12 @@ void KernelTimer::reset() {
 // The counting sort and the lists.  all == 0 (inside a step) leaves static
 // boundary particles without a list; lists_state_ records which kind of search
 // ran last, so that list downloads can complete them first.
-int Batch::search_impl(int all) {
-  launch_fill_i32(d.cell_count, (long)C_total_ + 1, 0, stream);
+int Batch::search_impl(int all, int begin) {
+  launch_begin(dref(), begin, (long)C_total_ + 1, stream);
   TIMED(K_CELL_COUNT, launch_cell_count(dref(), blk(K_CELL_COUNT), stream));
   TIMED(K_SCAN, launch_scan(dref(), C_total_ + 1, stream));
   TIMED(K_BUCKET, launch_bucket(dref(), blk(K_BUCKET), stream));
-  TIMED(K_PLACE, launch_place(dref(), blk(K_PLACE), stream));
+  TIMED(K_PLACE, launch_place(dref(), blk(K_PLACE), begin == BEGIN_STEP, stream));
   swap_sort_buffers();
   TIMED(K_BUILD_LISTS, launch_build_lists(dref(), blk(K_BUILD_LISTS), lanes(K_BUILD_LISTS), all, stream));
   lists_state_ = all ? 2 : 1;
@@ -844,8 +844,7 @@ int Batch::search_impl(int all) {
 
 int Batch::search() {
   if (scenes.empty()) return NN_OK;
-  launch_step_begin(dref(), stream);
-  CHK(search_impl());
+  CHK(search_impl(1, BEGIN_STATUS));
   HIPCHK(hipGetLastError());
   CHK(gather_state());
   for (size_t k = 0; k < scenes.size(); k++) {
@@ -971,8 +970,7 @@ int Batch::build_stress_set(const std::vector<int>& which) {
 
 int Batch::init_scenes(const std::vector<int>& which) {
   if (scenes.empty()) return NN_OK;
-  launch_step_begin(dref(), stream);
-  CHK(search_impl());
+  CHK(search_impl(1, BEGIN_STATUS));
   launch_elastic_init(dref(), block, stream);
   HIPCHK(hipGetLastError());
   CHK(gather_state());
@@ -985,7 +983,7 @@ int Batch::init_scenes(const std::vector<int>& which) {
   CHK(build_stress_set(which));
   // the stress-set relayout does not carry neighbor lists (they hold absolute
   // slots); search again on the unchanged positions before the volume sweeps
-  CHK(search_impl());
+  CHK(search_impl(1, BEGIN_CELLS));
   launch_bvol(dref(), block, lanes(K_BVOL), 0, stream);
   launch_bvol(dref(), block, lanes(K_BVOL), 1, stream);
   HIPCHK(hipGetLastError());
@@ -1060,7 +1058,6 @@ int Batch::solver_loop(int which) {
 // plus two, then four -- with one report of the active-scene counter per chunk;
 // iterations past convergence are near-empty launches.
 int Batch::cg_start() {
-  launch_solver_begin(dref(), 2, stream);
   TIMED(K_CG_INIT, launch_cg_init(dref(), blk(K_CG_INIT), stream));
   if (any_warm_cg_) launch_scene_finish(dref(), 4, 1, nullptr, 0, stream);
   TIMED(K_CG_GUESS, launch_cg_guess(dref(), blk(K_CG_GUESS), stream));
@@ -1082,7 +1079,7 @@ int Batch::cg_solve(bool& done, bool& gave_up) {
   if (timer.on) timer.seen[K_CG_UPDATE]++;  // one launch does the work of both
   TIMED(K_CG_MATVEC, launch_cg_solve(dref(), scenes[0]->dev.wave_end, stream));
   unsigned bits = 0;
-  launch_report_active(dref(), 3, report_dev_, ++ticket_, stream);
+  launch_report_active(dref(), 1, report_dev_, ++ticket_, stream);
   CHK(await(1, bits));
   gave_up = bits != 0;
   done = !gave_up;
@@ -1125,7 +1122,7 @@ int Batch::cg_loop() {
     }
     if (k > last) break;
     unsigned active = 0;
-    launch_report_active(dref(), 2, report_dev_, ++ticket_, stream);
+    launch_report_active(dref(), 0, report_dev_, ++ticket_, stream);
     CHK(await(1, active));
     if (!active) break;
     chunk = 4;
@@ -1140,32 +1137,29 @@ int Batch::step(std::vector<nn_step_stats>* stats) {
       set_error("step before init");
       return NN_E_STATE;
     }
-  launch_step_begin(dref(), stream);
   // static particles get no list inside a step, except in batches with rigid
   // bodies: their ground collision moves positions after the search, so the
   // search positions would not survive to build those lists on demand
-  CHK(search_impl(any_rigid_ ? 1 : 0));                                // :917
+  CHK(search_impl(any_rigid_ ? 1 : 0, BEGIN_STEP));  // :917, :920
   if (any_elastic_ || any_rigid_) TIMED(K_BVOL, launch_bvol(dref(), blk(K_BVOL), lanes(K_BVOL), 1, stream));  // :918
-  TIMED(K_CLEAR_ACC, launch_clear_acc(dref(), blk(K_CLEAR_ACC), stream));             // :920
   if (any_fluid_) {  // DFSPHSolver.substep, :1546-1555
     TIMED(K_DENSITY_ALPHA, launch_density_alpha(dref(), blk(K_DENSITY_ALPHA), lanes(K_DENSITY_ALPHA), dep(K_DENSITY_ALPHA), stream));
-    if (any_div_) {
-      launch_solver_begin(dref(), 0, stream);
-      CHK(solver_loop(0));
-    }
+    if (any_div_) CHK(solver_loop(0));
     if (any_strain_) TIMED(K_STRAIN, launch_strain(dref(), blk(K_STRAIN), lanes(K_STRAIN), dep(K_STRAIN), stream));
     if (any_weiler_) {
       CHK(cg_start());
       bool done = false, gave_up = false;
       CHK(cg_solve(done, gave_up));
       if (!done) {
-        if (gave_up) CHK(cg_start());  // given up by k_cg_solve: from the start again
+        if (gave_up) {  // from the start again
+          launch_begin(dref(), BEGIN_CG, 0, stream);
+          CHK(cg_start());
+        }
         CHK(cg_loop());
       }
     }
     TIMED(K_NONPRESSURE, launch_nonpressure(dref(), blk(K_NONPRESSURE), lanes(K_NONPRESSURE), dep(K_NONPRESSURE), stream));
     std::swap(d.vel, d.vel_alt);
-    launch_solver_begin(dref(), 1, stream);
     TIMED(K_PRESS_SOURCE, launch_press_source(dref(), blk(K_PRESS_SOURCE), lanes(K_PRESS_SOURCE), dep(K_PRESS_SOURCE), 0, stream));
     CHK(solver_loop(1));
   }
@@ -1444,7 +1438,7 @@ int Batch::upload_field(int k, int field, const void* host, size_t bytes) {
 // builds them in its search.)
 int Batch::complete_lists() {
   if (lists_state_ == 2) return NN_OK;
-  if (lists_state_ == 0) return search_impl(1);  // laid out since: search the current positions
+  if (lists_state_ == 0) return search_impl(1, BEGIN_CELLS);  // laid out since: search the current positions
   Dev at_search = d;
   at_search.pos = d.pos_alt;
   launch_build_lists(DevRef{at_search}, blk(K_BUILD_LISTS), lanes(K_BUILD_LISTS), 1, stream);

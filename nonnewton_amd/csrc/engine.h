@@ -176,7 +176,7 @@ struct Dev {
   const int2* cg_blocks;  // CG update workgroups: (scene, first wave), up to CG_UPD_WAVES waves of one scene each
   int* cg_list;           // 3 x W: waves of the scenes that iteration k leaves iterating, at k % 3
   int* cg_list_n;         // 3 counts
-  int* n_active;     // [0] divergence, [1] pressure, [2] cg, [3] k_cg_solve gave up waiting
+  int* n_active;     // [0] scenes whose CG iterates, [1] k_cg_solve gave up waiting
   // Weiler CG: 3-vectors packed at 12 bytes (the sweeps stream them and the
   // matvec gathers u and the position of every neighbor)
   float3* wx;  // iterate x
@@ -261,14 +261,13 @@ constexpr int SCAN_TILE_ITEMS = 2048;
 
 void launch_cell_count(const DevRef& d, int block, hipStream_t st);
 void launch_bucket(const DevRef& d, int block, hipStream_t st);
-void launch_place(const DevRef& d, int block, hipStream_t st);
+void launch_place(const DevRef& d, int block, int clear_acc, hipStream_t st);
 void launch_build_lists(const DevRef& d, int block, int lanes, int all, hipStream_t st);  // all = 0: no static lists
 void launch_bvol(const DevRef& d, int block, int lanes, int dynamic, hipStream_t st);
 
 void launch_density_alpha(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_div_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_div_source(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
-void launch_solver_begin(const DevRef& d, int which, hipStream_t st);
 void launch_strain(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_cg_init(const DevRef& d, int block, hipStream_t st);
 void launch_cg_guess(const DevRef& d, int block, hipStream_t st);
@@ -280,7 +279,6 @@ void launch_cg_solve(const DevRef& d, int waves, hipStream_t st);  // the whole 
 void launch_nonpressure(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_press_source(const DevRef& d, int block, int lanes, int depth, int reduce, hipStream_t st);
 void launch_press_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
-void launch_clear_acc(const DevRef& d, int block, hipStream_t st);
 void launch_elastic_init(const DevRef& d, int block, hipStream_t st);
 void launch_elastic_rot_stress(const DevRef& d, int lanes, hipStream_t st);
 void launch_elastic_force(const DevRef& d, int lanes, hipStream_t st);
@@ -292,7 +290,8 @@ void launch_rigid_sum(const DevRef& d, int pass, int r, int c, hipStream_t st);
 void launch_body_finish(const DevRef& d, int pass, int r, int c, hipStream_t st);
 void launch_rigid_place(const DevRef& d, int r, int c, hipStream_t st);
 void launch_advect(const DevRef& d, int block, hipStream_t st);
-void launch_step_begin(const DevRef& d, hipStream_t st);
+enum { BEGIN_CELLS, BEGIN_STATUS, BEGIN_STEP, BEGIN_CG };
+void launch_begin(const DevRef& d, int begin, long cells, hipStream_t st);
 void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* host, unsigned long long* report,
                     unsigned ticket, hipStream_t st);
 // reports whether n_active[which] is not zero (which < 0: only the ticket)

@@ -7,6 +7,8 @@
 // average density error per scene; k_scene_finish adds them and decides
 // termination, clearing the scene's active flag; later launches of a finished
 // scene return at once.
+#include <algorithm>
+
 #include "device_common.h"
 
 namespace nn {
@@ -18,20 +20,37 @@ __device__ __forceinline__ float alpha_press(const SceneDev& sc, float a) {
   return (sc.flags & SF_DIVERGENCE) ? ((a * sc.inv_dt) * sc.dt) * sc.inv_dt2 : a * sc.inv_dt2;
 }
 
-__global__ void k_step_begin(Dev d) {
-  for (int s = threadIdx.x; s < d.nscenes; s += blockDim.x) {
-    d.state[s].status = 0;
+// Before a search: the cell counts to zero and the scenes' state as `begin`
+// says: BEGIN_STATUS (a search by itself), BEGIN_STEP (also the three solvers'),
+// BEGIN_CG (only the CG's, before a solve is repeated; no cells).  One launch
+// for what were five: 1.5 to 3 us each, and the gaps between them.
+__global__ void k_begin(Dev d, int begin, long cells) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < cells) d.cell_count[i] = 0;
+  if (i < d.nscenes && begin != BEGIN_CELLS) {
+    const SceneDev& sc = d.scenes[i];
+    SceneState& st = d.state[i];
+    if (begin != BEGIN_CG) st.status = 0;
+    if (begin == BEGIN_STEP) {
+      st.active_v = (sc.flags & SF_HAS_FLUID) && (sc.flags & SF_DIVERGENCE) ? 1 : 0;
+      st.iter_v = 0;
+      st.err_v = 0.0;
+      st.active_p = (sc.flags & SF_HAS_FLUID) ? 1 : 0;
+      st.iter_p = 0;
+      st.err_p = 0.0;
+    }
+    if (begin != BEGIN_STATUS) {  // cg_init activates scenes
+      st.active_cg = 0;
+      st.cg_stop_at = 0;
+      st.iter_cg = 0;
+      st.cg_rr = 0.0;
+      st.cg_bb = 0.0;
+    }
   }
-}
-
-// clear_accelerations_kernel, :945-951
-__global__ void k_clear_acc(Dev d) {
-  int i, s;
-  if (!slot_scene(d, i, s)) return;
-  const SceneDev& sc = d.scenes[s];
-  if (i >= sc.p_begin + sc.n) return;
-  const bool stat = kind_of(d.info[i]) == KIND_STATIC;
-  d.acc[i] = stat ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(sc.gx, sc.gy, sc.gz, 0.f);
+  if (i == 0 && begin >= BEGIN_STEP) {
+    d.cg_list_n[0] = d.cg_list_n[1] = d.cg_list_n[2] = 0;
+    d.n_active[0] = d.n_active[1] = 0;
+  }
 }
 
 // compute_densities (:962-984), compute_DFSPH_factor (:1569-1608) and the first
@@ -155,42 +174,6 @@ __global__ __launch_bounds__(PUBLISH_THREADS) void k_publish(Dev d, int list_lan
   host[s] = st;
   // after the state: released to the host
   __hip_atomic_store(report + s, (unsigned long long)ticket << 32, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// which: 0 divergence, 1 pressure, 2 cg (cg_init activates scenes)
-__global__ void k_solver_begin(Dev d, int which) {
-  __shared__ int cnt;
-  if (threadIdx.x == 0) cnt = 0;
-  __syncthreads();
-  for (int s = threadIdx.x; s < d.nscenes; s += blockDim.x) {
-    const SceneDev& sc = d.scenes[s];
-    SceneState& st = d.state[s];
-    int act = 0;
-    if (which == 0) {
-      act = (sc.flags & SF_HAS_FLUID) && (sc.flags & SF_DIVERGENCE) ? 1 : 0;
-      st.active_v = act;
-      st.iter_v = 0;
-      st.err_v = 0.0;
-    } else if (which == 1) {
-      act = (sc.flags & SF_HAS_FLUID) ? 1 : 0;
-      st.active_p = act;
-      st.iter_p = 0;
-      st.err_p = 0.0;
-    } else {
-      st.active_cg = 0;
-      st.cg_stop_at = 0;
-      st.iter_cg = 0;
-      st.cg_rr = 0.0;
-      st.cg_bb = 0.0;
-      if (s == 0) d.cg_list_n[0] = d.cg_list_n[1] = d.cg_list_n[2] = 0;
-    }
-    if (act) atomicAdd(&cnt, 1);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    d.n_active[which] = cnt;
-    if (which == 2) d.n_active[3] = 0;
-  }
 }
 
 // sum_j of the velocity changes both solvers' updates make (:1721-1760,
@@ -574,7 +557,6 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
     if (err <= sc.eta_v || ran >= sc.max_iter_v) {
       st->active_v = 0;
       if (!(err <= sc.eta_v)) st->status |= ST_NOCONV;
-      atomicSub(&d.n_active[0], 1);
     }
     if (report) report_word(report + s, ticket, !(err <= sc.eta_v || ran >= sc.max_iter_v));
   } else if (which == 1) {
@@ -585,7 +567,6 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
     if (err <= sc.eta_p || ran >= sc.max_iter_p) {
       st->active_p = 0;
       if (!(err <= sc.eta_p)) st->status |= ST_NOCONV;
-      atomicSub(&d.n_active[1], 1);
     }
     if (report) report_word(report + s, ticket, !(err <= sc.eta_p || ran >= sc.max_iter_p));
   } else if (which == 4) {
@@ -602,7 +583,7 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
     const int act = (tot[0] > 0.0 && tot[1] > sc.cg_tol2 * tot[0]) ? 1 : 0;
     st->active_cg = act;
     st->cg_stop_at = 0;
-    if (act) atomicAdd(&d.n_active[2], 1);
+    if (act) atomicAdd(&d.n_active[0], 1);
   }
 }
 
@@ -705,8 +686,9 @@ __global__ void k_advect(Dev d) {
 
 static inline dim3 grid_of(const DevRef& d, int block) { return dim3((d.h.Pn + block - 1) / block); }
 
-void launch_step_begin(const DevRef& d, hipStream_t st) {
-  NN_LAUNCH(k_step_begin, dim3(1), dim3(256), 0, st, d.h);
+void launch_begin(const DevRef& d, int begin, long cells, hipStream_t st) {
+  const long n = std::max(cells, (long)d.h.nscenes);
+  if (n > 0) NN_LAUNCH(k_begin, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, d.h, begin, cells);
 }
 void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* host, unsigned long long* report,
                     unsigned ticket, hipStream_t st) {
@@ -716,14 +698,8 @@ void launch_publish(const DevRef& d, int list_lanes, int rho_lanes, SceneState* 
 void launch_report_active(const DevRef& d, int which, unsigned long long* report, unsigned ticket, hipStream_t st) {
   NN_LAUNCH(k_report_active, dim3(1), dim3(64), 0, st, d.h, which, report, ticket);
 }
-void launch_clear_acc(const DevRef& d, int block, hipStream_t st) {
-  NN_LAUNCH(k_clear_acc, grid_of(d, block), dim3(block), 0, st, d.h);
-}
 void launch_density_alpha(const DevRef& d, int block, int lanes, int depth, hipStream_t st) {
   SWEEP_LAUNCH(k_density_alpha, lanes, depth, d.h.Pn, block, st, d.h);
-}
-void launch_solver_begin(const DevRef& d, int which, hipStream_t st) {
-  NN_LAUNCH(k_solver_begin, dim3(1), dim3(256), 0, st, d.h, which);
 }
 void launch_div_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st) {
   SWEEP_LAUNCH_4(k_div_update, lanes, depth, d.h.Pn, block, st, d.h);

@@ -111,19 +111,8 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_reduce(const int* in, int n, in
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(SCAN_T) void k_scan_top(int* sums, int nb) {
-  __shared__ int lds[SCAN_T / 64];
-  int carry = 0;
-  for (int base = 0; base < nb; base += SCAN_T) {
-    int i = base + threadIdx.x;
-    int v = i < nb ? sums[i] : 0;
-    int total;
-    int ex = block_excl_scan(v, lds, total);
-    if (i < nb) sums[i] = ex + carry;
-    carry += total;
-  }
-}
-
+// (each block adds the sums of those before it: one block scanning them first
+// was a launch of 3 us)
 __global__ __launch_bounds__(SCAN_T) void k_scan_down(const int* in, int n, const int* sums, int* out) {
   __shared__ int lds[SCAN_T / 64];
   long base = (long)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_I;
@@ -134,8 +123,11 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_down(const int* in, int n, cons
     v[k] = (base + k < n) ? in[base + k] : 0;
     s += v[k];
   }
-  int total;
-  int ex = block_excl_scan(s, lds, total) + sums[blockIdx.x];
+  int before = 0;
+  for (int k = threadIdx.x; k < (int)blockIdx.x; k += SCAN_T) before += sums[k];
+  int total, all_before;
+  block_excl_scan(before, lds, all_before);
+  int ex = block_excl_scan(s, lds, total) + all_before;
 #pragma unroll
   for (int k = 0; k < SCAN_I; k++) {
     if (base + k < n) out[base + k] = ex;
@@ -147,7 +139,6 @@ __global__ __launch_bounds__(SCAN_T) void k_scan_down(const int* in, int n, cons
 void launch_scan_i32(const int* in, int n, int* tmp, int* out, hipStream_t st) {
   int nb = (n + SCAN_TILE - 1) / SCAN_TILE;
   NN_LAUNCH(k_scan_reduce, dim3(nb), dim3(SCAN_T), 0, st, in, n, tmp);
-  NN_LAUNCH(k_scan_top, dim3(1), dim3(SCAN_T), 0, st, tmp, nb);
   NN_LAUNCH(k_scan_down, dim3(nb), dim3(SCAN_T), 0, st, in, n, tmp, out);
 }
 
@@ -212,10 +203,13 @@ __global__ void k_bucket(Dev d) {
   if (!slot_scene(d, i, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (i >= sc.p_begin + sc.n) return;
-  d.bucket[d.cell_start[d.key[i]] + d.rank[i]] = i;
+  d.bucket[d.cell_start[d.key[i]] + d.rank[i]] = id_of(d.info[i]);
 }
 
-__global__ void k_place(Dev d) {
+// Particles to their places: in its cell, a particle's place is the number of
+// lower ids there.  clear_acc: the accelerations of a step start here
+// (clear_accelerations_kernel, :945-951; a launch of its own took 3.5 to 5 us).
+__global__ void k_place(Dev d, int clear_acc) {
   int i, s;
   if (!slot_scene(d, i, s)) return;
   const SceneDev& sc = d.scenes[s];
@@ -225,12 +219,14 @@ __global__ void k_place(Dev d) {
   const int inf = d.info[i];
   const int my = id_of(inf);
   int r = 0;
-  for (int k = cs; k < ce; k++) r += id_of(d.info[d.bucket[k]]) < my ? 1 : 0;
+  for (int k = cs; k < ce; k++) r += d.bucket[k] < my ? 1 : 0;
   const int dest = sc.shift + cs + r;
   d.pos_alt[dest] = d.pos[i];
   d.vel_alt[dest] = d.vel[i];
   d.info_alt[dest] = inf;
   if (sc.flags & SF_WARM_CG) d.vdiff_alt[dest] = d.vdiff[i];
+  if (clear_acc)
+    d.acc[dest] = kind_of(inf) == KIND_STATIC ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(sc.gx, sc.gy, sc.gz, 0.f);
   d.inv[sc.p_begin + my] = dest - sc.p_begin;
 }
 
@@ -360,8 +356,8 @@ void launch_cell_count(const DevRef& d, int block, hipStream_t st) {
 void launch_bucket(const DevRef& d, int block, hipStream_t st) {
   NN_LAUNCH(k_bucket, dim3((d.h.Pn + block - 1) / block), dim3(block), 0, st, d.h);
 }
-void launch_place(const DevRef& d, int block, hipStream_t st) {
-  NN_LAUNCH(k_place, dim3((d.h.Pn + block - 1) / block), dim3(block), 0, st, d.h);
+void launch_place(const DevRef& d, int block, int clear_acc, hipStream_t st) {
+  NN_LAUNCH(k_place, dim3((d.h.Pn + block - 1) / block), dim3(block), 0, st, d.h, clear_acc);
 }
 void launch_build_lists(const DevRef& d, int block, int lanes, int all, hipStream_t st) {
   const dim3 g((unsigned)(((long)d.h.Pn * lanes + block - 1) / block)), b(block);

@@ -443,7 +443,7 @@ __device__ __forceinline__ bool cg_decide(const Dev& d, const SceneDev& sc, Scen
       st->cg_rr = rr;
       st->cg_stop_at = k;
       if (!conv) st->status |= ST_NOCONV;
-      atomicSub(&d.n_active[2], 1);
+      atomicSub(&d.n_active[0], 1);
     }
     return false;
   }
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(UPD_THREADS) void k_cg_update(Dev d, int k) {
 //
 // The wait is bounded (CG_SOLVE_POLLS): should a workgroup not have been
 // scheduled by then -- the device held by other work -- the waiting ones set
-// n_active[3] and leave, every later wait of the launch ends the same way, and
+// n_active[1] and leave, every later wait of the launch ends the same way, and
 // the host repeats the solve with k_cg_update and k_cg_matvec.  Nothing that
 // such a repetition starts from is written here.
 //
@@ -713,7 +713,7 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_cg_solve(Dev d) {
         }
       }
       if (__syncthreads_or(late)) {
-        if (t == 0) atomicOr(&d.n_active[3], 1);
+        if (t == 0) atomicOr(&d.n_active[1], 1);
         return;
       }
 #pragma unroll
@@ -844,7 +844,7 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_cg_solve(Dev d) {
     st->iter_cg = k - 1;
     st->cg_rr = rr;
     if (!(rr <= sc.cg_tol2 * bb)) st->status |= ST_NOCONV;
-    d.n_active[2] = 0;
+    d.n_active[0] = 0;
   }
 }
 
