@@ -143,7 +143,6 @@ class Batch {
   int n_cg_blocks_ = 0;  // entries of d.cg_blocks
   int solve_waves_ = -1;  // waves k_cg_solve may have (-1: not looked up yet)
   std::vector<void*> deferred_;
-  int scan_blocks_ = 0;
   // pinned, h_state_cap_ entries each, with their device addresses: scene states
   // and report words (ticket in the high half), and the fields' staging memory
   SceneState *h_state_ = nullptr, *state_dev_ = nullptr;

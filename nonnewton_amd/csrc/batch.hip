@@ -493,7 +493,7 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   nd.nbodies = NB;
   nd.nscenes = (int)scenes.size();
   const int ncell_entries = Cc + 1;
-  const int nscan = (ncell_entries + 2047) / 2048;
+  const size_t nscan = (size_t)scan_tmp_ints(ncell_entries);
   std::vector<std::pair<void**, size_t>> req;
   auto A = [&](auto*& p, size_t count) {
     using T = std::remove_reference_t<decltype(*p)>;
@@ -586,7 +586,6 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   C_cap_ = Cc;
   NB_cap_ = NBc;
   scene_cap_ = Sc;
-  scan_blocks_ = nscan;
   // pinned host copies of the scene states and their report words, for as many
   // scenes as the layout holds (a staging batch holds one; hipHostFree
   // synchronizes the device)

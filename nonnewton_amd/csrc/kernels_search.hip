@@ -100,46 +100,80 @@ __device__ __forceinline__ int block_excl_scan(int v, int* lds, int& total) {
   return off + incl - v;
 }
 
-__global__ __launch_bounds__(SCAN_T) void k_scan_reduce(const int* in, int n, int* sums) {
-  __shared__ int lds[SCAN_T / 64];
-  long base = (long)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_I;
-  int s = 0;
+// a thread's SCAN_I items from `base` on (16-byte loads where they may be);
+// nz: 1 for an item that is not zero
+__device__ __forceinline__ void scan_items(const int* in, int n, long base, int nz, int* v) {
+  if (base + SCAN_I <= n && ((uintptr_t)in & 15) == 0) {
+    const int4* q = reinterpret_cast<const int4*>(in + base);
 #pragma unroll
-  for (int k = 0; k < SCAN_I; k++) s += (base + k < n) ? in[base + k] : 0;
+    for (int k = 0; k < SCAN_I / 4; k++) {
+      const int4 t = q[k];
+      v[4 * k] = t.x;
+      v[4 * k + 1] = t.y;
+      v[4 * k + 2] = t.z;
+      v[4 * k + 3] = t.w;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < SCAN_I; k++) v[k] = base + k < n ? in[base + k] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < SCAN_I; k++) v[k] = nz ? v[k] != 0 : v[k];
+}
+
+__global__ __launch_bounds__(SCAN_T) void k_scan_reduce(const int* in, int n, int nz, int* sums) {
+  __shared__ int lds[SCAN_T / 64];
+  int v[SCAN_I], s = 0;
+  scan_items(in, n, (long)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_I, nz, v);
+#pragma unroll
+  for (int k = 0; k < SCAN_I; k++) s += v[k];
   int total;
   block_excl_scan(s, lds, total);
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// (each block adds the sums of those before it: one block scanning them first
-// was a launch of 3 us)
-__global__ __launch_bounds__(SCAN_T) void k_scan_down(const int* in, int n, const int* sums, int* out) {
+// scanned: sums holds the blocks' offsets; else each block adds the sums of
+// those before it (one block scanning them first was a launch of 3 us)
+__global__ __launch_bounds__(SCAN_T) void k_scan_down(const int* in, int n, int nz, const int* sums, int scanned, int total_out,
+                                                      int* out) {
   __shared__ int lds[SCAN_T / 64];
-  long base = (long)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_I;
-  int v[SCAN_I];
-  int s = 0;
+  const long base = (long)blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_I;
+  int v[SCAN_I], s = 0;
+  scan_items(in, n, base, nz, v);
 #pragma unroll
-  for (int k = 0; k < SCAN_I; k++) {
-    v[k] = (base + k < n) ? in[base + k] : 0;
-    s += v[k];
+  for (int k = 0; k < SCAN_I; k++) s += v[k];
+  int total, offset;
+  if (scanned) {
+    offset = sums[blockIdx.x];
+  } else {
+    int before = 0;
+    for (int k = threadIdx.x; k < (int)blockIdx.x; k += SCAN_T) before += sums[k];
+    block_excl_scan(before, lds, offset);
   }
-  int before = 0;
-  for (int k = threadIdx.x; k < (int)blockIdx.x; k += SCAN_T) before += sums[k];
-  int total, all_before;
-  block_excl_scan(before, lds, all_before);
-  int ex = block_excl_scan(s, lds, total) + all_before;
+  int ex = block_excl_scan(s, lds, total) + offset;
 #pragma unroll
   for (int k = 0; k < SCAN_I; k++) {
     if (base + k < n) out[base + k] = ex;
     ex += v[k];
   }
+  if (total_out && blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_T - 1) out[n] = ex;
 }
 
-// exclusive scan of in[0..n) into out, with ceil(n / SCAN_TILE) ints of tmp
-void launch_scan_i32(const int* in, int n, int* tmp, int* out, hipStream_t st) {
-  int nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-  NN_LAUNCH(k_scan_reduce, dim3(nb), dim3(SCAN_T), 0, st, in, n, tmp);
-  NN_LAUNCH(k_scan_down, dim3(nb), dim3(SCAN_T), 0, st, in, n, tmp, out);
+// Exclusive scan of in[0..n) -- with nz of (in[i] != 0) -- into out[0..n), which
+// may be in; with total also out[n].  scan_tmp_ints(n) ints of tmp.  Up to
+// SCAN_DIRECT blocks add the sums before theirs, 32 loads a thread on average;
+// beyond that the sums are scanned by this first.
+constexpr int SCAN_DIRECT = 16384;
+long scan_tmp_ints(long n) {
+  const long nb = (n + SCAN_TILE - 1) / SCAN_TILE;
+  return (nb + 63) / 64 * 64 + (nb > SCAN_DIRECT ? scan_tmp_ints(nb) : 0);
+}
+void launch_scan_i32(const int* in, int n, int* tmp, int* out, hipStream_t st, int nz, int total) {
+  const int nb = (n + SCAN_TILE - 1) / SCAN_TILE;
+  const int scanned = nb > SCAN_DIRECT;
+  NN_LAUNCH(k_scan_reduce, dim3(nb), dim3(SCAN_T), 0, st, in, n, nz, tmp);
+  if (scanned) launch_scan_i32(tmp, nb, tmp + (nb + 63) / 64 * 64, tmp, st, 0, 0);
+  NN_LAUNCH(k_scan_down, dim3(nb), dim3(SCAN_T), 0, st, in, n, nz, tmp, scanned, total, out);
 }
 
 void launch_scan(const DevRef& d, int n, hipStream_t st) {

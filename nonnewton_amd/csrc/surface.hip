@@ -46,7 +46,6 @@ constexpr int MAX_PER_VOXEL = 64;  // max_num_particle_per_voxel, srtool.py:685
 constexpr double FIX_SCALE = 4294967296.0;
 constexpr double FIX_INV = 1.0 / 4294967296.0;
 constexpr float MAX_CONTRIB = 1048576.0f;  // |contribution| bound keeping the int64 sums exact
-constexpr int SCAN_TILE = 1024;
 
 enum { ERR_OUT_OF_GRID = 1, ERR_VOXEL_OVERFLOW = 2, ERR_RANGE = 4 };
 
@@ -67,7 +66,8 @@ struct K {
   unsigned char* active;
   float4* rec;  // REC_QUADS per entry of vlist
   float *field0, *field, *tmp;
-  int *flag, *cube_id, *tcount, *tstart;
+  int *flag, *cube_id;      // per vertex of the grid: its cube's code and mesh vertex + 1
+  int *cubes, *tcount, *tstart;  // per mesh vertex: its cube, its triangles
   float *verts, *normals;
   int* faces;
   int* err;
@@ -149,11 +149,11 @@ __device__ __forceinline__ long gidx(const K& k, int gx, int gy, int gz) {
 __device__ __forceinline__ long bidx(const K& k, int gx, int gy, int gz) {
   return ((long)(gx / BLOCK) * k.bdim[1] + gy / BLOCK) * k.bdim[2] + gz / BLOCK;
 }
-// value at vertex (x, y, z) (absolute vertex coordinates); 0 if unwritten
+// value at vertex (x, y, z) (absolute vertex coordinates); 0 if unwritten (the
+// fields hold 0 in blocks that no box touches)
 __device__ __forceinline__ float val_at(const K& k, const float* f, int x, int y, int z) {
   const int gx = x - k.glo[0], gy = y - k.glo[1], gz = z - k.glo[2];
   if (gx < 0 || gy < 0 || gz < 0 || gx >= k.gdim[0] || gy >= k.gdim[1] || gz >= k.gdim[2]) return 0.0f;
-  if (!k.active[bidx(k, gx, gy, gz)]) return 0.0f;
   return f[gidx(k, gx, gy, gz)];
 }
 // get_mapped_position (:795-796)
@@ -187,33 +187,6 @@ __device__ __forceinline__ unsigned long long fix_of(float v) {
 __device__ __forceinline__ int mult_axis(int v, int c, int off, int R) {
   const int lo = c - off, hi = c - off + R - 1;
   return (v >= lo && v <= hi) + (v - 1 >= lo && v - 1 <= hi);
-}
-
-// ------------------------------------------------------------------ scan
-// exclusive prefix sum of in[0, L) into out[0, L), total into out[L];
-// tiles of 1024 scanned in LDS, tile sums scanned recursively, added back
-
-__global__ __launch_bounds__(SCAN_TILE) void k_scan_tile(const int* in, int* out, int* tsum, long L) {
-  __shared__ int s[SCAN_TILE];
-  const long i = (long)blockIdx.x * SCAN_TILE + threadIdx.x;
-  const int v = i < L ? in[i] : 0;
-  s[threadIdx.x] = v;
-  __syncthreads();
-  for (int d = 1; d < SCAN_TILE; d <<= 1) {
-    const int t = threadIdx.x >= d ? s[threadIdx.x - d] : 0;
-    __syncthreads();
-    s[threadIdx.x] += t;
-    __syncthreads();
-  }
-  if (i < L) out[i] = s[threadIdx.x] - v;
-  if (threadIdx.x == SCAN_TILE - 1) tsum[blockIdx.x] = s[SCAN_TILE - 1];
-}
-__global__ void k_scan_add(int* out, const int* toff, long L) {
-  const long i = (long)blockIdx.x * SCAN_TILE + threadIdx.x;
-  if (i < L) out[i] += toff[blockIdx.x];
-}
-__global__ void k_scan_total(const int* in, int* out, long L) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) out[L] = L > 0 ? out[L - 1] + in[L - 1] : 0;
 }
 
 // ------------------------------------------------------------------ stages
@@ -904,16 +877,27 @@ __global__ __launch_bounds__(ST_THREADS) void k_stats(K k, int which, double* pa
   const float mean = (float)k.stats[2];
   double a = 0.0;
   int c = 0;
-  for (int l = t; l < BLOCK * BLOCK * BLOCK; l += ST_THREADS) {
-    const int gx = bx * BLOCK + (l >> 10), gy = by * BLOCK + ((l >> 5) & 31), gz = bz * BLOCK + (l & 31);
-    const float v = k.field[gidx(k, gx, gy, gz)];
-    if (v < 0.0f) {
-      if (which == 0) {
-        a += (double)v;
-        c++;
-      } else {
-        const double d = (double)(v - mean);
-        a += d * d;
+  // few blocks, so few wavefronts: 32 loads in flight each, 11 to 14 us (a
+  // block's 128 a lane one after the other took 34 to 37)
+  constexpr int DEEP = 32;
+  const float* f = k.field + gidx(k, bx * BLOCK, by * BLOCK + (t >> 5), bz * BLOCK + (t & 31));
+  for (int j0 = 0; j0 < BLOCK * BLOCK * BLOCK / ST_THREADS; j0 += DEEP) {
+    float v[DEEP];
+#pragma unroll
+    for (int j = 0; j < DEEP; j++) {  // vertex l = t + 256 (j0 + j)
+      const int row = (j0 + j) * (ST_THREADS / BLOCK);
+      v[j] = f[((long)(row >> 5) * k.gdim[1] + (row & 31)) * k.gdim[2]];
+    }
+#pragma unroll
+    for (int j = 0; j < DEEP; j++) {
+      if (v[j] < 0.0f) {
+        if (which == 0) {
+          a += (double)v[j];
+          c++;
+        } else {
+          const double d = (double)(v[j] - mean);
+          a += d * d;
+        }
       }
     }
   }
@@ -931,14 +915,27 @@ __global__ __launch_bounds__(ST_THREADS) void k_stats(K k, int which, double* pa
 }
 
 // blocks added in block order; which 0 sets the mean, which 1 the sd
-__global__ void k_stats_final(K k, int which, const double* part, const long long* pcount) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ __launch_bounds__(ST_THREADS) void k_stats_final(K k, int which, const double* part, const long long* pcount) {
+  __shared__ double ps[ST_THREADS];
+  __shared__ long long pc[ST_THREADS];
+  const int t = threadIdx.x;
   double s = 0.0;
   long long c = 0;
-  for (long b = 0; b < k.nblock; b++) {
-    s += part[b];
-    c += pcount[b];
+  for (long b0 = 0; b0 < k.nblock; b0 += ST_THREADS) {
+    const int n = (int)min((long)ST_THREADS, k.nblock - b0);
+    if (t < n) {
+      ps[t] = part[b0 + t];
+      pc[t] = pcount[b0 + t];
+    }
+    __syncthreads();
+    if (t == 0)
+      for (int b = 0; b < n; b++) {
+        s += ps[b];
+        c += pc[b];
+      }
+    __syncthreads();
   }
+  if (t != 0) return;
   if (which == 0) {
     k.stats[0] = s;
     k.stats[1] = (double)c;
@@ -961,19 +958,26 @@ __global__ void k_smooth(K k, const float* in, float* out) {
   const float sd = (float)k.stats[3];
   const int i = gx + k.glo[0], j = gy + k.glo[1], l = gz + k.glo[2];
   const float vc = in[q];
+  const float den = 2.0f * sd * sd, tt = k.c2pi * sd * sd, scale = tt * sqrtf(tt);
   float avg = 0.0f, weight = 0.0f;
-  for (int dx = -1; dx <= 1; dx++)
-    for (int dy = -1; dy <= 1; dy++)
-      for (int dz = -1; dz <= 1; dz++) {
-        const int x = i + dx, y = j + dy, z = l + dz;
-        if (x < 0 || y < 0 || z < 0) continue;
-        const float vn = val_at(k, in, x, y, z);
-        const float d = fabsf(vc - vn);
-        const float tt = k.c2pi * sd * sd;
-        const float gw = sr_expf(-d * d / (2.0f * sd * sd)) / (tt * sqrtf(tt));
-        avg += gw * vn;
-        weight += gw;
-      }
+#pragma unroll
+  for (int dx = -1; dx <= 1; dx++) {  // nine loads in flight
+    float vn[9];
+    bool on[9];
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+      const int dy = e / 3 - 1, dz = e % 3 - 1;
+      on[e] = min(i + dx, min(j + dy, l + dz)) >= 0;
+      vn[e] = val_at(k, in, i + dx, j + dy, l + dz);
+    }
+#pragma unroll
+    for (int e = 0; e < 9; e++) {
+      const float d = fabsf(vc - vn[e]);
+      const float gw = on[e] ? sr_expf(-d * d / den) / scale : 0.0f;
+      avg += gw * vn[e];
+      weight += gw;
+    }
+  }
   if (weight != 0.0f) avg /= weight;
   out[q] = avg;
 }
@@ -990,47 +994,42 @@ __constant__ int ADJ[3][3][3] = {
     {{0, -1, 0}, {-1, -1, 0}, {-1, 0, 0}},
 };
 
-// cube index bits (value < isolevel) << 12 | crossed-edge mask (the
-// marching-cubes edge table, derived: an edge is crossed when its corners differ)
-__device__ __forceinline__ int cube_setup(const K& k, int x, int y, int z, float* cv, float (*cp)[3]) {
-  int ci = 0;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    cv[j] = val_at(k, k.field, x + CORNER[j][0], y + CORNER[j][1], z + CORNER[j][2]);
-    vpos(k, x + CORNER[j][0], y + CORNER[j][1], z + CORNER[j][2], cp[j]);
-    if (cv[j] < k.iso) ci |= 1 << j;
-  }
-  int mask = 0;
-#pragma unroll
-  for (int w = 0; w < 12; w++)
-    if (((ci >> EDGE[w][0]) & 1) != ((ci >> EDGE[w][1]) & 1)) mask |= 1 << w;
-  return (ci << 12) | mask;
-}
-
+// Code of every cube (its vertex of the grid): 0 without a crossing, else the
+// bits (corner value < isolevel) << 12 | crossed-edge mask (the marching-cubes
+// edge table, derived: an edge is crossed when its corners differ).
 __global__ void k_cube_flag(K k) {
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= k.nvert) return;
   const int gz = (int)(q % k.gdim[2]), gy = (int)((q / k.gdim[2]) % k.gdim[1]), gx = (int)(q / ((long)k.gdim[1] * k.gdim[2]));
-  int f = 0;
+  int code = 0;
   if (k.active[bidx(k, gx, gy, gz)]) {
-    float cv[8], cp[8][3];
-    f = (cube_setup(k, gx + k.glo[0], gy + k.glo[1], gz + k.glo[2], cv, cp) & 0xFFF) != 0;
+    int ci = 0;
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (val_at(k, k.field, gx + k.glo[0] + CORNER[j][0], gy + k.glo[1] + CORNER[j][1], gz + k.glo[2] + CORNER[j][2]) < k.iso)
+        ci |= 1 << j;
+    int mask = 0;
+#pragma unroll
+    for (int w = 0; w < 12; w++)
+      if (((ci >> EDGE[w][0]) & 1) != ((ci >> EDGE[w][1]) & 1)) mask |= 1 << w;
+    if (mask) code = (ci << 12) | mask;
   }
-  k.flag[q] = f;
+  k.flag[q] = code;
 }
 
+// cube_id held the number of crossing cubes before each cube: a crossing cube's
+// vertex number + 1 (0 for the others), and the cubes by vertex number
 __global__ void k_cube_id(K k) {
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= k.nvert) return;
-  k.cube_id[q] = k.flag[q] ? k.cube_id[q] + 1 : 0;  // cube_id holds the exclusive scan of flag
+  const bool on = k.flag[q] != 0;
+  const int m = k.cube_id[q];
+  if (on) k.cubes[m] = (int)q;
+  k.cube_id[q] = on ? m + 1 : 0;
 }
 
 // calc_vertex_normal (:1307-1321) with normalize (:1413-1417)
-__device__ __forceinline__ void vertex_normal(const K& k, int x, int y, int z, float* n) {
-  const float* f = k.field;
-  n[0] = x == 0 ? -val_at(k, f, x + 1, y, z) : val_at(k, f, x - 1, y, z) - val_at(k, f, x + 1, y, z);
-  n[1] = y == 0 ? -val_at(k, f, x, y + 1, z) : val_at(k, f, x, y - 1, z) - val_at(k, f, x, y + 1, z);
-  n[2] = z == 0 ? -val_at(k, f, x, y, z + 1) : val_at(k, f, x, y, z - 1) - val_at(k, f, x, y, z + 1);
+__device__ __forceinline__ void unit_or_zero(float* n) {
   const float nr = norm3f(n[0], n[1], n[2]);
   if (nr != 0.0f) {
     n[0] /= nr;
@@ -1040,6 +1039,13 @@ __device__ __forceinline__ void vertex_normal(const K& k, int x, int y, int z, f
     n[0] = n[1] = n[2] = 0.0f;
   }
 }
+__device__ __forceinline__ void vertex_normal(const K& k, int x, int y, int z, float* n) {
+  const float* f = k.field;
+  n[0] = x == 0 ? -val_at(k, f, x + 1, y, z) : val_at(k, f, x - 1, y, z) - val_at(k, f, x + 1, y, z);
+  n[1] = y == 0 ? -val_at(k, f, x, y + 1, z) : val_at(k, f, x, y - 1, z) - val_at(k, f, x, y + 1, z);
+  n[2] = z == 0 ? -val_at(k, f, x, y, z + 1) : val_at(k, f, x, y, z - 1) - val_at(k, f, x, y, z + 1);
+  unit_or_zero(n);
+}
 // process_normal_at (:1336-1349)
 __device__ __forceinline__ void normal_at(const K& k, const float* p, float* out) {
   int v[3];
@@ -1048,8 +1054,24 @@ __device__ __forceinline__ void normal_at(const K& k, const float* p, float* out
   vpos(k, v[0], v[1], v[2], base);
   const float xd = (p[0] - base[0]) / k.vs, yd = (p[1] - base[1]) / k.vs, zd = (p[2] - base[2]) / k.vs;
   float c[8][3];
+  const int gx = v[0] - k.glo[0], gy = v[1] - k.glo[1], gz = v[2] - k.glo[2];
+  // the 4^3 vertices around the voxel lie in the grid
+  if (min(gx, min(gy, gz)) >= 1 && gx + 2 < k.gdim[0] && gy + 2 < k.gdim[1] && gz + 2 < k.gdim[2]) {
+    const long sy = k.gdim[2], sx = (long)k.gdim[1] * k.gdim[2];
+    const float* f = k.field + gidx(k, gx, gy, gz);
 #pragma unroll
-  for (int j = 0; j < 8; j++) vertex_normal(k, v[0] + (j >> 2), v[1] + ((j >> 1) & 1), v[2] + (j & 1), c[j]);
+    for (int j = 0; j < 8; j++) {
+      const float* at = f + (j >> 2) * sx + ((j >> 1) & 1) * sy + (j & 1);
+      c[j][0] = at[-sx] - at[sx];
+      c[j][1] = at[-sy] - at[sy];
+      c[j][2] = at[-1] - at[1];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) unit_or_zero(c[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; j++) vertex_normal(k, v[0] + (j >> 2), v[1] + ((j >> 1) & 1), v[2] + (j & 1), c[j]);
+  }
   float r[3];
 #pragma unroll
   for (int a = 0; a < 3; a++) {
@@ -1188,29 +1210,65 @@ __device__ __forceinline__ int cube_vertex(const K& k, int x, int y, int z) {
 }
 
 // dual_contouring_impl (:1532-1596) for the cubes with a crossing, and the
-// number of triangles each emits (dual_contouring_polygen, :1708-1763)
-__global__ void k_dc_point(K k) {
-  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= k.nvert) return;
-  const int id = k.cube_id[q];
-  if (!id) {
-    k.tcount[q] = 0;
-    return;
+// number of triangles each emits (dual_contouring_polygen, :1708-1763).
+//
+// A lane per edge of a cube (16 lanes, three of the others for the faces) forms
+// the crossing point and its normal, the longest part (64 field values), into
+// LDS; then a lane per cube folds them in edge order and solves, the
+// workgroup's first wavefront for its 64 cubes.  Microseconds at 5,013, 46,166
+// and 66,148 cubes: 26, 71 and 101; with a thread per vertex of the grid, few of
+// a wavefront's lanes on a cube, 248, 530 and 450.
+constexpr int DC_CUBES = 64;
+constexpr int DC_THREADS = 16 * DC_CUBES;
+__global__ __launch_bounds__(DC_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_dc_point(K k, int nv) {
+  __shared__ float pn[12][6][DC_CUBES + 1];  // crossing point and normal of an edge
+  const int e = threadIdx.x & 15, c = threadIdx.x >> 4;
+  const int m = blockIdx.x * DC_CUBES + c;
+  if (m < nv) {
+    const int q = k.cubes[m];
+    const int mask = k.flag[q] & 0xFFF;
+    const int gz = q % k.gdim[2], gy = (q / k.gdim[2]) % k.gdim[1], gx = q / (k.gdim[1] * k.gdim[2]);
+    const int x = gx + k.glo[0], y = gy + k.glo[1], z = gz + k.glo[2];
+    bool quad = false;
+    if (e < 12) {
+      if (mask & (1 << e)) {
+        float cv[2], cp[2][3], p[3], n[3];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          const int* o = CORNER[EDGE[e][s]];
+          cv[s] = val_at(k, k.field, x + o[0], y + o[1], z + o[2]);
+          vpos(k, x + o[0], y + o[1], z + o[2], cp[s]);
+        }
+        vinterp(k.iso, cp[0], cp[1], cv[0], cv[1], p);
+        normal_at(k, p, n);
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+          pn[e][a][c] = p[a];
+          pn[e][3 + a][c] = n[a];
+        }
+      }
+    } else if (e < 15) {
+      const int (&adj)[3][3] = ADJ[e - 12];
+      quad = (mask & (1 << ADJ_W[e - 12])) && cube_vertex(k, x + adj[0][0], y + adj[0][1], z + adj[0][2]) &&
+             cube_vertex(k, x + adj[1][0], y + adj[1][1], z + adj[1][2]) &&
+             cube_vertex(k, x + adj[2][0], y + adj[2][1], z + adj[2][2]);
+    }
+    const int quads = __popcll(__ballot(quad) >> (threadIdx.x & 48) & 0x7000ull);
+    if (e == 0) k.tcount[m] = 2 * quads;
   }
-  const int gz = (int)(q % k.gdim[2]), gy = (int)((q / k.gdim[2]) % k.gdim[1]), gx = (int)(q / ((long)k.gdim[1] * k.gdim[2]));
-  const int x = gx + k.glo[0], y = gy + k.glo[1], z = gz + k.glo[2];
-  float cv[8], cp[8][3];
-  const int cm = cube_setup(k, x, y, z, cv, cp);
-  const int mask = cm & 0xFFF;
+  __syncthreads();
+  if (threadIdx.x >= DC_CUBES) return;
+  const int t = threadIdx.x, mt = blockIdx.x * DC_CUBES + t;
+  if (mt >= nv) return;
+  const int q = k.cubes[mt];
+  const int mask = k.flag[q] & 0xFFF;
   float mean[3] = {0.0f, 0.0f, 0.0f};
   int cnt = 0;
   for (int w = 0; w < 12; w++) {
     if (!(mask & (1 << w))) continue;
-    float p[3];
-    vinterp(k.iso, cp[EDGE[w][0]], cp[EDGE[w][1]], cv[EDGE[w][0]], cv[EDGE[w][1]], p);
-    mean[0] += p[0];
-    mean[1] += p[1];
-    mean[2] += p[2];
+    mean[0] += pn[w][0][t];
+    mean[1] += pn[w][1][t];
+    mean[2] += pn[w][2][t];
     cnt++;
   }
   const float fc = (float)cnt;
@@ -1222,53 +1280,34 @@ __global__ void k_dc_point(K k) {
   for (int a = 0; a < 16; a++) R[a] = 0.0f;
   for (int w = 0; w < 12; w++) {
     if (!(mask & (1 << w))) continue;
-    float p[3], n[3];
-    vinterp(k.iso, cp[EDGE[w][0]], cp[EDGE[w][1]], cv[EDGE[w][0]], cv[EDGE[w][1]], p);
-    normal_at(k, p, n);
-    const float d0 = p[0] - mean[0], d1 = p[1] - mean[1], d2 = p[2] - mean[2];
-    qef_add(R, n[0], n[1], n[2], n[0] * d0 + n[1] * d1 + n[2] * d2);
+    const float d0 = pn[w][0][t] - mean[0], d1 = pn[w][1][t] - mean[1], d2 = pn[w][2][t] - mean[2];
+    const float n0 = pn[w][3][t], n1 = pn[w][4][t], n2 = pn[w][5][t];
+    qef_add(R, n0, n1, n2, n0 * d0 + n1 * d1 + n2 * d2);
   }
   float r[3];
   qef_solve(R, r);
-  const float t[3] = {r[0] + mean[0], r[1] + mean[1], r[2] + mean[2]};
+  const float pt[3] = {r[0] + mean[0], r[1] + mean[1], r[2] + mean[2]};
   int v[3];
-  voxel_of(k, t, v);
-  float* out = k.verts + 3 * (long)(id - 1);
-  if (v[0] != x || v[1] != y || v[2] != z) {
-    out[0] = mean[0];
-    out[1] = mean[1];
-    out[2] = mean[2];
-  } else {
-    out[0] = r[0] + mean[0];
-    out[1] = r[1] + mean[1];
-    out[2] = r[2] + mean[2];
-  }
-  int nt = 0;
-  for (int e = 0; e < 3; e++) {
-    if (!(mask & (1 << ADJ_W[e]))) continue;
-    if (cube_vertex(k, x + ADJ[e][0][0], y + ADJ[e][0][1], z + ADJ[e][0][2]) &&
-        cube_vertex(k, x + ADJ[e][1][0], y + ADJ[e][1][1], z + ADJ[e][1][2]) &&
-        cube_vertex(k, x + ADJ[e][2][0], y + ADJ[e][2][1], z + ADJ[e][2][2]))
-      nt += 2;
-  }
-  k.tcount[q] = nt;
+  voxel_of(k, pt, v);
+  const int gz = q % k.gdim[2], gy = (q / k.gdim[2]) % k.gdim[1], gx = q / (k.gdim[1] * k.gdim[2]);
+  const bool in = v[0] == gx + k.glo[0] && v[1] == gy + k.glo[1] && v[2] == gz + k.glo[2];
+  float* out = k.verts + 3 * (long)mt;
+#pragma unroll
+  for (int a = 0; a < 3; a++) out[a] = in ? pt[a] : mean[a];
 }
 
-__global__ void k_faces(K k) {
-  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= k.nvert) return;
-  const int id = k.cube_id[q];
-  if (!id) return;
-  const int gz = (int)(q % k.gdim[2]), gy = (int)((q / k.gdim[2]) % k.gdim[1]), gx = (int)(q / ((long)k.gdim[1] * k.gdim[2]));
+__global__ void k_faces(K k, int nv) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m >= nv || !k.tcount[m]) return;
+  const int q = k.cubes[m];
+  const int gz = q % k.gdim[2], gy = (q / k.gdim[2]) % k.gdim[1], gx = q / (k.gdim[1] * k.gdim[2]);
   const int x = gx + k.glo[0], y = gy + k.glo[1], z = gz + k.glo[2];
-  float cv[8], cp[8][3];
-  const int cm = cube_setup(k, x, y, z, cv, cp);
-  const int mask = cm & 0xFFF, ci = cm >> 12;
-  int* f = k.faces + 3 * (long)k.tstart[q];
+  const int mask = k.flag[q] & 0xFFF, ci = k.flag[q] >> 12;
+  int* f = k.faces + 3 * (long)k.tstart[m];
   for (int e = 0; e < 3; e++) {
     const int w = ADJ_W[e];
     if (!(mask & (1 << w))) continue;
-    const int i1 = id;
+    const int i1 = m + 1;
     const int i2 = cube_vertex(k, x + ADJ[e][0][0], y + ADJ[e][0][1], z + ADJ[e][0][2]);
     const int i3 = cube_vertex(k, x + ADJ[e][1][0], y + ADJ[e][1][1], z + ADJ[e][1][2]);
     const int i4 = cube_vertex(k, x + ADJ[e][2][0], y + ADJ[e][2][1], z + ADJ[e][2][2]);
@@ -1288,8 +1327,7 @@ __global__ void k_faces(K k) {
 // get_velocity_at (:1352-1359): 0 outside written blocks
 __device__ __forceinline__ void vel_at(const K& k, int x, int y, int z, float* out) {
   const int gx = x - k.glo[0], gy = y - k.glo[1], gz = z - k.glo[2];
-  if (gx < 0 || gy < 0 || gz < 0 || gx >= k.gdim[0] || gy >= k.gdim[1] || gz >= k.gdim[2] ||
-      !k.active[bidx(k, gx, gy, gz)]) {
+  if (gx < 0 || gy < 0 || gz < 0 || gx >= k.gdim[0] || gy >= k.gdim[1] || gz >= k.gdim[2]) {
     out[0] = out[1] = out[2] = 0.0f;
     return;
   }
@@ -1358,7 +1396,7 @@ struct Surface {
   K k{};
   hipStream_t st = nullptr;
   DBuf<float> pos, vel, G, xbar, field0, field, tmp, verts, normals, vfield, mvel;
-  DBuf<int> vcount, vstart, vslot, vlist, pvox, flag, cube_id, tcount, tstart, faces, err, bounds, scratch;
+  DBuf<int> vcount, vstart, vslot, vlist, pvox, flag, cube_id, cubes, tcount, tstart, faces, err, bounds, scratch;
   DBuf<unsigned char> active;
   DBuf<float4> rec;
   DBuf<double> stats, part;
@@ -1370,7 +1408,7 @@ struct Surface {
 
   ~Surface() {
     for (auto* b : {&pos, &vel, &G, &xbar, &field0, &field, &tmp, &verts, &normals, &vfield, &mvel}) b->release();
-    for (auto* b : {&vcount, &vstart, &vslot, &vlist, &pvox, &flag, &cube_id, &tcount, &tstart, &faces, &err, &bounds, &scratch})
+    for (auto* b : {&vcount, &vstart, &vslot, &vlist, &pvox, &flag, &cube_id, &cubes, &tcount, &tstart, &faces, &err, &bounds, &scratch})
       b->release();
     active.release();
     rec.release();
@@ -1383,48 +1421,15 @@ struct Surface {
 
 static inline unsigned grid1(long n, int b) { return (unsigned)((n + b - 1) / b); }
 
-// exclusive scan of in[0, L) into out[0, L], total in out[L]
-static hipError_t scan(Surface& S, const int* in, int* out, long L) {
+// exclusive scan of in[0, L) (nz: of in[i] != 0) into out[0, L], total in out[L]
+static hipError_t scan(Surface& S, const int* in, int* out, long L, int nz = 0) {
   if (L <= 0) {
     hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, S.st, out, 0, 1L);
     return hipGetLastError();
   }
-  // levels: tile sums of each level kept in scratch
-  std::vector<long> len;
-  std::vector<long> offs;
-  long l = L, total = 0;
-  while (true) {
-    const long tiles = (l + SCAN_TILE - 1) / SCAN_TILE;
-    len.push_back(l);
-    offs.push_back(total);
-    total += tiles + 1;
-    if (tiles == 1) break;
-    l = tiles;
-  }
-  hipError_t e = S.scratch.ensure((size_t)total * 2);
+  hipError_t e = S.scratch.ensure((size_t)scan_tmp_ints(L));
   if (e != hipSuccess) return e;
-  int* base = S.scratch.p;
-  // level 0: in -> out; level j: tile sums of level j - 1 (at base + offs[j - 1]
-  // in the first half) scanned into the second half
-  const int* lin = in;
-  int* lout = out;
-  for (size_t j = 0; j < len.size(); j++) {
-    const long lj = len[j];
-    const long tiles = (lj + SCAN_TILE - 1) / SCAN_TILE;
-    int* tsum = base + offs[j];
-    hipLaunchKernelGGL(k_scan_tile, dim3((unsigned)tiles), dim3(SCAN_TILE), 0, S.st, lin, lout, tsum, lj);
-    lin = tsum;
-    lout = base + total + offs[j];
-  }
-  // add back from the top: level j's output gets the scanned tile sums of level j
-  for (size_t j = len.size() - 1; j-- > 0;) {
-    const long lj = len[j];
-    const long tiles = (lj + SCAN_TILE - 1) / SCAN_TILE;
-    int* tgt = j == 0 ? out : base + total + offs[j - 1];
-    const int* toff = base + total + offs[j];
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)tiles), dim3(SCAN_TILE), 0, S.st, tgt, toff, lj);
-  }
-  hipLaunchKernelGGL(k_scan_total, dim3(1), dim3(64), 0, S.st, in, out, L);
+  launch_scan_i32(in, (int)L, S.scratch.p, out, S.st, nz, 1);
   return hipGetLastError();
 }
 
@@ -1522,8 +1527,6 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   SR_HIP(S.tmp.ensure(nvert), "nn_surface_run: alloc");
   SR_HIP(S.flag.ensure(nvert), "nn_surface_run: alloc");
   SR_HIP(S.cube_id.ensure(nvert + 1), "nn_surface_run: alloc");
-  SR_HIP(S.tcount.ensure(nvert), "nn_surface_run: alloc");
-  SR_HIP(S.tstart.ensure(nvert + 1), "nn_surface_run: alloc");
   SR_HIP(S.part.ensure(nblock), "nn_surface_run: alloc");
   SR_HIP(S.pcount.ensure(nblock), "nn_surface_run: alloc");
   if (k.vel) {
@@ -1544,8 +1547,6 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   k.tmp = S.tmp.p;
   k.flag = S.flag.p;
   k.cube_id = S.cube_id.p;
-  k.tcount = S.tcount.p;
-  k.tstart = S.tstart.p;
   // hash
   hipLaunchKernelGGL(k_fill_i32, dim3(grid1(nvox, 256)), dim3(256), 0, S.st, k.vcount, 0, nvox);
   hipLaunchKernelGGL(k_vcount, dim3(grid1(n, 256)), dim3(256), 0, S.st, k);
@@ -1570,30 +1571,36 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   if ((rc = device_error(S))) return rc;
   // smoothing
   hipLaunchKernelGGL(k_stats, dim3((unsigned)nblock), dim3(ST_THREADS), 0, S.st, k, 0, S.part.p, S.pcount.p);
-  hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(64), 0, S.st, k, 0, S.part.p, S.pcount.p);
+  hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(ST_THREADS), 0, S.st, k, 0, S.part.p, S.pcount.p);
   hipLaunchKernelGGL(k_stats, dim3((unsigned)nblock), dim3(ST_THREADS), 0, S.st, k, 1, S.part.p, S.pcount.p);
-  hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(64), 0, S.st, k, 1, S.part.p, S.pcount.p);
+  hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(ST_THREADS), 0, S.st, k, 1, S.part.p, S.pcount.p);
   for (int it = 0; it < S.prm.smooth_iterations; it++) {
     hipLaunchKernelGGL(k_smooth, dim3(grid1(nvert, 256)), dim3(256), 0, S.st, k, k.field, k.tmp);
     std::swap(k.field, k.tmp);
   }
   // contour
   hipLaunchKernelGGL(k_cube_flag, dim3(grid1(nvert, 256)), dim3(256), 0, S.st, k);
-  SR_HIP(scan(S, k.flag, k.cube_id, nvert), "nn_surface_run: scan");
+  SR_HIP(scan(S, k.flag, k.cube_id, nvert, 1), "nn_surface_run: scan");
   int nv = 0;
   SR_HIP(hipMemcpyAsync(&nv, k.cube_id + nvert, sizeof(int), hipMemcpyDeviceToHost, S.st), "nn_surface_run: count");
-  hipLaunchKernelGGL(k_cube_id, dim3(grid1(nvert, 256)), dim3(256), 0, S.st, k);
   SR_HIP(hipStreamSynchronize(S.st), "nn_surface_run");
   SR_HIP(S.verts.ensure(3 * (size_t)nv), "nn_surface_run: alloc");
+  SR_HIP(S.cubes.ensure(nv), "nn_surface_run: alloc");
+  SR_HIP(S.tcount.ensure(nv), "nn_surface_run: alloc");
+  SR_HIP(S.tstart.ensure((size_t)nv + 1), "nn_surface_run: alloc");
   k.verts = S.verts.p;
-  hipLaunchKernelGGL(k_dc_point, dim3(grid1(nvert, 128)), dim3(128), 0, S.st, k);
-  SR_HIP(scan(S, k.tcount, k.tstart, nvert), "nn_surface_run: scan");
+  k.cubes = S.cubes.p;
+  k.tcount = S.tcount.p;
+  k.tstart = S.tstart.p;
+  hipLaunchKernelGGL(k_cube_id, dim3(grid1(nvert, 256)), dim3(256), 0, S.st, k);
+  if (nv > 0) hipLaunchKernelGGL(k_dc_point, dim3(grid1(nv, DC_CUBES)), dim3(DC_THREADS), 0, S.st, k, nv);
+  SR_HIP(scan(S, k.tcount, k.tstart, nv), "nn_surface_run: scan");
   int nt = 0;
-  SR_HIP(hipMemcpyAsync(&nt, k.tstart + nvert, sizeof(int), hipMemcpyDeviceToHost, S.st), "nn_surface_run: count");
+  SR_HIP(hipMemcpyAsync(&nt, k.tstart + nv, sizeof(int), hipMemcpyDeviceToHost, S.st), "nn_surface_run: count");
   SR_HIP(hipStreamSynchronize(S.st), "nn_surface_run");
   SR_HIP(S.faces.ensure(3 * (size_t)nt), "nn_surface_run: alloc");
   k.faces = S.faces.p;
-  hipLaunchKernelGGL(k_faces, dim3(grid1(nvert, 128)), dim3(128), 0, S.st, k);
+  if (nv > 0) hipLaunchKernelGGL(k_faces, dim3(grid1(nv, 128)), dim3(128), 0, S.st, k, nv);
   const int want_n = S.prm.normals ? 1 : 0, want_v = S.prm.velocity ? 1 : 0;
   if ((want_n || want_v) && nv > 0) {
     if (want_n) {
