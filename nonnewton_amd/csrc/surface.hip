@@ -571,18 +571,23 @@ __global__ void k_mark(K k) {
 // eighth of them: a lane holds the 8 vertices of one (x, y) column, so the
 // x and y parts of G d are formed once for 8 values, a vertex plane outside
 // the particle's box is skipped by the whole wavefront, and the multiplicity
-// of the reference's voxel-corner loop is a shift (1, 2, 4 or 8).  The
-// wavefronts' sums meet in LDS.  What bounds it is VALU issue: about 45
+// of the reference's voxel-corner loop is a factor (1, 2, 4 or 8).  The
+// wavefronts' sums meet in LDS.  What bounds it is VALU issue: about 36
 // instructions a value, in 26 of every 33 planes and 26^2 of every 33^2
-// columns; 128,000 particles take 4.3 ms against 10.7 with one vertex per
-// lane and every candidate evaluated at all 512.
+// columns; 128,000 particles take 3.3 ms (4.1 with int64 sums, 45 instructions
+// a value; 10.7 with one vertex per lane and every candidate evaluated at all
+// 512).
 // The fixed-point form of v: the double v + 1.5 2^20 has an ulp of 2^-32, so
-// its bits less those of 1.5 2^20 are rint(v 2^32), for |v| < 2^19.  Each lane
-// adds up |v|; only if some total reaches 2^19 or is not a number is the tile
-// summed again in the general form (fix_of, with its error flag).
+// (v + 1.5 2^20) - 1.5 2^20 is v rounded to a multiple of 2^-32, and sums of such
+// below 2^21 are exact in FP64.  Each staged particle adds a bound of its values
+// to a total; only if that reaches 2^18 (a value counts up to 8 times) or is not
+// a number is the tile summed again in the general form (fix_of in int64, with
+// its error flag).
 //
 // FIELD_VELOCITY: the poly6-weighted velocity of the particles within h
-// (generate_smooth_fluid_field_with_velocity_impl, :1160-1190), same layout.
+// (generate_smooth_fluid_field_with_velocity_impl, :1160-1190), same layout:
+// 30,011 particles take 0.235 ms, 0.35 with int64 sums and the full-range root
+// and division.
 //
 // Every tile then has the isotropic poly6 values added (in FIELD_ANISO or, for
 // the isotropic field, FIELD_ISO), one thread per vertex over the 27 voxels
@@ -592,11 +597,17 @@ constexpr int TILE = 8;
 constexpr int FIELD_THREADS = TILE * TILE * TILE;
 constexpr int FIELD_WAVES = FIELD_THREADS / 64;
 constexpr int MAX_COLS = 1536;  // (TILE + R)^2 columns, R + 1 <= 32
-constexpr float FIX_ROOM = 524288.0f;  // 2^19
+constexpr float FIX_ROOM = 262144.0f;  // 2^18
 
-__device__ __forceinline__ unsigned long long fix_fast(float v) {
-  const double t = (double)v + 1572864.0;  // 1.5 2^20
-  return (unsigned long long)__double_as_longlong(t) - 0x4138000000000000ull;
+// acc + mult v (half of that where not `whole`, which is uniform), v rounded to a
+// multiple of 2^-32, where that is exact; acc holds a double
+__device__ __forceinline__ unsigned long long fix_fast(unsigned long long acc, float v, double mult, bool whole) {
+  double r = ((double)v + 1572864.0) - 1572864.0;  // 1.5 2^20
+  if (__builtin_expect(!whole, 0)) r *= 0.5;
+  return (unsigned long long)__double_as_longlong(__builtin_fma(r, mult, __longlong_as_double((long long)acc)));
+}
+__device__ __forceinline__ unsigned long long fix_done(unsigned long long acc) {
+  return (unsigned long long)(long long)(__longlong_as_double((long long)acc) * FIX_SCALE);
 }
 
 // multiplicity of axis position v for a particle of voxel c, as a shift: 0, 1, or -1 for none
@@ -609,6 +620,13 @@ __device__ __forceinline__ float aniso_of(float c48d, float c16d, float q) {
   const float r = q <= 0.5f ? in : out;
   return 0.0f < q && q <= 1.0f ? r : 0.0f;
 }
+// the same for q > 0: past 1 (or not a number) 1 - q is clamped to 0, and the value is +-0
+__device__ __forceinline__ float aniso_mid(float c48d, float c16d, float q) {
+  const float in = c48d * (q * q * q - q * q) + 1.0f;
+  const float u = __builtin_amdgcn_fmed3f(1.0f - q, 0.0f, 1.0f);
+  const float out = c16d * u * u * u;
+  return q <= 0.5f ? in : out;
+}
 
 // one staged particle's values at the 8 vertices of each lane's column
 template <bool GENERAL>
@@ -616,59 +634,100 @@ __device__ __forceinline__ void aniso_column(const K& k, const float4 (&r)[REC_Q
                                              float py, unsigned long long (&acc)[TILE], float& total, bool& bad) {
   const int c0 = uniform(__float_as_int(r[2].w)), c1 = uniform(__float_as_int(r[3].w)), c2 = uniform(__float_as_int(r[4].x));
   const int sx = mult_shift(vx, c0, k.off, k.R), sy = mult_shift(vy, c1, k.off, k.R);
+  const float c48d = k.c48 * r[0].w, c16d = k.c16 * r[0].w;
+  // |q^3 - q^2| <= 1/8 up to q = 1/2, (1 - q)^3 <= 1/8 from there on
+  if (!GENERAL) total += fmaxf(fabsf(c48d), fabsf(c16d)) * 0.1251f + 1.001f;
   if (sx < 0 || sy < 0) return;
   const int sxy = sx + sy;
+  const double mult = (double)(2 << sxy);  // inside the box along z; half of it in its first and last plane
   const float dx = r[0].x - px, dy = r[0].y - py;
   const float ta = r[1].x * dx + r[1].y * dy, tb = r[2].x * dx + r[2].y * dy, tc = r[3].x * dx + r[3].y * dy;
-  const float c48d = k.c48 * r[0].w, c16d = k.c16 * r[0].w;
 #pragma unroll
   for (int z = 0; z < TILE; z++) {
-    const int sz = mult_shift(T[2] + z, c2, k.off, k.R);
-    if (sz < 0) continue;  // uniform
+    const unsigned rel = (unsigned)(T[2] + z - c2 + k.off);  // mult_shift, uniform: 0 .. R, 1 .. R - 1
+    if (rel > (unsigned)k.R) continue;
+    const bool inner = rel - 1u < (unsigned)k.R - 1u;
     const float dz = r[0].z - ((float)(T[2] + z) * k.vs + k.o[2]);
     const float a = ta + r[1].z * dz, b = tb + r[2].z * dz, c = tc + r[3].z * dz;
     const float ss = a * a + b * b + c * c;
-    if (!GENERAL && __all(ss > 1.0f)) continue;  // q = 1 gives 0 too
-    float q = GENERAL ? sqrtf(ss) : sqrt_mid(ss);
-    if (!GENERAL && __builtin_expect(ss < 1e-30f, 0)) q = sqrtf(ss);
-    const float w = k.vol * aniso_of(c48d, c16d, q);
     if (GENERAL) {
+      const float w = k.vol * aniso_of(c48d, c16d, sqrtf(ss));
       if (!(fabsf(w) <= MAX_CONTRIB)) bad = true;
-      else acc[z] += fix_of(w) << (sxy + sz);
+      else acc[z] += fix_of(w) << (sxy + inner);
     } else {
-      total += fabsf(w);
-      acc[z] += fix_fast(w) << (sxy + sz);
+      if (__all(ss > 1.0f)) continue;  // q = 1 gives 0 too
+      float f = aniso_mid(c48d, c16d, sqrt_mid(ss));
+      if (__builtin_expect(ss < 1e-30f, 0)) f = aniso_of(c48d, c16d, sqrtf(ss));
+      acc[z] = fix_fast(acc[z], k.vol * f, mult, inner);
     }
   }
 }
 
+// poly6's constants, with the shorter exact root and division where they hold: a
+// numerator below 2^-103 may round differently, but gives less than 2^-40 there
+// (den >= 2^-63), which times a velocity and voxel_size^3 of less than 2^6
+// rounds to 0 in either form
+struct Poly6 {
+  float h, h2, den, y;
+  bool mid;
+  __device__ __forceinline__ explicit Poly6(const K& k) : h(k.sr), h2(k.sr * k.sr) {
+    den = h2 * h2 * h2 * h2 * h;
+    y = recip_mid(den);
+    mid = k.mid && den > 0x1p-63f && den < 0x1p30f;
+  }
+};
+
 // one staged particle's poly6-weighted velocity at the 8 vertices of each lane's column
-__device__ __forceinline__ void velocity_column(const K& k, const float4& p4, const float4& v4, int c0, int c1, const int* T,
-                                                int vx, int vy, float px, float py, unsigned long long (&acc)[3][TILE],
-                                                bool& bad) {
+// (GENERAL: into the tile's sums at once)
+template <bool GENERAL>
+__device__ __forceinline__ void velocity_column(const K& k, const Poly6& w6, const float4& p4, const float4& v4, int c0, int c1,
+                                                const int* T, int vx, int vy, float px, float py,
+                                                unsigned long long (&acc)[3][TILE], unsigned long long (*sum)[FIELD_THREADS],
+                                                float& total, bool& bad) {
   const int sx = mult_shift(vx, c0, k.off, k.R), sy = mult_shift(vy, c1, k.off, k.R);
+  if (!GENERAL) total += fmaxf(fabsf(v4.x), fmaxf(fabsf(v4.y), fabsf(v4.z)));
   if (sx < 0 || sy < 0) return;
+  const double mult = (double)(2 << (sx + sy));
   const int c2 = uniform(__float_as_int(p4.x));
   const float rx = p4.y - px, ry = p4.z - py;
   if (__all(rx * rx + ry * ry > 1.0001f * k.sr * k.sr)) return;
-#pragma unroll
-  for (int z = 0; z < TILE; z++) {
-    const int sz = mult_shift(T[2] + z, c2, k.off, k.R);
-    if (sz < 0) continue;
+  const auto plane = [&](int z) {
+    const unsigned rel = (unsigned)(T[2] + z - c2 + k.off);  // as in aniso_column
+    if (rel > (unsigned)k.R) return;
+    const bool inner = rel - 1u < (unsigned)k.R - 1u;
     const float rz = p4.w - ((float)(T[2] + z) * k.vs + k.o[2]);
-    if (fabsf(rz) > 1.0001f * k.sr) continue;  // uniform; poly6 is 0 there
-    const float f = poly6(k, rx, ry, rz, k.sr) * k.cvs3;
-    const float u[3] = {v4.x * f, v4.y * f, v4.z * f};
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      if (!(fabsf(u[c]) <= MAX_CONTRIB)) bad = true;
-      else acc[c][z] += fix_of(u[c]) << (sx + sy + sz);
+    if (fabsf(rz) > 1.0001f * k.sr) return;  // uniform; poly6 is 0 there
+    if (GENERAL) {
+      const float f = poly6(k, rx, ry, rz, k.sr) * k.cvs3;
+      const float u[3] = {v4.x * f, v4.y * f, v4.z * f};
+      for (int c = 0; c < 3; c++) {
+        if (!(fabsf(u[c]) <= MAX_CONTRIB)) bad = true;
+        else atomicAdd(&sum[c][((threadIdx.x & 63) << 3) + z], fix_of(u[c]) << (sx + sy + inner));
+      }
+      return;
     }
+    const float ss = rx * rx + ry * ry + rz * rz;
+    const float rn = sqrt_mid(ss);
+    float res = w6.h2 - rn * rn;
+    res = res * res * res;
+    float f = rn <= w6.h ? div_mid(k.acoef * res, w6.den, w6.y) : 0.0f;
+    if (__builtin_expect(ss < 1e-30f, 0)) f = poly6(k, rx, ry, rz, k.sr);
+    f *= k.cvs3;
+    acc[0][z] = fix_fast(acc[0][z], v4.x * f, mult, inner);
+    acc[1][z] = fix_fast(acc[1][z], v4.y * f, mult, inner);
+    acc[2][z] = fix_fast(acc[2][z], v4.z * f, mult, inner);
+  };
+  if constexpr (GENERAL) {
+#pragma unroll 1
+    for (int z = 0; z < TILE; z++) plane(z);
+  } else {
+#pragma unroll
+    for (int z = 0; z < TILE; z++) plane(z);
   }
 }
 
 template <int MODE>
-__global__ __launch_bounds__(FIELD_THREADS) void k_field(K k) {
+__global__ __launch_bounds__(FIELD_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_field(K k) {
   constexpr int QUADS = MODE == FIELD_VELOCITY ? 3 : REC_QUADS;
   __shared__ int col_off[MODE == FIELD_ISO ? 1 : MAX_COLS + 1];
   __shared__ int col_begin[MODE == FIELD_ISO ? 1 : MAX_COLS];
@@ -773,12 +832,13 @@ __global__ __launch_bounds__(FIELD_THREADS) void k_field(K k) {
       thi[a] = (float)(T[a] + TILE - 1) * k.vs + k.o[a];
     }
     unsigned long long acc[MODE == FIELD_VELOCITY ? 3 : 1][TILE];
+    const Poly6 w6(k);
     // a second round, in the general form, only where the first was out of range
     for (int round = 0; round < 2; round++) {
       for (int c = 0; c < (MODE == FIELD_VELOCITY ? 3 : 1); c++)
 #pragma unroll
         for (int z = 0; z < TILE; z++) acc[c][z] = 0ull;
-      float abs_total = 0.0f;
+      float bound = 0.0f;
       for (int s0 = 0; s0 < total; s0 += FIELD_THREADS) {
         if (t == 0) kept = 0;
         __syncthreads();
@@ -821,17 +881,30 @@ __global__ __launch_bounds__(FIELD_THREADS) void k_field(K k) {
             float4 rr[REC_QUADS];
 #pragma unroll
             for (int e = 0; e < REC_QUADS; e++) rr[e] = stage[e * FIELD_THREADS + r];
-            if (round == 0) aniso_column<false>(k, rr, T, vx, vy, px, py, acc[0], abs_total, bad);
-            else aniso_column<true>(k, rr, T, vx, vy, px, py, acc[0], abs_total, bad);
+            if (round == 0) aniso_column<false>(k, rr, T, vx, vy, px, py, acc[0], bound, bad);
+            else aniso_column<true>(k, rr, T, vx, vy, px, py, acc[0], bound, bad);
           } else {
             const float4 c4 = stage[2 * FIELD_THREADS + r];
-            velocity_column(k, stage[r], stage[FIELD_THREADS + r], uniform(__float_as_int(c4.x)), uniform(__float_as_int(c4.y)),
-                            T, vx, vy, px, py, acc, bad);
+            const int v0 = uniform(__float_as_int(c4.x)), v1 = uniform(__float_as_int(c4.y));
+            if (round == 0)
+              velocity_column<false>(k, w6, stage[r], stage[FIELD_THREADS + r], v0, v1, T, vx, vy, px, py, acc, sum, bound, bad);
+            else
+              velocity_column<true>(k, w6, stage[r], stage[FIELD_THREADS + r], v0, v1, T, vx, vy, px, py, acc, sum, bound, bad);
           }
         }
         __syncthreads();
       }
-      if (MODE != FIELD_ANISO || !__syncthreads_or(!(abs_total < FIX_ROOM))) break;
+      if (round == 1) break;
+      // poly6 <= acoef h^6 / h^9
+      const bool fits = MODE == FIELD_ANISO ? fabsf(k.vol) * bound < FIX_ROOM
+                                            : w6.mid && fabsf(k.acoef * k.cvs3 / (w6.h2 * w6.h)) * 1.001f * bound < FIX_ROOM &&
+                                                  bound * k.cvs3 < 64.0f;
+      if (!__syncthreads_or(!fits)) {
+        for (int c = 0; c < (MODE == FIELD_VELOCITY ? 3 : 1); c++)
+#pragma unroll
+          for (int z = 0; z < TILE; z++) acc[c][z] = fix_done(acc[c][z]);
+        break;
+      }
     }
     for (int c = 0; c < (MODE == FIELD_VELOCITY ? 3 : 1); c++)
 #pragma unroll

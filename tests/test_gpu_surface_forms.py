@@ -1,6 +1,8 @@
-"""The contour over compacted cubes against the oracle bit for bit: cube counts
-around a workgroup's 64, and a voxel grid whose scan needs its block sums scanned
-first (more than 2^25 voxels)."""
+"""The smooth field's FP64 tile sums and the contour over compacted cubes against
+the oracle bit for bit: velocities whose sums fit and whose sums take the
+general form, a smooth radius below the range of the short poly6 quotient, cube
+counts around a workgroup's 64, and a voxel grid whose scan needs its block sums
+scanned first (more than 2^25 voxels)."""
 import numpy as np
 import pytest
 
@@ -30,6 +32,17 @@ def block(n, seed, sp):
     k = np.arange(n)
     x = np.stack([k // (a * a), k // a % a, k % a], 1) * sp + 10.5 * sp
     return (x + np.random.Generator(np.random.PCG64(seed)).uniform(-0.15 * sp, 0.15 * sp, x.shape)).astype(np.float32)
+
+
+@pytest.mark.parametrize("scale,sp", [(1.0, 0.02), (1e7, 0.02), (1.0, 0.0016)])
+def test_velocity_sums(scale, sp):
+    """h = 0.05 and 0.004 (h^9 below 2^-63)."""
+    x = block(600, 3, sp)
+    u = (scale * np.random.Generator(np.random.PCG64(4)).uniform(-1, 1, x.shape)).astype(np.float32)
+    small = sp < 0.01  # no negative values there: nothing to smooth by
+    o = check(x, u, voxel_size=sp / 2, particle_radius=sp, smooth_radius=2.5 * sp, normals=True,
+              isolevel=0.2 if small else 0.0, smooth_iterations=0 if small else 1)
+    assert np.any(o["mesh_velocity"] != 0)
 
 
 @pytest.mark.parametrize("voxel", [0.05, 0.045, 0.04, 0.036, 0.03])
