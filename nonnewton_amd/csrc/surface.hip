@@ -64,7 +64,8 @@ struct K {
   int *vcount, *vstart, *vslot, *vlist;
   float *G, *xbar;
   unsigned char* active;
-  float4* rec;  // REC_QUADS per entry of vlist
+  float4* sorted;  // per entry of vlist: position, particle
+  float4* rec;     // REC_QUADS per entry of vlist
   float *field0, *field, *tmp;
   int *flag, *cube_id;      // per vertex of the grid: its cube's code and mesh vertex + 1
   int *cubes, *tcount, *tstart;  // per mesh vertex: its cube, its triangles
@@ -101,32 +102,6 @@ __device__ __forceinline__ float sr_expf(float x) {
 
 // cyclic Jacobi eigen-decomposition of a symmetric 3x3 (Golub & Van Loan,
 // Alg. 8.5.2), 6 sweeps; ev = the diagonal, V = the accumulated rotations
-__device__ __forceinline__ void jrot(float* S, float* V, int p, int q) {
-  const float apq = S[3 * p + q];
-  if (apq == 0.0f) return;
-  const float theta = (S[3 * q + q] - S[3 * p + p]) / (2.0f * apq);
-  const float t = (theta >= 0.0f ? 1.0f : -1.0f) / (fabsf(theta) + sqrtf(theta * theta + 1.0f));
-  const float c = 1.0f / sqrtf(t * t + 1.0f);
-  const float s = t * c;
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    const float a = S[3 * k + p], b = S[3 * k + q];
-    S[3 * k + p] = c * a - s * b;
-    S[3 * k + q] = s * a + c * b;
-  }
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    const float a = S[3 * p + k], b = S[3 * q + k];
-    S[3 * p + k] = c * a - s * b;
-    S[3 * q + k] = s * a + c * b;
-  }
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    const float a = V[3 * k + p], b = V[3 * k + q];
-    V[3 * k + p] = c * a - s * b;
-    V[3 * k + q] = s * a + c * b;
-  }
-}
 __device__ __forceinline__ void eig3(const float* A, float* ev, float* V) {
   float S[9];
 #pragma unroll
@@ -134,9 +109,9 @@ __device__ __forceinline__ void eig3(const float* A, float* ev, float* V) {
 #pragma unroll
   for (int k = 0; k < 9; k++) V[k] = (k % 4) == 0 ? 1.0f : 0.0f;
   for (int sweep = 0; sweep < 6; sweep++) {
-    jrot(S, V, 0, 1);
-    jrot(S, V, 0, 2);
-    jrot(S, V, 1, 2);
+    jacobi_rot(S, V, 0, 1);
+    jacobi_rot(S, V, 0, 2);
+    jacobi_rot(S, V, 1, 2);
   }
   ev[0] = S[0];
   ev[1] = S[4];
@@ -261,117 +236,33 @@ __global__ void k_vcount(K k) {
   k.vslot[i] = slot;
 }
 
-__global__ void k_vplace(K k) {
+__global__ void k_vplace(K k, int* bucket) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= k.n) return;
   int v[3];
   voxel_of(k, k.pos + 3 * (long)i, v);
-  k.vlist[k.vstart[vkey(k, v)] + k.vslot[i]] = i;
+  bucket[k.vstart[vkey(k, v)] + k.vslot[i]] = i;
 }
 
-// a voxel's list in increasing particle index (insertion sort, <= 64 entries)
-__global__ void k_vsort(K k) {
-  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= k.nvox) return;
-  const int b = k.vstart[q], e = k.vstart[q + 1];
-  for (int m = b + 1; m < e; m++) {
-    const int x = k.vlist[m];
-    int j = m - 1;
-    while (j >= b && k.vlist[j] > x) {
-      k.vlist[j + 1] = k.vlist[j];
-      j--;
-    }
-    k.vlist[j + 1] = x;
+// a voxel's particles in increasing index (a particle's place is the number of
+// lower indices there; a voxel with too many is reported, k_vcount): vlist, and
+// their positions in the same order
+__global__ void k_vsort(K k, const int* bucket) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= k.n) return;
+  const int i = bucket[t];
+  const float* x = k.pos + 3 * (long)i;
+  int v[3];
+  voxel_of(k, x, v);
+  const long key = vkey(k, v);
+  const int b = k.vstart[key], e = k.vstart[key + 1];
+  int dest = t;
+  if (e - b <= MAX_PER_VOXEL) {
+    dest = b;
+    for (int m = b; m < e; m++) dest += bucket[m] < i;
   }
-}
-
-__device__ __forceinline__ void vrange(const K& k, int x, int y, int z, int& b, int& e) {
-  const int a = x - k.vlo[0], c = y - k.vlo[1], d = z - k.vlo[2];
-  if (a < 0 || c < 0 || d < 0 || a >= k.vdim[0] || c >= k.vdim[1] || d >= k.vdim[2]) {
-    b = e = 0;
-    return;
-  }
-  const long q = ((long)a * k.vdim[1] + c) * k.vdim[2] + d;
-  b = k.vstart[q];
-  e = k.vstart[q + 1];
-}
-
-template <int G, int U>
-__device__ __forceinline__ int lane_bcast_i(int v) {
-  return __float_as_int(lane_bcast<G, U>(__int_as_float(v)));
-}
-// lane r's (first, shift) of G runs laid end to end: the shift of the run that holds candidate c
-template <int G, int U>
-__device__ __forceinline__ int shift_at(int c, int first, int shift, int sh) {
-  if constexpr (U < G) {
-    const int f = lane_bcast_i<G, U>(first), s = lane_bcast_i<G, U>(shift);
-    return shift_at<G, U + 1>(c, first, shift, c >= f ? s : sh);
-  }
-  return sh;
-}
-
-// The particles a sweep of pre_process_data visits, in its order (voxel dx,
-// dy, dz nested, z fastest, then the voxel's list), restricted to the voxels
-// that can hold a particle closer than r2: a voxel's particles are contiguous
-// in vlist and the voxels of one (x, y) column are consecutive, so each
-// column is one range.  A skipped particle has w = 0 and adds +0 to every sum
-// (rows and column ends are trimmed with a margin of 1e-3 voxel around each
-// voxel and 1e-4 of r2), so the sums are those of the full loop bit for bit.
-//
-// G lanes per particle (4 or 16): they find the ranges of G columns at a time,
-// lay them end to end, and take candidates q, q + G, ...; term(entry of vlist
-// or -1, t) forms a candidate's N terms and the group adds them in order.
-template <int G, int N, typename Term>
-__device__ __forceinline__ void for_reach(const K& k, int q, const int* v, float x0, float x1, float x2, float r2,
-                                          float (&acc)[N], Term term) {
-  const int R = k.R, off = k.off;
-  const float reach = r2 * 1.0001f;
-  const float reach2 = reach * reach;
-  const float m = 1e-3f * k.vs;
-  for (int col0 = 0; col0 < R * R; col0 += G) {
-    const int col = col0 + q;
-    int b = 0, len = 0;
-    const int x = v[0] + col / R - off, y = v[1] + col % R - off;
-    if (col < R * R && x >= 0 && x >= k.vlo[0] && x < k.vlo[0] + k.vdim[0] && y >= 0 && y >= k.vlo[1] && y < k.vlo[1] + k.vdim[1]) {
-      const float lx = (float)x * k.vs + k.o[0] - m, hx = lx + k.vs + 2.0f * m;
-      const float gx = fmaxf(0.0f, fmaxf(lx - x0, x0 - hx));
-      const float ly = (float)y * k.vs + k.o[1] - m, hy = ly + k.vs + 2.0f * m;
-      const float gy = fmaxf(0.0f, fmaxf(ly - x1, x1 - hy));
-      const float rest = reach2 - (gx * gx + gy * gy);
-      if (rest > 0.0f) {
-        const float zr = sqrtf(rest);
-        int z0 = (int)floorf((x2 - zr - k.o[2]) / k.vs) - 1;
-        int z1 = (int)floorf((x2 + zr - k.o[2]) / k.vs) + 1;
-        z0 = max(max(z0, v[2] - off), max(0, k.vlo[2]));
-        z1 = min(min(z1, v[2] - off + R - 1), k.vlo[2] + k.vdim[2] - 1);
-        if (z0 <= z1) {
-          const long base = ((long)(x - k.vlo[0]) * k.vdim[1] + (y - k.vlo[1])) * k.vdim[2] - k.vlo[2];
-          b = k.vstart[base + z0];
-          len = k.vstart[base + z1 + 1] - b;
-        }
-      }
-    }
-    // inclusive scan of the lengths over the group
-    int incl = len;
-#pragma unroll
-    for (int d = 1; d < G; d <<= 1) {
-      const int u = __shfl_up(incl, d, G);
-      if (q >= d) incl += u;
-    }
-    const int first = incl - len, shift = b - first;
-    const int total = lane_bcast_i<G, G - 1>(incl);
-    for (int c0 = 0; c0 < total; c0 += G) {
-      const int c = c0 + q;
-      const int e = c + shift_at<G, 0>(c, first, shift, 0);
-      float t[N];
-      term(c < total ? e : -1, t);
-      auto add = [&](const float (&b)[N], bool) {
-#pragma unroll
-        for (int n = 0; n < N; n++) acc[n] += b[n];
-      };
-      add_in_order<G, N, 0>(t, G, add);
-    }
-  }
+  k.vlist[dest] = i;
+  k.sorted[dest] = make_float4(x[0], x[1], x[2], __int_as_float(i));
 }
 
 // Record of list entry m (particle j = vlist[m]), for the field's tiles:
@@ -381,28 +272,182 @@ __device__ __forceinline__ void for_reach(const K& k, int q, const int* v, float
 // |G d| > 1.  G = V diag(1 / (h s)) V^T with V orthonormal to FP32 rounding,
 // so |G d| >= |d| / (h max |s|) less a few ulp; 1% covers them.
 constexpr int REC_QUADS = 5;
-constexpr int ANISO_THREADS = 64;
-constexpr long ANISO_WIDE = 32768;  // 16 lanes and 4 take the same time at 32,000 particles
+// Lists and sums of k_aniso, a workgroup of one wavefront with 16 lanes per
+// particle.  Data crosses lanes of a group through LDS, which a wavefront's
+// accesses reach in order; wave_order() keeps the compiler to that order.
+constexpr int AN_GROUPS = 4;   // particles of a workgroup
+constexpr int AN_CAND = 128;   // candidates laid out at a time
+constexpr int AN_LIST = 1024;  // neighbors held for the second pass
+constexpr int AN_BATCH = 32;   // neighbors whose terms are formed together
+struct AnisoLds {
+  int cand[AN_GROUPS][AN_CAND];
+  unsigned short list[AN_GROUPS][AN_LIST];  // less a base
+  float term[AN_GROUPS][6][AN_BATCH + 4];
+};
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The particles within r2 (to 1e-5) of one at x in the order of pre_process_data
+// (voxel dx, dy, dz nested, z fastest, then the voxel's list), as entries of
+// vlist less `base`, into the group's list; full(count) takes the list whenever
+// it may not hold the next 64.  Returns the entries left in the list.
+//
+// A voxel's particles are contiguous in vlist and the voxels of one (x, y)
+// column are consecutive, so a column is one range: the lanes find those of 32
+// columns at a time, restricted to the voxels that can hold a particle closer
+// than r2 (rows and column ends are trimmed with a margin of 1e-3 voxel around
+// each voxel and 1e-4 of r2), lay their entries end to end, and test 16 a round.
+// Particles left out have weight 0 and would add +0 to every sum.
+template <typename Full>
+__device__ __forceinline__ int find_neighbors(const K& k, AnisoLds& lds, int g, int q, const int* v, float4 x, float r2,
+                                              int& base, Full full) {
+  const int R = k.R, off = k.off;
+  const float reach = r2 * 1.0001f;
+  const float reach2 = reach * reach;
+  const float m = 1e-3f * k.vs;
+  int* cand = lds.cand[g];
+  unsigned short* list = lds.list[g];
+  const int base_lane = threadIdx.x & 48;
+  const float within = r2 * 1.00001f, within2 = within * within;
+  int cnt = 0;
+  for (int col0 = 0; col0 < R * R; col0 += 32) {
+    int b[2], len[2];
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      const int col = col0 + 2 * q + s;
+      b[s] = len[s] = 0;
+      const int cx = v[0] + col / R - off, cy = v[1] + col % R - off;
+      if (col < R * R && cx >= max(0, k.vlo[0]) && cx < k.vlo[0] + k.vdim[0] && cy >= max(0, k.vlo[1]) &&
+          cy < k.vlo[1] + k.vdim[1]) {
+        const float lx = (float)cx * k.vs + k.o[0] - m, hx = lx + k.vs + 2.0f * m;
+        const float gx = fmaxf(0.0f, fmaxf(lx - x.x, x.x - hx));
+        const float ly = (float)cy * k.vs + k.o[1] - m, hy = ly + k.vs + 2.0f * m;
+        const float gy = fmaxf(0.0f, fmaxf(ly - x.y, x.y - hy));
+        const float rest = reach2 - (gx * gx + gy * gy);
+        if (rest > 0.0f) {
+          const float zr = sqrtf(rest);
+          int z0 = (int)floorf((x.z - zr - k.o[2]) / k.vs) - 1;
+          int z1 = (int)floorf((x.z + zr - k.o[2]) / k.vs) + 1;
+          z0 = max(max(z0, v[2] - off), max(0, k.vlo[2]));
+          z1 = min(min(z1, v[2] - off + R - 1), k.vlo[2] + k.vdim[2] - 1);
+          if (z0 <= z1) {
+            const long at = ((long)(cx - k.vlo[0]) * k.vdim[1] + (cy - k.vlo[1])) * k.vdim[2] - k.vlo[2];
+            b[s] = k.vstart[at + z0];
+            len[s] = k.vstart[at + z1 + 1] - b[s];
+          }
+        }
+      }
+    }
+    int incl = len[0] + len[1];  // scanned over the group
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1) {
+      const int u = __shfl_up(incl, d, 16);
+      if (q >= d) incl += u;
+    }
+    const int total = __float_as_int(lane_bcast<16, 15>(__int_as_float(incl)));
+    const int first[2] = {incl - len[0] - len[1], incl - len[1]};
+    for (int c0 = 0; c0 < total; c0 += AN_CAND) {
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+        for (int t = max(0, c0 - first[s]); t < min(len[s], c0 + AN_CAND - first[s]); t++) cand[first[s] + t - c0] = b[s] + t;
+      wave_order();
+      const int n = min(AN_CAND, total - c0);
+      for (int r = 0, lim; r < n; r = lim) {
+        lim = min(r + 64, n);  // entries increase along the sequence
+        if (cnt + 64 > AN_LIST || cand[lim - 1] - base > 0xFFFF) {
+          if (cnt) full(cnt);
+          cnt = 0;
+          base = cand[r];
+          while (cand[lim - 1] - base > 0xFFFF) lim--;
+        }
+        int e[4];
+        float4 p[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const int c = r + 16 * u + q;
+          e[u] = cand[c < lim ? c : r];
+          p[u] = k.sorted[e[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const float dx = x.x - p[u].x, dy = x.y - p[u].y, dz = x.z - p[u].z;
+          const bool hit = r + 16 * u + q < lim && dx * dx + dy * dy + dz * dz < within2;
+          const int hits = (int)(__ballot(hit) >> base_lane) & 0xFFFF;
+          if (hit) list[cnt + __popc(hits & ((1 << q) - 1))] = (unsigned short)(e[u] - base);
+          cnt += __popc(hits);
+        }
+      }
+      wave_order();  // cand is written again
+    }
+  }
+  return cnt;
+}
+
+// N sums over `cnt` entries of the group's list, in order: every lane forms the
+// terms of its entries, lane n < N adds up sum n.
+template <int N, typename Term>
+__device__ __forceinline__ void add_neighbors(const K& k, AnisoLds& lds, int g, int q, int base, int cnt, float& acc,
+                                              Term term) {
+  const unsigned short* list = lds.list[g];
+  for (int c0 = 0; c0 < cnt; c0 += AN_BATCH) {
+    float4 p[AN_BATCH / 16];
+#pragma unroll
+    for (int u = 0; u < AN_BATCH / 16; u++) {
+      const int c = c0 + 16 * u + q;
+      p[u] = k.sorted[base + list[c < cnt ? c : 0]];
+    }
+#pragma unroll
+    for (int u = 0; u < AN_BATCH / 16; u++) {
+      float t[N];
+      const bool on = c0 + 16 * u + q < cnt;
+      term(p[u], on, t);
+#pragma unroll
+      for (int n = 0; n < N; n++) lds.term[g][n][16 * u + q] = on ? t[n] : NEUTRAL;
+    }
+    wave_order();
+    if (q < N) {
+      const float4* row = reinterpret_cast<const float4*>(lds.term[g][q]);
+#pragma unroll
+      for (int h = 0; h < AN_BATCH / 4; h++) {
+        const float4 t = row[h];
+        acc += t.x;
+        acc += t.y;
+        acc += t.z;
+        acc += t.w;
+      }
+    }
+    wave_order();  // the terms are written again
+  }
+}
 
 // pre_process_data (:1007-1112) for particle i >= 1 (particle 0 keeps G = 0,
 // x_bar = 0: the reference's loop starts at 1 and reset() zeroes both), in
-// the order of the voxel lists.  16 lanes per particle while they are few, 4
-// once the device is full (a lane repeats its group's additions and searches
-// its group's columns): 2,000 particles take 0.14 ms against 2.0 with one lane
-// each walking about 900 neighbors twice, 128,000 take 1.78 with 4 lanes, 2.60
-// with 16 and 3.05 with one.
-template <int L>
-__global__ void k_aniso(K k) {
-  const int m = (blockIdx.x * blockDim.x + threadIdx.x) / L, q = threadIdx.x & (L - 1);
+// the order of the voxel lists.  16 lanes per particle find its neighbors once
+// into LDS and walk them twice; a sum's additions, serial by their order, are
+// one lane's.  What bounds it is issue, and at 2,000 particles the chain of
+// loads.  Milliseconds at 2,000 / 30,011 / 128,000 particles: 0.067 / 0.145 /
+// 1.19; with the columns searched twice and every lane of a group repeating its
+// additions 0.140 / 0.312 / 1.77; lists of 4-byte entries leave six workgroups
+// to a CU instead of eleven and take 0.066 / 0.211 / 1.89.
+__global__ __launch_bounds__(16 * AN_GROUPS) void k_aniso(K k) {
+  __shared__ __align__(16) AnisoLds lds;
+  const int grp = threadIdx.x >> 4, q = threadIdx.x & 15;
+  const int m = blockIdx.x * AN_GROUPS + grp;
   if (m >= k.n) return;  // whole groups leave together
-  const int i = k.vlist[m];
+  const float4 own = k.sorted[m];
+  const int i = __float_as_int(own.w);
   float* G = k.G + 9 * (long)i;
   float* xb = k.xbar + 3 * (long)i;
   float4* rec = k.rec + (long)REC_QUADS * m;
-  const float* xi = k.pos + 3 * (long)i;
-  const float x0 = xi[0], x1 = xi[1], x2 = xi[2];
+  const float x0 = own.x, x1 = own.y, x2 = own.z;
   int v[3];
-  voxel_of(k, xi, v);
+  {
+    const float xi[3] = {x0, x1, x2};
+    voxel_of(k, xi, v);
+  }
   if (i == 0) {
     if (q == 0) {
       for (int a = 0; a < 9; a++) G[a] = 0.0f;
@@ -417,8 +462,8 @@ __global__ void k_aniso(K k) {
   }
   const float r2 = 2.0f * k.sr;
   const float r2y = recip_mid(r2);
-  auto weight = [&](float y0, float y1, float y2) {
-    const float dx = x0 - y0, dy = x1 - y1, dz = x2 - y2;
+  const auto weight = [&](const float4& y) {
+    const float dx = x0 - y.x, dy = x1 - y.y, dz = x2 - y.z;
     const float ss = dx * dx + dy * dy + dz * dz;
     float nr = sqrt_mid(ss);
     float t = div_mid(nr, r2, r2y);
@@ -428,16 +473,29 @@ __global__ void k_aniso(K k) {
     }
     return nr < r2 ? 1.0f - t * t * t : 0.0f;
   };
-  float sw[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for_reach<L, 4>(k, q, v, x0, x1, x2, r2, sw, [&](int e, float (&t)[4]) {
-    const float* xj = k.pos + 3 * (long)(e >= 0 ? k.vlist[e] : i);
-    const float y0 = xj[0], y1 = xj[1], y2 = xj[2];
-    const float w = weight(y0, y1, y2);
-    t[0] = e >= 0 ? w : NEUTRAL;
-    t[1] = e >= 0 ? w * y0 : NEUTRAL;
-    t[2] = e >= 0 ? w * y1 : NEUTRAL;
-    t[3] = e >= 0 ? w * y2 : NEUTRAL;
+  float sum = 0.0f;
+  int nn = 0;  // neighbors: w > 0
+  bool whole = true;  // the list has held them all
+  constexpr int NO_BASE = -0x10000;  // farther below every entry than the list reaches
+  int base = NO_BASE;
+  const auto first_pass = [&](int cnt) {
+    add_neighbors<4>(k, lds, grp, q, base, cnt, sum, [&](const float4& y, bool on, float (&t)[4]) {
+      const float w = weight(y);
+      nn += on && w > 0.0f;
+      t[0] = w;
+      t[1] = w * y.x;
+      t[2] = w * y.y;
+      t[3] = w * y.z;
+    });
+  };
+  const int left = find_neighbors(k, lds, grp, q, v, own, r2, base, [&](int cnt) {
+    wave_order();
+    first_pass(cnt);
+    whole = false;
   });
+  wave_order();
+  first_pass(left);
+  const float sw[4] = {lane_bcast<16, 0>(sum), lane_bcast<16, 1>(sum), lane_bcast<16, 2>(sum), lane_bcast<16, 3>(sum)};
   const float tw = sw[0];
   float w0 = sw[1], w1 = sw[2], w2 = sw[3];
   if (tw != 0.0f) {
@@ -446,23 +504,35 @@ __global__ void k_aniso(K k) {
     w2 /= tw;
   }
   const float b0 = k.lam1 * x0 + k.lam * w0, b1 = k.lam1 * x1 + k.lam * w1, b2 = k.lam1 * x2 + k.lam * w2;
-  // C is symmetric bit for bit (w (a b) and w (b a)): six sums, and the
-  // neighbors (w > 0) counted beside them
-  int nn = 0;
-  float cs[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-  for_reach<L, 6>(k, q, v, x0, x1, x2, r2, cs, [&](int e, float (&t)[6]) {
-    const float* xj = k.pos + 3 * (long)(e >= 0 ? k.vlist[e] : i);
-    const float y0 = xj[0], y1 = xj[1], y2 = xj[2];
-    const float w = weight(y0, y1, y2);
-    const bool on = e >= 0 && w > 0.0f;
-    nn += __popc((unsigned)(__ballot(on) >> (threadIdx.x & 63 & ~(L - 1))) & ((1u << L) - 1u));
-    const float dp[3] = {y0 - w0, y1 - w1, y2 - w2};
-    int n = 0;
+  // C is symmetric bit for bit (w (a b) and w (b a)): six sums
+  sum = 0.0f;
+  const auto second_pass = [&](int cnt) {
+    add_neighbors<6>(k, lds, grp, q, base, cnt, sum, [&](const float4& y, bool, float (&t)[6]) {
+      const float w = weight(y);
+      const float dp[3] = {y.x - w0, y.y - w1, y.z - w2};
+      int n = 0;
 #pragma unroll
-    for (int a = 0; a < 3; a++)
+      for (int a = 0; a < 3; a++)
 #pragma unroll
-      for (int c = a; c < 3; c++) t[n++] = on ? w * (dp[a] * dp[c]) : NEUTRAL;
-  });
+        for (int c = a; c < 3; c++) t[n++] = w * (dp[a] * dp[c]);
+    });
+  };
+  if (whole) {
+    second_pass(left);
+  } else {
+    base = NO_BASE;
+    const int rest = find_neighbors(k, lds, grp, q, v, own, r2, base, [&](int cnt) {
+      wave_order();
+      second_pass(cnt);
+    });
+    wave_order();
+    second_pass(rest);
+  }
+  // the lanes' counts
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) nn += __shfl_xor(nn, d, 16);
+  const float cs[6] = {lane_bcast<16, 0>(sum), lane_bcast<16, 1>(sum), lane_bcast<16, 2>(sum),
+                       lane_bcast<16, 3>(sum), lane_bcast<16, 4>(sum), lane_bcast<16, 5>(sum)};
   float C[9] = {cs[0], cs[1], cs[2], cs[1], cs[3], cs[4], cs[2], cs[4], cs[5]};
   if (tw != 0.0f)
 #pragma unroll
@@ -765,8 +835,8 @@ __global__ __launch_bounds__(FIELD_THREADS) __attribute__((amdgpu_waves_per_eu(4
         for (int y = max(vy - 1, k.vlo[1]); y <= min(vy + 1, k.vlo[1] + k.vdim[1] - 1); y++) {
           const long base = ((long)(x - k.vlo[0]) * k.vdim[1] + (y - k.vlo[1])) * k.vdim[2] - k.vlo[2];
           for (int m = k.vstart[base + z0]; m < k.vstart[base + z1 + 1]; m++) {
-            const float* xj = k.pos + 3 * (long)k.vlist[m];
-            const float w = k.vol * poly6(k, xj[0] - p[0], xj[1] - p[1], xj[2] - p[2], k.sr);
+            const float4 xj = k.sorted[m];
+            const float w = k.vol * poly6(k, xj.x - p[0], xj.y - p[1], xj.z - p[2], k.sr);
             if (!(fabsf(w) <= MAX_CONTRIB)) bad = true;
             else acc += fix_of(w);
           }
@@ -1471,7 +1541,7 @@ struct Surface {
   DBuf<float> pos, vel, G, xbar, field0, field, tmp, verts, normals, vfield, mvel;
   DBuf<int> vcount, vstart, vslot, vlist, pvox, flag, cube_id, cubes, tcount, tstart, faces, err, bounds, scratch;
   DBuf<unsigned char> active;
-  DBuf<float4> rec;
+  DBuf<float4> rec, sorted;
   DBuf<double> stats, part;
   DBuf<long long> pcount;
   long nverts = 0, ntris = 0, nactive = 0;
@@ -1485,6 +1555,7 @@ struct Surface {
       b->release();
     active.release();
     rec.release();
+    sorted.release();
     stats.release();
     part.release();
     pcount.release();
@@ -1590,6 +1661,7 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   SR_HIP(S.vstart.ensure(nvox + 1), "nn_surface_run: alloc");
   SR_HIP(S.vslot.ensure(n), "nn_surface_run: alloc");
   SR_HIP(S.vlist.ensure(n), "nn_surface_run: alloc");
+  SR_HIP(S.sorted.ensure(n), "nn_surface_run: alloc");
   SR_HIP(S.pvox.ensure(3 * n), "nn_surface_run: alloc");
   SR_HIP(S.G.ensure(9 * n), "nn_surface_run: alloc");
   SR_HIP(S.xbar.ensure(3 * n), "nn_surface_run: alloc");
@@ -1614,6 +1686,7 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   k.G = S.G.p;
   k.xbar = S.xbar.p;
   k.rec = S.rec.p;
+  k.sorted = S.sorted.p;
   k.active = S.active.p;
   k.field0 = S.field0.p;
   k.field = S.field.p;
@@ -1624,14 +1697,12 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   hipLaunchKernelGGL(k_fill_i32, dim3(grid1(nvox, 256)), dim3(256), 0, S.st, k.vcount, 0, nvox);
   hipLaunchKernelGGL(k_vcount, dim3(grid1(n, 256)), dim3(256), 0, S.st, k);
   SR_HIP(scan(S, k.vcount, k.vstart, nvox), "nn_surface_run: scan");
-  hipLaunchKernelGGL(k_vplace, dim3(grid1(n, 256)), dim3(256), 0, S.st, k);
-  hipLaunchKernelGGL(k_vsort, dim3(grid1(nvox, 256)), dim3(256), 0, S.st, k);
+  int* bucket = reinterpret_cast<int*>(k.xbar);  // written by k_aniso, after this
+  hipLaunchKernelGGL(k_vplace, dim3(grid1(n, 256)), dim3(256), 0, S.st, k, bucket);
+  hipLaunchKernelGGL(k_vsort, dim3(grid1(n, 256)), dim3(256), 0, S.st, k, bucket);
   if ((rc = device_error(S))) return rc;
   // anisotropic kernel and field
-  if (k.aniso) {
-    if (n <= ANISO_WIDE) hipLaunchKernelGGL(k_aniso<16>, dim3(grid1(16 * n, ANISO_THREADS)), dim3(ANISO_THREADS), 0, S.st, k);
-    else hipLaunchKernelGGL(k_aniso<4>, dim3(grid1(4 * n, ANISO_THREADS)), dim3(ANISO_THREADS), 0, S.st, k);
-  }
+  if (k.aniso) hipLaunchKernelGGL(k_aniso, dim3(grid1(n, AN_GROUPS)), dim3(16 * AN_GROUPS), 0, S.st, k);
   hipLaunchKernelGGL(k_fill_u8, dim3(grid1(nblock, 256)), dim3(256), 0, S.st, k.active, nblock);
   hipLaunchKernelGGL(k_mark, dim3(grid1(n, 256)), dim3(256), 0, S.st, k);
   const dim3 tiles((unsigned)(nvert / FIELD_THREADS)), ft(FIELD_THREADS);
