@@ -204,6 +204,8 @@ int32_t nn_counts(nn_ctx *ctx, int64_t *n, int64_t *n_fluid);
  * many independent scenes resident in HBM in one concatenated, offset-indexed
  * particle array and advances all of them with one launch sequence per tick.
  * ------------------------------------------------------------------------- */
+/* Beside its scenes a pool holds up to an eighth of its budget in memory that
+ * scenes have left, for the next ones; nn_pool_destroy gives it back. */
 int32_t nn_pool_create(int64_t budget_bytes, nn_pool **out);
 /* nn_pool_create with flags.  NN_POOL_OWN_QUEUE: the pool's stream gets a
  * hardware queue of its own (a stream whose CU mask covers every CU), so that

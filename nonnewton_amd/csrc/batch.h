@@ -5,6 +5,7 @@
 // changes between ticks.
 #pragma once
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -81,9 +82,37 @@ struct KernelTimer {
   void reset();
 };
 
+// Device and pinned host memory that a pool's batches have given up, kept for
+// its next ones: an admission makes a staging batch and a later one frees it.
+// 64 admissions took 104 ms, 52 of them in hipMalloc, hipFree and their pinned
+// counterparts (the frees wait for the device); with these blocks, the upload
+// expanded on the device and no second search for scenes without a stress set,
+// 41 ms.  At most `limit` device bytes and 64 pinned blocks
+// are held, the oldest freed first, all of them when an allocation fails and when
+// the pool goes.  Any thread; a block is given only when no work on it is
+// pending, and taken for the device it is on.
+class Spares {
+ public:
+  explicit Spares(size_t limit) : limit_(limit) {}
+  ~Spares() { clear(); }
+  bool take(bool host, size_t bytes, void** p, size_t* got);
+  void give(bool host, void* p, size_t bytes);
+  void clear();
+
+ private:
+  struct Block {
+    void* p;
+    size_t bytes;
+    int device;
+  };
+  std::mutex mu_;
+  std::vector<Block> dev_, host_;
+  size_t held_ = 0, limit_;
+};
+
 class Batch {
  public:
-  explicit Batch(hipStream_t stream);
+  explicit Batch(hipStream_t stream, std::shared_ptr<Spares> spares = nullptr);
   ~Batch();
   Batch(const Batch&) = delete;
   Batch& operator=(const Batch&) = delete;
@@ -108,7 +137,11 @@ class Batch {
   // When set, arrays replaced by layout() are not freed but handed out by
   // take_deferred(), to be freed off the thread that steps the batch.
   bool defer_free_ = false;
-  void take_deferred(std::vector<void*>& out);
+  struct Alloc {
+    void* p;
+    size_t bytes;
+  };
+  void take_deferred(std::vector<Alloc>& out);
   int upload(int k, const float* x, const float* v, const int* kind);
   int init_scenes(const std::vector<int>& which);  // search, rest state, boundary volumes
   int search();
@@ -131,10 +164,9 @@ class Batch {
   KernelTimer timer;
 
  private:
-  struct Alloc {
-    void* p;
-    size_t bytes;
-  };
+  std::shared_ptr<Spares> spares_;
+  int alloc_host(void** p, size_t bytes);
+  void free_host(void* p, size_t bytes);
   std::vector<Alloc> allocs_;
   long long bytes_ = 0;
   int C_total_ = 0;  // cells in use
@@ -142,7 +174,7 @@ class Batch {
   int scene_cap_ = 0;
   int n_cg_blocks_ = 0;  // entries of d.cg_blocks
   int solve_waves_ = -1;  // waves k_cg_solve may have (-1: not looked up yet)
-  std::vector<void*> deferred_;
+  std::vector<Alloc> deferred_;
   // pinned, h_state_cap_ entries each, with their device addresses: scene states
   // and report words (ticket in the high half), and the fields' staging memory
   SceneState *h_state_ = nullptr, *state_dev_ = nullptr;
@@ -159,7 +191,7 @@ class Batch {
   int rigid_step();
   int max_iter_[3] = {1, 1, 1};
 
-  int alloc_arena(std::vector<std::pair<void**, size_t>>& req);
+  int alloc_arena(std::vector<std::pair<void**, size_t>>& req, bool& used);
   void release();
   int search_impl(int all, int begin);
   int complete_lists();
@@ -171,7 +203,7 @@ class Batch {
   int cg_start();
   int cg_solve(bool& done, bool& gave_up);
   int cg_loop();
-  int build_stress_set(const std::vector<int>& which);
+  int build_stress_set(const std::vector<int>& which, bool& any);
   int gather_state();
   void swap_sort_buffers();
   void derive_members();

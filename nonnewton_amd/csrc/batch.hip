@@ -229,41 +229,121 @@ long long scene_footprint(long long n, long long ns, long long cells) {
   return np * BYTES_PER_SLOT + nsp * BYTES_PER_MEMBER + (cells + 1) * 8 + 2048;
 }
 
-Batch::Batch(hipStream_t st) : stream(st) {}
+// Pinned memory through which the kernels read and write the fields of small
+// scenes themselves.  Microseconds of an upload / a download by field size,
+// this way and with a copy to or from device memory:
+//             5 KB      134 KB    329 KB    886 KB    1.9 MB     3.4 MB
+//   kernels   11 / 11   15 / 17   21 / 27   41 / 51   93 / 139   142 / 238
+//   copies    20 / 27   74 / 82   36 / 40   60 / 68   91 / 145   141 / 274
+constexpr size_t STAGE_BYTES = 1 << 20;
+static size_t state_bytes(int scenes) { return (sizeof(SceneState) + sizeof(unsigned long long)) * (size_t)scenes; }
+
+bool Spares::take(bool host, size_t bytes, void** p, size_t* got) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  std::lock_guard<std::mutex> lk(mu_);
+  auto& v = host ? host_ : dev_;
+  size_t best = v.size();
+  for (size_t k = 0; k < v.size(); k++)
+    if (v[k].device == dev && v[k].bytes >= bytes && v[k].bytes / 2 <= bytes + (1u << 20) &&
+        (best == v.size() || v[k].bytes < v[best].bytes))
+      best = k;
+  if (best == v.size()) return false;
+  *p = v[best].p;
+  *got = v[best].bytes;
+  if (!host) held_ -= *got;
+  v.erase(v.begin() + best);
+  return true;
+}
+
+void Spares::give(bool host, void* p, size_t bytes) {
+  std::vector<Block> out;
+  hipPointerAttribute_t at{};
+  int dev = 0;
+  if (hipPointerGetAttributes(&at, p) == hipSuccess) dev = at.device;
+  else (void)hipGetLastError();
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    auto& v = host ? host_ : dev_;
+    v.push_back({p, bytes, dev});
+    if (!host) held_ += bytes;
+    while (!v.empty() && (host ? v.size() > 64 : held_ > limit_)) {
+      if (!host) held_ -= v.front().bytes;
+      out.push_back(v.front());
+      v.erase(v.begin());
+    }
+  }
+  for (auto& b : out) (void)(host ? hipHostFree(b.p) : hipFree(b.p));
+}
+
+void Spares::clear() {
+  std::lock_guard<std::mutex> lk(mu_);
+  for (auto& b : dev_) (void)hipFree(b.p);
+  for (auto& b : host_) (void)hipHostFree(b.p);
+  dev_.clear();
+  host_.clear();
+  held_ = 0;
+}
+
+Batch::Batch(hipStream_t st, std::shared_ptr<Spares> spares) : stream(st), spares_(std::move(spares)) {}
 
 Batch::~Batch() {
   release();
-  if (h_state_) (void)hipHostFree(h_state_);
-  if (h_stage_) (void)hipHostFree(h_stage_);
+  free_host(h_state_, state_bytes(h_state_cap_));
+  free_host(h_stage_, STAGE_BYTES);
+}
+
+int Batch::alloc_host(void** p, size_t bytes) {
+  size_t got = 0;
+  if (spares_ && spares_->take(true, bytes, p, &got)) return NN_OK;
+  HIPCHK(hipHostMalloc(p, bytes, hipHostMallocDefault));
+  return NN_OK;
+}
+void Batch::free_host(void* p, size_t bytes) {  // after release(): no work is pending
+  if (!p) return;
+  if (spares_) spares_->give(true, p, bytes);
+  else (void)hipHostFree(p);
 }
 
 // The arrays of a layout are carved from one device allocation (256-byte
 // aligned sub-ranges): one hipMalloc and, when the batch is released or laid
-// out again, one hipFree, which synchronizes the device -- a pool admission
-// creates and later frees a staging batch, and with one allocation per array
-// it paid that synchronization some forty times.
-int Batch::alloc_arena(std::vector<std::pair<void**, size_t>>& req) {
+// out again, one hipFree, which synchronizes the device.  used: the memory held
+// other arrays before.
+int Batch::alloc_arena(std::vector<std::pair<void**, size_t>>& req, bool& used) {
   size_t total = 0;
   for (auto& r : req) total += (r.second + 255) & ~(size_t)255;
   void* q = nullptr;
-  hipError_t e = hipMalloc(&q, total);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    set_error(std::string("hipMalloc failed: ") + hipGetErrorString(e));
-    return NN_E_OOM;
+  size_t got = total;
+  used = spares_ && spares_->take(false, total, &q, &got);
+  if (!used) {
+    hipError_t e = hipMalloc(&q, total);
+    if (e == hipErrorOutOfMemory && spares_) {
+      (void)hipGetLastError();
+      spares_->clear();
+      e = hipMalloc(&q, total);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      set_error(std::string("hipMalloc failed: ") + hipGetErrorString(e));
+      return NN_E_OOM;
+    }
   }
   char* c = (char*)q;
   for (auto& r : req) {
     *r.first = c;
     c += (r.second + 255) & ~(size_t)255;
   }
-  allocs_.push_back({q, total});
-  bytes_ += (long long)total;
+  allocs_.push_back({q, got});
+  bytes_ += (long long)got;
   return NN_OK;
 }
 
 void Batch::release() {
-  for (auto& a : allocs_) (void)hipFree(a.p);
+  if (spares_ && !allocs_.empty()) (void)hipStreamSynchronize(stream);
+  for (auto& a : allocs_) {
+    if (spares_) spares_->give(false, a.p, a.bytes);
+    else (void)hipFree(a.p);
+  }
   allocs_.clear();
   bytes_ = 0;
 }
@@ -499,24 +579,33 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
     using T = std::remove_reference_t<decltype(*p)>;
     req.push_back({(void**)&p, (count ? count : 1) * sizeof(T)});
   };
-  SceneDev* scenes_dev = nullptr;
-  A(scenes_dev, Sc);
+  // arrays that start at zero, arrays that start at -1, and the others
   A(nd.state, Sc);
-  int* ws = nullptr;
-  A(ws, nd.W);
-  int* sws = nullptr;
-  A(sws, nd.SW);
   A(nd.pos, Pc);
   A(nd.pos_alt, Pc);
   A(nd.vel, Pc);
   A(nd.vel_alt, Pc);
-  A(nd.info, Pc);
-  A(nd.info_alt, Pc);
   A(nd.acc, Pc);
   A(nd.rho, Pc);
   A(nd.sa, Pc);
-  A(nd.nbr, (size_t)Pc * MAX_NB);
+  A(nd.gam, Pc);
+  A(nd.eta, Pc);
+  A(nd.x0, Pc);
+  A(nd.vdiff, Pc);
+  A(nd.vdiff_alt, Pc);  // swapped with vdiff also where the sort does not copy it
   A(nd.nnbr, Pc);
+  A(nd.rest_cnt, NSc);
+  A(nd.info, Pc);
+  A(nd.info_alt, Pc);
+  A(nd.s_of, Pc);
+  A(nd.s_pid, NSc);
+  SceneDev* scenes_dev = nullptr;
+  A(scenes_dev, Sc);
+  int* ws = nullptr;
+  A(ws, nd.W);
+  int* sws = nullptr;
+  A(sws, nd.SW);
+  A(nd.nbr, (size_t)Pc * MAX_NB);
   A(nd.key, Pc);
   A(nd.rank, Pc);
   A(nd.inv, Pc);
@@ -536,19 +625,11 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   A(nd.wp, Pc);
   A(nd.ws, Pc);
   A(nd.xu, Pc);
-  A(nd.vdiff_alt, Pc);
   A(nd.wd0, Pc);
   A(nd.wd1, Pc);
   A(nd.spair, (size_t)Pc * MAX_NB);
-  A(nd.vdiff, Pc);
   A(nd.mu, Pc);
-  A(nd.gam, Pc);
-  A(nd.eta, Pc);
-  A(nd.x0, Pc);
-  A(nd.s_of, Pc);
-  A(nd.s_pid, NSc);
   A(nd.rest, (size_t)NSc * MAX_REST);
-  A(nd.rest_cnt, NSc);
   A(nd.rs, 4 * (size_t)NSc);
   int* rpid = nullptr;
   A(rpid, NRc);
@@ -556,7 +637,8 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   A(rwb, NRc / 64);
   A(nd.rpartials, 9 * (size_t)(NRc / 64));
   A(nd.bodies, NBc);
-  const int rc = alloc_arena(req);
+  bool used = false;
+  const int rc = alloc_arena(req, used);
   if (rc != NN_OK) {
     release();
     allocs_.swap(old_allocs);
@@ -593,32 +675,18 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
     if (h_state_) HIPCHK(hipHostFree(h_state_));
     h_state_ = nullptr;
     const size_t cap = (size_t)std::max(Sc, 1);
-    HIPCHK(hipHostMalloc((void**)&h_state_, (sizeof(SceneState) + sizeof(*h_report_)) * cap, hipHostMallocDefault));
+    CHK(alloc_host((void**)&h_state_, state_bytes((int)cap)));
     h_report_ = reinterpret_cast<unsigned long long*>(h_state_ + cap);
     std::fill(h_report_, h_report_ + cap, 0ull);
     h_state_cap_ = (int)cap;
     HIPCHK(hipHostGetDevicePointer((void**)&state_dev_, h_state_, 0));
     report_dev_ = reinterpret_cast<unsigned long long*>(state_dev_ + cap);
   }
+  // memory that was in use before starts at zero throughout, as new memory does
+  const long zeros = (long)((used ? (char*)allocs_.back().p + allocs_.back().bytes : (char*)nd.info) - (char*)nd.state);
+  launch_fill_f4(reinterpret_cast<float4*>(nd.state), zeros / 16, make_float4(0.f, 0.f, 0.f, 0.f), stream);
+  launch_fill_i32(nd.info, (long)((char*)scenes_dev - (char*)nd.info) / 4, -1, stream);
   CHK(upload_tables(nd));
-  HIPCHK(hipMemsetAsync(nd.state, 0, sizeof(SceneState) * std::max<size_t>(Sc, 1), stream));
-  launch_fill_i32(nd.info, Pc, -1, stream);
-  launch_fill_i32(nd.info_alt, Pc, -1, stream);
-  launch_fill_i32(nd.s_of, Pc, -1, stream);
-  launch_fill_i32(nd.s_pid, NSc, -1, stream);
-  launch_fill_i32(nd.rest_cnt, NSc, 0, stream);
-  launch_fill_i32(nd.nnbr, Pc, 0, stream);
-  launch_fill_f4(nd.pos, Pc, make_float4(0.f, 0.f, 0.f, 0.f), stream);
-  launch_fill_f4(nd.pos_alt, Pc, make_float4(0.f, 0.f, 0.f, 0.f), stream);
-  launch_fill_f4(nd.vel, Pc, make_float4(0.f, 0.f, 0.f, 0.f), stream);
-  launch_fill_f4(nd.vel_alt, Pc, make_float4(0.f, 0.f, 0.f, 0.f), stream);
-  launch_fill_f4(nd.x0, Pc, make_float4(0.f, 0.f, 0.f, 0.f), stream);
-  launch_fill_f4(nd.vdiff, Pc, make_float4(0.f, 0.f, 0.f, 0.f), stream);
-  HIPCHK(hipMemsetAsync(nd.rho, 0, sizeof(float) * std::max(Pc, 1), stream));
-  HIPCHK(hipMemsetAsync(nd.sa, 0, sizeof(float2) * std::max(Pc, 1), stream));
-  HIPCHK(hipMemsetAsync(nd.gam, 0, sizeof(float) * std::max(Pc, 1), stream));
-  HIPCHK(hipMemsetAsync(nd.eta, 0, sizeof(float) * std::max(Pc, 1), stream));
-  HIPCHK(hipMemsetAsync(nd.acc, 0, sizeof(float4) * std::max(Pc, 1), stream));
   // copy persistent state of relocated scenes
   for (size_t k = 0; k < scenes.size(); k++)
     if (src[k].b) CHK(copy_scene_state(nd, *scenes[k], src[k].b, src[k].pb, src[k].sb, src[k].ns));
@@ -626,7 +694,7 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   // the old arrays are freed by the caller's choice: now, or later (off the
   // thread that steps the batch; hipFree waits for the device)
   if (defer_free_) {
-    for (auto& al : old_allocs) deferred_.push_back(al.p);
+    for (auto& al : old_allocs) deferred_.push_back(al);
   } else {
     for (auto& al : old_allocs) (void)hipFree(al.p);
   }
@@ -702,7 +770,7 @@ int Batch::append_in_place(const std::vector<std::shared_ptr<SceneHost>>& member
   return NN_OK;
 }
 
-void Batch::take_deferred(std::vector<void*>& out) {
+void Batch::take_deferred(std::vector<Alloc>& out) {
   out.insert(out.end(), deferred_.begin(), deferred_.end());
   deferred_.clear();
 }
@@ -725,21 +793,24 @@ int Batch::refresh_scene_table() {
 int Batch::upload(int k, const float* x, const float* v, const int* kind) {
   SceneHost& s = *scenes[k];
   const int n = s.n, pb = s.p_begin;
-  const float V0 = s.dev.vol0;  // :607, :741
-  std::vector<float4> hp(n), hv(n);
-  std::vector<int> hi(n), hinv(n);
-  for (int i = 0; i < n; i++) {
-    const int kd = kind[i] >= KIND_RIGID ? KIND_RIGID : kind[i];
-    hp[i] = make_float4(x[3 * i], x[3 * i + 1], x[3 * i + 2], kd == KIND_FLUID ? V0 : -V0);
-    hv[i] = v ? make_float4(v[3 * i], v[3 * i + 1], v[3 * i + 2], 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
-    hi[i] = (kd << 28) | i;
-    hinv[i] = i;
+  // expanded on the device, from staging memory or (larger scenes) from a copy
+  // in the pair scalars, which only a step uses
+  const size_t words = (size_t)(v ? 7 : 4) * n;
+  float* raw = d.spair;
+  if (4 * words <= STAGE_BYTES) {
+    CHK(stage());
+    std::memcpy(h_stage_, x, sizeof(float) * 3 * n);
+    std::memcpy(h_stage_ + 3 * (size_t)n, kind, sizeof(int) * n);
+    if (v) std::memcpy(h_stage_ + 4 * (size_t)n, v, sizeof(float) * 3 * n);
+    raw = stage_dev_;
+  } else {
+    HIPCHK(hipMemcpyAsync(raw, x, sizeof(float) * 3 * n, hipMemcpyHostToDevice, stream));
+    HIPCHK(hipMemcpyAsync(raw + 3 * (size_t)n, kind, sizeof(int) * n, hipMemcpyHostToDevice, stream));
+    if (v) HIPCHK(hipMemcpyAsync(raw + 4 * (size_t)n, v, sizeof(float) * 3 * n, hipMemcpyHostToDevice, stream));
   }
-  HIPCHK(hipMemcpyAsync(d.pos + pb, hp.data(), sizeof(float4) * n, hipMemcpyHostToDevice, stream));
-  HIPCHK(hipMemcpyAsync(d.vel + pb, hv.data(), sizeof(float4) * n, hipMemcpyHostToDevice, stream));
-  HIPCHK(hipMemcpyAsync(d.info + pb, hi.data(), sizeof(int) * n, hipMemcpyHostToDevice, stream));
-  HIPCHK(hipMemcpyAsync(d.inv + pb, hinv.data(), sizeof(int) * n, hipMemcpyHostToDevice, stream));
-  launch_fill_f4(d.vdiff + pb, n, make_float4(0.f, 0.f, 0.f, 0.f), stream);
+  launch_expand(dref(), pb, n, s.dev.vol0, raw, reinterpret_cast<const int*>(raw + 3 * (size_t)n),
+                v ? raw + 4 * (size_t)n : nullptr, stream);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(stream));
   s.initialized = false;
   s.stepped = false;
@@ -896,8 +967,8 @@ int Batch::gather_state() {
 
 // stress set: elastic particles and their rest neighbors (first search), with
 // rest lists capped at 50 (Elasticity.initValues_kernel, :1220-1236)
-int Batch::build_stress_set(const std::vector<int>& which) {
-  bool any = false;
+int Batch::build_stress_set(const std::vector<int>& which, bool& any) {
+  any = false;
   for (int k : which) {
     SceneHost& s = *scenes[k];
     s.s_pid.clear();
@@ -979,10 +1050,11 @@ int Batch::init_scenes(const std::vector<int>& which) {
     if (stt & ST_CELL_OVERFLOW) { set_error("more than 50 particles in a cell"); return NN_E_CELL_OVERFLOW; }
     if (stt & ST_NEIGHBOR_OVERFLOW) { set_error("more than 60 neighbors"); return NN_E_NEIGHBOR_OVERFLOW; }
   }
-  CHK(build_stress_set(which));
+  bool relayout = false;
+  CHK(build_stress_set(which, relayout));
   // the stress-set relayout does not carry neighbor lists (they hold absolute
   // slots); search again on the unchanged positions before the volume sweeps
-  CHK(search_impl(1, BEGIN_CELLS));
+  if (relayout) CHK(search_impl(1, BEGIN_CELLS));
   launch_bvol(dref(), block, lanes(K_BVOL), 0, stream);
   launch_bvol(dref(), block, lanes(K_BVOL), 1, stream);
   HIPCHK(hipGetLastError());
@@ -1246,16 +1318,9 @@ static int field_width(int field) {
   }
 }
 
-// Pinned memory through which the kernels read and write the fields of small
-// scenes themselves.  Microseconds of an upload / a download by field size,
-// this way and with a copy to or from device memory:
-//             5 KB      134 KB    329 KB    886 KB    1.9 MB     3.4 MB
-//   kernels   11 / 11   15 / 17   21 / 27   41 / 51   93 / 139   142 / 238
-//   copies    20 / 27   74 / 82   36 / 40   60 / 68   91 / 145   141 / 274
-constexpr size_t STAGE_BYTES = 1 << 20;
 int Batch::stage() {
   if (h_stage_) return NN_OK;
-  HIPCHK(hipHostMalloc((void**)&h_stage_, STAGE_BYTES, hipHostMallocDefault));
+  CHK(alloc_host((void**)&h_stage_, STAGE_BYTES));
   HIPCHK(hipHostGetDevicePointer((void**)&stage_dev_, h_stage_, 0));
   return NN_OK;
 }

@@ -397,7 +397,8 @@ struct nn_pool {
   // device memory no longer used by the batch, freed by the next admission
   // (hipFree waits for the device, so not on the thread that ticks)
   std::vector<std::unique_ptr<Batch>> graveyard;
-  std::vector<void*> dead_arrays;
+  std::vector<Batch::Alloc> dead_arrays;
+  std::shared_ptr<nn::Spares> spares;
   // a tick in flight (nn_pool_tick_async): its thread, and what nn_pool_sync returns
   std::thread async;
   bool async_on = false;
@@ -406,17 +407,17 @@ struct nn_pool {
   std::vector<nn_step_stats> async_stats;
 };
 
-// frees what the ticks left behind; called outside the pool lock
+// gives up what the ticks left behind; called outside the pool lock
 static void pool_free_dead(nn_pool* p) {
   std::vector<std::unique_ptr<Batch>> dead;
-  std::vector<void*> arrays;
+  std::vector<Batch::Alloc> arrays;
   {
     std::lock_guard<std::mutex> lk(p->mu);
     dead.swap(p->graveyard);
     arrays.swap(p->dead_arrays);
   }
   dead.clear();
-  for (void* a : arrays) (void)hipFree(a);
+  for (auto& a : arrays) p->spares->give(false, a.p, a.bytes);  // the layout that replaced them waited for its stream
 }
 
 extern "C" {
@@ -464,7 +465,8 @@ int32_t nn_pool_create_ex(int64_t budget_bytes, int32_t flags, nn_pool** out) {
     return nn::hip_fail(e, "hipStreamCreate");
   }
   p->budget = budget_bytes;
-  p->main.reset(new Batch(p->stream));
+  p->spares = std::make_shared<nn::Spares>((size_t)budget_bytes / 8);
+  p->main.reset(new Batch(p->stream, p->spares));
   p->main->defer_free_ = true;
   p->slots.resize(POOL_CAPACITY);
   *out = p;
@@ -558,7 +560,7 @@ int32_t nn_pool_admit(nn_pool* p, const nn_params* params, const float* x, const
     const int rc2 = staging_stream(&sst);
     if (rc2 < 0) return fail(rc2);
   }
-  std::unique_ptr<Batch> stg(new Batch(sst));
+  std::unique_ptr<Batch> stg(new Batch(sst, p->spares));
   stg->block = p->block;
   std::copy(p->kblock, p->kblock + nn::K_COUNT, stg->kblock);
   std::copy(p->kdepth, p->kdepth + nn::K_COUNT, stg->kdepth);

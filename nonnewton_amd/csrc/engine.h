@@ -253,6 +253,8 @@ void launch_fill_i32(int* p, long n, int v, hipStream_t st);
 void launch_fill_f4(float4* p, long n, float4 v, hipStream_t st);
 // x, y, z of a scene's particles between cell order (slots) and original order
 void launch_gather3(const float4* slots, const int* inv, int n, float* ordered, hipStream_t st);
+// a scene's slots [pb, pb + n) from x, kind and v (or none) in original order
+void launch_expand(const DevRef& d, int pb, int n, float V0, const float* x, const int* kind, const float* v, hipStream_t st);
 void launch_scatter3(const float* ordered, const int* inv, int n, float4* slots, hipStream_t st);
 void launch_scan(const DevRef& d, int n, hipStream_t st);  // cell_start = exclusive scan(cell_count)
 // exclusive scan of in[0..n) into out; tmp holds ceil(n / 2048) ints

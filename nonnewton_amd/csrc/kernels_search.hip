@@ -59,6 +59,22 @@ __global__ void k_scatter3(const float* ordered, const int* inv, int n, float4* 
   p->y = ordered[3 * (long)id + 1];
   p->z = ordered[3 * (long)id + 2];
 }
+__global__ void k_expand(Dev d, int pb, int n, float V0, const float* x, const int* kind, const float* v) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int kd = min(kind[i], (int)KIND_RIGID);  // a rigid particle's kind holds its body
+  const float* xi = x + 3 * (long)i;
+  d.pos[pb + i] = make_float4(xi[0], xi[1], xi[2], kd == KIND_FLUID ? V0 : -V0);  // :607, :741
+  float4 vi = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (v) vi = make_float4(v[3 * (long)i], v[3 * (long)i + 1], v[3 * (long)i + 2], 0.f);
+  d.vel[pb + i] = vi;
+  d.vdiff[pb + i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  d.info[pb + i] = (kd << 28) | i;
+  d.inv[pb + i] = i;
+}
+void launch_expand(const DevRef& d, int pb, int n, float V0, const float* x, const int* kind, const float* v, hipStream_t st) {
+  if (n > 0) NN_LAUNCH(k_expand, dim3((n + 255) / 256), dim3(256), 0, st, d.h, pb, n, V0, x, kind, v);
+}
 void launch_gather3(const float4* slots, const int* inv, int n, float* ordered, hipStream_t st) {
   if (n > 0) NN_LAUNCH(k_gather3, dim3((n + 255) / 256), dim3(256), 0, st, slots, inv, n, ordered);
 }
