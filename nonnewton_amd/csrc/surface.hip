@@ -1089,7 +1089,9 @@ __global__ __launch_bounds__(ST_THREADS) void k_stats_final(K k, int which, cons
   }
 }
 
-// smooth_sdf_impl (:1459-1484), radius 1
+// smooth_sdf_impl (:1459-1484), radius 1.  Bound by issue: 27 exponentials and as
+// many pairs of quotients a vertex; 2.5 million vertices take 87 us, 95 with
+// full-range divisions.
 __global__ void k_smooth(K k, const float* in, float* out) {
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= k.nvert) return;
@@ -1102,6 +1104,12 @@ __global__ void k_smooth(K k, const float* in, float* out) {
   const int i = gx + k.glo[0], j = gy + k.glo[1], l = gz + k.glo[2];
   const float vc = in[q];
   const float den = 2.0f * sd * sd, tt = k.c2pi * sd * sd, scale = tt * sqrtf(tt);
+  // the shorter exact quotients where the denominators let them be used.  A
+  // numerator so small that they may round differently gives an exponent whose
+  // e^x is 1 in either form; one too large, or a weight too small, takes the
+  // full-range division.
+  const bool mid = den > 0x1p-40f && den < 0x1p40f && scale > 0x1p-40f && scale < 0x1p40f;
+  const float yd = recip_mid(den), ys = recip_mid(scale);
   float avg = 0.0f, weight = 0.0f;
 #pragma unroll
   for (int dx = -1; dx <= 1; dx++) {  // nine loads in flight
@@ -1116,7 +1124,14 @@ __global__ void k_smooth(K k, const float* in, float* out) {
 #pragma unroll
     for (int e = 0; e < 9; e++) {
       const float d = fabsf(vc - vn[e]);
-      const float gw = on[e] ? sr_expf(-d * d / den) / scale : 0.0f;
+      const float dd = -d * d;
+      float ex = sr_expf(div_mid(dd, den, yd));
+      float gw = div_mid(ex, scale, ys);
+      if (__builtin_expect(!mid || !(dd > -0x1p60f) || (ex < 0x1p-60f && ex > 0.0f), 0)) {
+        ex = sr_expf(dd / den);
+        gw = ex / scale;
+      }
+      gw = on[e] ? gw : 0.0f;
       avg += gw * vn[e];
       weight += gw;
     }
