@@ -30,6 +30,7 @@
 // expression is FP32 in the reference's operation order (-ffp-contract=off).
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cmath>
 #include <cstdint>
 #include <string>
@@ -173,6 +174,12 @@ __global__ void k_fill_i32(int* p, int v, long n) {
 __global__ void k_fill_u8(unsigned char* p, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
+}
+
+__global__ void k_start(K k) {
+  const int t = threadIdx.x;
+  if (t < 6) k.bounds[t] = t < 3 ? INT32_MAX : INT32_MIN;
+  if (t == 6) *k.err = 0;
 }
 
 // voxel range of the particles: a workgroup min/max in LDS, then one atomic
@@ -691,6 +698,7 @@ __device__ __forceinline__ float aniso_of(float c48d, float c16d, float q) {
   return 0.0f < q && q <= 1.0f ? r : 0.0f;
 }
 // the same for q > 0: past 1 (or not a number) 1 - q is clamped to 0, and the value is +-0
+// (the inner form under a wavefront's branch instead: 3.30 -> 3.47 ms)
 __device__ __forceinline__ float aniso_mid(float c48d, float c16d, float q) {
   const float in = c48d * (q * q * q - q * q) + 1.0f;
   const float u = __builtin_amdgcn_fmed3f(1.0f - q, 0.0f, 1.0f);
@@ -1549,6 +1557,33 @@ struct DBuf {
   }
 };
 
+// What the host reads between the launches, written by k_report into pinned
+// memory: the ticket last.
+struct Report {
+  unsigned long long ticket;
+  double stats[4];
+  int err, count, bounds[6];
+  long long active;
+};
+__global__ __launch_bounds__(256) void k_report(K k, const int* count, int active, Report* host, unsigned long long ticket) {
+  __shared__ int red[4];
+  const int t = threadIdx.x;
+  int na = 0;
+  if (active)
+    for (long b = t; b < k.nblock; b += 256) na += k.active[b];
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) na += __shfl_xor(na, off, 64);
+  if ((t & 63) == 0) red[t >> 6] = na;
+  __syncthreads();
+  if (t != 0) return;
+  host->err = *k.err;
+  host->count = count ? *count : 0;
+  host->active = (long long)red[0] + red[1] + red[2] + red[3];
+  for (int a = 0; a < 6; a++) host->bounds[a] = k.bounds[a];
+  for (int a = 0; a < 4; a++) host->stats[a] = k.stats[a];
+  __hip_atomic_store(&host->ticket, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 struct Surface {
   nn_surface_params prm{};
   K k{};
@@ -1563,6 +1598,8 @@ struct Surface {
   double sd = 0.0;
   bool have = false;
   int64_t budget = 0;  // device bytes a run may use (0 = no limit)
+  Report *report = nullptr, *report_dev = nullptr;  // pinned, and its device address
+  unsigned long long ticket = 0;
 
   ~Surface() {
     for (auto* b : {&pos, &vel, &G, &xbar, &field0, &field, &tmp, &verts, &normals, &vfield, &mvel}) b->release();
@@ -1574,6 +1611,7 @@ struct Surface {
     stats.release();
     part.release();
     pcount.release();
+    if (report) (void)hipHostFree(report);
     if (st) (void)hipStreamDestroy(st);
   }
 };
@@ -1600,10 +1638,22 @@ static int fail(hipError_t e, const char* what) { return hip_fail(e, what); }
     if (e__ != hipSuccess) return fail(e__, what); \
   } while (0)
 
-static int device_error(Surface& S) {
-  int err = 0;
-  SR_HIP(hipMemcpyAsync(&err, S.err.p, sizeof(int), hipMemcpyDeviceToHost, S.st), "nn_surface_run: error flag");
-  SR_HIP(hipStreamSynchronize(S.st), "nn_surface_run");
+// Launches k_report and waits for it (as Batch::await: polled, a long wait left to
+// the stream's), then returns the error the launches so far have flagged.
+static int report(Surface& S, const int* count = nullptr, bool active = false) {
+  hipLaunchKernelGGL(k_report, dim3(1), dim3(256), 0, S.st, S.k, count, active ? 1 : 0, S.report_dev, ++S.ticket);
+  SR_HIP(hipGetLastError(), "nn_surface_run: launch");
+  const auto start = std::chrono::steady_clock::now();
+  for (int polls = 1; __atomic_load_n(&S.report->ticket, __ATOMIC_ACQUIRE) != S.ticket; polls++) {
+    if (polls % 64 == 0 && std::chrono::steady_clock::now() - start > std::chrono::microseconds(300)) {
+      SR_HIP(hipStreamSynchronize(S.st), "nn_surface_run");
+      if (__atomic_load_n(&S.report->ticket, __ATOMIC_ACQUIRE) == S.ticket) break;
+      set_error("nn_surface_run: a launch did not report its end");
+      return NN_E_HIP;
+    }
+    __builtin_ia32_pause();
+  }
+  const int err = S.report->err;
   if (err & ERR_OUT_OF_GRID) {
     set_error("nn_surface_run: a particle lies below the bounding box's first voxel, or its position is not finite");
     return NN_E_OUT_OF_GRID;
@@ -1631,14 +1681,16 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   k.err = S.err.p;
   k.bounds = S.bounds.p;
   k.stats = S.stats.p;
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, S.st, k.err, 0, 1L);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, S.st, k.bounds, INT32_MAX, 3L);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, S.st, k.bounds + 3, INT32_MIN, 3L);
+  if (!S.report) {
+    SR_HIP(hipHostMalloc((void**)&S.report, sizeof(Report), hipHostMallocDefault), "nn_surface_run: alloc");
+    S.report->ticket = 0;
+    SR_HIP(hipHostGetDevicePointer((void**)&S.report_dev, S.report, 0), "nn_surface_run");
+  }
+  hipLaunchKernelGGL(k_start, dim3(1), dim3(64), 0, S.st, k);
   hipLaunchKernelGGL(k_bounds, dim3(grid1(n, BOUNDS_THREADS)), dim3(BOUNDS_THREADS), 0, S.st, k);
-  int hb[6];
-  SR_HIP(hipMemcpyAsync(hb, k.bounds, sizeof(hb), hipMemcpyDeviceToHost, S.st), "nn_surface_run: bounds");
-  int rc = device_error(S);
+  int rc = report(S);
   if (rc) return rc;
+  const int* hb = S.report->bounds;
   // voxel range and the vertex grid (blocks that the field passes can write)
   long nvox = 1;
   for (int a = 0; a < 3; a++) {
@@ -1715,7 +1767,7 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   int* bucket = reinterpret_cast<int*>(k.xbar);  // written by k_aniso, after this
   hipLaunchKernelGGL(k_vplace, dim3(grid1(n, 256)), dim3(256), 0, S.st, k, bucket);
   hipLaunchKernelGGL(k_vsort, dim3(grid1(n, 256)), dim3(256), 0, S.st, k, bucket);
-  if ((rc = device_error(S))) return rc;
+  if ((rc = report(S))) return rc;  // before sweeps over voxels that may hold any number
   // anisotropic kernel and field
   if (k.aniso) hipLaunchKernelGGL(k_aniso, dim3(grid1(n, AN_GROUPS)), dim3(16 * AN_GROUPS), 0, S.st, k);
   hipLaunchKernelGGL(k_fill_u8, dim3(grid1(nblock, 256)), dim3(256), 0, S.st, k.active, nblock);
@@ -1727,7 +1779,6 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
     hipLaunchKernelGGL(k_check_velocities, dim3(grid1(3 * n, 256)), dim3(256), 0, S.st, k);
     hipLaunchKernelGGL(k_field<FIELD_VELOCITY>, tiles, ft, 0, S.st, k);
   }
-  if ((rc = device_error(S))) return rc;
   // smoothing
   hipLaunchKernelGGL(k_stats, dim3((unsigned)nblock), dim3(ST_THREADS), 0, S.st, k, 0, S.part.p, S.pcount.p);
   hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(ST_THREADS), 0, S.st, k, 0, S.part.p, S.pcount.p);
@@ -1740,9 +1791,8 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   // contour
   hipLaunchKernelGGL(k_cube_flag, dim3(grid1(nvert, 256)), dim3(256), 0, S.st, k);
   SR_HIP(scan(S, k.flag, k.cube_id, nvert, 1), "nn_surface_run: scan");
-  int nv = 0;
-  SR_HIP(hipMemcpyAsync(&nv, k.cube_id + nvert, sizeof(int), hipMemcpyDeviceToHost, S.st), "nn_surface_run: count");
-  SR_HIP(hipStreamSynchronize(S.st), "nn_surface_run");
+  if ((rc = report(S, k.cube_id + nvert))) return rc;
+  const int nv = S.report->count;
   SR_HIP(S.verts.ensure(3 * (size_t)nv), "nn_surface_run: alloc");
   SR_HIP(S.cubes.ensure(nv), "nn_surface_run: alloc");
   SR_HIP(S.tcount.ensure(nv), "nn_surface_run: alloc");
@@ -1754,9 +1804,10 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   hipLaunchKernelGGL(k_cube_id, dim3(grid1(nvert, 256)), dim3(256), 0, S.st, k);
   if (nv > 0) hipLaunchKernelGGL(k_dc_point, dim3(grid1(nv, DC_CUBES)), dim3(DC_THREADS), 0, S.st, k, nv);
   SR_HIP(scan(S, k.tcount, k.tstart, nv), "nn_surface_run: scan");
-  int nt = 0;
-  SR_HIP(hipMemcpyAsync(&nt, k.tstart + nv, sizeof(int), hipMemcpyDeviceToHost, S.st), "nn_surface_run: count");
-  SR_HIP(hipStreamSynchronize(S.st), "nn_surface_run");
+  if ((rc = report(S, k.tstart + nv, true))) return rc;
+  const int nt = S.report->count;
+  S.nactive = (long)S.report->active;  // the written blocks and the deviation, for the caller's statistics
+  S.sd = S.report->stats[3];
   SR_HIP(S.faces.ensure(3 * (size_t)nt), "nn_surface_run: alloc");
   k.faces = S.faces.p;
   if (nv > 0) hipLaunchKernelGGL(k_faces, dim3(grid1(nv, 128)), dim3(128), 0, S.st, k, nv);
@@ -1772,19 +1823,10 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
     }
     hipLaunchKernelGGL(k_vertex_attrs, dim3(grid1(nv, 128)), dim3(128), 0, S.st, k, (long)nv, want_n, want_v);
   }
-  double st4[4];
-  SR_HIP(hipMemcpyAsync(st4, k.stats, sizeof(st4), hipMemcpyDeviceToHost, S.st), "nn_surface_run: stats");
-  SR_HIP(hipStreamSynchronize(S.st), "nn_surface_run");
   SR_HIP(hipGetLastError(), "nn_surface_run: launch");
-  // active-block count for the caller's statistics
-  std::vector<unsigned char> act(nblock);
-  SR_HIP(hipMemcpy(act.data(), k.active, nblock, hipMemcpyDeviceToHost), "nn_surface_run: active");
-  long na = 0;
-  for (unsigned char c : act) na += c;
-  S.nactive = na;
+  if ((rc = report(S))) return rc;
   S.nverts = nv;
   S.ntris = nt;
-  S.sd = st4[3];
   S.have = true;
   return NN_OK;
 }
