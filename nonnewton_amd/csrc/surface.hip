@@ -33,6 +33,8 @@
 #include <chrono>
 #include <cmath>
 #include <cstdint>
+#include <cstring>
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -1600,6 +1602,8 @@ struct Surface {
   int64_t budget = 0;  // device bytes a run may use (0 = no limit)
   Report *report = nullptr, *report_dev = nullptr;  // pinned, and its device address
   unsigned long long ticket = 0;
+  int *stage = nullptr, *stage_dev = nullptr;  // pinned, STAGE_BYTES
+  bool stage_read = false;                     // a kernel may still read it
 
   ~Surface() {
     for (auto* b : {&pos, &vel, &G, &xbar, &field0, &field, &tmp, &verts, &normals, &vfield, &mvel}) b->release();
@@ -1612,6 +1616,7 @@ struct Surface {
     part.release();
     pcount.release();
     if (report) (void)hipHostFree(report);
+    if (stage) (void)hipHostFree(stage);
     if (st) (void)hipStreamDestroy(st);
   }
 };
@@ -1630,6 +1635,28 @@ static hipError_t scan(Surface& S, const int* in, int* out, long L, int nz = 0) 
   return hipGetLastError();
 }
 
+// Caller's arrays of up to STAGE_BYTES together cross through pinned memory that
+// kernels read and write: a copy of 60 to 130 KB to or from pageable memory takes
+// 40 to 80 us, this 11 to 17 (fields of that size).
+constexpr size_t STAGE_BYTES = 1 << 20;
+struct Piece {
+  void* p;     // device side
+  void* host;  // caller's side
+  size_t bytes;
+};
+struct Pieces {
+  int* dev[3];
+  long end[3];  // words of the pieces up to this one
+};
+__global__ void k_stage(Pieces c, int* stage, int in) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= c.end[2]) return;
+  const int a = i < c.end[0] ? 0 : i < c.end[1] ? 1 : 2;
+  int* d = c.dev[a] + (i - (a ? c.end[a - 1] : 0));
+  if (in) *d = stage[i];
+  else stage[i] = *d;
+}
+
 static int fail(hipError_t e, const char* what) { return hip_fail(e, what); }
 
 #define SR_HIP(expr, what)                      \
@@ -1639,8 +1666,13 @@ static int fail(hipError_t e, const char* what) { return hip_fail(e, what); }
   } while (0)
 
 // Launches k_report and waits for it (as Batch::await: polled, a long wait left to
-// the stream's), then returns the error the launches so far have flagged.
-static int report(Surface& S, const int* count = nullptr, bool active = false) {
+// the stream's); report() then returns the error the launches so far have flagged.
+static int wait_report(Surface& S, const int* count, bool active) {
+  if (!S.report) {
+    SR_HIP(hipHostMalloc((void**)&S.report, sizeof(Report), hipHostMallocDefault), "nn_surface_run: alloc");
+    S.report->ticket = 0;
+    SR_HIP(hipHostGetDevicePointer((void**)&S.report_dev, S.report, 0), "nn_surface_run");
+  }
   hipLaunchKernelGGL(k_report, dim3(1), dim3(256), 0, S.st, S.k, count, active ? 1 : 0, S.report_dev, ++S.ticket);
   SR_HIP(hipGetLastError(), "nn_surface_run: launch");
   const auto start = std::chrono::steady_clock::now();
@@ -1653,6 +1685,13 @@ static int report(Surface& S, const int* count = nullptr, bool active = false) {
     }
     __builtin_ia32_pause();
   }
+  S.stage_read = false;
+  return NN_OK;
+}
+
+static int report(Surface& S, const int* count = nullptr, bool active = false) {
+  const int rc = wait_report(S, count, active);
+  if (rc) return rc;
   const int err = S.report->err;
   if (err & ERR_OUT_OF_GRID) {
     set_error("nn_surface_run: a particle lies below the bounding box's first voxel, or its position is not finite");
@@ -1669,6 +1708,55 @@ static int report(Surface& S, const int* count = nullptr, bool active = false) {
   return NN_OK;
 }
 
+// Copies pieces in (before a run) or out (after one); in: the run waits for it.
+static int transfer(Surface& S, bool in, std::initializer_list<Piece> pieces, const char* what) {
+  size_t total = 0;
+  bool host = true;  // memory that the CPU can use
+  for (const Piece& q : pieces) {
+    total += q.bytes;
+    hipPointerAttribute_t at{};
+    if (q.bytes == 0) continue;
+    if (hipPointerGetAttributes(&at, q.host) != hipSuccess) (void)hipGetLastError();
+    else host = host && at.type != hipMemoryTypeDevice;
+  }
+  if (total == 0) return NN_OK;
+  if (!host || total > STAGE_BYTES) {
+    for (const Piece& q : pieces) {
+      if (q.bytes == 0) continue;
+      if (in) SR_HIP(hipMemcpyAsync(q.p, q.host, q.bytes, hipMemcpyHostToDevice, S.st), what);
+      else SR_HIP(hipMemcpy(q.host, q.p, q.bytes, hipMemcpyDeviceToHost), what);
+    }
+    return NN_OK;
+  }
+  if (!S.stage) {
+    SR_HIP(hipHostMalloc((void**)&S.stage, STAGE_BYTES, hipHostMallocDefault), what);
+    SR_HIP(hipHostGetDevicePointer((void**)&S.stage_dev, S.stage, 0), what);
+  }
+  if (S.stage_read) SR_HIP(hipStreamSynchronize(S.st), what);  // by a run that ended before its first report
+  S.stage_read = in;
+  Pieces c{};
+  long words = 0;
+  int a = 0;
+  for (const Piece& q : pieces) {
+    if (in && q.bytes) std::memcpy(S.stage + words, q.host, q.bytes);
+    words += (long)(q.bytes / 4);
+    c.dev[a] = static_cast<int*>(q.p);
+    c.end[a++] = words;
+  }
+  for (; a < 3; a++) c.end[a] = words;
+  hipLaunchKernelGGL(k_stage, dim3(grid1(words, 256)), dim3(256), 0, S.st, c, S.stage_dev, in ? 1 : 0);
+  SR_HIP(hipGetLastError(), what);
+  if (in) return NN_OK;
+  const int rc = wait_report(S, nullptr, false);
+  if (rc) return rc;
+  words = 0;
+  for (const Piece& q : pieces) {
+    if (q.bytes) std::memcpy(q.host, S.stage + words, q.bytes);
+    words += (long)(q.bytes / 4);
+  }
+  return NN_OK;
+}
+
 static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   K& k = S.k;
   S.have = false;
@@ -1681,11 +1769,6 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   k.err = S.err.p;
   k.bounds = S.bounds.p;
   k.stats = S.stats.p;
-  if (!S.report) {
-    SR_HIP(hipHostMalloc((void**)&S.report, sizeof(Report), hipHostMallocDefault), "nn_surface_run: alloc");
-    S.report->ticket = 0;
-    SR_HIP(hipHostGetDevicePointer((void**)&S.report_dev, S.report, 0), "nn_surface_run");
-  }
   hipLaunchKernelGGL(k_start, dim3(1), dim3(64), 0, S.st, k);
   hipLaunchKernelGGL(k_bounds, dim3(grid1(n, BOUNDS_THREADS)), dim3(BOUNDS_THREADS), 0, S.st, k);
   int rc = report(S);
@@ -1977,8 +2060,8 @@ int32_t nn_surface_run(nn_surface* s, const float* pos, int64_t n) {
   }
   hipError_t e = S->pos.ensure(3 * (size_t)n);
   if (e != hipSuccess) return nn::hip_fail(e, "nn_surface_run: alloc");
-  e = hipMemcpyAsync(S->pos.p, pos, sizeof(float) * 3 * (size_t)n, hipMemcpyHostToDevice, S->st);
-  if (e != hipSuccess) return nn::hip_fail(e, "nn_surface_run: upload");
+  const int rc = nn::sr::transfer(*S, true, {{S->pos.p, const_cast<float*>(pos), sizeof(float) * 3 * (size_t)n}}, "nn_surface_run: upload");
+  if (rc) return rc;
   return nn::sr::run(*S, S->pos.p, nullptr, (long)n);
 }
 
@@ -1995,9 +2078,10 @@ int32_t nn_surface_run_velocity(nn_surface* s, const float* pos, const float* ve
   hipError_t e = S->pos.ensure(3 * (size_t)n);
   if (e == hipSuccess) e = S->vel.ensure(3 * (size_t)n);
   if (e != hipSuccess) return nn::hip_fail(e, "nn_surface_run_velocity: alloc");
-  e = hipMemcpyAsync(S->pos.p, pos, sizeof(float) * 3 * (size_t)n, hipMemcpyHostToDevice, S->st);
-  if (e == hipSuccess) e = hipMemcpyAsync(S->vel.p, vel, sizeof(float) * 3 * (size_t)n, hipMemcpyHostToDevice, S->st);
-  if (e != hipSuccess) return nn::hip_fail(e, "nn_surface_run_velocity: upload");
+  const size_t bytes = sizeof(float) * 3 * (size_t)n;
+  const int rc = nn::sr::transfer(*S, true, {{S->pos.p, const_cast<float*>(pos), bytes}, {S->vel.p, const_cast<float*>(vel), bytes}},
+                                  "nn_surface_run_velocity: upload");
+  if (rc) return rc;
   return nn::sr::run(*S, S->pos.p, S->vel.p, (long)n);
 }
 
@@ -2011,11 +2095,7 @@ int32_t nn_surface_mesh_velocity(nn_surface* s, float* out) {
     nn::set_error("nn_surface_mesh_velocity: no completed run with the velocity channels");
     return NN_E_STATE;
   }
-  if (S->nverts) {
-    hipError_t e = hipMemcpy(out, S->k.mvel, sizeof(float) * 3 * S->nverts, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return nn::hip_fail(e, "nn_surface_mesh_velocity");
-  }
-  return NN_OK;
+  return nn::sr::transfer(*S, false, {{S->k.mvel, out, sizeof(float) * 3 * S->nverts}}, "nn_surface_mesh_velocity");
 }
 
 int32_t nn_surface_info(nn_surface* s, int64_t* out, double* sd) {
@@ -2057,13 +2137,11 @@ int32_t nn_surface_mesh(nn_surface* s, float* vertices, int32_t* faces, float* n
     nn::set_error("nn_surface_mesh: normals were not requested (nn_surface_params.normals)");
     return NN_E_STATE;
   }
-  hipError_t e = hipSuccess;
-  if (S->nverts) e = hipMemcpy(vertices, S->k.verts, sizeof(float) * 3 * S->nverts, hipMemcpyDeviceToHost);
-  if (e == hipSuccess && S->ntris) e = hipMemcpy(faces, S->k.faces, sizeof(int) * 3 * S->ntris, hipMemcpyDeviceToHost);
-  if (e == hipSuccess && normals && S->nverts)
-    e = hipMemcpy(normals, S->k.normals, sizeof(float) * 3 * S->nverts, hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return nn::hip_fail(e, "nn_surface_mesh");
-  return NN_OK;
+  return nn::sr::transfer(*S, false,
+                          {{S->k.verts, vertices, sizeof(float) * 3 * S->nverts},
+                           {S->k.faces, faces, sizeof(int) * 3 * S->ntris},
+                           {S->k.normals, normals, normals ? sizeof(float) * 3 * S->nverts : 0}},
+                          "nn_surface_mesh");
 }
 
 int32_t nn_surface_field(nn_surface* s, int32_t which, float* out, size_t count) {
