@@ -546,6 +546,8 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
       if (f) d.cg_waves[sc.wave_begin + at] = j0 + t;
       __syncthreads();
     }
+    // the rest names some wave, for lanes that request one before they know n
+    for (int j = sc.wave_begin + n + t; j < sc.wave_end; j += FINISH_THREADS) d.cg_waves[j] = sc.wave_begin;
     if (t == 0) st->cg_nw = n;
   }
   if (t != 0) return;

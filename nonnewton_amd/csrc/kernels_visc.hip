@@ -268,6 +268,7 @@ __global__ void k_cg_guess(Dev d) {
 // are added in list order whatever D is.  A pair with s_ij = 0 -- every
 // neighbor that is not fluid -- adds nothing and is skipped, so the neighbor's
 // u is never read there.  Returns u.w of the particle (lane 0; else 0).
+// (Slots without a particle are of no kind, so validity needs no scene word.)
 template <int D>
 __device__ __forceinline__ double matvec_row(const Dev& d, const SceneDev& sc, int i, int q) {
   const long P = d.P;
@@ -284,7 +285,7 @@ __device__ __forceinline__ double matvec_row(const Dev& d, const SceneDev& sc, i
   const XU own = d.xu[i];
   const int cnt = d.nnbr[i];
   const float rho = d.rho[i];
-  const bool valid = i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID;
+  const bool valid = kind_of(d.info[i]) == KIND_FLUID;
   float ax = 0.f, ay = 0.f, az = 0.f;
   const float3 xi = own.p, ui = own.u;
   if (valid) {
@@ -479,7 +480,8 @@ __device__ __forceinline__ void cg_list_scene(const Dev& d, const SceneDev& sc, 
 // 20 MB in and out at 131,072 particles: 4.3 us at the rate of a large copy,
 // and a chain of loads through the tables and the sums before it.  Requested
 // after the decision, with the sums' loads four at a time, the vectors made the
-// update take 11.8 us; requested before it, with the sums' loads together, 10.6
+// update take 11.8 us; requested before it, with the sums' loads together, 10.6;
+// with the wave's number requested beside the tables' words as well, 10.5
 // (workgroups of 4 or 16 waves: 10.9, 10.1).  Waves without fluid, a fifth
 // there and half of a small scene's, made up a tenth of a 64-scene pool's tick.
 constexpr int UPD_THREADS = 64 * CG_UPD_WAVES;
@@ -501,6 +503,7 @@ __global__ __launch_bounds__(UPD_THREADS) void k_cg_update(Dev d, int k) {
   const SceneDev& sc = d.scenes[s];
   SceneState* st = d.state + s;
   const int t = threadIdx.x;
+  const int w = d.cg_waves[min(e.y + (t >> 6), d.W - 1)];  // with the tables' words, not after them
   if (blockIdx.x == 0 && t == 0) d.cg_list_n[(k + 1) % 3] = 0;  // for iteration k + 1
   const int stop = st->cg_stop_at;
   if (!st->active_cg || (stop != 0 && stop < k)) return;  // uniform over the workgroup
@@ -508,8 +511,7 @@ __global__ __launch_bounds__(UPD_THREADS) void k_cg_update(Dev d, int k) {
   const int m0 = e.y - sc.wave_begin, m = m0 + (t >> 6), nw = st->cg_nw;
   if (m0 != 0 && m0 >= nw) return;
   // the particle's vectors are requested before the decision that scales them
-  const int w = d.cg_waves[sc.wave_begin + min(m, nw - 1)];
-  const int i = w * 64 + (t & 63);
+  const int i = (m < nw ? w : sc.wave_begin) * 64 + (t & 63);
   const int inf = d.info[i];
   const float3 ww = d.ww[i], po = d.wp[i], so = d.ws[i];
   float3 x = d.wx[i], r = d.wr[i];
