@@ -184,6 +184,9 @@ class Batch {
   float *h_stage_ = nullptr, *stage_dev_ = nullptr;
   int stage();
   int await(int n, unsigned& bits);
+  int await(int n, unsigned& bits, unsigned ticket, bool later);
+  template <typename Launch>
+  int field_pieces(int n, float* out, const float* in, Launch launch);
   bool any_fluid_ = false, any_elastic_ = false, any_weiler_ = false, any_strain_ = false, any_div_ = false;
   bool any_warm_cg_ = false, any_rigid_ = false;
   int max_body_ = 0, max_coupling_ = 0, max_body_waves_ = 0;  // over the scenes with rigid bodies

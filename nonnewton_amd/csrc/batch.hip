@@ -229,12 +229,12 @@ long long scene_footprint(long long n, long long ns, long long cells) {
   return np * BYTES_PER_SLOT + nsp * BYTES_PER_MEMBER + (cells + 1) * 8 + 2048;
 }
 
-// Pinned memory through which the kernels read and write the fields of small
-// scenes themselves.  Microseconds of an upload / a download by field size,
-// this way and with a copy to or from device memory:
-//             5 KB      134 KB    329 KB    886 KB    1.9 MB     3.4 MB
-//   kernels   11 / 11   15 / 17   21 / 27   41 / 51   93 / 139   142 / 238
-//   copies    20 / 27   74 / 82   36 / 40   60 / 68   91 / 145   141 / 274
+// Pinned memory through which the kernels read and write fields, larger ones in
+// pieces.  Microseconds of an upload / a download by field size, this way and
+// with a copy to or from device memory:
+//             5 KB      134 KB    329 KB    886 KB    1.9 MB     3.4 MB      6.5 MB
+//   kernels   11 / 11   15 / 17   21 / 27   41 / 51   68 / 93    111 / 157   196 / 291
+//   copies    20 / 27   74 / 82   36 / 40   60 / 68   91 / 140   136 / 256   228 / 473
 constexpr size_t STAGE_BYTES = 1 << 20;
 static size_t state_bytes(int scenes) { return (sizeof(SceneState) + sizeof(unsigned long long)) * (size_t)scenes; }
 
@@ -926,19 +926,20 @@ int Batch::search() {
   return NN_OK;
 }
 
-// Waits until each of the first n report words carries the last ticket; bits:
-// the or of what they report.  Polling them costs 6 us less than a copy of the
+// Waits until each of the first n report words carries the ticket, the last one
+// given out by default (later: or one after it); bits: the or of what they report.  Polling them costs 6 us less than a copy of the
 // counter and a wait for the stream (six small launches and the wait: 19.5 us
 // against 26); a wait that lasts is left to the stream's, which also returns
 // the errors of launches that cannot report.
-int Batch::await(int n, unsigned& bits) {
+int Batch::await(int n, unsigned& bits) { return await(n, bits, ticket_, false); }
+int Batch::await(int n, unsigned& bits, unsigned ticket, bool later) {
   HIPCHK(hipGetLastError());
   bits = 0;
   bool synced = false;
   const auto start = std::chrono::steady_clock::now();
   for (int k = 0, polls = 0; k < n;) {
     const unsigned long long v = __atomic_load_n(h_report_ + k, __ATOMIC_ACQUIRE);
-    if ((unsigned)(v >> 32) == ticket_) {
+    if ((unsigned)(v >> 32) == ticket || (later && (int)((unsigned)(v >> 32) - ticket) > 0)) {
       bits |= (unsigned)v;
       k++;
     } else if (synced) {
@@ -1325,6 +1326,33 @@ int Batch::stage() {
   return NN_OK;
 }
 
+// A three-component field of n particles through the two halves of the staging
+// memory: a piece is copied by the host while the kernel of the next one runs.
+// launch(first particle, particles, device address of the half) reads or writes.
+template <typename Launch>
+int Batch::field_pieces(int n, float* out, const float* in, Launch launch) {
+  CHK(stage());
+  constexpr int PIECE = (int)(STAGE_BYTES / 2 / 12);
+  const int pieces = (n + PIECE - 1) / PIECE;
+  const unsigned before = ticket_;  // piece c reports ticket before + 1 + c
+  ticket_ += pieces;
+  const auto count = [&](int c) { return std::min(PIECE, n - c * PIECE); };
+  const auto half = [&](int c) { return (size_t)(c & 1) * (STAGE_BYTES / 2 / 4); };
+  const auto start = [&](int c) {
+    if (in) std::memcpy(h_stage_ + half(c), in + 3 * (size_t)c * PIECE, 12 * (size_t)count(c));
+    launch(c * PIECE, count(c), stage_dev_ + half(c));
+    launch_report_active(dref(), -1, report_dev_, before + 1 + c, stream);
+  };
+  for (int c = 0; c < std::min(pieces, 2); c++) start(c);
+  for (int c = 0; c < pieces; c++) {
+    unsigned none = 0;
+    CHK(await(1, none, before + 1 + c, true));
+    if (out) std::memcpy(out + 3 * (size_t)c * PIECE, h_stage_ + half(c), 12 * (size_t)count(c));
+    if (c + 2 < pieces) start(c + 2);
+  }
+  return NN_OK;
+}
+
 int Batch::download(int k, int field, void* host, size_t bytes) {
   SceneHost& s = *scenes[k];
   const int w = field_width(field);
@@ -1338,8 +1366,7 @@ int Batch::download(int k, int field, void* host, size_t bytes) {
     return NN_E_ARG;
   }
   if (field == NN_FIELD_NUM_NEIGHBORS) CHK(complete_lists());
-  // three-component fields: into original order on the device (vel_alt is free
-  // between steps), then one copy
+  // three-component fields: into original order by the kernel that writes them
   if (field == NN_FIELD_X || field == NN_FIELD_V || field == NN_FIELD_ACCELERATION || field == NN_FIELD_VISC_DIFF) {
     const float4* p = field == NN_FIELD_V ? d.vel : field == NN_FIELD_ACCELERATION ? d.acc : field == NN_FIELD_VISC_DIFF ? d.vdiff : d.pos;
     if (bytes <= STAGE_BYTES) {
@@ -1351,12 +1378,8 @@ int Batch::download(int k, int field, void* host, size_t bytes) {
       std::memcpy(host, h_stage_, bytes);
       return NN_OK;
     }
-    float* ordered = reinterpret_cast<float*>(d.vel_alt + pb);
-    launch_gather3(p + pb, d.inv + pb, n, ordered, stream);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(host, ordered, bytes, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    return NN_OK;
+    return field_pieces(n, static_cast<float*>(host), nullptr,
+                        [&](int at, int m, float* dev) { launch_gather3(p + pb, d.inv + pb + at, m, dev, stream); });
   }
   std::vector<int> info(n);
   HIPCHK(hipMemcpyAsync(info.data(), d.info + pb, sizeof(int) * n, hipMemcpyDeviceToHost, stream));
@@ -1488,12 +1511,8 @@ int Batch::upload_field(int k, int field, const void* host, size_t bytes) {
     unsigned none = 0;
     return await(1, none);
   }
-  float* ordered = reinterpret_cast<float*>(d.vel_alt + pb);  // free between steps
-  HIPCHK(hipMemcpyAsync(ordered, host, bytes, hipMemcpyHostToDevice, stream));
-  launch_scatter3(ordered, d.inv + pb, n, p + pb, stream);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(stream));
-  return NN_OK;
+  return field_pieces(n, nullptr, static_cast<const float*>(host),
+                      [&](int at, int m, float* dev) { launch_scatter3(dev, d.inv + pb + at, m, p + pb, stream); });
 }
 
 // After a step, the static particles' lists are built on demand, from the

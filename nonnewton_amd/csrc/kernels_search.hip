@@ -38,11 +38,9 @@ void launch_fill_f4(float4* p, long n, float4 v, hipStream_t st) {
   NN_LAUNCH(k_fill_f4, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n, v);
 }
 
-// Fields of float[n][3] in original order (inv: slot of an id).  Reordered by
-// the host, particle by particle over two arrays copied each way, an upload of
-// 168,218 particles took 402 us and a download 360 us; through these kernels
-// (3 to 5 us) and one copy of 12 bytes a particle, 86 and 152 us.  `ordered` may
-// be host memory.
+// Fields of float[n][3] in original order (inv: slot of an id); `ordered` is pinned
+// host memory.  (Reordered by the host, particle by particle over two arrays
+// copied each way, an upload of 168,218 particles took 402 us and a download 360.)
 __global__ void k_gather3(const float4* slots, const int* inv, int n, float* ordered) {
   const int id = blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= n) return;

@@ -66,3 +66,23 @@ def test_fields_on_either_side_of_the_staging_size(n):
     assert np.array_equal(ctx.download(L.FIELD_V).reshape(-1, 3).view(np.uint32), marks)
     assert np.array_equal(ctx.download(L.FIELD_X).reshape(-1, 3), sc.x)
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [131070, 131072, 175000])
+def test_fields_in_pieces(n):
+    """Pieces of 43,690 particles through the halves of the staging memory."""
+    sc = scenes.tiny_box(seed=2, fluid_counts=(3, 3, 3), cells=(120, 120, 120))
+    rng = np.random.Generator(np.random.PCG64(n))
+    x = scenes.lattice((0.1, 0.1, 0.1), (56, 56, 56)).astype(np.float32)
+    sc.x = np.ascontiguousarray(x[rng.permutation(len(x))[:n]])
+    sc.kind, sc.v = np.zeros(n, np.int32), np.zeros((n, 3), np.float32)
+    ctx = L.Context(sc.params, sc.n)
+    ctx.upload(sc.x, sc.kind, sc.v)
+    ctx.init()
+    assert np.array_equal(ctx.download(L.FIELD_X).reshape(-1, 3), sc.x)
+    for k in (1, 3):
+        marks = (k * np.arange(3 * n, dtype=np.uint32) * 2654435761 & 0x7FFFFFFF).reshape(-1, 3)
+        ctx.upload_field(L.FIELD_V, marks.view(np.float32))
+        assert np.array_equal(ctx.download(L.FIELD_V).reshape(-1, 3).view(np.uint32), marks)
+    assert np.array_equal(ctx.download(L.FIELD_X).reshape(-1, 3), sc.x)
+    ctx.close()
