@@ -4,7 +4,8 @@ Two shapes per kernel: the workgroup size, and the gather depth (how many
 neighbor-list entries a lane loads before using them).  Neither changes a
 result: the per-particle arithmetic, the order of every sum and the grouping of
 the FP64 partial sums are fixed per wavefront.  So shapes are tuned on the live
-workload:
+workload (a sweep over few particles runs 16 lanes per particle at one depth,
+and the elastic sweeps at one workgroup size: their choice changes nothing):
   1. workgroup sizes: one tick per candidate size (all kernels at that size),
      rounds in alternating order, every kernel timed with HIP events; the time
      of a solver kernel is divided by its work in that tick (particles x

@@ -35,8 +35,8 @@ constexpr int WAVE = 64;
 // Workgroup sizes of the per-scene reductions.  Smaller workgroups find room
 // on a CU sooner while other pools' sweeps occupy the device (lanes): with 8
 // waves per CG-update workgroup and 256 threads per scene finish the mixed
-// batch ticks in 3.11 ms in three lanes against 3.23 with 16 waves and 1,024
-// threads (3.54 against 3.59 in one pool), with the same bits.
+// batch ticked in 3.11 ms in three lanes against 3.23 with 16 waves and 1,024
+// threads (3.54 against 3.59 in one pool; now 2.78 and 3.17), with the same bits.
 #ifndef NN_UPD_WAVES
 #define NN_UPD_WAVES 8
 #endif
