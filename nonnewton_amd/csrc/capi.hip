@@ -485,6 +485,7 @@ int32_t nn_pool_destroy(nn_pool* p) {
   for (auto& s : p->slots) {
     s.staging.reset();
   }
+  p->spares->clear();  // before the stream goes
   if (p->stream) (void)hipStreamDestroy(p->stream);
   delete p;
   return NN_OK;

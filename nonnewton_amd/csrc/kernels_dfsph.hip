@@ -162,16 +162,19 @@ __global__ __launch_bounds__(PUBLISH_THREADS) void k_publish(Dev d, int list_lan
   }
   __syncthreads();
   if (t != 0) return;
-  SceneState st = d.state[s];
-  st.pairs = st.pairs_fluid = 0ull;
+  unsigned long long pairs = 0, pairs_fluid = 0;
   m = 0.0f;
   for (int w = 0; w < PUBLISH_THREADS / 64; w++) {
-    st.pairs += (unsigned long long)red[0][w];
-    st.pairs_fluid += (unsigned long long)red[1][w];
+    pairs += (unsigned long long)red[0][w];
+    pairs_fluid += (unsigned long long)red[1][w];
     m = fmaxf(m, rmax[w]);
   }
-  st.max_rho_bits = __float_as_uint(m);
-  host[s] = st;
+  // copied first and completed in place: completed as a local copy, it lay in
+  // scratch, for which every queue of a step would have to keep memory
+  host[s] = d.state[s];
+  host[s].pairs = pairs;
+  host[s].pairs_fluid = pairs_fluid;
+  host[s].max_rho_bits = __float_as_uint(m);
   // after the state: released to the host
   __hip_atomic_store(report + s, (unsigned long long)ticket << 32, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
