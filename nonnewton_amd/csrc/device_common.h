@@ -345,6 +345,20 @@ __device__ __forceinline__ void lane_partials(const Dev& d, int i, double (&v)[N
   }
 }
 
+// Entries of list[b, e) below `id`, eight loads in flight (one at a time, each
+// member of a cell costs a trip to the L2).
+__device__ __forceinline__ int lower_ids(const int* list, int b, int e, int id) {
+  int n = 0;
+  for (int k = b; k < e; k += 8) {
+    int v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = list[min(k + u, e - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; u++) n += k + u < e && v[u] < id ? 1 : 0;
+  }
+  return n;
+}
+
 // Four-lane sweeps: lanes 4i..4i+3 share particle slot i, lane q walks list
 // positions k = q, q+4, ...; a wavefront covers 16 particles.  `hw` is the
 // hardware wavefront index used for the partial sums.

@@ -267,8 +267,7 @@ __global__ void k_vsort(K k, const int* bucket) {
   const int b = k.vstart[key], e = k.vstart[key + 1];
   int dest = t;
   if (e - b <= MAX_PER_VOXEL) {
-    dest = b;
-    for (int m = b; m < e; m++) dest += bucket[m] < i;
+    dest = b + lower_ids(bucket, b, e, i);
   }
   k.vlist[dest] = i;
   k.sorted[dest] = make_float4(x[0], x[1], x[2], __int_as_float(i));
