@@ -58,16 +58,17 @@ __global__ void k_begin(Dev d, int begin, long cells) {
 // read the same neighbors and none reads what another writes.
 template <int G, int B>
 __global__ void k_density_alpha(Dev d) {
+  const Ahead<G, B> own(d);
   int i, q, s;
   if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (!(sc.flags & SF_HAS_FLUID)) return;
   float rho_out = 0.0f;
-  if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
+  if (i < sc.p_begin + sc.n && kind_of(own.info(d, i)) == KIND_FLUID) {
     const KernH kh(sc);
-    const float4 xi = d.pos[i];
+    const float4 xi = own.pos(d, i);
     const float4 vi = d.vel[i];
-    const int cnt = d.nnbr[i];
+    const int cnt = own.count(d, i);
     const bool comp = (sc.flags & SF_COMPENSATED) != 0;
     KSum den{0.0f, 0.0f};
     float gix = 0.f, giy = 0.f, giz = 0.f, sk = 0.f, rd = 0.f;
@@ -99,7 +100,8 @@ __global__ void k_density_alpha(Dev d) {
           giy += t[3];
           giz += t[4];
           rd += t[5];
-        });
+        },
+        &own);
     float rho = xi.w * sc.W0;
     rho += den.s;
     rho *= sc.rho0;
@@ -185,11 +187,12 @@ __global__ __launch_bounds__(PUBLISH_THREADS) void k_publish(Dev d, int list_lan
 // neighbor's factor.  SIGNED where the sums start at a velocity, which may be
 // -0, and not at +0.
 template <int G, int B, bool SIGNED, typename KJ>
-__device__ __forceinline__ void velocity_push(const Dev& d, const SceneDev& sc, const KernH& kh, int i, int q, int cnt,
-                                              float4 xi, float ki, KJ kj, float& ax, float& ay, float& az) {
+__device__ __forceinline__ void velocity_push(const Dev& d, const SceneDev& sc, const KernH& kh, int i, int q,
+                                              const Ahead<G, B>& own, float ki, KJ kj, float& ax, float& ay, float& az) {
+  const float4 xi = own.pos(d, i);
   const bool solid_on = fabsf(ki) > sc.eps;
   for_pairs<G, B, 3>(
-      d, i, q, cnt, [&](int j) { const float2 t = d.sa[j]; return PosSrc{d.pos[j], t.x, t.y}; },
+      d, i, q, own.count(d, i), [&](int j) { const float2 t = d.sa[j]; return PosSrc{d.pos[j], t.x, t.y}; },
       [&](int, const PosSrc& nj, bool live, float (&t)[3]) {
         const float4 xj = nj.x;
         const bool fluid = xj.w > 0.0f;
@@ -210,7 +213,8 @@ __device__ __forceinline__ void velocity_push(const Dev& d, const SceneDev& sc, 
         ax += t[0];
         ay += t[1];
         az += t[2];
-      });
+      },
+      &own);
 }
 
 // divergence_solver_iteration_kernel, :1721-1760 (Jacobi: reads rho-dot and
@@ -218,18 +222,18 @@ __device__ __forceinline__ void velocity_push(const Dev& d, const SceneDev& sc, 
 // clear_accelerations (:1552) erases them.
 template <int G, int B>
 __global__ void k_div_update(Dev d) {
+  const Ahead<G, B> own(d);
   int i, q, s;
   if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (!d.state[s].active_v) return;
-  if (i >= sc.p_begin + sc.n || kind_of(d.info[i]) != KIND_FLUID) return;
+  if (i >= sc.p_begin + sc.n || kind_of(own.info(d, i)) != KIND_FLUID) return;
   const KernH kh(sc);
-  const float4 xi = d.pos[i];
   const float2 sai = d.sa[i];
   const float ki = sai.x * alpha_div(sc, sai.y);
   float dvx = 0.f, dvy = 0.f, dvz = 0.f;
-  velocity_push<G, B, false>(d, sc, kh, i, q, d.nnbr[i], xi, ki, [&](const PosSrc& nj) { return nj.src * alpha_div(sc, nj.alpha); },
-                      dvx, dvy, dvz);
+  velocity_push<G, B, false>(d, sc, kh, i, q, own, ki, [&](const PosSrc& nj) { return nj.src * alpha_div(sc, nj.alpha); },
+                             dvx, dvy, dvz);
   if (q != 0) return;
   float4 v = d.vel[i];
   v.x += dvx;
@@ -238,12 +242,12 @@ __global__ void k_div_update(Dev d) {
   d.vel[i] = v;
 }
 
-// sum_j V_j (v_i - v_j) . gradW_ij over all neighbors, and the count
+// sum_j V_j (v_i - v_j) . gradW_ij over all neighbors
 template <int G, int B>
-__device__ __forceinline__ float velocity_divergence(const Dev& d, const SceneDev& sc, int i, int q, float4 xi, int& cnt) {
+__device__ __forceinline__ float velocity_divergence(const Dev& d, const SceneDev& sc, int i, int q, const Ahead<G, B>& own) {
   const KernH kh(sc);
-  const float4 vi = d.vel[i];
-  cnt = d.nnbr[i];
+  const float4 xi = own.pos(d, i), vi = d.vel[i];
+  const int cnt = own.count(d, i);
   float acc = 0.f;
   for_pairs<G, B, 1>(
       d, i, q, cnt, [&](int j) { return PosVel{d.pos[j], d.vel[j]}; },
@@ -253,7 +257,7 @@ __device__ __forceinline__ float velocity_divergence(const Dev& d, const SceneDe
         const float dvx = vi.x - vj.x, dvy = vi.y - vj.y, dvz = vi.z - vj.z;
         t[0] = live ? fabsf(xj.w) * (dvx * g.x + dvy * g.y + dvz * g.z) : NEUTRAL;
       },
-      [&](const float (&t)[1], bool) { acc += t[0]; });
+      [&](const float (&t)[1], bool) { acc += t[0]; }, &own);
   return acc;
 }
 
@@ -261,17 +265,17 @@ __device__ __forceinline__ float velocity_divergence(const Dev& d, const SceneDe
 // and the loop test of divergence_solve (:1695-1703)
 template <int G, int B>
 __global__ void k_div_source(Dev d) {
+  const Ahead<G, B> own(d);
   int i, q, s;
   if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   SceneState* st = d.state + s;
   if (!st->active_v) return;
   double v[1] = {0.0};
-  if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
-    int cnt;
-    float rd = velocity_divergence<G, B>(d, sc, i, q, d.pos[i], cnt);
+  if (i < sc.p_begin + sc.n && kind_of(own.info(d, i)) == KIND_FLUID) {
+    float rd = velocity_divergence<G, B>(d, sc, i, q, own);
     rd = rd > 0.0f ? rd : 0.0f;
-    if (cnt < 20) rd = 0.0f;
+    if (own.count(d, i) < 20) rd = 0.0f;
     if (q == 0) d.sa[i].x = rd;
     v[0] = (double)sc.rho0 * (double)rd - 0.0;
   }
@@ -285,11 +289,12 @@ __global__ void k_div_source(Dev d) {
 // reads vel and writes vel_alt.
 template <int G, int B>
 __global__ void k_nonpressure(Dev d) {
+  const Ahead<G, B> own(d);
   int i, q, s;
   if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (i >= sc.p_begin + sc.n) return;
-  const int kind = kind_of(d.info[i]);
+  const int kind = kind_of(own.info(d, i));
   const float4 vi = d.vel[i];
   if (!(sc.flags & SF_HAS_FLUID)) {
     if (q == 0) d.vel_alt[i] = vi;
@@ -301,7 +306,7 @@ __global__ void k_nonpressure(Dev d) {
   const bool bnu_on = vis_on && sc.bnu != 0.0f;
   if (kind == KIND_FLUID) {
     const KernH kh(sc);
-    const float4 xi = d.pos[i];
+    const float4 xi = own.pos(d, i);
     const bool st_on = (sc.flags & SF_SURFACE_TENSION) != 0;
     const float rhoi = d.rho[i];
     float sx = 0.f, sy = 0.f, sz = 0.f, wvx = 0.f, wvy = 0.f, wvz = 0.f;
@@ -313,7 +318,7 @@ __global__ void k_nonpressure(Dev d) {
         float4 x, v;
         float rho;
       };
-      const int cnt = d.nnbr[i];
+      const int cnt = own.count(d, i);
       for_pairs<G, B, 6>(
           d, i, q, cnt, [&](int j) { return NJ{d.pos[j], d.vel[j], d.rho[j]}; },
           [&](int, const NJ& nj, bool live, float (&t)[6]) {
@@ -347,9 +352,10 @@ __global__ void k_nonpressure(Dev d) {
             wvx += t[3];
             wvy += t[4];
             wvz += t[5];
-          });
+          },
+          &own);
     } else if (st_on) {
-      const int cnt = d.nnbr[i];
+      const int cnt = own.count(d, i);
       for_pairs<G, B, 3>(
           d, i, q, cnt, [&](int j) { return d.pos[j]; },
           [&](int, const float4& xj, bool live, float (&t)[3]) {
@@ -366,7 +372,8 @@ __global__ void k_nonpressure(Dev d) {
             sx += t[0];
             sy += t[1];
             sz += t[2];
-          });
+          },
+          &own);
     }
     if (q != 0) return;
     float ax = sc.gx, ay = sc.gy, az = sc.gz;
@@ -440,15 +447,15 @@ __global__ void k_nonpressure(Dev d) {
 // test of pressure_solve (:1778-1784)
 template <int G, int B>
 __global__ void k_press_source(Dev d, int reduce) {
+  const Ahead<G, B> own(d);
   int i, q, s;
   if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   SceneState* st = d.state + s;
   if (!st->active_p) return;
   double v[1] = {0.0};
-  if (i < sc.p_begin + sc.n && kind_of(d.info[i]) == KIND_FLUID) {
-    int cnt;
-    const float delta = velocity_divergence<G, B>(d, sc, i, q, d.pos[i], cnt);
+  if (i < sc.p_begin + sc.n && kind_of(own.info(d, i)) == KIND_FLUID) {
+    const float delta = velocity_divergence<G, B>(d, sc, i, q, own);
     float da = d.rho[i] / sc.rho0 + sc.dt * delta;
     da = da > 1.0f ? da : 1.0f;
     if (q == 0) d.sa[i].x = da;
@@ -597,18 +604,19 @@ __global__ __launch_bounds__(FINISH_THREADS) void k_scene_finish(Dev d, int whic
 // -vel_change/dt of every fluid neighbor (:1835-1841) into their acceleration.
 template <int G, int B>
 __global__ void k_press_update(Dev d) {
+  const Ahead<G, B> own(d);
   int i, q, s;
   if (!lane_slot_scene<G>(d, i, q, s)) return;
   const SceneDev& sc = d.scenes[s];
   if (!d.state[s].active_p) return;
   if (i >= sc.p_begin + sc.n) return;
-  const int kind = kind_of(d.info[i]);
+  const int kind = kind_of(own.info(d, i));
   if (kind == KIND_FLUID) {
     const KernH kh(sc);
     const float2 sai = d.sa[i];
     const float ki = (sai.x - 1.0f) * alpha_press(sc, sai.y);
     float4 v = d.vel[i];
-    velocity_push<G, B, true>(d, sc, kh, i, q, d.nnbr[i], d.pos[i], ki,
+    velocity_push<G, B, true>(d, sc, kh, i, q, own, ki,
                               [&](const PosSrc& nj) { return (nj.src - 1.0f) * alpha_press(sc, nj.alpha); }, v.x, v.y, v.z);
     if (q == 0) d.vel[i] = v;
   } else if (dyn_solid(kind)) {
