@@ -320,7 +320,8 @@ typedef struct nn_surface_params {
  * of 4 * smooth_radius / voxel_size + 2 vertices exceeds 32 per axis. */
 int32_t nn_surface_create(const nn_surface_params *params, nn_surface **out);
 int32_t nn_surface_destroy(nn_surface *s);
-/* Cap on the device bytes a run's grids may take (0 = none): NN_E_OOM above it. */
+/* Cap on the device bytes of a run's grids, lists, input copies and mesh
+ * (0 = none): NN_E_OOM above it. */
 int32_t nn_surface_set_budget(nn_surface *s, int64_t bytes);
 /* SRTool.dual_contouring(isolevel, smooth_radius, num_particles, pos)
  * (srtool.py:1264-1304) on n host positions (x, y, z float triples).

@@ -1799,13 +1799,24 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   k.nvox = nvox;
   k.nvert = nvert;
   k.nblock = nblock;
-  const double need = (double)nvox * 8 + (double)nvert * (k.vel ? 72 : 36) + (double)n * 64 + (double)nblock * 20;
+  // the device bytes of the buffers below, the inputs' copies (pos, vel) and the
+  // scans' partials; the mesh's are added once its size is known
+  double need = (double)nvox * 8 + (double)nvert * (k.vel ? 32 : 20) + (double)nblock * 17 +
+                (double)n * (84 + (k.aniso ? 16 * REC_QUADS : 0)) + 4.0 * (double)scan_tmp_ints(std::max(nvox, nvert));
+  if (dpos == S.pos.p) need += 12.0 * (double)n;
+  if (dvel) need += 12.0 * (double)n;
   // int32 scans: up to 6 triangles per cube must stay below 2^31
   if (nvert > (1L << 28) || nvox > (1L << 30) || (S.budget > 0 && need > (double)S.budget)) {
     set_error("nn_surface_run: the vertex grid over the particles' extent exceeds the device budget (" +
-              std::to_string(nvert) + " vertices)");
+              std::to_string(nvert) + " vertices, " + std::to_string(n) + " particles)");
     return NN_E_OOM;
   }
+  const auto mesh_fits = [&](double bytes) {
+    need += bytes;
+    if (!(S.budget > 0 && need > (double)S.budget)) return true;
+    set_error("nn_surface_run: the mesh exceeds the device budget");
+    return false;
+  };
   SR_HIP(S.vcount.ensure(nvox), "nn_surface_run: alloc");
   SR_HIP(S.vstart.ensure(nvox + 1), "nn_surface_run: alloc");
   SR_HIP(S.vslot.ensure(n), "nn_surface_run: alloc");
@@ -1875,6 +1886,8 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   SR_HIP(scan(S, k.flag, k.cube_id, nvert, 1), "nn_surface_run: scan");
   if ((rc = report(S, k.cube_id + nvert))) return rc;
   const int nv = S.report->count;
+  // verts, cubes, tcount, tstart; normals and velocities
+  if (!mesh_fits((double)nv * (24 + (S.prm.normals ? 12 : 0) + (S.prm.velocity ? 12 : 0)))) return NN_E_OOM;
   SR_HIP(S.verts.ensure(3 * (size_t)nv), "nn_surface_run: alloc");
   SR_HIP(S.cubes.ensure(nv), "nn_surface_run: alloc");
   SR_HIP(S.tcount.ensure(nv), "nn_surface_run: alloc");
@@ -1890,6 +1903,7 @@ static int run(Surface& S, const float* dpos, const float* dvel, long n) {
   const int nt = S.report->count;
   S.nactive = (long)S.report->active;  // the written blocks and the deviation, for the caller's statistics
   S.sd = S.report->stats[3];
+  if (!mesh_fits(12.0 * (double)nt)) return NN_E_OOM;
   SR_HIP(S.faces.ensure(3 * (size_t)nt), "nn_surface_run: alloc");
   k.faces = S.faces.p;
   if (nv > 0) hipLaunchKernelGGL(k_faces, dim3(grid1(nv, 128)), dim3(128), 0, S.st, k, nv);
