@@ -207,11 +207,12 @@ int32_t nn_counts(nn_ctx *ctx, int64_t *n, int64_t *n_fluid);
 /* Beside its scenes a pool holds up to an eighth of its budget in memory that
  * scenes have left, for the next ones; nn_pool_destroy gives it back. */
 int32_t nn_pool_create(int64_t budget_bytes, nn_pool **out);
-/* nn_pool_create with flags.  NN_POOL_OWN_QUEUE: the pool's stream gets a
- * hardware queue of its own (a stream whose CU mask covers every CU), so that
- * pools ticked concurrently from several threads (lanes) never share a queue;
- * with plain streams the device maps streams onto a few shared hardware
- * queues, and two pools on one queue serialize. */
+/* nn_pool_create with flags.  NN_POOL_OWN_QUEUE marks a pool that is ticked
+ * concurrently with others (a lane); it is accepted and has no effect: every
+ * pool has a plain stream, and the device maps streams onto a few shared
+ * hardware queues (4 by default; GPU_MAX_HW_QUEUES), on which up to three lanes
+ * and the admissions find one each.  (Streams with a CU mask have a queue of
+ * their own, but pools on them did not always return from nn_pool_destroy.) */
 #define NN_POOL_OWN_QUEUE 1
 int32_t nn_pool_create_ex(int64_t budget_bytes, int32_t flags, nn_pool **out);
 int32_t nn_pool_destroy(nn_pool *pool);

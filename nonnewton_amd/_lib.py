@@ -371,8 +371,8 @@ class Pool:
     """Many resident scenes stepped together (nn_pool)."""
 
     def __init__(self, budget_bytes: int, own_queue: bool = False):
-        """own_queue: the pool's stream gets a hardware queue of its own
-        (NN_POOL_OWN_QUEUE), for pools stepped concurrently (lanes)."""
+        """own_queue: the pool is stepped concurrently with others (a lane;
+        NN_POOL_OWN_QUEUE, which has no effect at present)."""
         self.lib = load()
         h = ctypes.c_void_p()
         check(self.lib.nn_pool_create_ex(int(budget_bytes), POOL_OWN_QUEUE if own_queue else 0, ctypes.byref(h)),

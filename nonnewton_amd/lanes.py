@@ -12,9 +12,9 @@ every sum is per scene in a fixed order, so a scene gives the same bits in any
 lane and beside any other lanes.
 
 Scenes go to the lane with the smallest load (particles resident, or the cost
-the caller gives).  With more than one lane each pool's stream has a hardware
-queue of its own (NN_POOL_OWN_QUEUE): the device maps plain streams onto a few
-shared queues, and two lanes on one queue would run one after the other.
+the caller gives).  The device maps streams onto a few shared hardware queues
+(4 by default): three lanes and the admissions' stream find one each, and of
+more lanes two share one and run one after the other.
 """
 from __future__ import annotations
 
@@ -37,9 +37,7 @@ class LanePool:
         if lanes < 1:
             raise ValueError("lanes must be at least 1")
         self.budget = int(budget_bytes)
-        # each lane may use the whole budget; admit() keeps the sum within it.
-        # With several lanes every pool's stream gets a hardware queue of its
-        # own: lanes that shared one would run one after the other.
+        # each lane may use the whole budget; admit() keeps the sum within it
         self.pools: List[_lib.Pool] = []
         try:
             for _ in range(lanes):
