@@ -265,6 +265,17 @@ int32_t nn_set_kernel_block(nn_ctx *ctx, int32_t kernel, int32_t block);
 int32_t nn_pool_set_kernel_depth(nn_pool *pool, int32_t kernel, int32_t depth);
 int32_t nn_set_kernel_depth(nn_ctx *ctx, int32_t kernel, int32_t depth);
 
+/* The forms of a context's Weiler solves so far (no counterpart in the
+ * reference): solves[0] in one launch (a scene of at most 256 waves of 64
+ * slots), solves[1] in two launches an iteration, and of these solves[2] that a
+ * one-launch solve had begun and left, having waited in vain for a workgroup
+ * that the device did not run.  The results are the same bits in every form. */
+int32_t nn_cg_forms(nn_ctx *ctx, int64_t *solves);
+/* Exchanges that a one-launch solve waits for: at the next one it leaves at once
+ * (0: at its first).  Negative: no limit, the default.  For tests of what
+ * follows a wait in vain. */
+int32_t nn_set_cg_patience(nn_ctx *ctx, int32_t exchanges);
+
 /* Per-kernel timing with HIP events recorded around launches on the stream the
  * kernel runs on (no counterpart in the reference).  enable != 0 turns it on
  * for every launch of every kernel and clears the totals.  The _mask forms

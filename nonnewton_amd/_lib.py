@@ -171,6 +171,8 @@ def load():
         "nn_profile": (i32, [vp, i32]),
         "nn_set_kernel_block": (i32, [vp, i32, i32]),
         "nn_set_kernel_depth": (i32, [vp, i32, i32]),
+        "nn_cg_forms": (i32, [vp, P(i64)]),
+        "nn_set_cg_patience": (i32, [vp, i32]),
         "nn_pool_set_kernel_depth": (i32, [vp, i32, i32]),
         "nn_pool_set_kernel_block": (i32, [vp, i32, i32]),
         "nn_profile_mask": (i32, [vp, ctypes.c_uint32, i32]),
@@ -348,6 +350,15 @@ class Context:
 
     def set_kernel_depth(self, kernel: str, depth: int):
         check(self.lib.nn_set_kernel_depth(self.h, kernel_names().index(kernel), int(depth)), "nn_set_kernel_depth")
+
+    def cg_forms(self):
+        """Weiler solves (in one launch, in two launches an iteration, of these begun in one launch and left)."""
+        n = (ctypes.c_int64 * 3)()
+        check(self.lib.nn_cg_forms(self.h, n), "nn_cg_forms")
+        return tuple(int(v) for v in n)
+
+    def set_cg_patience(self, exchanges: int):
+        check(self.lib.nn_set_cg_patience(self.h, int(exchanges)), "nn_set_cg_patience")
 
     def profile(self, enable: bool = True, kernels=None, stride: int = 1):
         """Time every launch of every kernel (kernels None), or every stride-th

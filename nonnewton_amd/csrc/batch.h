@@ -4,6 +4,7 @@
 // Batch of one, the pool of the serving form is a Batch whose membership
 // changes between ticks.
 #pragma once
+#include <climits>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -158,6 +159,8 @@ class Batch {
   int kdepth[K_COUNT] = {};    // per-kernel gather depth (0 = the kernel's default), set by the autotuner
   int blk(int id) const { return kblock[id] ? kblock[id] : block; }
   int dep(int id) const { return kdepth[id]; }
+  int cg_patience = INT_MAX;       // exchanges a one-launch CG solve waits for
+  long long cg_forms[3] = {0, 0, 0};  // solves in one launch; in two an iteration; of those, left by the first form
   int lanes(int id) const;  // lanes per particle of list sweep `id`
   hipStream_t stream;
   Dev d{};

@@ -1159,7 +1159,7 @@ int Batch::cg_solve(bool& done, bool& gave_up) {
   if (dep(K_CG_MATVEC) != 0) return NN_OK;  // a gather depth was asked for: it is k_cg_matvec's
   if (scenes.size() != 1 || scenes[0]->dev.wave_begin != 0 || scenes[0]->dev.wave_end > solve_waves_) return NN_OK;
   if (timer.on) timer.seen[K_CG_UPDATE]++;  // one launch does the work of both
-  TIMED(K_CG_MATVEC, launch_cg_solve(dref(), scenes[0]->dev.wave_end, stream));
+  TIMED(K_CG_MATVEC, launch_cg_solve(dref(), scenes[0]->dev.wave_end, cg_patience, stream));
   unsigned bits = 0;
   launch_report_active(dref(), 1, report_dev_, ++ticket_, stream);
   CHK(await(1, bits));
@@ -1232,6 +1232,8 @@ int Batch::step(std::vector<nn_step_stats>* stats) {
       CHK(cg_start());
       bool done = false, gave_up = false;
       CHK(cg_solve(done, gave_up));
+      cg_forms[done ? 0 : 1]++;
+      cg_forms[2] += gave_up;
       if (!done) {
         if (gave_up) {  // from the start again
           launch_begin(dref(), BEGIN_CG, 0, stream);

@@ -330,6 +330,18 @@ int32_t nn_set_kernel_depth(nn_ctx* ctx, int32_t kernel, int32_t depth) {
   return NN_OK;
 }
 
+int32_t nn_cg_forms(nn_ctx* ctx, int64_t* solves) {
+  if (!ctx || !solves) return NN_E_ARG;
+  std::copy(ctx->batch->cg_forms, ctx->batch->cg_forms + 3, solves);
+  return NN_OK;
+}
+
+int32_t nn_set_cg_patience(nn_ctx* ctx, int32_t exchanges) {
+  if (!ctx) return NN_E_ARG;
+  ctx->batch->cg_patience = exchanges < 0 ? INT_MAX : exchanges;
+  return NN_OK;
+}
+
 int32_t nn_set_kernel_block(nn_ctx* ctx, int32_t kernel, int32_t block) {
   if (!ctx || kernel < 0 || kernel >= nn::K_COUNT) return NN_E_ARG;
   if (block != 0 && (block < 64 || block > 1024 || (block & (block - 1)))) return NN_E_ARG;

@@ -278,7 +278,8 @@ void launch_cg_matvec_start(const DevRef& d, int block, int depth, hipStream_t s
 void launch_cg_update(const DevRef& d, int nblocks, int k, hipStream_t st);  // iteration k >= 1
 void launch_cg_matvec(const DevRef& d, int depth, int k, int grid, hipStream_t st);
 constexpr int CG_SOLVE_WAVES = 256;  // one workgroup per compute unit of the device
-void launch_cg_solve(const DevRef& d, int waves, hipStream_t st);  // the whole solve of a batch of one scene
+// the whole solve of a batch of one scene; after `patience` exchanges it gives up
+void launch_cg_solve(const DevRef& d, int waves, int patience, hipStream_t st);
 void launch_nonpressure(const DevRef& d, int block, int lanes, int depth, hipStream_t st);
 void launch_press_source(const DevRef& d, int block, int lanes, int depth, int reduce, hipStream_t st);
 void launch_press_update(const DevRef& d, int block, int lanes, int depth, hipStream_t st);

@@ -570,7 +570,8 @@ __global__ __launch_bounds__(UPD_THREADS) void k_cg_update(Dev d, int k) {
 // matvec launch an iteration takes 13 to 15 us at these sizes, as one launch
 // that recomputes the neighbors' updates 9 to 11.
 //
-// The wait is bounded (CG_SOLVE_POLLS): should a workgroup not have been
+// The wait is bounded (CG_SOLVE_POLLS polls, and none after `patience`
+// exchanges, which is for the tests of what follows a wait in vain): should a workgroup not have been
 // scheduled by then -- the device held by other work -- the waiting ones set
 // n_active[1] and leave, every later wait of the launch ends the same way, and
 // the host repeats the solve with k_cg_update and k_cg_matvec.  Nothing that
@@ -618,7 +619,7 @@ struct CgExchange {
   }
 };
 
-__global__ __launch_bounds__(SOLVE_THREADS) void k_cg_solve(Dev d) {
+__global__ __launch_bounds__(SOLVE_THREADS) void k_cg_solve(Dev d, int patience) {
   __shared__ double red[3][SUM_THREADS / 64];
   __shared__ double part[3][SOLVE_THREADS / 64];
   __shared__ float fixed[SOLVE_KEEP][9][SOLVE_THREADS];  // a lane's neighbors' position and M
@@ -686,8 +687,9 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_cg_solve(Dev d) {
       if (t < CG_SOLVE_WAVES) {
         const unsigned long long* from = words + 6L * ((k - 1) & 1) * d.W + t;
         bool there = t >= nw;  // the words of workgroup t are in
+        const int limit = k - 1 > patience ? 0 : CG_SOLVE_POLLS;
         for (int polls = 0; !__all(there); polls++) {
-          if (polls >= CG_SOLVE_POLLS) {
+          if (polls >= limit) {
             late = true;
             break;
           }
@@ -886,8 +888,8 @@ void launch_cg_matvec(const DevRef& d, int depth, int k, int grid, hipStream_t s
 void launch_cg_update(const DevRef& d, int nblocks, int k, hipStream_t st) {
   if (nblocks > 0) NN_LAUNCH(k_cg_update, dim3(nblocks), dim3(UPD_THREADS), 0, st, d.h, k);
 }
-void launch_cg_solve(const DevRef& d, int waves, hipStream_t st) {
-  NN_LAUNCH(k_cg_solve, dim3(waves), dim3(SOLVE_THREADS), 0, st, d.h);
+void launch_cg_solve(const DevRef& d, int waves, int patience, hipStream_t st) {
+  NN_LAUNCH(k_cg_solve, dim3(waves), dim3(SOLVE_THREADS), 0, st, d.h, patience);
 }
 
 }  // namespace nn
