@@ -1148,6 +1148,7 @@ int Batch::cg_start() {
   return NN_OK;
 }
 
+constexpr int SOLVE_REST = 256;
 int Batch::cg_solve(bool& done, bool& gave_up) {
   done = gave_up = false;
   if (solve_waves_ < 0) {  // its workgroups wait for one another: no more than compute units
@@ -1156,6 +1157,7 @@ int Batch::cg_solve(bool& done, bool& gave_up) {
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     solve_waves_ = std::min(cus, CG_SOLVE_WAVES);
   }
+  if (solve_rest_ > 0 && solve_rest_-- > 0) return NN_OK;
   if (dep(K_CG_MATVEC) != 0) return NN_OK;  // a gather depth was asked for: it is k_cg_matvec's
   if (scenes.size() != 1 || scenes[0]->dev.wave_begin != 0 || scenes[0]->dev.wave_end > solve_waves_) return NN_OK;
   if (timer.on) timer.seen[K_CG_UPDATE]++;  // one launch does the work of both
@@ -1165,7 +1167,9 @@ int Batch::cg_solve(bool& done, bool& gave_up) {
   CHK(await(1, bits));
   gave_up = bits != 0;
   done = !gave_up;
-  if (!done) solve_waves_ = 0;  // the device is shared: this batch does not try again
+  // the device was busy: a wait in vain takes about 15 ms, a solve in one launch
+  // saves about 0.5 ms, so the next try comes after SOLVE_REST solves
+  if (gave_up) solve_rest_ = SOLVE_REST;
   return NN_OK;
 }
 

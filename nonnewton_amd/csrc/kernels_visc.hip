@@ -573,8 +573,8 @@ __global__ __launch_bounds__(UPD_THREADS) void k_cg_update(Dev d, int k) {
 // The wait is bounded (CG_SOLVE_POLLS polls, and none after `patience`
 // exchanges, which is for the tests of what follows a wait in vain): should a workgroup not have been
 // scheduled by then -- the device held by other work -- the waiting ones set
-// n_active[1] and leave, every later wait of the launch ends the same way, and
-// the host repeats the solve with k_cg_update and k_cg_matvec.  Nothing that
+// n_active[1] and leave, a workgroup that comes later finds it at its 64th poll
+// (about 60 us) instead of waiting as long again, and the host repeats the solve with k_cg_update and k_cg_matvec.  Nothing that
 // such a repetition starts from is written here.
 //
 // Order: lane 4 q + a takes list positions q + 4 a + 16 b, so the four lanes of
@@ -683,13 +683,14 @@ __global__ __launch_bounds__(SOLVE_THREADS) void k_cg_solve(Dev d, int patience)
     } else {
       // every workgroup's r, w, s and partials of iteration k - 1 are there
       bool late = false;
+      const auto gave_up = [&] { return __any(__hip_atomic_load(&d.n_active[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0); };
       double mine[3] = {0.0, 0.0, 0.0};
       if (t < CG_SOLVE_WAVES) {
         const unsigned long long* from = words + 6L * ((k - 1) & 1) * d.W + t;
         bool there = t >= nw;  // the words of workgroup t are in
         const int limit = k - 1 > patience ? 0 : CG_SOLVE_POLLS;
         for (int polls = 0; !__all(there); polls++) {
-          if (polls >= limit) {
+          if (polls >= limit || ((polls & 63) == 63 && gave_up())) {
             late = true;
             break;
           }

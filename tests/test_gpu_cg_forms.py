@@ -62,3 +62,20 @@ def test_way_back_at_the_iteration_limit(patience):
     ib, b, forms = run(sc, patience=patience)
     assert all(i == 5 and s & 32 for i, _, _, s in ia) and forms[2] >= 1
     assert ia == ib and all(np.array_equal(p, q) for p, q in zip(a, b))
+
+
+def test_tried_again_later():
+    """A solve left once is tried again after 256 others."""
+    sc = column((4, 4, 4), (10, 10, 10))
+    ctx = L.Context(sc.params, sc.n)
+    ctx.set_cg_patience(0)
+    ctx.upload(sc.x, sc.kind, sc.v)
+    ctx.init()
+    ctx.step()
+    assert ctx.cg_forms() == (0, 1, 1)
+    ctx.set_cg_patience(-1)
+    ctx.step(256)
+    assert ctx.cg_forms() == (0, 257, 1)
+    ctx.step(3)
+    assert ctx.cg_forms() == (3, 257, 1)
+    ctx.close()
