@@ -176,7 +176,7 @@ class Batch {
   int C_cap_ = 0;    // cells allocated
   int scene_cap_ = 0;
   int n_cg_blocks_ = 0;  // entries of d.cg_blocks
-  int solve_waves_ = -1;  // waves k_cg_solve may have (-1: not looked up yet)
+  int device_ = 0, cus_ = -1;  // of the solves: the device and its compute units (-1: not looked up yet)
   int solve_rest_ = 0;    // solves to take in two launches an iteration before the next try
   std::vector<Alloc> deferred_;
   // pinned, h_state_cap_ entries each, with their device addresses: scene states

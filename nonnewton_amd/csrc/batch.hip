@@ -4,6 +4,7 @@
 #include "batch.h"
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -1149,19 +1150,35 @@ int Batch::cg_start() {
 }
 
 constexpr int SOLVE_REST = 256;
+// Workgroups of the one-launch solves under way, by device.  Each holds a compute
+// unit and waits for the others of its solve, so solves of several contexts run
+// at once only while there is a compute unit for every workgroup: three of 200
+// waves in three threads left a solve each after a wait in vain (0.68 ms for a
+// step of all three over the first 60, 0.56 with this; later steps the same).
+constexpr int SOLVE_DEVICES = 64;
+static std::atomic<int> solving[SOLVE_DEVICES];
+
 int Batch::cg_solve(bool& done, bool& gave_up) {
   done = gave_up = false;
-  if (solve_waves_ < 0) {  // its workgroups wait for one another: no more than compute units
-    int dev = 0, cus = 0;
-    HIPCHK(hipGetDevice(&dev));
-    HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    solve_waves_ = std::min(cus, CG_SOLVE_WAVES);
+  if (cus_ < 0) {
+    HIPCHK(hipGetDevice(&device_));
+    HIPCHK(hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, device_));
   }
   if (solve_rest_ > 0 && solve_rest_-- > 0) return NN_OK;
   if (dep(K_CG_MATVEC) != 0) return NN_OK;  // a gather depth was asked for: it is k_cg_matvec's
-  if (scenes.size() != 1 || scenes[0]->dev.wave_begin != 0 || scenes[0]->dev.wave_end > solve_waves_) return NN_OK;
+  if (scenes.size() != 1 || scenes[0]->dev.wave_begin != 0) return NN_OK;
+  const int waves = scenes[0]->dev.wave_end;
+  if (waves > std::min(cus_, CG_SOLVE_WAVES) || device_ >= SOLVE_DEVICES) return NN_OK;
+  struct Share {
+    std::atomic<int>& all;
+    const int mine;
+    const bool fits;
+    Share(std::atomic<int>& a, int n, int limit) : all(a), mine(n), fits(a.fetch_add(n) + n <= limit) {}
+    ~Share() { all.fetch_sub(mine); }
+  } share(solving[device_], waves, cus_);
+  if (!share.fits) return NN_OK;
   if (timer.on) timer.seen[K_CG_UPDATE]++;  // one launch does the work of both
-  TIMED(K_CG_MATVEC, launch_cg_solve(dref(), scenes[0]->dev.wave_end, cg_patience, stream));
+  TIMED(K_CG_MATVEC, launch_cg_solve(dref(), waves, cg_patience, stream));
   unsigned bits = 0;
   launch_report_active(dref(), 1, report_dev_, ++ticket_, stream);
   CHK(await(1, bits));

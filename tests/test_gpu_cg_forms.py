@@ -1,6 +1,8 @@
 """Which form a Weiler solve takes, and the way back from the one-launch form: a
 solve that leaves after 0, 1, 2 or 5 exchanges is repeated with the two-launch
 form and gives that form's bits, iteration counts and status."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -79,3 +81,27 @@ def test_tried_again_later():
     ctx.step(3)
     assert ctx.cg_forms() == (3, 257, 1)
     ctx.close()
+
+
+@pytest.mark.parametrize("waves", [(200, 200, 200), (200, 40, 120)])
+def test_contexts_in_threads(waves):
+    """Contexts stepped at once from their own threads, with more waves in all
+    than the device has compute units: the bits of each alone, and no solve
+    begun in one launch that had to be left."""
+    scs = [cut(column((22, 30, 20), (40, 40, 40)), w) for w in waves]
+    want = [run(sc, 40) for sc in scs]
+    got = [None] * len(scs)
+    start = threading.Barrier(len(scs))
+
+    def work(k):
+        start.wait()
+        got[k] = run(scs[k], 40)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(scs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for (ia, a, _), (ib, b, forms) in zip(want, got):
+        assert ia == ib and all(np.array_equal(p, q) for p, q in zip(a, b))
+        assert forms[0] + forms[1] == 40 and forms[2] == 0
