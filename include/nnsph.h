@@ -204,8 +204,12 @@ int32_t nn_counts(nn_ctx *ctx, int64_t *n, int64_t *n_fluid);
  * many independent scenes resident in HBM in one concatenated, offset-indexed
  * particle array and advances all of them with one launch sequence per tick.
  * ------------------------------------------------------------------------- */
-/* Beside its scenes a pool holds up to an eighth of its budget in memory that
- * scenes have left, for the next ones; nn_pool_destroy gives it back. */
+/* Memory that scenes have left is kept for the next ones, by one store for all
+ * pools of the process: at most an eighth of the largest budget, with the pools'
+ * scenes no more than that budget, and 128 MiB of pinned blocks.  It is
+ * given back when an allocation of the library fails (a context's or surface's
+ * too) and when the last pool goes.  nn_pool_kept_bytes: the device bytes kept,
+ * with what reused blocks have beyond their need. */
 int32_t nn_pool_create(int64_t budget_bytes, nn_pool **out);
 /* nn_pool_create with flags.  NN_POOL_OWN_QUEUE marks a pool that is ticked
  * concurrently with others (a lane); it is accepted and has no effect: every
@@ -246,6 +250,7 @@ int64_t nn_pool_steps(nn_pool *pool, int32_t slot);
 int32_t nn_pool_read(nn_pool *pool, int32_t slot, int32_t field, void *host, size_t bytes);
 int32_t nn_pool_info(nn_pool *pool, int32_t *resident, int32_t *pending, int64_t *bytes_in_use);
 int32_t nn_pool_capacity(void);
+int64_t nn_pool_kept_bytes(void);
 /* Launch shape used by the sweep kernels (block size, power of two 64..1024);
  * the autotuner sets it.  0 = library default. */
 int32_t nn_pool_set_block(nn_pool *pool, int32_t block);

@@ -166,6 +166,7 @@ def load():
         "nn_pool_read": (i32, [vp, i32, i32, vp, sz]),
         "nn_pool_info": (i32, [vp, P(i32), P(i32), P(i64)]),
         "nn_pool_capacity": (i32, []),
+        "nn_pool_kept_bytes": (i64, []),
         "nn_pool_set_block": (i32, [vp, i32]),
         "nn_kernel_name": (ctypes.c_char_p, [i32]),
         "nn_profile": (i32, [vp, i32]),
@@ -222,6 +223,11 @@ def device_name() -> str:
     cus = ctypes.c_int32()
     check(lib.nn_device_info(buf, 256, ctypes.byref(hbm), ctypes.byref(cus)), "nn_device_info")
     return buf.value.decode(errors="replace")
+
+
+def pool_kept_bytes() -> int:
+    """Device bytes that the process's pools keep for their next scenes (nn_pool_kept_bytes)."""
+    return int(load().nn_pool_kept_bytes())
 
 
 def kernel_mask(kernels) -> int:

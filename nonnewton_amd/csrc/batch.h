@@ -83,22 +83,29 @@ struct KernelTimer {
   void reset();
 };
 
-// Device and pinned host memory that a pool's batches have given up, kept for
-// its next ones: an admission makes a staging batch and a later one frees it.
+// Device and pinned host memory that the pools' batches have given up, kept for
+// their next ones: an admission makes a staging batch and a later one frees it.
 // 64 admissions took 104 ms, 52 of them in hipMalloc, hipFree and their pinned
 // counterparts (the frees wait for the device); with these blocks, the upload
 // expanded on the device and no second search for scenes without a stress set,
-// 41 ms.  At most `limit` device bytes and 64 pinned blocks
-// are held, the oldest freed first, all of them when an allocation fails and when
-// the pool goes.  Any thread; a block is given only when no work on it is
-// pending, and taken for the device it is on.
+// 41 ms.  One store for all pools of the process (the lanes of one budget would
+// hold a part of it each): the idle blocks and what blocks in use have beyond
+// their need are at most an eighth of the largest budget of the pools there are,
+// and with the pools' scenes no more than that budget; pinned blocks 128 MiB (64
+// admissions leave 65; with 64 blocks of any size they took 10 ms longer).  The
+// oldest go first, all of them when an allocation of the library fails (any
+// object's: free_kept) and when the last pool goes.  Any thread; a block is given
+// only when no work on it is pending, and taken for the device it is on.
 class Spares {
  public:
-  explicit Spares(size_t limit) : limit_(limit) {}
-  ~Spares() { clear(); }
+  static Spares& get();
+  void pool_begins(int64_t budget);
+  void pool_ends(int64_t budget);
+  void scenes(long long bytes);  // more (or fewer) bytes of the pools' scenes
   bool take(bool host, size_t bytes, void** p, size_t* got);
-  void give(bool host, void* p, size_t bytes);
-  void clear();
+  void give(bool host, void* p, size_t bytes, size_t need);  // need: what take or the allocation was asked for
+  bool clear();  // whether there was anything to free
+  long long kept();
 
  private:
   struct Block {
@@ -106,14 +113,20 @@ class Spares {
     size_t bytes;
     int device;
   };
+  size_t limit() const;
+  void evict(std::vector<Block>& dev, std::vector<Block>& host);
+  static void release(const std::vector<Block>& dev, const std::vector<Block>& host);
   std::mutex mu_;
   std::vector<Block> dev_, host_;
-  size_t held_ = 0, limit_;
+  std::vector<int64_t> budgets_;
+  long long held_ = 0, excess_ = 0, scenes_ = 0, pinned_ = 0;
 };
+// Frees the kept memory; true if there was any, so that a failed allocation is worth another try.
+inline bool free_kept() { return Spares::get().clear(); }
 
 class Batch {
  public:
-  explicit Batch(hipStream_t stream, std::shared_ptr<Spares> spares = nullptr);
+  explicit Batch(hipStream_t stream, bool keep = false);  // keep: memory through Spares
   ~Batch();
   Batch(const Batch&) = delete;
   Batch& operator=(const Batch&) = delete;
@@ -140,7 +153,7 @@ class Batch {
   bool defer_free_ = false;
   struct Alloc {
     void* p;
-    size_t bytes;
+    size_t bytes, need;
   };
   void take_deferred(std::vector<Alloc>& out);
   int upload(int k, const float* x, const float* v, const int* kind);
@@ -167,9 +180,10 @@ class Batch {
   KernelTimer timer;
 
  private:
-  std::shared_ptr<Spares> spares_;
-  int alloc_host(void** p, size_t bytes);
-  void free_host(void* p, size_t bytes);
+  const bool keep_;
+  int alloc_host(void** p, size_t bytes, size_t& got);
+  void free_host(void* p, size_t got);
+  void free_arena(const Alloc& a);
   std::vector<Alloc> allocs_;
   long long bytes_ = 0;
   int C_total_ = 0;  // cells in use
@@ -184,6 +198,7 @@ class Batch {
   SceneState *h_state_ = nullptr, *state_dev_ = nullptr;
   unsigned long long *h_report_ = nullptr, *report_dev_ = nullptr;
   int h_state_cap_ = 0;
+  size_t h_state_bytes_ = 0, h_stage_bytes_ = 0;  // of their blocks
   unsigned ticket_ = 0;
   float *h_stage_ = nullptr, *stage_dev_ = nullptr;
   int stage();

@@ -239,71 +239,147 @@ long long scene_footprint(long long n, long long ns, long long cells) {
 constexpr size_t STAGE_BYTES = 1 << 20;
 static size_t state_bytes(int scenes) { return (sizeof(SceneState) + sizeof(unsigned long long)) * (size_t)scenes; }
 
+Spares& Spares::get() {
+  static Spares* s = new Spares();  // not destroyed: the runtime may be gone by then
+  return *s;
+}
+
+size_t Spares::limit() const {
+  int64_t most = 0;
+  for (int64_t b : budgets_) most = std::max(most, b);
+  return (size_t)std::max<long long>(0, std::min<long long>(most / 8, most - scenes_));
+}
+
+void Spares::evict(std::vector<Block>& dev, std::vector<Block>& host) {
+  while (!dev_.empty() && held_ + excess_ > (long long)limit()) {
+    held_ -= (long long)dev_.front().bytes;
+    dev.push_back(dev_.front());
+    dev_.erase(dev_.begin());
+  }
+  while (!host_.empty() && pinned_ > (budgets_.empty() ? 0 : 128 << 20)) {
+    pinned_ -= (long long)host_.front().bytes;
+    host.push_back(host_.front());
+    host_.erase(host_.begin());
+  }
+}
+
+void Spares::release(const std::vector<Block>& dev, const std::vector<Block>& host) {
+  for (auto& b : dev) (void)hipFree(b.p);
+  for (auto& b : host) (void)hipHostFree(b.p);
+}
+
+void Spares::pool_begins(int64_t budget) {
+  std::lock_guard<std::mutex> lk(mu_);
+  budgets_.push_back(budget);
+}
+
+void Spares::pool_ends(int64_t budget) {
+  std::vector<Block> dev, host;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    budgets_.erase(std::find(budgets_.begin(), budgets_.end(), budget));
+    evict(dev, host);
+  }
+  release(dev, host);
+}
+
+void Spares::scenes(long long bytes) {
+  std::vector<Block> dev, host;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    scenes_ += bytes;
+    evict(dev, host);
+  }
+  release(dev, host);
+}
+
 bool Spares::take(bool host, size_t bytes, void** p, size_t* got) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return false;
   std::lock_guard<std::mutex> lk(mu_);
   auto& v = host ? host_ : dev_;
+  const size_t room = host ? 4096 : 1u << 20;  // a block may have twice the bytes asked for and twice this more
   size_t best = v.size();
   for (size_t k = 0; k < v.size(); k++)
-    if (v[k].device == dev && v[k].bytes >= bytes && v[k].bytes / 2 <= bytes + (1u << 20) &&
+    if (v[k].device == dev && v[k].bytes >= bytes && v[k].bytes / 2 <= bytes + room &&
         (best == v.size() || v[k].bytes < v[best].bytes))
       best = k;
   if (best == v.size()) return false;
   *p = v[best].p;
   *got = v[best].bytes;
-  if (!host) held_ -= *got;
+  if (!host) {
+    held_ -= (long long)*got;
+    excess_ += (long long)(*got - bytes);
+  } else {
+    pinned_ -= (long long)*got;
+  }
   v.erase(v.begin() + best);
   return true;
 }
 
-void Spares::give(bool host, void* p, size_t bytes) {
-  std::vector<Block> out;
+void Spares::give(bool host, void* p, size_t bytes, size_t need) {
+  std::vector<Block> dev, pinned;
   hipPointerAttribute_t at{};
-  int dev = 0;
-  if (hipPointerGetAttributes(&at, p) == hipSuccess) dev = at.device;
+  int device = 0;
+  if (hipPointerGetAttributes(&at, p) == hipSuccess) device = at.device;
   else (void)hipGetLastError();
   {
     std::lock_guard<std::mutex> lk(mu_);
-    auto& v = host ? host_ : dev_;
-    v.push_back({p, bytes, dev});
-    if (!host) held_ += bytes;
-    while (!v.empty() && (host ? v.size() > 64 : held_ > limit_)) {
-      if (!host) held_ -= v.front().bytes;
-      out.push_back(v.front());
-      v.erase(v.begin());
+    (host ? host_ : dev_).push_back({p, bytes, device});
+    if (!host) {
+      held_ += (long long)bytes;
+      excess_ -= (long long)(bytes - need);
+    } else {
+      pinned_ += (long long)bytes;
     }
+    evict(dev, pinned);
   }
-  for (auto& b : out) (void)(host ? hipHostFree(b.p) : hipFree(b.p));
+  release(dev, pinned);
 }
 
-void Spares::clear() {
+bool Spares::clear() {
+  std::vector<Block> dev, host;
+  {
+    std::lock_guard<std::mutex> lk(mu_);
+    dev.swap(dev_);
+    host.swap(host_);
+    held_ = pinned_ = 0;
+  }
+  release(dev, host);
+  return !dev.empty() || !host.empty();
+}
+
+long long Spares::kept() {
   std::lock_guard<std::mutex> lk(mu_);
-  for (auto& b : dev_) (void)hipFree(b.p);
-  for (auto& b : host_) (void)hipHostFree(b.p);
-  dev_.clear();
-  host_.clear();
-  held_ = 0;
+  return held_ + excess_;
 }
 
-Batch::Batch(hipStream_t st, std::shared_ptr<Spares> spares) : stream(st), spares_(std::move(spares)) {}
+Batch::Batch(hipStream_t st, bool keep) : stream(st), keep_(keep) {}
 
 Batch::~Batch() {
   release();
-  free_host(h_state_, state_bytes(h_state_cap_));
-  free_host(h_stage_, STAGE_BYTES);
+  free_host(h_state_, h_state_bytes_);
+  free_host(h_stage_, h_stage_bytes_);
 }
 
-int Batch::alloc_host(void** p, size_t bytes) {
-  size_t got = 0;
-  if (spares_ && spares_->take(true, bytes, p, &got)) return NN_OK;
-  HIPCHK(hipHostMalloc(p, bytes, hipHostMallocDefault));
-  return NN_OK;
+int Batch::alloc_host(void** p, size_t bytes, size_t& got) {
+  got = bytes;
+  if (keep_ && Spares::get().take(true, bytes, p, &got)) return NN_OK;
+  hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
+  if (e != hipSuccess && free_kept()) {
+    (void)hipGetLastError();
+    e = hipHostMalloc(p, bytes, hipHostMallocDefault);
+  }
+  return e == hipSuccess ? NN_OK : hip_fail(e, "hipHostMalloc");
 }
-void Batch::free_host(void* p, size_t bytes) {  // after release(): no work is pending
+void Batch::free_host(void* p, size_t got) {  // no work on it is pending
   if (!p) return;
-  if (spares_) spares_->give(true, p, bytes);
+  if (keep_) Spares::get().give(true, p, got, got);
   else (void)hipHostFree(p);
+}
+void Batch::free_arena(const Alloc& a) {  // no work on it is pending, or (not kept) hipFree waits for it
+  if (keep_) Spares::get().give(false, a.p, a.bytes, a.need);
+  else (void)hipFree(a.p);
 }
 
 // The arrays of a layout are carved from one device allocation (256-byte
@@ -315,12 +391,11 @@ int Batch::alloc_arena(std::vector<std::pair<void**, size_t>>& req, bool& used) 
   for (auto& r : req) total += (r.second + 255) & ~(size_t)255;
   void* q = nullptr;
   size_t got = total;
-  used = spares_ && spares_->take(false, total, &q, &got);
+  used = keep_ && Spares::get().take(false, total, &q, &got);
   if (!used) {
     hipError_t e = hipMalloc(&q, total);
-    if (e == hipErrorOutOfMemory && spares_) {
+    if (e == hipErrorOutOfMemory && free_kept()) {
       (void)hipGetLastError();
-      spares_->clear();
       e = hipMalloc(&q, total);
     }
     if (e != hipSuccess) {
@@ -334,7 +409,7 @@ int Batch::alloc_arena(std::vector<std::pair<void**, size_t>>& req, bool& used) 
     *r.first = c;
     c += (r.second + 255) & ~(size_t)255;
   }
-  allocs_.push_back({q, got});
+  allocs_.push_back({q, got, total});
   bytes_ += (long long)got;
   return NN_OK;
 }
@@ -346,15 +421,12 @@ int Batch::alloc_arena(std::vector<std::pair<void**, size_t>>& req, bool& used) 
 // closed) took 1.39 ms with it and takes 0.72 at 1,082 particles, 2.33 and 0.85
 // at 22,530.
 void Batch::release() {
-  if (spares_ && !allocs_.empty()) {
+  if (keep_ && !allocs_.empty()) {
     bool asked = false;
     for (; hipStreamQuery(stream) == hipErrorNotReady; asked = true) __builtin_ia32_pause();
     if (asked) (void)hipGetLastError();  // hipErrorNotReady
   }
-  for (auto& a : allocs_) {
-    if (spares_) spares_->give(false, a.p, a.bytes);
-    else (void)hipFree(a.p);
-  }
+  for (auto& a : allocs_) free_arena(a);
   allocs_.clear();
   bytes_ = 0;
 }
@@ -683,10 +755,11 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   // scenes as the layout holds (a staging batch holds one; hipHostFree
   // synchronizes the device)
   if (!h_state_ || h_state_cap_ < Sc) {
-    if (h_state_) HIPCHK(hipHostFree(h_state_));
+    if (h_state_) HIPCHK(hipStreamSynchronize(stream));
+    free_host(h_state_, h_state_bytes_);
     h_state_ = nullptr;
     const size_t cap = (size_t)std::max(Sc, 1);
-    CHK(alloc_host((void**)&h_state_, state_bytes((int)cap)));
+    CHK(alloc_host((void**)&h_state_, state_bytes((int)cap), h_state_bytes_));
     h_report_ = reinterpret_cast<unsigned long long*>(h_state_ + cap);
     std::fill(h_report_, h_report_ + cap, 0ull);
     h_state_cap_ = (int)cap;
@@ -707,7 +780,7 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   if (defer_free_) {
     for (auto& al : old_allocs) deferred_.push_back(al);
   } else {
-    for (auto& al : old_allocs) (void)hipFree(al.p);
+    for (auto& al : old_allocs) free_arena(al);
   }
   d = nd;
   lists_state_ = 0;
@@ -1354,7 +1427,7 @@ static int field_width(int field) {
 
 int Batch::stage() {
   if (h_stage_) return NN_OK;
-  CHK(alloc_host((void**)&h_stage_, STAGE_BYTES));
+  CHK(alloc_host((void**)&h_stage_, STAGE_BYTES, h_stage_bytes_));
   HIPCHK(hipHostGetDevicePointer((void**)&stage_dev_, h_stage_, 0));
   return NN_OK;
 }

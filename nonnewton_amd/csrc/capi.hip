@@ -410,7 +410,6 @@ struct nn_pool {
   // (hipFree waits for the device, so not on the thread that ticks)
   std::vector<std::unique_ptr<Batch>> graveyard;
   std::vector<Batch::Alloc> dead_arrays;
-  std::shared_ptr<nn::Spares> spares;
   // a tick in flight (nn_pool_tick_async): its thread, and what nn_pool_sync returns
   std::thread async;
   bool async_on = false;
@@ -429,7 +428,7 @@ static void pool_free_dead(nn_pool* p) {
     arrays.swap(p->dead_arrays);
   }
   dead.clear();
-  for (auto& a : arrays) p->spares->give(false, a.p, a.bytes);  // the layout that replaced them waited for its stream
+  for (auto& a : arrays) nn::Spares::get().give(false, a.p, a.bytes, a.need);  // the layout that replaced them waited for its stream
 }
 
 extern "C" {
@@ -448,6 +447,8 @@ int32_t nn_surface_run_context(nn_surface* s, nn_ctx* ctx) {
 
 int32_t nn_pool_capacity(void) { return POOL_CAPACITY; }
 
+int64_t nn_pool_kept_bytes(void) { return nn::Spares::get().kept(); }
+
 int32_t nn_pool_create(int64_t budget_bytes, nn_pool** out) { return nn_pool_create_ex(budget_bytes, 0, out); }
 
 int32_t nn_pool_create_ex(int64_t budget_bytes, int32_t flags, nn_pool** out) {
@@ -464,8 +465,8 @@ int32_t nn_pool_create_ex(int64_t budget_bytes, int32_t flags, nn_pool** out) {
     return nn::hip_fail(e, "hipStreamCreate");
   }
   p->budget = budget_bytes;
-  p->spares = std::make_shared<nn::Spares>((size_t)budget_bytes / 8);
-  p->main.reset(new Batch(p->stream, p->spares));
+  nn::Spares::get().pool_begins(budget_bytes);
+  p->main.reset(new Batch(p->stream, true));
   p->main->defer_free_ = true;
   p->slots.resize(POOL_CAPACITY);
   *out = p;
@@ -484,7 +485,8 @@ int32_t nn_pool_destroy(nn_pool* p) {
   for (auto& s : p->slots) {
     s.staging.reset();
   }
-  p->spares->clear();  // before the stream goes
+  nn::Spares::get().scenes(-p->in_use);
+  nn::Spares::get().pool_ends(p->budget);  // before the stream goes
   if (p->stream) (void)hipStreamDestroy(p->stream);
   delete p;
   return NN_OK;
@@ -546,6 +548,7 @@ int32_t nn_pool_admit(nn_pool* p, const nn_params* params, const float* x, const
     p->slots[s_id].steps = 0;
     p->in_use += fp;
   }
+  nn::Spares::get().scenes(fp);
   PoolSlot& ps = p->slots[s_id];
   auto fail = [&](int code) {
     std::lock_guard<std::mutex> lk(p->mu);
@@ -553,6 +556,7 @@ int32_t nn_pool_admit(nn_pool* p, const nn_params* params, const float* x, const
     ps.scene.reset();
     ps.used = false;
     p->in_use -= fp;
+    nn::Spares::get().scenes(-fp);
     return code;
   };
   hipStream_t sst = nullptr;
@@ -560,7 +564,7 @@ int32_t nn_pool_admit(nn_pool* p, const nn_params* params, const float* x, const
     const int rc2 = staging_stream(&sst);
     if (rc2 < 0) return fail(rc2);
   }
-  std::unique_ptr<Batch> stg(new Batch(sst, p->spares));
+  std::unique_ptr<Batch> stg(new Batch(sst, true));
   stg->block = p->block;
   std::copy(p->kblock, p->kblock + nn::K_COUNT, stg->kblock);
   std::copy(p->kdepth, p->kdepth + nn::K_COUNT, stg->kdepth);
@@ -643,6 +647,7 @@ static int pool_apply_membership(nn_pool* p) {
       s.used = false;
       s.retired = false;
       p->in_use -= s.bytes;
+      nn::Spares::get().scenes(-s.bytes);
       s.bytes = 0;
       continue;
     }

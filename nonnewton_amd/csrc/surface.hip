@@ -1548,6 +1548,10 @@ struct DBuf {
     cap = 0;
     const size_t c = n > 0 ? n : 1;
     hipError_t e = hipMalloc(&p, c * sizeof(T));
+    if (e == hipErrorOutOfMemory && free_kept()) {
+      (void)hipGetLastError();
+      e = hipMalloc(&p, c * sizeof(T));
+    }
     if (e == hipSuccess) cap = c;
     return e;
   }
