@@ -213,7 +213,7 @@ class Batch {
   int rigid_step();
   int max_iter_[3] = {1, 1, 1};
 
-  int alloc_arena(std::vector<std::pair<void**, size_t>>& req, bool& used);
+  int alloc_arena(std::vector<std::pair<void**, size_t>>& req);
   void release();
   int search_impl(int all, int begin);
   int complete_lists();

@@ -384,15 +384,13 @@ void Batch::free_arena(const Alloc& a) {  // no work on it is pending, or (not k
 
 // The arrays of a layout are carved from one device allocation (256-byte
 // aligned sub-ranges): one hipMalloc and, when the batch is released or laid
-// out again, one hipFree, which synchronizes the device.  used: the memory held
-// other arrays before.
-int Batch::alloc_arena(std::vector<std::pair<void**, size_t>>& req, bool& used) {
+// out again, one hipFree, which synchronizes the device.
+int Batch::alloc_arena(std::vector<std::pair<void**, size_t>>& req) {
   size_t total = 0;
   for (auto& r : req) total += (r.second + 255) & ~(size_t)255;
   void* q = nullptr;
   size_t got = total;
-  used = keep_ && Spares::get().take(false, total, &q, &got);
-  if (!used) {
+  if (!(keep_ && Spares::get().take(false, total, &q, &got))) {
     hipError_t e = hipMalloc(&q, total);
     if (e == hipErrorOutOfMemory && free_kept()) {
       (void)hipGetLastError();
@@ -720,8 +718,7 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
   A(rwb, NRc / 64);
   A(nd.rpartials, 9 * (size_t)(NRc / 64));
   A(nd.bodies, NBc);
-  bool used = false;
-  const int rc = alloc_arena(req, used);
+  const int rc = alloc_arena(req);
   if (rc != NN_OK) {
     release();
     allocs_.swap(old_allocs);
@@ -766,9 +763,11 @@ int Batch::layout(const std::vector<const Batch*>& from, double slack, int scene
     HIPCHK(hipHostGetDevicePointer((void**)&state_dev_, h_state_, 0));
     report_dev_ = reinterpret_cast<unsigned long long*>(state_dev_ + cap);
   }
-  // memory that was in use before starts at zero throughout, as new memory does
-  const long zeros = (long)((used ? (char*)allocs_.back().p + allocs_.back().bytes : (char*)nd.info) - (char*)nd.state);
-  launch_fill_f4(reinterpret_cast<float4*>(nd.state), zeros / 16, make_float4(0.f, 0.f, 0.f, 0.f), stream);
+  // nothing else is read before it is written (device memory comes as it was
+  // left, new or used again; every GPU test gives the same with the rest filled
+  // with NaN and, where it holds indices, with 1)
+  launch_fill_f4(reinterpret_cast<float4*>(nd.state), (long)((char*)nd.info - (char*)nd.state) / 16,
+                 make_float4(0.f, 0.f, 0.f, 0.f), stream);
   launch_fill_i32(nd.info, (long)((char*)scenes_dev - (char*)nd.info) / 4, -1, stream);
   CHK(upload_tables(nd));
   // copy persistent state of relocated scenes
