@@ -207,7 +207,7 @@ class Batch {
   template <typename Launch>
   int field_pieces(int n, float* out, const float* in, Launch launch);
   bool any_fluid_ = false, any_elastic_ = false, any_weiler_ = false, any_strain_ = false, any_div_ = false;
-  bool any_warm_cg_ = false, any_rigid_ = false;
+  bool any_warm_cg_ = false, any_rigid_ = false, any_velocity_terms_ = false;
   int max_body_ = 0, max_coupling_ = 0, max_body_waves_ = 0;  // over the scenes with rigid bodies
   int NB_cap_ = 0;                       // body-table entries allocated
   int rigid_step();

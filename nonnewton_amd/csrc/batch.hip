@@ -434,22 +434,43 @@ DevRef Batch::dref() { return DevRef{d}; }
 // Lanes per particle of a list sweep, by the slots in use.  A sweep is bound by
 // its longest chain (a lane walking its list) until the device is full of
 // wavefronts, and by instructions after that, where every lane of a group
-// repeats the additions.  Microseconds a launch with 1 / 4 / 16 lanes, by
-// slots in use (one scene; the last column the 64-scene pool):
-//                  2,554          46,346         162,570        1,616,737
-//   build_lists    37 / 15 / 8    44 / 22 / 16   58 / 43 / 44   246 / 240 / 296
-//   density_alpha  13 / 9 / 7     15 / 12 / 17   22 / 25 / 51    96 / 129 / 385
-//   div_source     11 / 7 / 7     12 /  8 /  7   20 / 17 / 20    81 /  82 / 137
-//   nonpressure    24 / 11 / 8    28 / 16 / 15   46 / 34 / 39   156 / 176 / 258
-//   strain         13 / 9 / 6     16 / 12 / 15   27 / 24 / 39    97 / 118 / 231
-// (nonpressure of a scene with explicit viscosity.)  The search's limit is
-// higher: its lanes share candidates and repeat nothing.  One lane is left to
-// the three sweeps with the most sums, where four were slower.
+// repeats the additions.  Microseconds a launch with 4 / 16 lanes (or 1 / 4), by
+// slots (one scene; the last columns 8 and 64 mixed scenes in a pool):
+//   4 / 16 lanes        11,970       19,170       28,514       36,066
+//   build_lists         21 / 11      21 / 11      24 / 13      22 / 14
+//   density_alpha       8.5 / 7.8    8.7 / 8.7    9.5 / 10.6   9.6 / 12.5
+//   strain              11.4 / 9.5   10.8 / 11.1  12.2 / 12.3  11.6 / 14.0
+//   nonpressure         10.3 / 6.9   10.6 / 7.7   12.1 / 9.4   12.1 / 10.0
+//   press_source        7.3 / 6.4    6.9 / 5.9    7.4 / 5.5    7.7 / 6.1
+//                       86,754       118,178      153,954      202,594
+//   build_lists         31 / 26      34 / 34      42 / 44      55 / 56
+//   press_source        9.6 / 9.8    12.0 / 12.8  14.1 / 16.4  18.6 / 20.6
+//   1 / 4 lanes         86,754       118,178      202,594      572,130      1,288,930    248,122      1,616,737
+//   density_alpha       16.7 / 15.3  18.0 / 19.3  24.0 / 28.2  58 / 67      124 / 142    24.7 / 26.6  90 / 124
+//   strain              18.1 / 16.9  21.0 / 21.0  29.3 / 28.3  66 / 63      138 / 132    29.3 / 27.5  92 / 113
+//   nonpressure, with velocities   (explicit or boundary viscosity)
+//                       31 / 18      34 / 23      46 / 36      109 / 87     238 / 185
+//   nonpressure, positions only    (surface tension beside the implicit solve)
+//                       18.5 / 15.1  19.5 / 17.4  25.1 / 29.6  62 / 69      161 / 193    30.9 / 34.5  154 / 173
+//                       members of the stress set, 4 / 16 lanes
+//                       4,096        13,824       24,576       30,720       40,960
+//   elastic_rot_stress  18.5 / 18.9  19.9 / 20.3  23 / 38      24 / 38      28 / 53
+//   elastic_force       10.2 / 7.9   11.4 / 8.2   14.0 / 13.5  14.5 / 13.4  16.1 / 18.1
+// The search's lanes share candidates and repeat nothing, so its limit is the
+// highest; the sums of density and strain are the most, so theirs are the
+// lowest, and one lane is left to them and to the position-only sweep.
 int Batch::lanes(int id) const {
-  const int slots = id == K_ELASTIC_ROT_STRESS || id == K_ELASTIC_FORCE ? d.NSn : d.Pn;
-  if (slots <= (id == K_BUILD_LISTS ? 131072 : 32768)) return 16;
-  const bool many_sums = id == K_DENSITY_ALPHA || id == K_NONPRESSURE || id == K_STRAIN;
-  return many_sums && d.Pn > 196608 ? 1 : 4;
+  const bool members = id == K_ELASTIC_ROT_STRESS || id == K_ELASTIC_FORCE;
+  const int slots = members ? d.NSn : d.Pn;
+  int wide = 32768, one = INT_MAX;  // 16 lanes up to, 1 lane above
+  switch (id) {
+    case K_BUILD_LISTS: wide = 131072; break;
+    case K_DENSITY_ALPHA: wide = 16384; one = 98304; break;
+    case K_STRAIN: wide = 16384; one = 1048576; break;
+    case K_NONPRESSURE: one = any_velocity_terms_ ? INT_MAX : 196608; break;
+    case K_ELASTIC_ROT_STRESS: wide = 16384; break;
+  }
+  return slots <= wide ? 16 : slots > one ? 1 : 4;
 }
 
 void Batch::swap_sort_buffers() {
@@ -459,12 +480,18 @@ void Batch::swap_sort_buffers() {
   std::swap(d.vdiff, d.vdiff_alt);
 }
 
+// the non-pressure sweep forms viscosity terms of this scene (k_nonpressure)
+static bool velocity_terms(const SceneDev& c) {
+  return (c.flags & SF_HAS_FLUID) && (c.flags & SF_VISCOSITY) && (!(c.flags & SF_WEILER) || c.bnu != 0.0f);
+}
+
 // Per-scene fields that depend on the scenes' order and offsets (p_begin,
 // cell_begin and s_begin must be set): the slot shift used by the sort, the
 // wave range, and the batch-wide feature flags.
 void Batch::derive_members() {
   long base = 0;
   any_fluid_ = any_elastic_ = any_weiler_ = any_strain_ = any_div_ = any_warm_cg_ = any_rigid_ = false;
+  any_velocity_terms_ = false;
   max_body_ = max_coupling_ = max_body_waves_ = 0;
   max_iter_[0] = max_iter_[1] = max_iter_[2] = 1;
   for (auto& sp : scenes) {
@@ -479,6 +506,7 @@ void Batch::derive_members() {
     s.dev.body_begin = s.body_begin;
     base += s.n;
     const int f = s.dev.flags;
+    any_velocity_terms_ |= velocity_terms(s.dev);
     if (f & SF_HAS_FLUID) {
       any_fluid_ = true;
       if (f & SF_DIVERGENCE) any_div_ = true;
@@ -864,7 +892,9 @@ int Batch::refresh_scene_table() {
   if (!hs.empty())
     HIPCHK(hipMemcpyAsync((void*)d.scenes, hs.data(), sizeof(SceneDev) * hs.size(), hipMemcpyHostToDevice, stream));
   max_iter_[0] = max_iter_[1] = max_iter_[2] = 1;
+  any_velocity_terms_ = false;
   for (auto& sp : scenes) {
+    any_velocity_terms_ |= velocity_terms(sp->dev);
     max_iter_[0] = std::max(max_iter_[0], sp->dev.max_iter_v);
     max_iter_[1] = std::max(max_iter_[1], sp->dev.max_iter_p);
     max_iter_[2] = std::max(max_iter_[2], sp->dev.max_iter_cg);

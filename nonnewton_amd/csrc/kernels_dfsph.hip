@@ -302,8 +302,9 @@ __global__ void k_nonpressure(Dev d) {
   }
   const bool vis_on = (sc.flags & SF_VISCOSITY) != 0;
   const bool weiler = vis_on && (sc.flags & SF_WEILER);
-  const bool expl = vis_on && !weiler;
-  const bool bnu_on = vis_on && sc.bnu != 0.0f;
+  // one lane per particle: only for batches without velocity terms (Batch::lanes)
+  const bool expl = G != 1 && vis_on && !weiler;
+  const bool bnu_on = G != 1 && vis_on && sc.bnu != 0.0f;
   if (kind == KIND_FLUID) {
     const KernH kh(sc);
     const float4 xi = own.pos(d, i);
