@@ -264,7 +264,8 @@ int32_t nn_set_kernel_block(nn_ctx *ctx, int32_t kernel, int32_t block);
  * before using them (0 = the kernel's default; 1..16, a power of two).  The
  * neighbor sweeps take 4, 8 or 16 (default 8), cg_matvec 1, 2, 4 or 8 (default
  * 2); other values select the default; a sweep over few particles, with 16
- * lanes on each, has one depth.  A depth for cg_matvec also asks for the
+ * lanes on each, has one depth, and one over so many that each has one lane 4
+ * and 8.  A depth for cg_matvec also asks for the
  * two-launch iteration where one small scene's solve would run in a single
  * launch.  Results do not depend on it. */
 int32_t nn_pool_set_kernel_depth(nn_pool *pool, int32_t kernel, int32_t depth);
