@@ -308,6 +308,13 @@ int32_t nn_pool_kernel_launches(nn_pool *pool, int64_t *seen, int32_t n);
  * its timed interval minus this. */
 int32_t nn_event_overhead(int32_t reps, double *ms);
 
+/* A check of the device (no counterpart in the reference): the sweeps' shortened
+ * square root against the correctly rounded one for every float in
+ * [2^-100, 2^100), and their shortened division against the correctly rounded
+ * one for `rounds` pairs in each of 2^20 threads, over the exponents that the
+ * sweeps use it for.  *roots, *quotients: the results that differ (0). */
+int32_t nn_check_roundings(int32_t rounds, int64_t *roots, int64_t *quotients);
+
 /* ------------------------------------------------------------------------
  * Surface reconstruction: the particle-to-mesh path of SRTool
  * (SPH/surf_recon/srtool.py), a dual-contouring mesh of the particles'

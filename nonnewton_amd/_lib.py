@@ -184,6 +184,7 @@ def load():
         "nn_pool_kernel_launches": (i32, [vp, P(i64), i32]),
         "nn_pool_kernel_times": (i32, [vp, P(ctypes.c_double), P(i64), i32]),
         "nn_event_overhead": (i32, [i32, P(ctypes.c_double)]),
+        "nn_check_roundings": (i32, [i32, P(i64), P(i64)]),
         "nn_surface_create": (i32, [P(NnSurfaceParams), P(vp)]),
         "nn_surface_destroy": (i32, [vp]),
         "nn_surface_set_budget": (i32, [vp, i64]),
@@ -213,6 +214,14 @@ def event_overhead_ms(reps: int = 200) -> float:
     ms = ctypes.c_double()
     check(load().nn_event_overhead(int(reps), ctypes.byref(ms)), "nn_event_overhead")
     return float(ms.value)
+
+
+def check_roundings(rounds: int = 1024):
+    """(square roots, quotients) of the shortened forms that differ from the
+    correctly rounded ones on this device (nn_check_roundings)."""
+    r, q = ctypes.c_int64(), ctypes.c_int64()
+    check(load().nn_check_roundings(int(rounds), ctypes.byref(r), ctypes.byref(q)), "nn_check_roundings")
+    return int(r.value), int(q.value)
 
 
 def device_name() -> str:

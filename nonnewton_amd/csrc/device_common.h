@@ -78,13 +78,16 @@ __device__ __forceinline__ long nb_word(long P, int i, int k) { return 4 * ((lon
 // scaling (operands near overflow or underflow) a pair of particles never
 // needs.  Where a scene's h lies in [2^-20, 2^20] (SF_MIDRANGE) and a pair's
 // squared distance is above 1e-10 with no component in (0, 2^-100), the
-// sequences below give the same bits:
-//   sqrt_mid   x rsq(x) and one residual correction (compared on this device
-//              with the correctly rounded root of every float in [2^-100, 2^100))
+// sequences below give the same bits (nn_check_roundings compares them on the
+// device at hand, a root for every float of the range):
+//   sqrt_mid   x rsq(x) and one residual correction
 //   recip_mid  v_rcp_f32 and one Newton step, shared by every quotient of one
 //              denominator
 //   div_mid    a y, then two residual corrections q + (a - b q) y (Markstein,
-//              IBM J. R&D 34, 1990); -0 / b comes out as +0, which only a sum
+//              IBM J. R&D 34, 1990), for quotients in the normal range (a
+//              component's below it, which takes h > 2^13, is multiplied by the
+//              kernel's factor of less than 2^-35 and gives 0 in either form);
+//              -0 / b comes out as +0, which only a sum
 //              that may itself be -0 can tell (pair_grad's SIGNED)
 // A gradient has one square root and four quotients of two denominators (h
 // and r h), about half of its instructions.
