@@ -98,7 +98,8 @@ typedef struct nn_params {
     int32_t coupling_interval; /* rigid-body substeps per step (Parameter.coupling_interval, :616) */
 } nn_params;
 
-/* Per-step statistics (what the reference prints each step, :916,1548,1704,1785). */
+/* Per-step statistics (what the reference prints each step, :916,1548,1704,1785).
+ * The iterations and errors of a solver that the scene does not use are 0. */
 typedef struct nn_step_stats {
     int32_t iterations_v;  /* divergence-solver iterations run */
     int32_t iterations_p;  /* pressure-solver iterations run */
