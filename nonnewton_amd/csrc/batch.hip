@@ -909,6 +909,7 @@ int Batch::upload(int k, const float* x, const float* v, const int* kind) {
   // expanded on the device, from staging memory or (larger scenes) from a copy
   // in the pair scalars, which only a step uses
   const size_t words = (size_t)(v ? 7 : 4) * n;
+  (void)hipGetLastError();  // what another call left on this thread is not this one's error
   float* raw = d.spair;
   if (4 * words <= STAGE_BYTES) {
     CHK(stage());
@@ -1500,6 +1501,7 @@ int Batch::download(int k, int field, void* host, size_t bytes) {
     set_error("buffer size does not match n * width * 4");
     return NN_E_ARG;
   }
+  (void)hipGetLastError();  // as in upload
   if (field == NN_FIELD_NUM_NEIGHBORS) CHK(complete_lists());
   // three-component fields: into original order by the kernel that writes them
   if (field == NN_FIELD_X || field == NN_FIELD_V || field == NN_FIELD_ACCELERATION || field == NN_FIELD_VISC_DIFF) {
@@ -1638,6 +1640,7 @@ int Batch::upload_field(int k, int field, const void* host, size_t bytes) {
     return NN_E_ARG;
   }
   float4* p = field == NN_FIELD_X ? d.pos : field == NN_FIELD_V ? d.vel : d.vdiff;
+  (void)hipGetLastError();  // as in upload
   if (bytes <= STAGE_BYTES) {
     CHK(stage());
     std::memcpy(h_stage_, host, bytes);

@@ -1713,6 +1713,7 @@ static int report(Surface& S, const int* count = nullptr, bool active = false) {
 
 // Copies pieces in (before a run) or out (after one); in: the run waits for it.
 static int transfer(Surface& S, bool in, std::initializer_list<Piece> pieces, const char* what) {
+  (void)hipGetLastError();  // what another call left on this thread is not this one's error
   size_t total = 0;
   bool host = true;  // memory that the CPU can use
   for (const Piece& q : pieces) {
