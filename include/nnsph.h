@@ -183,7 +183,7 @@ int32_t nn_neighbors(nn_ctx *ctx, int32_t *nbr, int32_t *count, int32_t cap);
  * `stream` (a hipStream_t; NULL = the default stream) and asynchronous: the
  * outputs, status included, are valid once the stream reaches that point.
  * Allocates nothing: the search's scratch is one fixed __device__ array of
- * 42 MB per GPU, held from the first call on that GPU until the process ends;
+ * 59 MB per GPU, held from the first call on that GPU until the process ends;
  * n above 1048576 or a grid above 4194304 cells is NN_E_ARG.  Every call on a
  * GPU shares that GPU's scratch: calls that overlap on one GPU (on different
  * streams or threads) race. */
@@ -292,7 +292,7 @@ int32_t nn_set_cg_patience(nn_ctx *ctx, int32_t exchanges);
  * of timed launches of kernel ids 0..n-1 (names from nn_kernel_name,
  * NN_KERNEL_COUNT ids); nn_*_kernel_launches the number of launches of every
  * kernel made while timing was on, timed or not, masked or not. */
-#define NN_KERNEL_COUNT 21
+#define NN_KERNEL_COUNT 21 /* "clear_acc" is kept for its number and never launched */
 const char *nn_kernel_name(int32_t id);
 int32_t nn_profile(nn_ctx *ctx, int32_t enable);
 int32_t nn_profile_mask(nn_ctx *ctx, uint32_t mask, int32_t stride);

@@ -58,7 +58,7 @@ long long scene_footprint(long long n, long long ns, long long cells);
 
 // Per-kernel durations from HIP events recorded around each launch on the
 // batch stream (enabled on request; read after the step's final sync).
-enum KernelId {
+enum KernelId {  // K_CLEAR_ACC keeps its place in the public numbering; k_place does its work
   K_CELL_COUNT, K_SCAN, K_BUCKET, K_PLACE, K_BUILD_LISTS, K_BVOL, K_CLEAR_ACC, K_DENSITY_ALPHA,
   K_DIV_UPDATE, K_DIV_SOURCE, K_STRAIN, K_CG_INIT, K_CG_MATVEC, K_CG_UPDATE, K_NONPRESSURE,
   K_PRESS_SOURCE, K_PRESS_UPDATE, K_ELASTIC_ROT_STRESS, K_ELASTIC_FORCE, K_ADVECT, K_CG_GUESS, K_COUNT

@@ -1048,10 +1048,11 @@ int Batch::search() {
 }
 
 // Waits until each of the first n report words carries the ticket, the last one
-// given out by default (later: or one after it); bits: the or of what they report.  Polling them costs 6 us less than a copy of the
-// counter and a wait for the stream (six small launches and the wait: 19.5 us
-// against 26); a wait that lasts is left to the stream's, which also returns
-// the errors of launches that cannot report.
+// given out by default (later: or one after it); bits: the or of what they
+// report.  Polling them costs 6 us less than a copy of the counter and a wait for
+// the stream (six small launches and the wait: 19.5 us against 26); a wait that
+// lasts is left to the stream's, which also returns the errors of launches that
+// cannot report.
 int Batch::await(int n, unsigned& bits) { return await(n, bits, ticket_, false); }
 int Batch::await(int n, unsigned& bits, unsigned ticket, bool later) {
   HIPCHK(hipGetLastError());
@@ -1248,7 +1249,7 @@ int Batch::solver_loop(int which) {
 // the scene sums of iteration k - 1 and stops converged scenes) and matvec k,
 // for k = 1 .. limit, then update limit + 1, which only tests the last
 // residual.  Enqueued in chunks -- first the previous step's iteration count
-// plus two, then four -- with one report of the active-scene counter per chunk;
+// plus three, then four -- with one report of the active-scene counter per chunk;
 // iterations past convergence are near-empty launches.
 int Batch::cg_start() {
   TIMED(K_CG_INIT, launch_cg_init(dref(), blk(K_CG_INIT), stream));

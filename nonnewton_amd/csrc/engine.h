@@ -257,7 +257,7 @@ void launch_gather3(const float4* slots, const int* inv, int n, float* ordered, 
 void launch_expand(const DevRef& d, int pb, int n, float V0, const float* x, const int* kind, const float* v, hipStream_t st);
 void launch_scatter3(const float* ordered, const int* inv, int n, float4* slots, hipStream_t st);
 void launch_scan(const DevRef& d, int n, hipStream_t st);  // cell_start = exclusive scan(cell_count)
-// exclusive scan of in[0..n) into out; tmp holds ceil(n / 2048) ints
+// exclusive scan of in[0..n) into out; tmp holds scan_tmp_ints(n) ints
 long scan_tmp_ints(long n);
 void launch_scan_i32(const int* in, int n, int* tmp, int* out, hipStream_t st, int nz = 0, int total = 0);
 constexpr int SCAN_TILE_ITEMS = 2048;

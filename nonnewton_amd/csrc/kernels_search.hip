@@ -4,8 +4,8 @@
 //
 // Pipeline per step:
 //   cell_count  : cell key of every particle, per-cell arrival counter (atomic)
-//   scan        : exclusive prefix sum of the cell counts (block scans over LDS
-//                 with wavefront shuffles, three passes)
+//   scan        : exclusive prefix sum of the cell counts (block sums, then block
+//                 scans with wavefront shuffles over the sums before theirs)
 //   bucket      : every particle into its cell's range of a bucket array
 //   place       : final slot = cell start + number of cell-mates with a smaller
 //                 original index; state is moved into the new order

@@ -23,9 +23,10 @@
 // (vertex (x, y, z) at origin + (x, y, z) * voxel_size, z fastest), one byte per
 // block for "written" (the reference's sparse leaf blocks: its loops visit
 // exactly those, and an unwritten vertex reads 0).  The field is accumulated in
-// 2^-32 fixed point (int64 atomics), so its value does not depend on the order
-// in which the particles' contributions are added (a per-vertex gather here, a
-// per-particle scatter in the reference), then rounded once to FP32.  The
+// 2^-32 fixed point (FP64 sums of each tile where they are exact, int64 sums
+// elsewhere), so its value does not depend on the order in which the particles'
+// contributions are added (a gather per tile here, a scatter per particle in the
+// reference), then rounded once to FP32.  The
 // reference adds FP32 with atomics in no defined order.  Every other
 // expression is FP32 in the reference's operation order (-ffp-contract=off).
 #include <hip/hip_runtime.h>
